@@ -30,6 +30,7 @@ struct candy_hip_llama final : candy_hip_decoder {
     int8_t *xq = nullptr;           // planar Q8_0 quants of the current activation
     candy::Q8Scale *xs = nullptr;
     void *attn_scratch = nullptr;                 // attention split partials
+    uint8_t *kv_parts = nullptr;                  // prompts, f32 cache: a layer's K and V as the attention kernel contracts them
     int n_splits = 1;
     // prompt buffers: [n][width] activations
     struct Prompt {
@@ -355,6 +356,8 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
     int rc;
     P.k = P.q + (size_t)n * qd;  // q, k and v of this pass end to end, whatever the buffer's capacity
     P.v = P.k + (size_t)n * c.n_kv_heads * c.head_dim;
+    if (!m->kv_f16 && !kv_parts && (rc = decoder_alloc(m, &kv_parts, attn_prefill_parts_bytes(c.n_kv_heads, c.head_dim, c.max_pos))))
+        return rc;
     if ((rc = embed(prompt_ids, n, P.h))) return rc;
     // A projection that splits K leaves its partial copies for the launch that follows: the norm launch behind o / down
     // sums them, adds the residual and writes P.h before it normalizes, the rope launch behind q / k / v sums them on
@@ -399,11 +402,11 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
             if ((rc = launch_contract(dev, L.wv, P.xq, P.xs, n, P.v, xh_for(L.wv)))) return rc;
         }
         rc = launch_prefill_rope_kv(dev, P.q, P.k, P.v, m->cos_t, m->sin_t, kc, vc, m->kv_f16, n, pos0, c.n_heads,
-                                    c.n_kv_heads, c.head_dim, cache_stride, &pend);
+                                    c.n_kv_heads, c.head_dim, cache_stride, kv_parts, &pend);
         pend.n_split = 0;
         if (rc) return rc;
-        _Float16 *att_xh = xh_for(L.wo) && mmq_fuses_residual(L.wo, n) && attn_prefill_writes_half(dev, c.head_dim) ? P.xh : nullptr;
-        if ((rc = launch_attn_prefill(dev, P.q, kc, vc, m->kv_f16, P.att, n, pos0, c.n_heads, c.n_kv_heads, c.head_dim,
+        _Float16 *att_xh = xh_for(L.wo) && mmq_fuses_residual(L.wo, n) && attn_prefill_writes_half(dev) ? P.xh : nullptr;
+        if ((rc = launch_attn_prefill(dev, P.q, kc, vc, m->kv_f16, kv_parts, P.att, n, pos0, c.n_heads, c.n_kv_heads, c.head_dim,
                                       cache_stride, scale, att_xh)))
             return rc;
         if (!att_xh && (rc = launch_quantize_q8(dev, P.att, n, qd, P.xq, P.xs, nullptr, xh_for(L.wo)))) return rc;

@@ -6,9 +6,9 @@
 // the same arithmetic as n successive decode steps, evaluated tile by tile here.
 //   k_prefill_rope_kv   Rope (reduce.go:3987-4006: pairs (j, j + d/2)) on q in place and on k, and the
 //                       new k / v rows written into the f32 cache [kv_head][position][head_dim]
-//   k_attn_prefill      causal attention of 32 queries of one head against the cache, f32 on the
-//                       vector ALU with K / V / probabilities tiled through LDS, online softmax (head_dim 64)
-//   k_attn_prefill_mfma the same for head_dim 128 on the matrix cores, 64 queries per workgroup
+//   k_kv_parts          cache rows of earlier positions as the sums of 16-bit parts the matrix cores contract
+//   k_attn_prefill_mfma causal attention of 64 or 128 queries of one head against the cache on the matrix cores
+//   k_attn_prefill      the same on the vector ALU (comparison runs)
 #include <cstdlib>
 
 #include "blocks.h"
@@ -66,15 +66,44 @@ __global__ __launch_bounds__(256) void k_prefill_rope_kv(float *__restrict__ q, 
     }
 }
 
+// The first P parts of four values, part_stride apart: each the rounding of what the parts before it leave.
+template <class T, int P>
+__device__ __forceinline__ void store_parts(T *dst, int64_t part_stride, float4 x) {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    float rest[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        t4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[e] = (T)rest[e];
+            rest[e] -= (float)o[e];
+        }
+        *(t4 *)(dst + (size_t)p * part_stride) = o;
+    }
+}
+
+// `count` cache rows of every kv head -> the parts k_attn_prefill_mfma reads, in rows like the cache's.
+template <class T, int P>
+__global__ __launch_bounds__(256) void k_kv_parts(const float *__restrict__ k_cache, const float *__restrict__ v_cache, int64_t cache_stride,
+                                                  T *__restrict__ kparts, T *__restrict__ vparts, int64_t part_stride, int lo, int count, int c4) {
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (row, four values)
+    if (idx >= (int64_t)count * c4) return;
+    const size_t at = (size_t)blockIdx.y * cache_stride + ((size_t)lo * c4 + idx) * 4;
+    store_parts<T, P>((blockIdx.z ? vparts : kparts) + at, part_stride, *(const float4 *)((blockIdx.z ? v_cache : k_cache) + at));
+}
+
 // The same four pairs per thread, for q, k and v rows that lie end to end in `src` ([n][q heads], [n][kv heads] twice),
 // optionally still as the n_split partial copies of a contraction split along K, `stride` floats apart, summed here in
-// the order of the separate split sum.  q is written to `q` (which may be `src`), k and v go to the cache only.
-template <class KV>
+// the order of the separate split sum.  q is written to `q` (which may be `src`), k and v go to the cache and, with an
+// f32 cache (P > 0), as parts to the rows the attention kernel reads: a launch and a pass less than k_kv_parts behind it.
+template <class KV, class T, int P>
 __global__ __launch_bounds__(256) void k_prefill_rope_kv4(float *q, const float *src, int n_split, size_t stride,
                                                           const float *__restrict__ cos_t,
                                                           const float *__restrict__ sin_t, KV *__restrict__ k_cache,
                                                           KV *__restrict__ v_cache, int n, int pos0, int n_heads,
-                                                          int n_kv_heads, int head_dim, int64_t cache_stride) {
+                                                          int n_kv_heads, int head_dim, int64_t cache_stride,
+                                                          T *__restrict__ kparts, T *__restrict__ vparts, int64_t part_stride) {
     const int half = head_dim >> 1, hq = half >> 2;
     const int slots = n_heads + 2 * n_kv_heads;  // q heads, then k heads, then v heads
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -102,9 +131,12 @@ __global__ __launch_bounds__(256) void k_prefill_rope_kv4(float *q, const float 
     if (slot >= n_heads + n_kv_heads) {
         const int h = slot - n_heads - n_kv_heads;
         const size_t off = v_base + ((size_t)i * n_kv_heads + h) * head_dim + j;
-        KV *dst = v_cache + (size_t)h * cache_stride + (size_t)pos * head_dim + j;
-        store(dst, load(off));
-        store(dst + half, load(off + half));
+        const size_t at = (size_t)h * cache_stride + (size_t)pos * head_dim + j;
+        const float4 x = load(off), y = load(off + half);
+        store(v_cache + at, x);
+        store(v_cache + at + half, y);
+        store_parts<T, P>(vparts + at, part_stride, x);
+        store_parts<T, P>(vparts + at + half, part_stride, y);
         return;
     }
     const float4 c = *(const float4 *)(cos_t + (size_t)pos * half + j), s = *(const float4 *)(sin_t + (size_t)pos * half + j);
@@ -118,9 +150,11 @@ __global__ __launch_bounds__(256) void k_prefill_rope_kv4(float *q, const float 
         *(float4 *)(q + off) = lo;
         *(float4 *)(q + off + half) = hi;
     } else {
-        KV *dst = k_cache + (size_t)h * cache_stride + (size_t)pos * head_dim + j;
-        store(dst, lo);
-        store(dst + half, hi);
+        const size_t at = (size_t)h * cache_stride + (size_t)pos * head_dim + j;
+        store(k_cache + at, lo);
+        store(k_cache + at + half, hi);
+        store_parts<T, P>(kparts + at, part_stride, lo);
+        store_parts<T, P>(kparts + at + half, part_stride, hi);
     }
 }
 
@@ -225,298 +259,308 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float *__restrict__ 
 }
 
 // ------------------------------------------------------------------ causal attention on the matrix cores
-// head_dim 128.  grid (n_heads, ceil(n / 64)), 4 wavefronts, wavefront w owns query rows 16w .. 16w+15 of
-// the tile.  Keys and values are walked in tiles of 32 positions through LDS.  Scores S = Q.K^T and
-// outputs O += P.V run on v_mfma_f32_16x16x32_f16 with every f32 operand split into an fp16 head and an
-// fp16 tail (x = hi + lo, |lo| <= 2^-11 |x|): hi.hi + hi.lo + lo.hi carries 22 bits of each operand into
-// the f32 accumulators, so the result stays at f32-like distance from the CPU composition while the
-// vector ALU only does the softmax.  (The arithmetic being replaced is MatMul / FastSoftmax / MatMul,
-// backend.go:78,147; online softmax as in the vector-ALU kernel above.)
+// An f32 operand meets the matrix cores as a sum of parts, each part the rounding of what the parts before it leave:
+//   head_dim 128, f32 cache   two fp16 parts of q, K, V and the weights (22 bits), three products
+//   head_dim 64, f32 cache    three bfloat16 parts (24 bits and f32's range: what the vector ALU had), six products
+//   fp16 cache                K and V are their own single part; q in two fp16 parts (three for head_dim 64), the weights in two
+// K and V parts lie in memory as rows like the cache's (k_kv_parts; a fp16 cache is read as it is), so that a tile goes
+// to LDS by direct loads and no workgroup converts what the others of its head convert as well.
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4h __attribute__((ext_vector_type(4)));
-typedef _Float16 half2h __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-struct HiLo { _Float16 hi, lo; };
-__device__ __forceinline__ HiLo split_half(float x) {
-    HiLo r;
-    r.hi = (_Float16)x;
-    r.lo = (_Float16)(x - (float)r.hi);
-    return r;
+template <class T> struct PartVec;
+template <> struct PartVec<_Float16> { typedef half8 v8; typedef half4h v4; };
+template <> struct PartVec<__bf16> { typedef __bf16 v8 __attribute__((ext_vector_type(8))); typedef __bf16 v4 __attribute__((ext_vector_type(4))); };
+
+__device__ __forceinline__ float4v mfma16(half8 a, half8 b, float4v c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ float4v mfma16(PartVec<__bf16>::v8 a, PartVec<__bf16>::v8 b, float4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+// four rows of a 16-bit matrix in LDS, transposed: lane l of 16 receives column l (lane l points at row l / 4, values
+// 4 (l % 4) .. + 3)
+__device__ __forceinline__ half4h lds_columns(const _Float16 *p) {
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(half4h, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)p));
+}
+__device__ __forceinline__ PartVec<__bf16>::v4 lds_columns(const __bf16 *p) {
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(PartVec<__bf16>::v4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)p));
 }
 
-// 16-lane row reductions on the DPP path (C-layout columns live in the 16 lanes of a row)
-__device__ __forceinline__ float row16_max(float v) {
-    v = fmaxf(v, dpp_move<0xB1>(v));
-    v = fmaxf(v, dpp_move<0x4E>(v));
-    v = fmaxf(v, dpp_move<0x141>(v));
-    v = fmaxf(v, dpp_move<0x140>(v));
-    return v;
+// over the four lanes 16 apart that share a query
+__device__ __forceinline__ float quad16_max(float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float row16_sum(float v) {
-    v += dpp_move<0xB1>(v);
-    v += dpp_move<0x4E>(v);
-    v += dpp_move<0x141>(v);
-    v += dpp_move<0x140>(v);
-    return v;
+__device__ __forceinline__ float quad16_sum(float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// GROUPS = 2: two groups of four wavefronts share the workgroup's 64 queries and take alternate key tiles, each with
-// tile buffers of its own, and merge their (max, sum, output) per row at the end: a short prompt has about one
-// workgroup per CU and the launch lasts as long as the last query tile's walk over all the keys, which this halves.
-template <class KV, int GROUPS>
-__global__ __launch_bounds__(256 * GROUPS) void k_attn_prefill_mfma(const float *__restrict__ q, const KV *__restrict__ k_cache,
-                                                                    const KV *__restrict__ v_cache, float *__restrict__ out,
-                                                                    int n, int pos0, int n_heads, int n_kv_heads,
-                                                                    int64_t cache_stride, float scale,
-                                                                    _Float16 *__restrict__ xh_out) {
-    constexpr int HD = 128, QT = 64, KT = 32;
-    constexpr bool HALF_KV = std::is_same<KV, _Float16>::value;  // cache values are their own fp16 head: no tail tiles
-    constexpr int KP = HD + 8;   // K tile pitch in halves (272 bytes: the 16 rows of an operand read hit distinct banks)
-    constexpr int VP = KT + 8;   // V^T tile pitch in halves (80 bytes, same property)
-    constexpr int PP = KT + 8;   // P tile pitch
-    constexpr int K_HALVES = 2 * KT * KP, VT_HALVES = 2 * HD * VP, P_HALVES = 4 * 2 * 16 * PP;
-    constexpr int GROUP_HALVES = K_HALVES + VT_HALVES + P_HALVES;
-    static_assert(GROUP_HALVES * 2 >= 40 * 256 * 4, "a group's buffers hold the other group's state at the merge");
-    __shared__ __align__(16) _Float16 s_all[GROUPS * GROUP_HALVES];
-    const int grp = GROUPS == 1 ? 0 : (int)(threadIdx.x >> 8);
-    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-    _Float16 *const s_kb = s_all + grp * GROUP_HALVES;   // [hi/lo][key][d]
-    _Float16 *const s_vtb = s_kb + K_HALVES;              // [hi/lo][d][key]
-    _Float16 *const s_pb = s_vtb + VT_HALVES;             // per wavefront [hi/lo][row][key]
-    _Float16 *const s_k[2] = {s_kb, s_kb + KT * KP};
-    _Float16 *const s_vt[2] = {s_vtb, s_vtb + HD * VP};
-    const int r16 = lane & 15, c4 = lane >> 4;
-    const int head = blockIdx.x, i0 = blockIdx.y * QT;
-    const int kvh = head / (n_heads / n_kv_heads);
-    const KV *kh = k_cache + (size_t)kvh * cache_stride, *vh = v_cache + (size_t)kvh * cache_stride;
-    const int n_keys = pos0 + min(i0 + QT, n);   // positions the tile's last query may see
-    const int wave_last = pos0 + i0 + 16 * wave + 15;  // last position any row of this wavefront may see
-
-    // Q as the A operand (row = query r16, 8 consecutive d per k-step), pre-scaled by scale * log2(e) (the softmax
-    // runs on powers of two: one v_exp_f32 per value), split hi / lo
-    half8 qh[4], ql[4];
+template <int HD, class T, int KVP, int QP, int PP, int QH, int KG>
+__global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * KG == 4 ? 1 : 2) void k_attn_prefill_mfma(const float *__restrict__ q, const T *__restrict__ kparts, const T *__restrict__ vparts,
+                                                              int64_t part_stride, int64_t head_stride, float *__restrict__ out, int n, int pos0,
+                                                              int n_heads, int group, int q_tiles, float scale,
+                                                              _Float16 *__restrict__ xh_out) {
+    typedef typename PartVec<T>::v8 v8;
+    typedef typename PartVec<T>::v4 v4;
+    constexpr int THREADS = 64 * QH * KG, QT = 32 * QH, R = 32 * KG, C = HD / 8, KS = HD / 32, DT = HD / 16;
+    constexpr int ARR = R * C, STEP = 2 * KVP * ARR;  // 16-byte pieces of one part of K or V, and of everything a step stages
+    constexpr int IT = ARR / THREADS;
+    static_assert(ARR % THREADS == 0 && (HD == 64 || HD == 128), "whole pieces per thread");
+    constexpr int MERGE = KG == 1 ? 0 : (4 + 2 * 4 * DT) * 16 * QH;  // the second key group's state at the end
+    __shared__ __align__(16) uint4 s_all[2 * STEP > MERGE ? 2 * STEP : MERGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int qh = wave % QH, kg = wave / QH;
+    // The workgroups of neighbouring heads (which share K and V) on one XCD, the longest walks first.
+    int head, qt0;
     {
-        const int i = min(i0 + 16 * wave + r16, n - 1);
-        const float *qr = q + ((size_t)i * n_heads + head) * HD;
+        const int id = blockIdx.x;
+        if ((n_heads & 7) == 0) {
+            const int per = n_heads >> 3, s = id >> 3;
+            head = (id & 7) * per + s % per;
+            qt0 = q_tiles - 1 - s / per;
+        } else {
+            head = id % n_heads;
+            qt0 = q_tiles - 1 - id / n_heads;
+        }
+    }
+    const int i0 = qt0 * QT;
+    const T *kh = kparts + (size_t)(head / group) * head_stride, *vh = vparts + (size_t)(head / group) * head_stride;
+    const int n_keys = pos0 + min(i0 + QT, n);  // positions the tile's last query may see
+    const int wq0 = pos0 + i0 + 32 * qh;         // first position of this wavefront's 32 queries
+
+    // q as the B operand (column = query, 8 consecutive d per lane), scaled for a softmax on powers of two
+    v8 qf[2][KS][QP];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const float4 a = *(const float4 *)(qr + ks * 32 + c4 * 8), b = *(const float4 *)(qr + ks * 32 + c4 * 8 + 4);
+    for (int t = 0; t < 2; ++t) {
+        const float *qr = q + ((size_t)min(i0 + 32 * qh + 16 * t + r16, n - 1) * n_heads + head) * HD;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const float4 a = *(const float4 *)(qr + ks * 32 + g * 8), b = *(const float4 *)(qr + ks * 32 + g * 8 + 4);
             const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const HiLo t = split_half(v[e] * (scale * 1.44269504088896341f));
-                qh[ks][e] = t.hi;
-                ql[ks][e] = t.lo;
+                float rest = v[e] * (scale * 1.44269504088896341f);
+#pragma unroll
+                for (int p = 0; p < QP; ++p) {
+                    qf[t][ks][p][e] = (T)rest;
+                    rest -= (float)qf[t][ks][p][e];
+                }
             }
         }
     }
-    // C layout: lane holds rows 4*c4 + j (j = 0..3) of the wavefront's 16 queries, column r16
-    float m_run[4], l_run[4];
-    float4v o[8];
+    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};  // the sum is over this lane's keys until the end
+    float4v o[2][DT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) { m_run[j] = -INFINITY; l_run[j] = 0.0f; }
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < DT; ++d) o[t][d] = float4v{0.f, 0.f, 0.f, 0.f};
 
-    // global -> register requests of a tile: K: thread -> (key, 4 consecutive d), 4 passes; V: thread -> (key pair,
-    // 4 consecutive d), 2 passes.  The next tile is requested before the current one is consumed.
-    float4 kreg[4], vreg[2][2];
-    auto request = [&](int p0) __attribute__((always_inline)) {
+    // Rows of a tile lie end to end in LDS; piece c of row r sits in slot c ^ turn(r), which keeps both the fragment
+    // reads of K (16 rows, one piece each) and the column reads of V (8 rows, two pieces each) off each other's banks.
+    auto turn = [](int r) { return HD == 128 ? ((r & 7) << 1) | ((r >> 3) & 1) : (((r >> 1) & 3) << 1) | ((r >> 3) & 1); };
+    auto stage = [&](int p0, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int e = tid + it * 256, key = e >> 5, d4 = e & 31;
-            kreg[it] = kv_load4(kh + (size_t)min(p0 + key, n_keys - 1) * HD + 4 * d4);
-        }
+        for (int a = 0; a < 2 * KVP; ++a) {
+            const T *src = (a < KVP ? kh : vh) + (size_t)(a < KVP ? a : a - KVP) * part_stride;
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            // a wavefront's lanes: 16 key pairs x 4 neighbouring d4.  With the 32 d4 of one key pair per half wavefront
-            // the transposed stores below put 32 lanes on two LDS banks (a row of V^T is 80 bytes: 4 rows are 320,
-            // a multiple of 64) - 16-way conflicts on every one of them: 512 prompt tokens 48 -> 42.5 us per launch
-            const int e = tid + it * 256, kp = e & 15, d4 = e >> 4;
-            vreg[it][0] = kv_load4(vh + (size_t)min(p0 + 2 * kp, n_keys - 1) * HD + 4 * d4);
-            vreg[it][1] = kv_load4(vh + (size_t)min(p0 + 2 * kp + 1, n_keys - 1) * HD + 4 * d4);
+            for (int it = 0; it < IT; ++it) {
+                const int e = it * THREADS + tid, row = e / C, c = (e % C) ^ turn(row);
+                const T *from = src + (size_t)min(p0 + row, n_keys - 1) * HD + c * 8;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from,
+                                                 (__attribute__((address_space(3))) void *)&s_all[buf * STEP + a * ARR + it * THREADS + wave * 64], 16, 0, 0);
+            }
         }
     };
-    // every group runs the same number of rounds (the barriers are the workgroup's); a group without a tile in the
-    // last round sits it out
-    const int n_rounds = ((n_keys + KT - 1) / KT + GROUPS - 1) / GROUPS;
-    if (grp * KT < n_keys) request(grp * KT);
-    for (int round = 0; round < n_rounds; ++round) {
-        const int p0 = (round * GROUPS + grp) * KT;
-        __syncthreads();  // previous tile fully consumed
-        if (GROUPS > 1 && p0 >= n_keys) {
-            __syncthreads();
-            continue;
+    const int k_turn = turn(r16), v_row = 4 * g + (r16 >> 2), v_turn = turn(v_row), v_half = (r16 & 3) >> 1;
+    const int n_steps = (n_keys + R - 1) / R;
+    stage(0, 0);
+    for (int step = 0; step < n_steps; ++step) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // the tile has landed for every wavefront, and the other buffer is consumed
+        if (step + 1 < n_steps) stage((step + 1) * R, (step + 1) & 1);
+        const int p0 = step * R + 32 * kg;  // this wavefront's 32 keys
+        if (p0 > wq0 + 31 || p0 >= n_keys) continue;
+        const uint4 *base = s_all + (step & 1) * STEP + 32 * kg * C;
+        // ---- scores, transposed: rows are keys, a lane holds those of query r16, keys 16 kt + 4 g + j
+        float4v s[2][2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) s[t][kt] = float4v{0.f, 0.f, 0.f, 0.f};
+        constexpr int TOP = QP > KVP ? QP : KVP;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+            v8 kf[KS][KVP];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int p = 0; p < KVP; ++p) kf[ks][p] = __builtin_bit_cast(v8, base[p * ARR + (kt * 16 + r16) * C + ((ks * 4 + g) ^ k_turn)]);
+#pragma unroll
+            for (int sum = TOP - 1; sum >= 0; --sum)  // the smallest products first
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                    for (int p = 0; p < KVP; ++p)
+                        if (sum - p >= 0 && sum - p < QP) {
+#pragma unroll
+                            for (int t = 0; t < 2; ++t) s[t][kt] = mfma16(kf[ks][p], qf[t][ks][sum - p], s[t][kt]);
+                        }
         }
+        // ---- online softmax: every score of a query is in the four lanes 16 apart
+        v8 pf[2][PP];
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int e = tid + it * 256, key = e >> 5, d4 = e & 31;
-            const float4 kv = kreg[it];
-            half4h hi, lo;
-            const float kvv[4] = {kv.x, kv.y, kv.z, kv.w};
+        for (int t = 0; t < 2; ++t) {
+            const int qpos = wq0 + 16 * t + r16;
+            if (p0 + 31 > wq0 + 16 * t) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const HiLo t = split_half(kvv[c]);
-                hi[c] = t.hi;
-                lo[c] = t.lo;
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s[t][kt][j] = p0 + kt * 16 + 4 * g + j <= qpos ? s[t][kt][j] : -INFINITY;
             }
-            *(half4h *)&s_k[0][key * KP + 4 * d4] = hi;
-            if (!HALF_KV) *(half4h *)&s_k[1][key * KP + 4 * d4] = lo;
-        }
-        // V transposed: two keys of one d share a 32-bit store
+            float mx = fmaxf(fmaxf(fmaxf(s[t][0][0], s[t][0][1]), fmaxf(s[t][0][2], s[t][0][3])),
+                             fmaxf(fmaxf(s[t][1][0], s[t][1][1]), fmaxf(s[t][1][2], s[t][1][3])));
+            const float m_new = fmaxf(m_run[t], quad16_max(mx));
+            const float m_at = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible yet: all weights are 2^-inf = 0
+            const float corr = __builtin_amdgcn_exp2f(m_run[t] - m_at);
+            m_run[t] = m_new;
+            float sum = 0.0f;
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int e = tid + it * 256, kp = e & 15, d4 = e >> 4;
-            const float4 v0 = vreg[it][0], v1 = vreg[it][1];
-            const float a[4] = {v0.x, v0.y, v0.z, v0.w}, b[4] = {v1.x, v1.y, v1.z, v1.w};
+            for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                half2h hi, lo;
-                const HiLo ta = split_half(a[c]), tb = split_half(b[c]);
-                hi[0] = ta.hi; lo[0] = ta.lo;
-                hi[1] = tb.hi; lo[1] = tb.lo;
-                *(half2h *)&s_vt[0][(4 * d4 + c) * VP + 2 * kp] = hi;
-                if (!HALF_KV) *(half2h *)&s_vt[1][(4 * d4 + c) * VP + 2 * kp] = lo;
+                for (int j = 0; j < 4; ++j) {
+                    float w = __builtin_amdgcn_exp2f(s[t][kt][j] - m_at);
+                    sum += w;
+#pragma unroll
+                    for (int p = 0; p < PP; ++p) {
+                        pf[t][p][kt * 4 + j] = (T)w;
+                        w -= (float)pf[t][p][kt * 4 + j];
+                    }
+                }
+            l_run[t] = l_run[t] * corr + sum;
+            if (__any(corr != 1.0f)) {  // the maxima settle after the first tiles
+#pragma unroll
+                for (int d = 0; d < DT; ++d) o[t][d] *= corr;
             }
         }
-        if (p0 + GROUPS * KT < n_keys) request(p0 + GROUPS * KT);
-        __syncthreads();
-        if (p0 > wave_last) continue;  // every key of the tile is in the future of all 16 rows (the barriers above stay uniform)
-
-        // ---- S = Q.K^T for 32 keys: two 16-key column tiles
-        float4v s_acc[2];
+        // ---- outputs, transposed: O^T += V^T P^T; K index 8 g + e stands for key 4 g + e (e < 4) or 16 + 4 g + e - 4
+        constexpr int TOPV = PP > KVP ? PP : KVP;
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-            float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < DT; ++d) {
+            v8 vf[KVP];
+            const int at = v_row * C + ((2 * d + v_half) ^ v_turn);
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const int off = (nt * 16 + r16) * KP + ks * 32 + c4 * 8;
-                const half8 kh8 = *(const half8 *)&s_k[0][off];
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[ks], kh8, acc, 0, 0, 0);
-                if (!HALF_KV) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], *(const half8 *)&s_k[1][off], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[ks], kh8, acc, 0, 0, 0);
-            }
-            s_acc[nt] = acc;
-        }
-        // ---- online softmax per row
-        float corr[4];
-        _Float16 *ph = s_pb + wave * 2 * 16 * PP, *pl = ph + 16 * PP;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int qpos = pos0 + i0 + 16 * wave + 4 * c4 + j;
-            float sv[2];
-            float mx = -INFINITY;
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const bool ok = p0 + nt * 16 + r16 <= qpos;
-                sv[nt] = ok ? s_acc[nt][j] : -INFINITY;
-                mx = fmaxf(mx, sv[nt]);
-            }
-            mx = row16_max(mx);
-            // position 0 is visible to every row: with one group finite from the first tile on; a second group's first
-            // tile may lie in a row's future altogether
-            const float m_new = fmaxf(m_run[j], mx);
-            const bool seen = GROUPS == 1 || m_new != -INFINITY;
-            corr[j] = seen ? __builtin_amdgcn_exp2f(m_run[j] - m_new) : 1.0f;
-            float ps = 0.0f;
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const float pw = seen ? __builtin_amdgcn_exp2f(sv[nt] - m_new) : 0.0f;  // 2^-inf = 0 for masked keys
-                ps += pw;
-                const HiLo t = split_half(pw);
-                ph[(4 * c4 + j) * PP + nt * 16 + r16] = t.hi;
-                pl[(4 * c4 + j) * PP + nt * 16 + r16] = t.lo;
-            }
-            ps = row16_sum(ps);
-            l_run[j] = l_run[j] * corr[j] + ps;
-            m_run[j] = m_new;
-        }
-        // the running maxima settle after the first tiles: most rounds have nothing to rescale
-        if (__any(corr[0] != 1.0f || corr[1] != 1.0f || corr[2] != 1.0f || corr[3] != 1.0f)) {
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) o[dt][j] *= corr[j];
-        }
-        // the wavefront's own P tile: its LDS operations complete in order, no workgroup barrier needed
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // ---- O += P.V: P as the A operand (row r16, keys 8*c4 .. +7), V^T rows as the B operand
-        const half8 pa_h = *(const half8 *)&ph[r16 * PP + c4 * 8], pa_l = *(const half8 *)&pl[r16 * PP + c4 * 8];
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            const int off = (dt * 16 + r16) * VP + c4 * 8;
-            const half8 vh8 = *(const half8 *)&s_vt[0][off];
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa_l, vh8, o[dt], 0, 0, 0);
-            if (!HALF_KV) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa_h, *(const half8 *)&s_vt[1][off], o[dt], 0, 0, 0);
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa_h, vh8, o[dt], 0, 0, 0);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    if constexpr (GROUPS == 2) {
-        // the second group's state goes through its own tile buffers (value k of thread t at k * 256 + t); the first
-        // group, whose tiles hold position 0, always has a finite maximum
-        float *st = (float *)(s_all + GROUP_HALVES);
-        __syncthreads();
-        if (grp == 1) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                st[j * 256 + tid] = m_run[j];
-                st[(4 + j) * 256 + tid] = l_run[j];
+            for (int p = 0; p < KVP; ++p) {
+                const T *a = (const T *)(base + (KVP + p) * ARR + at) + (r16 & 1) * 4;
+                const v4 lo = lds_columns(a), hi = lds_columns(a + 16 * HD);
+                vf[p] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
             }
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
+            for (int sum = TOPV - 1; sum >= 0; --sum)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) st[(8 + 4 * dt + j) * 256 + tid] = o[dt][j];
-        }
-        __syncthreads();
-        if (grp == 1) return;
+                for (int p = 0; p < KVP; ++p)
+                    if (sum - p >= 0 && sum - p < PP) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float m1 = st[j * 256 + tid], l1 = st[(4 + j) * 256 + tid];
-            const float m = fmaxf(m_run[j], m1);
-            const float f0 = __builtin_amdgcn_exp2f(m_run[j] - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
-            l_run[j] = l_run[j] * f0 + l1 * f1;
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt) o[dt][j] = o[dt][j] * f0 + st[(8 + 4 * dt + j) * 256 + tid] * f1;
+                        for (int t = 0; t < 2; ++t) o[t][d] = mfma16(vf[p], pf[t][sum - p], o[t][d]);
+                    }
         }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int i = i0 + 16 * wave + 4 * c4 + j;
-        if (i >= n) continue;
-        const float inv = 1.0f / l_run[j];
+    for (int t = 0; t < 2; ++t) l_run[t] = quad16_sum(l_run[t]);
+    if constexpr (KG == 2) {  // value k of thread t of the second group at k * 64 QH + t
+        float *st = (float *)s_all;
+        const int at = tid & (64 * QH - 1);
+        __syncthreads();
+        if (kg == 1) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                st[t * 64 * QH + at] = m_run[t];
+                st[(2 + t) * 64 * QH + at] = l_run[t];
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) st[(4 + (t * DT + d) * 4 + j) * 64 * QH + at] = o[t][d][j];
+            }
+        }
+        __syncthreads();
+        if (kg == 1) return;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const float m1 = st[t * 64 * QH + at], l1 = st[(2 + t) * 64 * QH + at];
+            const float m = fmaxf(m_run[t], m1);  // finite: position 0 is in the first group
+            const float f0 = __builtin_amdgcn_exp2f(m_run[t] - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
+            l_run[t] = l_run[t] * f0 + l1 * f1;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[t][d][j] = o[t][d][j] * f0 + st[(4 + (t * DT + d) * 4 + j) * 64 * QH + at] * f1;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int i = i0 + 32 * qh + 16 * t + r16;
+        const float inv = 1.0f / l_run[t];
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[t][d] *= inv;
         if (xh_out) {
-            // The output row leaves as the fp16 image of its Q8_0 quantization (what the o projection's fp16 tiles
-            // contract with), the arithmetic of quantize_q8_lane4 + q8_lane4_to_half value by value: a 32-value block
-            // is columns 32 b .. 32 b + 31 = this 16-lane row's o[2 b] and o[2 b + 1].
+            // The row leaves as the fp16 image of its Q8_0 quantization (what the o projection's fp16 tiles contract
+            // with), the arithmetic of quantize_q8_lane4 + q8_lane4_to_half value by value: a 32-value block is
+            // o[2 b] and o[2 b + 1] of the four lanes that share the query.
             const int K = n_heads * HD;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const float v0 = o[2 * b][j] * inv, v1 = o[2 * b + 1][j] * inv;
-                const float amax = row16_max(fmaxf(fabsf(v0), fabsf(v1)));
-                const float d = amax / 127.0f;
-                const int q0 = amax != 0.0f ? q8_level(v0, d) : 0, q1 = amax != 0.0f ? q8_level(v1, d) : 0;
-                const float df = __half2float(__float2half_rn(d));
-                const int col = head * HD + 32 * b + r16;
-                xh_out[xh_index4(i, col >> 2, K) * 4 + (col & 3)] = (_Float16)(df * (float)q0);
-                xh_out[xh_index4(i, (col + 16) >> 2, K) * 4 + (col & 3)] = (_Float16)(df * (float)q1);
-            }
-            continue;
-        }
-        float *dst = out + ((size_t)i * n_heads + head) * HD + r16;
+            for (int b = 0; b < DT / 2; ++b) {
+                float amax = 0.0f;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) dst[dt * 16] = o[dt][j] * inv;
+                for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(o[t][2 * b + (e >> 2)][e & 3]));
+                amax = quad16_max(amax);
+                const float dq = amax / 127.0f, df = __half2float(__float2half_rn(dq));
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf) {
+                    half4h w;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) w[j] = (_Float16)(df * (float)(amax != 0.0f ? q8_level(o[t][2 * b + hf][j], dq) : 0));
+                    const int col = head * HD + 32 * b + 16 * hf + 4 * g;
+                    if (i < n) *(half4h *)(xh_out + xh_index4(i, col >> 2, K) * 4) = w;
+                }
+            }
+        } else if (i < n) {
+            float *dst = out + ((size_t)i * n_heads + head) * HD + 4 * g;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) *(float4v *)(dst + 16 * d) = o[t][d];
+        }
     }
+}
+
+// The parts of K and V the matrix-core kernel contracts, for an f32 cache: three bfloat16 or two fp16 ones per value.
+size_t attn_prefill_parts_bytes(int n_kv_heads, int head_dim, int max_pos) {
+    return (size_t)2 * (head_dim == 64 ? 3 : 2) * n_kv_heads * max_pos * head_dim * 2;
+}
+
+static int launch_kv_parts(candy_hip_device *dev, const float *k_cache, const float *v_cache, void *parts, int lo, int count, int n_kv_heads,
+                           int head_dim, int64_t cache_stride) {
+    const int64_t part_stride = (int64_t)n_kv_heads * cache_stride;
+    const dim3 grid((unsigned)(((int64_t)count * (head_dim / 4) + 255) / 256), (unsigned)n_kv_heads, 2);
+    if (head_dim == 64)
+        hipLaunchKernelGGL((k_kv_parts<__bf16, 3>), grid, dim3(256), 0, dev->stream, k_cache, v_cache, cache_stride, (__bf16 *)parts,
+                           (__bf16 *)parts + 3 * part_stride, part_stride, lo, count, head_dim / 4);
+    else
+        hipLaunchKernelGGL((k_kv_parts<_Float16, 2>), grid, dim3(256), 0, dev->stream, k_cache, v_cache, cache_stride, (_Float16 *)parts,
+                           (_Float16 *)parts + 2 * part_stride, part_stride, lo, count, head_dim / 4);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
 }
 
 int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, const float *v, const float *cos_t,
                            const float *sin_t, void *k_cache, void *v_cache, bool kv_f16, int n, int pos0, int n_heads,
-                           int n_kv_heads, int head_dim, int64_t cache_stride, const SplitPending *sp) {
+                           int n_kv_heads, int head_dim, int64_t cache_stride, void *parts, const SplitPending *sp) {
+    const int64_t part_stride = (int64_t)n_kv_heads * cache_stride;
     const size_t q_count = (size_t)n * n_heads * head_dim, kv_count = (size_t)n * n_kv_heads * head_dim;
     const bool pending = sp && sp->n_split > 0;
     if (pending) CANDY_REQUIRE(sp->y == q && !sp->res && sp->count == q_count + 2 * kv_count, "internal: pending split sum of another shape");
@@ -527,14 +571,15 @@ int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, cons
         const float *src = pending ? sp->part : q;
         const int n_split = pending ? sp->n_split : 1;
         const size_t stride = pending ? sp->stride : 0;
-        if (kv_f16)
-            hipLaunchKernelGGL(k_prefill_rope_kv4<_Float16>, grid4, dim3(256), 0, dev->stream, q, src, n_split, stride, cos_t,
-                               sin_t, (_Float16 *)k_cache, (_Float16 *)v_cache, n, pos0, n_heads, n_kv_heads, head_dim,
-                               cache_stride);
-        else
-            hipLaunchKernelGGL(k_prefill_rope_kv4<float>, grid4, dim3(256), 0, dev->stream, q, src, n_split, stride, cos_t,
-                               sin_t, (float *)k_cache, (float *)v_cache, n, pos0, n_heads, n_kv_heads, head_dim,
-                               cache_stride);
+#define CANDY_ROPE4(KV, T, P)                                                                                                            \
+    hipLaunchKernelGGL((k_prefill_rope_kv4<KV, T, P>), grid4, dim3(256), 0, dev->stream, q, src, n_split, stride, cos_t, sin_t,          \
+                       (KV *)k_cache, (KV *)v_cache, n, pos0, n_heads, n_kv_heads, head_dim, cache_stride, (T *)parts,                   \
+                       (T *)parts + P * part_stride, part_stride)
+        if (kv_f16) CANDY_ROPE4(_Float16, _Float16, 0);
+        else if (!parts) CANDY_ROPE4(float, _Float16, 0);
+        else if (head_dim == 64) CANDY_ROPE4(float, __bf16, 3);
+        else CANDY_ROPE4(float, _Float16, 2);
+#undef CANDY_ROPE4
         CANDY_LAUNCH_CHECK();
         return CANDY_HIP_OK;
     }
@@ -549,55 +594,76 @@ int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, cons
         hipLaunchKernelGGL(k_prefill_rope_kv<float>, grid, dim3(256), 0, dev->stream, q, k, v, cos_t, sin_t,
                            (float *)k_cache, (float *)v_cache, n, pos0, n_heads, n_kv_heads, head_dim, cache_stride);
     CANDY_LAUNCH_CHECK();
-    return CANDY_HIP_OK;
+    return parts && !kv_f16 ? launch_kv_parts(dev, (const float *)k_cache, (const float *)v_cache, parts, pos0, n, n_kv_heads, head_dim, cache_stride)
+                            : CANDY_HIP_OK;
 }
 
-template <class KV>
-static void launch_attn_prefill_kv(candy_hip_device *dev, const float *q, const KV *k_cache, const KV *v_cache, float *out,
-                                   int n, int pos0, int n_heads, int n_kv_heads, int head_dim, int64_t cache_stride,
-                                   float scale, _Float16 *xh_out) {
-    const dim3 grid((unsigned)n_heads, (unsigned)((n + 31) / 32));
-    const bool valu_only = dev->opt.prefill_attention_valu != 0;  // comparison runs
-    if (head_dim == 128 && !valu_only) {
-        // Two key-tile groups per workgroup where the launch lasts as long as its longest workgroup: a grid of about one
-        // workgroup per CU and a walk of more than four key tiles.  A larger grid fills the CUs with several of the
-        // smaller workgroups, a shorter walk does not pay for the merge.
-        const dim3 tiles((unsigned)n_heads, (unsigned)((n + 63) / 64));
-        const int64_t wgs = (int64_t)tiles.x * tiles.y;
-        const int groups = dev->opt.prefill_attention_groups ? dev->opt.prefill_attention_groups
-                                                             : (n > 128 && 2 * wgs <= 3 * (int64_t)dev->num_cus ? 2 : 1);
-        if (groups == 2)
-            hipLaunchKernelGGL((k_attn_prefill_mfma<KV, 2>), tiles, dim3(512), 0, dev->stream, q, k_cache, v_cache, out, n,
-                               pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
-        else
-            hipLaunchKernelGGL((k_attn_prefill_mfma<KV, 1>), tiles, dim3(256), 0, dev->stream, q, k_cache, v_cache, out, n,
-                               pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
-    } else if (head_dim == 128)
-        hipLaunchKernelGGL((k_attn_prefill<128, KV>), grid, dim3(256), 0, dev->stream, q, k_cache, v_cache, out, n, pos0,
-                           n_heads, n_kv_heads, cache_stride, scale);
-    else
-        hipLaunchKernelGGL((k_attn_prefill<64, KV>), grid, dim3(256), 0, dev->stream, q, k_cache, v_cache, out, n, pos0,
-                           n_heads, n_kv_heads, cache_stride, scale);
+template <int HD, class T, int KVP, int QP, int PP>
+static void launch_attn_mfma(candy_hip_device *dev, const float *q, const T *kparts, const T *vparts, int64_t part_stride, float *out, int n,
+                             int pos0, int n_heads, int n_kv_heads, int64_t cache_stride, float scale, _Float16 *xh_out) {
+    // Two key groups per workgroup (64 queries, alternate tiles of 32 keys) where the launch lasts as long as its longest
+    // walk; 128 queries and one group where there are workgroups enough to fill the chip twice over.
+    // 64 queries per workgroup and two groups of wavefronts on alternate tiles of 32 keys, because a launch lasts as long
+    // as its longest walk; 128 queries where the tiles of an f32 cache (96 or 128 KB for two steps) leave a CU room for
+    // one workgroup and there are more than two of the small ones per CU.  us, 64 / 128 queries: head_dim 64, f32 cache,
+    // 32 heads, 700 tokens 30.6 / 36.5, 1500 95 / 75; head_dim 128 512 tokens 29.4 / 34.3, 1024 60.4 / 61.7, 2048 180 / 133;
+    // fp16 cache, head_dim 64, 1500 38.3 / 44.2.  (One group: 1500 91, 2048 147.)
+    const int64_t small = (int64_t)n_heads * ((n + 63) / 64);
+    const int form = dev->opt.prefill_attention_groups;
+#define CANDY_ATTN(QH, KG)                                                                                                            \
+    do {                                                                                                                              \
+        const int tiles = (n + 32 * QH - 1) / (32 * QH);                                                                              \
+        hipLaunchKernelGGL((k_attn_prefill_mfma<HD, T, KVP, QP, PP, QH, KG>), dim3((unsigned)(n_heads * tiles)), dim3(64 * QH * KG),  \
+                           0, dev->stream, q, kparts, vparts, part_stride, cache_stride, out, n, pos0, n_heads, n_heads / n_kv_heads, \
+                           tiles, scale, xh_out);                                                                                     \
+    } while (0)
+    if (form == 1) CANDY_ATTN(4, 1);
+    else if (form == 2 || KVP == 1 || small <= 2 * (int64_t)dev->num_cus) CANDY_ATTN(2, 2);
+    else CANDY_ATTN(4, 2);
+#undef CANDY_ATTN
 }
 
 // The matrix-core kernel can leave its output as the fp16 image of the quantized rows instead of f32 (no separate
 // quantize launch in front of an o projection that runs on the fp16 tiles).
-bool attn_prefill_writes_half(const candy_hip_device *dev, int head_dim) {
-    return head_dim == 128 && !dev->opt.prefill_attention_valu && dev->opt.prefill_fold_split_sums;
+bool attn_prefill_writes_half(const candy_hip_device *dev) {
+    return !dev->opt.prefill_attention_valu && dev->opt.prefill_fold_split_sums;
 }
 
-int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cache, const void *v_cache, bool kv_f16,
+int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cache, const void *v_cache, bool kv_f16, void *parts,
                         float *out, int n, int pos0, int n_heads, int n_kv_heads, int head_dim, int64_t cache_stride,
                         float scale, _Float16 *xh_out) {
     CANDY_REQUIRE(head_dim == 64 || head_dim == 128, "head_dim must be 64 or 128");
     CANDY_REQUIRE(n > 0 && pos0 >= 0 && n_heads % n_kv_heads == 0, "invalid attention shape");
-    CANDY_REQUIRE(!xh_out || attn_prefill_writes_half(dev, head_dim), "internal: this attention kernel writes f32 only");
-    if (kv_f16)
-        launch_attn_prefill_kv(dev, q, (const _Float16 *)k_cache, (const _Float16 *)v_cache, out, n, pos0, n_heads,
-                               n_kv_heads, head_dim, cache_stride, scale, xh_out);
-    else
-        launch_attn_prefill_kv(dev, q, (const float *)k_cache, (const float *)v_cache, out, n, pos0, n_heads, n_kv_heads,
-                               head_dim, cache_stride, scale, xh_out);
+    CANDY_REQUIRE(!xh_out || attn_prefill_writes_half(dev), "internal: this attention kernel writes f32 only");
+    const float *kf = (const float *)k_cache, *vf = (const float *)v_cache;
+    const _Float16 *kh = (const _Float16 *)k_cache, *vh = (const _Float16 *)v_cache;
+    if (dev->opt.prefill_attention_valu) {  // comparison runs
+        const dim3 grid((unsigned)n_heads, (unsigned)((n + 31) / 32));
+#define CANDY_VALU(HD, KV, K, V)                                                                                              \
+    hipLaunchKernelGGL((k_attn_prefill<HD, KV>), grid, dim3(256), 0, dev->stream, q, K, V, out, n, pos0, n_heads, n_kv_heads, \
+                       cache_stride, scale)
+        if (head_dim == 64 && kv_f16) CANDY_VALU(64, _Float16, kh, vh);
+        else if (head_dim == 64) CANDY_VALU(64, float, kf, vf);
+        else if (kv_f16) CANDY_VALU(128, _Float16, kh, vh);
+        else CANDY_VALU(128, float, kf, vf);
+#undef CANDY_VALU
+    } else if (kv_f16) {
+        if (head_dim == 64)
+            launch_attn_mfma<64, _Float16, 1, 3, 2>(dev, q, kh, vh, 0, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
+        else
+            launch_attn_mfma<128, _Float16, 1, 2, 2>(dev, q, kh, vh, 0, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
+    } else {
+        // the rope launch has left the new rows' parts; those of the positions in front may be another layer's
+        if (pos0 > 0)
+            if (int rc = launch_kv_parts(dev, kf, vf, parts, 0, pos0, n_kv_heads, head_dim, cache_stride)) return rc;
+        const int64_t ps = (int64_t)n_kv_heads * cache_stride;
+        const __bf16 *pb = (const __bf16 *)parts;
+        const _Float16 *ph = (const _Float16 *)parts;
+        if (head_dim == 64)
+            launch_attn_mfma<64, __bf16, 3, 3, 3>(dev, q, pb, pb + 3 * ps, ps, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
+        else
+            launch_attn_mfma<128, _Float16, 2, 2, 2>(dev, q, ph, ph + 2 * ps, ps, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
+    }
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }

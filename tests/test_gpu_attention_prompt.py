@@ -1,0 +1,72 @@
+"""Prompt attention on the matrix cores against the vector-ALU kernel, at the edges of its tiles: one-layer models whose
+feed-forward is switched off (zero weights), so that the hidden rows are x + Wo . q8(attention)."""
+import numpy as np
+import pytest
+
+from candy_amd import hip, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = hip.Device(0)
+    yield d
+    d.close()
+
+
+def one_layer(dev, heads, kv_heads, head_dim, max_pos):
+    d = heads * head_dim
+    cfg = dict(n_layers=1, d_model=d, n_heads=heads, n_kv_heads=kv_heads, head_dim=head_dim, d_ffn=256, vocab=256, max_pos=max_pos,
+               rms_eps=1e-5, rope_base=10000.0)
+    model, kd, f = hip.Llama(dev, **cfg), kv_heads * head_dim, synth.Q8_0
+    scale = synth.unit_scale(f)
+    for i, (kind, rows, cols) in enumerate(((hip.W_Q, d, d), (hip.W_K, kd, d), (hip.W_V, kd, d), (hip.W_O, d, d), (hip.W_GATE, 256, d),
+                                            (hip.W_UP, 256, d), (hip.W_HEAD, 256, d), (hip.W_EMBED, 256, d))):
+        layer = -1 if kind in (hip.W_HEAD, hip.W_EMBED) else 0
+        # q and k wide enough that the weights of a row differ by orders of magnitude
+        model.set_qweight(kind, layer, dev.qtensor(f, rows, cols, synth.random_weight(f, rows, cols, 50 + i, scale * (2 if i < 2 else 1))))
+    model.set_qweight(hip.W_DOWN, 0, dev.qtensor(f, d, 256, np.zeros(synth.weight_nbytes(f, d, 256), np.uint8)))
+    for kind, layer in ((hip.W_ATTN_NORM, 0), (hip.W_FFN_NORM, 0), (hip.W_OUT_NORM, -1)):
+        model.set_norm(kind, layer, np.ones(d, np.float32))
+    return model
+
+
+# (heads, kv heads, head_dim): shared kv heads; heads that do not divide over the XCDs; no sharing; and a head count with
+# which a long prompt takes the 128-query form
+SHAPES = [(8, 2, 64), (6, 2, 128), (4, 4, 64), (32, 4, 64), (8, 8, 128)]
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("heads,kv_heads,head_dim", SHAPES)
+def test_tiles_edges_against_the_vector_kernel(dev, heads, kv_heads, head_dim, f16):
+    lengths = [(1, 0), (31, 1), (32, 0), (33, 0), (64, 0), (65, 63), (130, 64), (300, 97)] + ([(1100, 1061)] if heads == 32 else [])
+    model = one_layer(dev, heads, kv_heads, head_dim, 1104)
+    if f16:
+        model.set_kv_f16(True)
+    rng = np.random.default_rng(heads * head_dim)
+    for n, cut in lengths:  # the whole prompt, and (cut > 0) the same in two passes
+        tokens = [int(t) for t in rng.integers(0, 256, n)]
+        got = {}
+        try:
+            for valu in (1, 0):
+                dev.set_option("prefill.attention_valu", valu)
+                model.prefill(tokens, 0, want_logits=False)
+                got[valu] = model.prompt_hidden(n)
+                if cut and not valu:
+                    model.prefill(tokens[:cut], 0, want_logits=False)
+                    model.prefill(tokens[cut:], cut, want_logits=False)
+                    got["cut"] = model.prompt_hidden(n - cut)
+        finally:
+            dev.set_option("prefill.attention_valu", 0)
+        # The two kernels agree to about 1e-6; a level of the quantizer behind them that falls the other way for it is
+        # 1/127 of its block's range in one of K = heads * head_dim products of random sign: 1/127/sqrt(K) of the largest
+        # result per level, and a few of a row's levels may move.
+        bar = 8 / 127 / np.sqrt(heads * head_dim)
+        top = np.max(np.abs(got[1]))
+        assert np.max(np.abs(got[0] - got[1])) <= bar * top, (n, "whole")
+        assert np.mean(np.abs(got[0] - got[1])) <= 1e-4 * top, (n, "whole, mean")
+        if cut:
+            # (below 256 rows and above it the projections round differently: fp16 operands, 3e-4 per contraction)
+            mixed = n >= 256
+            assert np.max(np.abs(got["cut"] - got[1][cut:])) <= (bar + 4e-3 if mixed else bar) * top, (n, cut)
