@@ -1,13 +1,16 @@
 // bfloat16 weights [rows, cols]: upload, row gather and the contraction y = epilogue(x . W^T).
 //   k_dense_mv      one activation row: every weight row is streamed once by one wavefront, the activations wait in LDS
 //                   (bfloat16 or f32 activations; HBM-bound).  Optional prologue: the norms in front of the contraction.
-//   k_dense_mm      prompt batches, bfloat16 activations: v_mfma_f32_16x16x32_bf16 over LDS tiles filled by direct
-//                   global-to-LDS loads, two stages; optionally split along K
+//   k_dense_mm      prompt batches of up to 64 rows, bfloat16 activations: v_mfma_f32_16x16x32_bf16 over LDS tiles filled
+//                   by direct global-to-LDS loads, two stages; optionally split along K
+//   k_dense_big     longer prompts: the same with tiles of 128 .. 256 x 128 or 256, fragments read a half stage ahead
 //   k_dense_mm_f32  prompt batches, f32 activations: v_mfma_f32_16x16x4_f32, weights widened exactly
 // Prompt batches also come with block-diagonal weights, and with their rows dealt to experts (GroupedRows).
 // Weights are stored with both sides padded to multiples of 64 by zeros, so no kernel has a ragged edge in K, and the
 // padded rows come out as epilogue(0) = 0.  (No counterpart in the reference, which has no bfloat16.)
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 #include "dense.h"
 
@@ -198,16 +201,16 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, con
 }
 
 // ------------------------------------------------------------------ prompt batches, bfloat16
-// Tile: BN = 128 weight rows x BM activation rows, 64 values of K per stage.  A row of a stage is 128 bytes = eight
+// Tile: BN = 128 weight rows x BM = 64 activation rows, 64 values of K per stage.  A row of a stage is 128 bytes = eight
 // 16-byte chunks; chunk c of row r sits in slot c ^ ((r >> 1) & 7), so that the 16 rows a fragment read touches spread
 // over all banks.  A direct load writes 64 consecutive 16-byte slots, so the permutation is in the addresses it reads.
 // GROUPED: the row tiles come from a list in device memory (of BM rows at most each), one expert's weights per tile.
-template <int BM, int EPI, bool GROUPED>
+template <int EPI, bool GROUPED>
 __global__ __launch_bounds__(256, 2) void k_dense_mm(const bf16 *__restrict__ W, const bf16 *__restrict__ X, void *__restrict__ yv,
                                                      int M, int Np, int ld, int ldx, int k_slice, int64_t ldy, int n_store,
                                                      size_t split_stride, int m_tiles, int n_tiles, int block_rows, const EpiArgs ea,
                                                      const GroupedRows gr) {
-    constexpr int BN = 128, BK = 64, ROWS = BN + BM, LOADS = ROWS / 32;
+    constexpr int BN = 128, BM = 64, BK = 64, ROWS = BN + BM, LOADS = ROWS / 32;
     constexpr int TN = 4, TM = BM / 32;
     __shared__ __align__(16) u32x4v s[2][ROWS * 8];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -289,6 +292,205 @@ __global__ __launch_bounds__(256, 2) void k_dense_mm(const bf16 *__restrict__ W,
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
         int m = m0 + wm - BN + j * 16 + r16;
+        if (m >= M) continue;
+        if (GROUPED) m = perm[m];
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+            const int n = n0 + wn + i * 16 + 4 * g;
+            f32x4 z = acc[i][j];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[e] = epilogue<EPI>(z[e], ea);
+            if (to_act(EPI)) {
+                if (n < n_store) *(bf16x4 *)((bf16 *)yv + (size_t)m * ldy + n) = __builtin_convertvector(z, bf16x4);
+            } else if (EPI == EPI_NONE) {
+                float *y = (float *)yv + blockIdx.y * split_stride + (size_t)m * ldy + n;
+                if (n + 3 < n_store && (ldy & 3) == 0) *(f32x4 *)y = z;
+                else
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < n_store) y[e] = z[e];
+            } else {
+                float *y = (float *)yv + (size_t)m * ldy + n;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < n_store) y[e] = z[e];
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------ prompt batches, bfloat16, large tiles
+// Tile: BN weight rows x BM activation rows, 64 values of K per stage, one workgroup of eight wavefronts (WN x WM) per CU;
+// a stage lies in LDS as in k_dense_mm.  What bounds it: the chip's power (the clock falls from 2.4 to 2.0 - 2.2 GHz) and, per
+// step of 256 x 256, 2 050 of 3 200 cycles of matrix instructions; without the loads the steps take 83 %, without the LDS
+// reads 91 % of the time.  Against two workgroups per CU of 128 x 128 tiles whose four wavefronts read all fragments of a
+// half stage and then multiply: a wavefront's tile is up to twice as large, so that a fragment read meets more matrix
+// instructions (an eighth to a quarter fewer LDS reads); the fragments of the next half stage are read while this one is
+// multiplied; a stage's loads are requested when its place is free and have a step (two with three stages) to arrive.
+// us, 128 x 128 -> the tile big_tile() picks: 2000 rows, 14336 x 4096 260 -> 215, 5120 x 4096 128 -> 91, 4096 x 4096 79 -> 72,
+// 4096 x 14336 248 -> 207; 512 rows, 14336 x 4096 80 -> 72, 4096 x 14336 79 -> 67.  The 32x32x16 instruction (same reads, half
+// the instructions) is 4 - 7 % slower, stages of 32 values with five of them in LDS no faster (fewer cycles, lower clock).
+struct BigArgs {
+    const bf16 *W, *X;           // from the tile's first rows and this workgroup's first value of K on
+    int64_t w_values, x_values;  // readable from there
+    const int *perm;             // grouped: the tile's rows
+    int x_div;
+    int rows, ld, ldx, n_it;     // activation rows, stages
+};
+constexpr int big_stages(int rows) { return 3 * rows * 128 <= 160 * 1024 ? 3 : 2; }
+
+// The products of one tile whose wavefronts hold TM fragments of 16 activation rows each, every WM-th from `wm` on.
+template <int BN, int WN, int TN, int TM, int TMAX, bool GROUPED>
+__device__ __forceinline__ void big_products(const BigArgs &a, u32x4v *s, f32x4 (&acc)[TN][TMAX], int wave, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+    constexpr int WM = 8 / WN, BK = 64, ROWS = BN + TM * WM * 16;
+    constexpr int PIECES = ROWS / 8, LOADS = (PIECES + 7) / 8;  // wavefront loads of 1 KB per stage, per wavefront
+    constexpr int STAGES = big_stages(ROWS);
+    // A wavefront load takes eight rows of one matrix through a buffer descriptor: rows past the matrix come as zeros, and
+    // the step along K is a scalar offset.  (Loads of the global_load_lds form count as LDS reads to the compiler's wait
+    // counting: every fragment read behind one would wait for all of them.)
+    auto describe = [](const bf16 *p, int64_t values) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, values >= 1ll << 31 ? -1 : (int)(uint32_t)(values * 2), 0x00027000);
+    };
+    const __amdgpu_buffer_rsrc_t rw = describe(a.W, a.w_values), rx = describe(a.X, a.x_values);
+    uint32_t off[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int piece = min(wave + 8 * i, PIECES - 1);  // a spare load repeats the last piece
+        const int r = piece * 8 + (lane >> 3);
+        const int c = (lane & 7) ^ ((r >> 1) & 7);
+        int row = r < BN ? r : r - BN;
+        if (GROUPED && r >= BN) row = a.perm[min(row, a.rows - 1)] / a.x_div;
+        off[i] = (uint32_t)row * (uint32_t)(r < BN ? a.ld : a.ldx) * 2 + c * 16;
+    }
+    int k_off = 0;
+    auto load = [&](int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int piece = min(wave + 8 * i, PIECES - 1);
+            auto *to = (__attribute__((address_space(3))) void *)(s + stage * ROWS * 8 + piece * 64);
+            if (8 * i + 7 < BN / 8) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, to, 16, off[i], k_off, 0, 0);
+            else if (8 * i >= BN / 8) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, to, 16, off[i], k_off, 0, 0);
+            else if (piece < BN / 8) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, to, 16, off[i], k_off, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, to, 16, off[i], k_off, 0, 0);
+        }
+        k_off += BK * 2;
+    };
+    const int wn = (wave / WM) * (BN / WN), wm = BN + (wave % WM) * 16;
+    const int r16 = lane & 15, g = lane >> 4;
+    const int sw = (r16 >> 1) & 7;
+    struct Frags { bf16x8 a[TN], b[TM]; };
+    auto read = [&](Frags &f, int stage, int kk) __attribute__((always_inline)) {
+        const u32x4v *p = s + stage * ROWS * 8 + r16 * 8 + ((kk * 4 + g) ^ sw);
+#pragma unroll
+        for (int i = 0; i < TN; ++i) f.a[i] = __builtin_bit_cast(bf16x8, p[(wn + i * 16) * 8]);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) f.b[j] = __builtin_bit_cast(bf16x8, p[(wm + j * WM * 16) * 8]);
+    };
+    auto multiply = [&](const Frags &f) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // s_waitcnt in the form the compiler's own counting sees: no LDS reads left, all vector loads or a stage's in flight
+    constexpr int ARRIVED = 0x0070, ARRIVED_BUT_ONE = 0x0070 | (LOADS & 15) | (LOADS >> 4) << 14;
+    const int n_it = a.n_it;
+    load(0);
+    if (n_it > 1) load(1);
+    if (n_it > 1) __builtin_amdgcn_s_waitcnt(ARRIVED_BUT_ONE);
+    else __builtin_amdgcn_s_waitcnt(ARRIVED);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    Frags f0, f1;
+    read(f0, 0, 0);
+    if (STAGES == 3 && n_it > 2) load(2);
+    int cur = 0, nxt = 1, last = 2;  // stage in use, the next one, and (three stages) the one behind that
+    // What a step does is fixed at compile time, so that the compiler's counts of reads in flight are exact.  fill: a
+    // further stage is requested; left: a stage is in flight behind the next one when that one's arrival is waited for
+    auto step = [&](auto fill, auto left, auto more) __attribute__((always_inline)) {
+        read(f1, cur, 1);
+        multiply(f0);
+        if (more) {
+            __builtin_amdgcn_s_waitcnt(left ? ARRIVED_BUT_ONE : ARRIVED);  // this stage is read, and the next one is there
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            read(f0, nxt, 0);
+            if (fill) load(cur);
+        }
+        multiply(f1);
+        const int was = cur;
+        cur = nxt;
+        nxt = STAGES == 3 ? last : was;
+        last = was;
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    int it = 0;
+    for (; it + STAGES < n_it; ++it) step(yes, std::bool_constant<STAGES == 3>{}, yes);
+    if (STAGES == 3 && it + 2 < n_it) { step(no, yes, yes); ++it; }
+    for (; it + 1 < n_it; ++it) step(no, no, yes);
+    step(no, no, no);
+#endif
+}
+
+template <int BN, int BM, int WN, int EPI, bool GROUPED>
+__global__ __launch_bounds__(512, 2) void k_dense_big(const bf16 *__restrict__ W, const bf16 *__restrict__ X, void *__restrict__ yv, int M, int Np,
+                                                      int ld, int ldx, int k_slice, int64_t ldy, int n_store, size_t split_stride, int m_tiles,
+                                                      int n_tiles, int block_rows, const EpiArgs ea, const GroupedRows gr) {
+    constexpr int WM = 8 / WN, TN = BN / WN / 16, TMAX = BM / WM / 16;
+    static_assert(BN % (16 * WN) == 0 && TMAX == 4, "whole fragments, four of them along the activation rows");
+    constexpr int most = std::max(std::max(big_stages(BN + BM / 4) * (BN + BM / 4), big_stages(BN + BM / 2) * (BN + BM / 2)),
+                                  std::max(big_stages(BN + BM / 4 * 3) * (BN + BM / 4 * 3), big_stages(BN + BM) * (BN + BM)));
+    __shared__ __align__(16) u32x4v s[most * 8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int n0, m0 = 0;
+    const int *perm = nullptr;
+    if (GROUPED) {
+        // expert by expert, an XCD taking neighbours; within one, its row tiles of one weight tile are neighbours
+        const int total = *gr.n_tiles * n_tiles, per = total >> 3, full = per << 3;
+        int t = blockIdx.x;
+        if (t >= total) return;
+        if (t < full) t = (t & 7) * per + (t >> 3);
+        GroupTile tile = gr.tiles[t / n_tiles];
+        const int local = t - tile.tile0 * n_tiles, nt = local / tile.of_expert;
+        n0 = nt * BN;
+        tile = gr.tiles[tile.tile0 + local - nt * tile.of_expert];
+        W += (size_t)tile.expert * Np * ld;
+        perm = gr.perm + tile.first;
+        M = tile.count;
+    } else {
+        int t = blockIdx.x;
+        const int total = m_tiles * n_tiles, per = total >> 3, full = per << 3;
+        if (t < full) t = (t & 7) * per + (t >> 3);
+        n0 = t / m_tiles * BN;
+        m0 = t % m_tiles * BM;
+    }
+    if (block_rows) X += (size_t)(n0 / block_rows) * ld;
+    const int kbeg = blockIdx.y * k_slice, kend = min(kbeg + k_slice, ld);
+    f32x4 acc[TN][TMAX];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TMAX; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int rows = min(M - m0, BM);
+    const BigArgs a{W + (size_t)n0 * ld + kbeg, X + (size_t)m0 * ldx + kbeg, (int64_t)(Np - n0) * ld - kbeg,
+                    GROUPED ? (int64_t)1 << 40 : (int64_t)(M - m0) * ldx - kbeg, perm, GROUPED ? gr.x_div : 1, rows, ld, ldx, (kend - kbeg) / 64};
+    // a tile of fewer rows takes as many quarters as it fills: the wavefronts share them fragment by fragment
+    switch ((rows + BM / 4 - 1) / (BM / 4)) {
+    case 1: big_products<BN, WN, TN, 1, TMAX, GROUPED>(a, s, acc, wave, lane); break;
+    case 2: big_products<BN, WN, TN, 2, TMAX, GROUPED>(a, s, acc, wave, lane); break;
+    case 3: big_products<BN, WN, TN, 3, TMAX, GROUPED>(a, s, acc, wave, lane); break;
+    default: big_products<BN, WN, TN, 4, TMAX, GROUPED>(a, s, acc, wave, lane); break;
+    }
+    const int r16 = lane & 15, g = lane >> 4, wn = (wave / WM) * (BN / WN);
+#pragma unroll
+    for (int j = 0; j < TMAX; ++j) {
+        int m = m0 + (j * WM + wave % WM) * 16 + r16;
         if (m >= M) continue;
         if (GROUPED) m = perm[m];
 #pragma unroll
@@ -456,40 +658,117 @@ int launch_dense_norm(candy_hip_device *dev, const DenseLaunch &L, const NormArg
     return L.f32 ? launch_mv<float>(dev, L, s, nv, np) : launch_mv<bf16>(dev, L, s, nv, np);
 }
 
-template <int BM>
+// A contraction's tile and how it is split along K.  big false: k_dense_mm, 128 x 64.
+struct MmPlan {
+    bool big = false;
+    int bn = 128, bm = 64, splits = 1;
+};
+struct BigTile {
+    int bn, bm;
+    float step;  // us a step of 64 values takes with every CU at work
+};
+constexpr BigTile BIG_TILES[] = {{256, 256, 1.52f}, {224, 256, 1.38f}, {192, 256, 1.24f}, {160, 256, 1.10f}, {128, 256, 0.92f},
+                                 {256, 128, 0.89f}, {192, 128, 0.74f}, {128, 128, 0.57f}};
+
+// The tile and split with the shortest time by the steps a CU has to take one after the other: rounds of workgroups x
+// steps x the step's measured time, plus a pass over the copies of a split (written here, read by the launch behind).
+// Over twelve shapes of 300 .. 4096 rows this finds the fastest of the tiles measured or one within 3 % of it.
+// row_tiles(bm): tiles along the activation rows.  few: of the tiles with 128 or 256 weight rows only; even: whose weight
+// rows divide `rows`.
+template <class RowTiles>
+static MmPlan big_tile(const candy_hip_device *dev, int64_t rows, int64_t K, RowTiles row_tiles, int64_t out_bytes, int max_splits, bool few,
+                       bool even) {
+    MmPlan best;
+    best.big = true;
+    float best_us = 1e30f;
+    for (const BigTile &t : BIG_TILES) {
+        if ((few && t.bn != 128 && t.bn != 256) || (even && rows % t.bn)) continue;
+        const int64_t tiles = row_tiles(t.bm) * ((rows + t.bn - 1) / t.bn);
+        for (int sp = 1; sp <= max_splits; ++sp) {
+            const int64_t steps = (K / 64 + sp - 1) / sp;
+            if (sp > 1 && steps < 8) break;
+            const float us = (float)((tiles * sp + dev->num_cus - 1) / dev->num_cus * steps) * t.step +
+                             (float)(sp - 1) * (float)out_bytes * 4e-7f;
+            if (us < best_us) {
+                best_us = us;
+                best.bn = t.bn;
+                best.bm = t.bm;
+                best.splits = sp;
+            }
+        }
+    }
+    return best;
+}
+
+template <int EPI, bool GROUPED, class... Args>
+static void launch_big(const MmPlan &p, dim3 g, hipStream_t stream, Args... args) {
+#define CANDY_BIG(BN, BM, WN)                                                                                       \
+    if (p.bn == BN && p.bm == BM) {                                                                                 \
+        hipLaunchKernelGGL((k_dense_big<BN, BM, WN, EPI, GROUPED>), g, dim3(512), 0, stream, args...);              \
+        return;                                                                                                     \
+    }
+    if constexpr (!GROUPED && (EPI == EPI_NONE || EPI == EPI_RELU2)) {
+        CANDY_BIG(224, 256, 2)
+        CANDY_BIG(192, 256, 2)
+        CANDY_BIG(160, 256, 2)
+        CANDY_BIG(192, 128, 4)
+    }
+    if constexpr (!GROUPED) {
+        CANDY_BIG(256, 256, 2)
+        CANDY_BIG(128, 256, 2)
+    }
+    CANDY_BIG(256, 128, 4)
+    CANDY_BIG(128, 128, 4)
+#undef CANDY_BIG
+}
+
 static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
-    const int m_tiles = (L.m + BM - 1) / BM, n_tiles = (int)((L.w->rows_pad + 127) / 128);
+    const int K = (int)L.w->ld;
+    const int64_t rows = L.w->rows_pad;
+    MmPlan p;
+    if (L.m <= 64) {
+        if (L.partial) {
+            // two workgroups fit a CU; a slice keeps at least 512 values of K
+            const int64_t room = 2 * (int64_t)dev->num_cus / ((rows + 127) / 128);
+            p.splits = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(room, 8), K / 512));
+        }
+    } else {
+        // block-diagonal: no tile may reach into a second block
+        const int64_t blocks = L.block_rows ? rows / L.block_rows : 1;
+        p = big_tile(dev, rows / blocks, K, [&](int bm) { return (L.m + bm - 1) / bm * blocks; }, (int64_t)L.m * rows * 4, L.partial ? 8 : 1,
+                     L.epi != EPI_NONE && L.epi != EPI_RELU2, L.block_rows != 0);
+    }
+    const int m_tiles = (L.m + p.bm - 1) / p.bm, n_tiles = (int)((rows + p.bn - 1) / p.bn);
     const int64_t tiles = (int64_t)m_tiles * n_tiles;
     CANDY_REQUIRE(tiles <= 0x7FFFFFFF, "matrix too large");
-    const int K = (int)L.w->ld;
-    int splits = 1;
     void *y = L.y;
     int64_t ldy = L.ldy, n_store = L.n_store;
     size_t stride = 0;
-    if (L.partial) {
-        // two workgroups fit a CU; a slice keeps at least 512 values of K
-        const int64_t room = 2 * (int64_t)dev->num_cus / tiles;
-        splits = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(room, 8), K / 512));
-        if (splits > 1) {
-            ldy = n_store = L.w->rows_pad;
-            stride = (size_t)L.m * ldy;
-            if (int rc = splitk_workspace(dev, stride * splits * sizeof(float), &y)) return rc;
-        }
+    if (p.splits > 1) {
+        ldy = n_store = rows;
+        stride = (size_t)L.m * ldy;
+        if (int rc = splitk_workspace(dev, stride * p.splits * sizeof(float), &y)) return rc;
     }
-    const int k_slice = (int)pad64((K + splits - 1) / splits);
-    splits = (K + k_slice - 1) / k_slice;
+    const int k_slice = (int)pad64((K + p.splits - 1) / p.splits);
+    const int splits = (K + k_slice - 1) / k_slice;
     if (L.partial) {
         L.partial->p = (const float *)y;
         L.partial->copies = splits;
         L.partial->stride = stride;
         L.partial->ld = (int)ldy;
     }
-    const dim3 g((unsigned)tiles, (unsigned)splits), b(256);
+    const dim3 g((unsigned)tiles, (unsigned)splits);
     const EpiArgs ea{L.scale, L.cap};
     const bf16 *W = (const bf16 *)L.w->data, *X = (const bf16 *)L.x;
-#define CANDY_MM(EPI)                                                                                                     \
-    hipLaunchKernelGGL((k_dense_mm<BM, EPI, false>), g, b, 0, dev->stream, W, X, y, L.m, (int)L.w->rows_pad, K, (int)L.ldx,   \
-                       k_slice, ldy, (int)n_store, stride, m_tiles, n_tiles, L.block_rows, ea, GroupedRows{})
+#define CANDY_MM(EPI)                                                                                                                 \
+    do {                                                                                                                              \
+        if (p.big)                                                                                                                    \
+            launch_big<EPI, false>(p, g, dev->stream, W, X, y, L.m, (int)rows, K, (int)L.ldx, k_slice, ldy, (int)n_store, stride,     \
+                                   m_tiles, n_tiles, L.block_rows, ea, GroupedRows{});                                                \
+        else                                                                                                                          \
+            hipLaunchKernelGGL((k_dense_mm<EPI, false>), g, dim3(256), 0, dev->stream, W, X, y, L.m, (int)rows, K, (int)L.ldx,        \
+                               k_slice, ldy, (int)n_store, stride, m_tiles, n_tiles, L.block_rows, ea, GroupedRows{});                \
+    } while (0)
     switch (L.epi) {
     case EPI_RELU2: CANDY_MM(EPI_RELU2); break;
     case EPI_CAP: CANDY_MM(EPI_CAP); break;
@@ -501,19 +780,40 @@ static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
     return CANDY_HIP_OK;
 }
 
+// 64-row tiles while experts have few rows each.  From 96 on tiles of 256 x 128, the longer ones' share in a launch that
+// reads every expert's weights either way: us, up / down, 128 x 128 tiles -> these, unevenly dealt rows: 64 experts of 1408 at
+// width 2048, 1024 tokens of 6 107 / 105 -> 107 / 102, 2048 134 / 149 -> 142 / 147; 16 of 2048 at 4096, 1024 tokens of 4
+// 144 / 128 -> 133 / 121, 2048 199 / 201 -> 194 / 196.  (256 rows: 127 / 114 and 220 / 194 in the second and last.)
+int grouped_tile_rows(int experts, int64_t slots, int64_t widest_x) {
+    // an activation row's place is a 32-bit offset in the large tiles' loads
+    return slots < 96 * (int64_t)experts || slots * widest_x * 2 > 0xFFFFFFFFll ? 64 : 128;
+}
+
 // Rows dealt to experts: the grid has room for max_tiles row tiles, workgroups past the list's end leave at once.
-template <int BM>
 static int launch_mm_grouped(candy_hip_device *dev, const DenseLaunch &L) {
     const GroupedRows &gr = *L.group;
-    const int n_tiles = (gr.expert_rows + 127) / 128, K = (int)L.w->ld;
+    const int K = (int)L.w->ld;
+    MmPlan p;
+    if (gr.tile_rows > 64) {
+        p.big = true;
+        p.bm = 128;
+        p.bn = gr.expert_rows > 128 ? 256 : 128;
+    }
+    const int n_tiles = (gr.expert_rows + p.bn - 1) / p.bn;
     const int64_t tiles = (int64_t)gr.max_tiles * n_tiles;
     CANDY_REQUIRE(tiles <= 0x7FFFFFFF, "matrix too large");
-    const dim3 g((unsigned)tiles), b(256);
+    const dim3 g((unsigned)tiles);
     const EpiArgs ea{L.scale, L.cap};
     const bf16 *W = (const bf16 *)L.w->data, *X = (const bf16 *)L.x;
-#define CANDY_MMG(EPI)                                                                                                       \
-    hipLaunchKernelGGL((k_dense_mm<BM, EPI, true>), g, b, 0, dev->stream, W, X, L.y, L.m, gr.expert_rows, K, (int)L.ldx, K,  \
-                       L.ldy, (int)L.n_store, (size_t)0, 0, n_tiles, 0, ea, gr)
+#define CANDY_MMG(EPI)                                                                                                                    \
+    do {                                                                                                                                  \
+        if (p.big)                                                                                                                        \
+            launch_big<EPI, true>(p, g, dev->stream, W, X, L.y, L.m, gr.expert_rows, K, (int)L.ldx, K, L.ldy, (int)L.n_store, (size_t)0, \
+                                  0, n_tiles, 0, ea, gr);                                                                                 \
+        else                                                                                                                              \
+            hipLaunchKernelGGL((k_dense_mm<EPI, true>), g, dim3(256), 0, dev->stream, W, X, L.y, L.m, gr.expert_rows, K, (int)L.ldx, K,   \
+                               L.ldy, (int)L.n_store, (size_t)0, 0, n_tiles, 0, ea, gr);                                                  \
+    } while (0)
     if (L.epi == EPI_RELU2) CANDY_MMG(EPI_RELU2);
     else CANDY_MMG(EPI_NONE);
 #undef CANDY_MMG
@@ -534,9 +834,8 @@ int launch_dense(candy_hip_device *dev, const DenseLaunch &L) {
         CANDY_REQUIRE((L.epi == EPI_NONE || L.epi == EPI_RELU2) && !L.partial && !L.block_rows && L.group->expert_rows % 64 == 0 &&
                           w->rows % L.group->expert_rows == 0 && L.group->max_tiles <= 65535,
                       "internal: grouped contraction");
-        if (!L.f32 && L.group->tile_rows == 128) return launch_mm_grouped<128>(dev, L);
-        CANDY_REQUIRE(L.group->tile_rows == 64, "internal: row tiles of 64");
-        if (!L.f32) return launch_mm_grouped<64>(dev, L);
+        CANDY_REQUIRE(L.group->tile_rows == 64 || (!L.f32 && L.group->tile_rows == 128), "internal: row tiles");
+        if (!L.f32) return launch_mm_grouped(dev, L);
     }
     if (L.partial) {
         L.partial->p = (const float *)L.y;
@@ -548,7 +847,7 @@ int launch_dense(candy_hip_device *dev, const DenseLaunch &L) {
         const MvShape s = mv_shape(dev, L.n_store);
         return L.f32 ? launch_mv<float>(dev, L, s) : launch_mv<bf16>(dev, L, s);
     }
-    if (!L.f32) return L.m <= 64 ? launch_mm<64>(dev, L) : launch_mm<128>(dev, L);
+    if (!L.f32) return launch_mm(dev, L);
     const dim3 g((unsigned)(out_rows / 64), (unsigned)(L.group ? L.group->max_tiles : (L.m + 63) / 64)), b(256);
     CANDY_REQUIRE((L.m + 63) / 64 <= 65535, "prompt too long for one pass");
     const EpiArgs ea{L.scale, L.cap};

@@ -372,9 +372,6 @@ int check_expert_spec(const candy_hip_expert_spec &s, int d) {
     return CANDY_HIP_OK;
 }
 
-static int deal_rows(const candy_hip_expert_spec &s, int n, bool f32) {
-    return !f32 && (int64_t)n * s.top >= 96 * (int64_t)s.n_experts ? 128 : 64;
-}
 static int deal_max_tiles(const candy_hip_expert_spec &s, int n, int rows) {
     const int64_t count = (int64_t)n * s.top;
     // an expert with members has at most one tile that is not full
@@ -385,7 +382,7 @@ size_t expert_list_ints(const candy_hip_expert_spec &s, int n) { return deal_per
 
 int launch_experts_prompt(candy_hip_device *dev, const ExpertLayer &A, int n) {
     const candy_hip_expert_spec &s = A.s;
-    const int rows = deal_rows(s, n, A.f32);
+    const int rows = A.f32 ? 64 : grouped_tile_rows(s.n_experts, (int64_t)n * s.top, std::max<int64_t>(A.ld_act, pad64(s.d_ff)));
     hipLaunchKernelGGL(k_route, dim3((unsigned)((n + ROUTE_T - 1) / ROUTE_T)), dim3(64 * ROUTE_W), route_lds(s), dev->stream, A.x, A.ldx,
                        (const bf16 *)A.w.router->data, (int)A.w.router->ld, s.n_experts, s.top, n, A.ids, A.weights);
     CANDY_LAUNCH_CHECK();
