@@ -4,7 +4,8 @@
 // first rope_dims dimensions of a head (pairs i, i + rope_dims / 2), the rest passes.
 //   k_rope_cache            projected q and k rows -> rotated q, and the new rows of both caches
 //   k_window_attn_row       one wavefront per (query, head), vector ALU: f32 activations, prompt and decode
-//   k_window_attn_prompt    bfloat16 prompts on the matrix cores, 64 queries of one head per workgroup
+//   k_window_attn_tiles     bfloat16 prompts on the matrix cores, 64 queries of one head per workgroup: rows of 64 and 128
+//   k_window_attn_prompt    the same for the other row widths
 //   k_window_attn_decode    bfloat16 decode: rotation, cache append and attention of the new token, split over the window
 //   k_window_attn_merge     its splits and the sink -> the head's output
 // Scores, weights and sums are f32; in the bfloat16 prompt kernel the weights meet V as the sum of two bfloat16 parts
@@ -14,6 +15,7 @@
 #include <cmath>
 #include <vector>
 
+#include "attention_tiles.h"
 #include "dense.h"
 
 namespace candy {
@@ -325,6 +327,65 @@ __global__ __launch_bounds__(256, 2) void k_window_attn_prompt(const WindowArgs 
     }
     if (h == a.H - 1)
         for (int i = a.H * a.dim + g; i < a.out_cols; i += 4) out[(size_t)qi * a.ldo + i] = (bf16)0.0f;
+}
+
+// Rows of 64 and 128 values: direct loads, two groups of wavefronts on alternate tiles of 32 keys, 32 queries per wavefront
+// (attention_tiles.h).  The kernel above spends its time converting layouts: V goes to LDS value pair by value pair, and a
+// fragment of K or V meets one query tile.  us, 32 heads of 128 over 8 with a cap, 2000 tokens, window 1536: 112 -> 84; two
+// thirds of that is the vector ALU (exp, rcp and exp per score), the rest the matrix cores.
+template <int DP, bool CAP>
+__global__ __launch_bounds__(256, 2) void k_window_attn_tiles(const WindowArgs a, const bf16 *__restrict__ q, const bf16 *__restrict__ kc,
+                                                              const bf16 *__restrict__ vc, bf16 *__restrict__ out, int n, int pos0, int q_tiles) {
+    typedef Bf16Tiles<DP, DP> Tiles;
+    __shared__ __align__(16) uint4 s[Tiles::LDS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    int h, tile;
+    attn_tile(blockIdx.x, a.H, q_tiles, h, tile);
+    const int kvh = h / (a.H / a.G), i0 = tile * Tiles::QT, wi = i0 + 32 * (wave & 1);
+    const bf16 *kh = kc + (size_t)kvh * a.kv_stride, *vh = vc + (size_t)kvh * a.kv_stride;
+    const int last = pos0 + min(i0 + Tiles::QT, n) - 1, first = max(0, pos0 + i0 - a.window + 1);
+    // capped: c_out tanh(y) = c_out - 2 c_out / (1 + exp(2 y)), like tanh_fast; else a negative scale turns the queries
+    const float c_in = CAP ? a.scale / a.cap * (2.0f * LOG2E) : tile_scale(a.scale * LOG2E), c_out = a.cap * LOG2E;
+    const bool turn = !CAP && a.scale < 0.0f;
+    Tiles T;
+    const bool sink = a.sink && wave < 2;  // the sink is in the first group's state
+    for (int t = 0; t < 2; ++t) {
+        T.m[t] = sink ? a.sink[h] * LOG2E : LOW;
+        T.l[t] = sink && g == 0 ? 1.0f : 0.0f;
+    }
+    bf16x8 qf[2][Tiles::KS];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int ks = 0; ks < Tiles::KS; ++ks) {
+            qf[t][ks] = *(const bf16x8 *)(q + ((size_t)min(wi + 16 * t + r16, n - 1) * a.H + h) * DP + ks * 32 + g * 8);
+            if (turn) qf[t][ks] = -qf[t][ks];
+        }
+    T.run(s, tid, pos0 + wi, first & ~(Tiles::R - 1), last, a.window, qf,
+          [&](int p, int c) { return kh + (size_t)p * DP + c * 8; }, [&](int p, int c) { return vh + (size_t)p * DP + c * 8; },
+          [&](float z) { return CAP ? __builtin_amdgcn_rcpf(-1.0f - __builtin_amdgcn_exp2f(z * c_in)) : z; }, CAP ? 2.0f * c_out : c_in,
+          CAP ? c_out : 0.0f);
+    if (wave >= 2) return;
+    for (int t = 0; t < 2; ++t) {
+        const int qi = wi + 16 * t + r16;
+        if (qi >= n) continue;
+        const float inv = 1.0f / T.l[t];
+        bf16 *dst = out + (size_t)qi * a.ldo + (size_t)h * a.dim;
+#pragma unroll
+        for (int d = 0; d < DP / 16; ++d) {
+            const int c = d * 16 + 4 * g;
+            const f32x4 v = T.o[t][d] * inv;
+            if ((a.dim & 3) == 0) {
+                if (c < a.dim) *(bf16x4 *)(dst + c) = __builtin_convertvector(v, bf16x4);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (c + j < a.dim) dst[c + j] = (bf16)v[j];
+            }
+        }
+        if (h == a.H - 1)
+            for (int i = a.H * a.dim + g; i < a.out_cols; i += 4) out[(size_t)qi * a.ldo + i] = (bf16)0.0f;
+    }
 }
 
 // ------------------------------------------------------------------ decode, bfloat16
@@ -687,11 +748,24 @@ int launch_window_prompt(candy_hip_device *dev, const WindowAttn &A, int n, int 
         hipLaunchKernelGGL((k_window_attn_prompt<DP>), g, b, 0, dev->stream, a, (const bf16 *)A.q, (const bf16 *)A.k_cache,        \
                            (const bf16 *)A.v_cache, (bf16 *)A.out, n, pos0);                                                      \
         break
+    // direct loads place 16-byte pieces in eights; the other widths keep the kernel that stages through registers (rows of
+    // 128, us: 112 there, 84 with direct loads)
+#define CANDY_WT(DP)                                                                                                              \
+    case DP:                                                                                                                      \
+        if (a.cap > 0.0f)                                                                                                          \
+            hipLaunchKernelGGL((k_window_attn_tiles<DP, true>), dim3(g.x * g.y), b, 0, dev->stream, a, (const bf16 *)A.q,          \
+                               (const bf16 *)A.k_cache, (const bf16 *)A.v_cache, (bf16 *)A.out, n, pos0, (int)g.y);                \
+        else                                                                                                                       \
+            hipLaunchKernelGGL((k_window_attn_tiles<DP, false>), dim3(g.x * g.y), b, 0, dev->stream, a, (const bf16 *)A.q,         \
+                               (const bf16 *)A.k_cache, (const bf16 *)A.v_cache, (bf16 *)A.out, n, pos0, (int)g.y);                \
+        break
     switch (A.row) {
-        CANDY_WP(32); CANDY_WP(64); CANDY_WP(96); CANDY_WP(128); CANDY_WP(192); CANDY_WP(256);
+        CANDY_WT(64); CANDY_WT(128);
+        CANDY_WP(32); CANDY_WP(96); CANDY_WP(192); CANDY_WP(256);
     default: return fail(CANDY_HIP_ERR_UNSUPPORTED, "no attention kernel for rows of %d values", A.row);
     }
 #undef CANDY_WP
+#undef CANDY_WT
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }

@@ -11,6 +11,7 @@
 //   k_attn_prefill      the same on the vector ALU (comparison runs)
 #include <cstdlib>
 
+#include "attention_tiles.h"
 #include "blocks.h"
 #include "internal.h"
 
@@ -277,31 +278,6 @@ __device__ __forceinline__ float4v mfma16(half8 a, half8 b, float4v c) { return 
 __device__ __forceinline__ float4v mfma16(PartVec<__bf16>::v8 a, PartVec<__bf16>::v8 b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-// four rows of a 16-bit matrix in LDS, transposed: lane l of 16 receives column l (lane l points at row l / 4, values
-// 4 (l % 4) .. + 3)
-__device__ __forceinline__ half4h lds_columns(const _Float16 *p) {
-    typedef short s4 __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(half4h, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)p));
-}
-__device__ __forceinline__ PartVec<__bf16>::v4 lds_columns(const __bf16 *p) {
-    typedef short s4 __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(PartVec<__bf16>::v4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)p));
-}
-
-// over the four lanes 16 apart that share a query
-__device__ __forceinline__ float quad16_max(float v) {
-    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float quad16_sum(float v) {
-    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 template <int HD, class T, int KVP, int QP, int PP, int QH, int KG>
 __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * KG == 4 ? 1 : 2) void k_attn_prefill_mfma(const float *__restrict__ q, const T *__restrict__ kparts, const T *__restrict__ vparts,
                                                               int64_t part_stride, int64_t head_stride, float *__restrict__ out, int n, int pos0,
@@ -318,19 +294,8 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int qh = wave % QH, kg = wave / QH;
-    // The workgroups of neighbouring heads (which share K and V) on one XCD, the longest walks first.
     int head, qt0;
-    {
-        const int id = blockIdx.x;
-        if ((n_heads & 7) == 0) {
-            const int per = n_heads >> 3, s = id >> 3;
-            head = (id & 7) * per + s % per;
-            qt0 = q_tiles - 1 - s / per;
-        } else {
-            head = id % n_heads;
-            qt0 = q_tiles - 1 - id / n_heads;
-        }
-    }
+    attn_tile(blockIdx.x, n_heads, q_tiles, head, qt0);
     const int i0 = qt0 * QT;
     const T *kh = kparts + (size_t)(head / group) * head_stride, *vh = vparts + (size_t)(head / group) * head_stride;
     const int n_keys = pos0 + min(i0 + QT, n);  // positions the tile's last query may see
@@ -363,9 +328,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[t][d] = float4v{0.f, 0.f, 0.f, 0.f};
 
-    // Rows of a tile lie end to end in LDS; piece c of row r sits in slot c ^ turn(r), which keeps both the fragment
-    // reads of K (16 rows, one piece each) and the column reads of V (8 rows, two pieces each) off each other's banks.
-    auto turn = [](int r) { return HD == 128 ? ((r & 7) << 1) | ((r >> 3) & 1) : (((r >> 1) & 3) << 1) | ((r >> 3) & 1); };
+    auto turn = [](int r) { return v_turn(C, r); };  // K and V alike
     auto stage = [&](int p0, int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int a = 0; a < 2 * KVP; ++a) {
@@ -379,7 +342,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
             }
         }
     };
-    const int k_turn = turn(r16), v_row = 4 * g + (r16 >> 2), v_turn = turn(v_row), v_half = (r16 & 3) >> 1;
+    const int k_at = turn(r16), v_row = 4 * g + (r16 >> 2), v_at = turn(v_row), v_half = (r16 & 3) >> 1;
     const int n_steps = (n_keys + R - 1) / R;
     stage(0, 0);
     for (int step = 0; step < n_steps; ++step) {
@@ -402,7 +365,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-                for (int p = 0; p < KVP; ++p) kf[ks][p] = __builtin_bit_cast(v8, base[p * ARR + (kt * 16 + r16) * C + ((ks * 4 + g) ^ k_turn)]);
+                for (int p = 0; p < KVP; ++p) kf[ks][p] = __builtin_bit_cast(v8, base[p * ARR + (kt * 16 + r16) * C + ((ks * 4 + g) ^ k_at)]);
 #pragma unroll
             for (int sum = TOP - 1; sum >= 0; --sum)  // the smallest products first
 #pragma unroll
@@ -455,7 +418,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             v8 vf[KVP];
-            const int at = v_row * C + ((2 * d + v_half) ^ v_turn);
+            const int at = v_row * C + ((2 * d + v_half) ^ v_at);
 #pragma unroll
             for (int p = 0; p < KVP; ++p) {
                 const T *a = (const T *)(base + (KVP + p) * ARR + at) + (r16 & 1) * 4;
