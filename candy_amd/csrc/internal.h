@@ -218,6 +218,9 @@ int launch_mmq_i8(candy_hip_device *dev, const candy_hip_qtensor *w, const int8_
 bool mmq_f16_big_covers(const candy_hip_qtensor *w, int64_t m, int min_m = 0);
 int launch_mmq_f16_big(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y,
                        const float *res = nullptr);
+// mmq_f16_rows.hip: the same for up to 128 rows, K dealt to the wavefronts of a workgroup
+bool mmq_f16_rows_covers(const candy_hip_qtensor *w, int64_t m);
+int launch_mmq_f16_rows(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res);
 // Two or three projections of the same activations on one grid (every tensor but the last: a multiple of 128 rows).
 bool mmq_f16_group_covers(const candy_hip_qtensor *const *ws, int count, int64_t m);
 int launch_mmq_f16_group(candy_hip_device *dev, const candy_hip_qtensor *const *ws, float *const *ys, int count,

@@ -1,0 +1,218 @@
+// 33 to 128 activation rows of Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 on the fp16 matrix cores, K dealt to wavefronts:
+// y[m, N] = x[m, K] . W^T with the operands of mmq_f16.hip.
+//
+// With so few rows a contraction should last as long as its weights take from memory, but in the role-split tiles of
+// mmq_f16.hip a step of K waits for a barrier and for the slower role (at 128 rows 1500 to 2200 cycles for 500 of matrix
+// instructions), 128-row tiles are N / 128 x splits workgroups, and the split's copies are added by a launch of its own.
+// Here nobody waits for anybody: a workgroup owns 16, 32 or 48 weight rows and all activation rows, and each of its eight
+// wavefronts takes every eighth super-block of K: weight blocks by direct loads into its own slice of LDS, dequantized into
+// matrix operands in registers, activation fragments straight from their image, each loaded by one wavefront of the
+// workgroup.  The wavefronts' sums meet in LDS at the end, in the order of the wavefronts (reproducible).  Kernel us, 77
+// rows, 11008 x 4096, before (with the split sum) -> now: Q4_K 22.8 + 4.5 -> 20.6, Q8_0 35.1 + 4.5 -> 24.0, Q4_0 33.4 + 4.5 ->
+// 21.2, Q5_K 31.5 + 4.5 -> 25.1; 2048 x 1024 Q8_0 13.0 + 4.1 -> 5.7.  What bounds it: the activations, which every CU reads
+// (655 KB here, 10 us), then the weights (48 MB of Q8_0, 8 us), half overlapped.
+#include <cstdlib>
+
+#include "f16_weights.h"
+#include "internal.h"
+
+namespace candy {
+
+template <class F>
+constexpr bool staged() { return F::BLOCK % 16 == 0; }
+
+template <class F, int RF, int MF>
+constexpr size_t lds_bytes() {
+    const size_t sums = (size_t)8 * RF * MF * 1024, slices = staged<F>() ? (size_t)8 * 1024 * ((RF * F::BLOCK / 16 + 3) / 4) : 0;
+    return sums > slices ? sums : slices;
+}
+
+template <class F, int RF, int MF>
+__global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restrict__ W, const _Float16 *__restrict__ xh, float *y,
+                                                         const float *res, int M, int N, int K) {
+    constexpr bool STAGED = staged<F>();
+    extern __shared__ __align__(16) uint8_t smem_raw[];
+    float4v *sums = (float4v *)smem_raw;  // [wave][RF][MF][lane]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, c = lane >> 4;
+    const int n0 = blockIdx.x * (16 * RF), first = wave;
+    const int count = ((K >> 8) - first + 7) >> 3;  // super-blocks first, first + 8, ... of this wavefront (may be none)
+    const size_t rb = (size_t)(K >> 8) * F::BLOCK, xrow = (size_t)(K >> 5) * 512;
+    const _Float16 *xl = xh + r16 * 32 + (F::RUN16 ? (c >> 1) * 512 + (c & 1) * 16 : c * 8);
+    constexpr int HALF = F::RUN16 ? 8 : 512;  // from a step's first chunk of K to its second
+
+    float4v acc[RF][MF];
+#pragma unroll
+    for (int i = 0; i < RF; ++i)
+#pragma unroll
+        for (int t = 0; t < MF; ++t) acc[i][t] = float4v{0.f, 0.f, 0.f, 0.f};
+    // A super-block of the workgroup's rows comes into the wavefront's own slice of LDS, 16-byte pieces in the order they
+    // lie in memory (requests of a lane for its own few bytes of a row cost the cache a line each: Q8_0 9 us per 16 rows of
+    // 4096 and CU, against 3 for the bytes themselves); from there to registers, which frees the slice for the next one.
+    // Q6_K blocks (210 bytes) are not whole pieces: their requests go straight to registers.
+    constexpr int PIECES = F::BLOCK / 16, IT = (RF * 16 * PIECES + 63) / 64;
+    uint4 *slice = (uint4 *)smem_raw + wave * (IT * 64);
+    uint32_t from[STAGED ? IT : 1];
+    if constexpr (STAGED) {
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int e = it * 64 + lane, row = min(e / PIECES, RF * 16 - 1);
+            from[it] = (uint32_t)(min(n0 + row, N - 1) - n0) * (uint32_t)rb + (uint32_t)(e % PIECES) * 16;
+        }
+    }
+    const uint8_t *w0 = W + (size_t)n0 * rb;
+    auto request = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int it = 0; it < IT; ++it)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(w0 + (size_t)sb * F::BLOCK + from[it]),
+                                             (__attribute__((address_space(3))) void *)(slice + it * 64), 16, 0, 0);
+    };
+    if (count > 0) {
+        typename F::Raw raw[STAGED ? 1 : 2][RF];
+        half8 xf[2][MF];
+        auto load_w = [&](int sb, int u) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < RF; ++i)
+                F::load(STAGED ? (const uint8_t *)slice + (16 * i + r16) * F::BLOCK
+                               : W + (size_t)min(n0 + 16 * i + r16, N - 1) * rb + (size_t)sb * F::BLOCK, c, raw[u][i]);
+        };
+        auto load_x = [&](int step, int h) __attribute__((always_inline)) {  // step: in 64s along K
+            const _Float16 *p = xl + (size_t)step * 1024 + h * HALF;
+#pragma unroll
+            for (int t = 0; t < MF; ++t) xf[h][t] = *(const half8 *)(p + t * xrow);
+        };
+        auto contract = [&](int sb, int u, int sb_next) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                load_x(sb * 4 + g, 1);
+                half8 a[RF][2];
+#pragma unroll
+                for (int i = 0; i < RF; ++i) {
+                    int k0, k1;
+                    F::dequant(raw[u][i], g, c, a[i][0], a[i][1], k0, k1);
+                }
+#pragma unroll
+                for (int t = 0; t < MF; ++t)
+#pragma unroll
+                    for (int i = 0; i < RF; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][0], xf[0][t], acc[i][t], 0, 0, 0);
+                load_x(g == 3 ? sb_next * 4 : sb * 4 + g + 1, 0);
+#pragma unroll
+                for (int t = 0; t < MF; ++t)
+#pragma unroll
+                    for (int i = 0; i < RF; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][1], xf[1][t], acc[i][t], 0, 0, 0);
+            }
+        };
+        if constexpr (STAGED) {
+            request(first);
+            load_x(first * 4, 0);
+            for (int k = 0; k < count; ++k) {
+                const int sb = first + 8 * k;
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the slice has landed
+                load_w(sb, 0);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and is in registers
+                if (k + 1 < count) request(sb + 8);
+                contract(sb, 0, k + 1 < count ? sb + 8 : sb);
+            }
+        } else {
+            load_w(first, 0);
+            if (count > 1) load_w(first + 8, 1);
+            load_x(first * 4, 0);
+            for (int k = 0; k < count; k += 2) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if (k + u >= count) break;
+                    const int sb = first + 8 * (k + u);
+                    contract(sb, u, k + u + 1 < count ? sb + 8 : sb);
+                    if (k + u + 2 < count) load_w(sb + 16, u);
+                }
+            }
+        }
+    }
+    __syncthreads();  // the slices are consumed
+#pragma unroll
+    for (int i = 0; i < RF; ++i)
+#pragma unroll
+        for (int t = 0; t < MF; ++t) sums[((wave * RF + i) * MF + t) * 64 + lane] = acc[i][t];
+    __syncthreads();
+    for (int f = wave; f < RF * MF; f += 8) {
+        const int m = (f % MF) * 16 + r16, n = n0 + (f / MF) * 16 + 4 * c;  // activation row; weight rows n .. n + 3
+        float4v s = sums[f * 64 + lane];
+#pragma unroll
+        for (int k = 1; k < 8; ++k) s += sums[(k * RF * MF + f) * 64 + lane];
+        if (m >= M) continue;
+        float *dst = y + (size_t)m * N + n;
+        const float *r = res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
+        if (n + 3 < N && (N & 3) == 0) {
+            if (r) s = *(const float4v *)r + s;
+            *(float4v *)dst = s;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (n + j < N) dst[j] = r ? r[j] + s[j] : s[j];
+        }
+    }
+}
+
+static int fragments(int64_t m) { return m <= 48 ? 3 : m <= 64 ? 4 : m <= 80 ? 5 : m <= 96 ? 6 : 8; }
+
+// 16-row weight fragments per workgroup with which one round of workgroups serves every row, 0: none (a second round would
+// read the activations again; wider workgroups than these have no registers for their sums)
+template <class F>
+static int weight_fragments(const candy_hip_device *dev, int64_t rows, int mf) {
+    for (int rf = 1; rf <= 3 && (rf < 3 || mf <= (staged<F>() ? 6 : 4)) && rf * mf <= 18; ++rf)
+        if ((rows + 16 * rf - 1) / (16 * rf) <= dev->num_cus) return rf;
+    return 0;
+}
+
+template <class F, int RF, int MF>
+static int launch_rf(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res) {
+    constexpr size_t smem = lds_bytes<F, RF, MF>();
+    void (*kern)(const uint8_t *, const _Float16 *, float *, const float *, int, int, int) = k_mmq_f16_rows<F, RF, MF>;
+    CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3((unsigned)((w->rows + 16 * RF - 1) / (16 * RF))), dim3(512), smem, dev->stream,
+                       (const uint8_t *)w->data, xh, y, res, (int)m, (int)w->rows, (int)w->cols);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+
+template <class F>
+static int launch_fmt(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res) {
+    const int mf = fragments(m), rf = weight_fragments<F>(dev, w->rows, mf);
+#define CANDY_RF(MF)                                                                      \
+    if (mf == MF) {                                                                       \
+        if (rf == 1) return launch_rf<F, 1, MF>(dev, w, xh, m, y, res);                   \
+        if (rf == 2) return launch_rf<F, 2, MF>(dev, w, xh, m, y, res);                   \
+        if constexpr (MF <= (staged<F>() ? 6 : 4))                                      \
+            if (rf == 3) return launch_rf<F, 3, MF>(dev, w, xh, m, y, res);               \
+    }
+    CANDY_RF(3) CANDY_RF(4) CANDY_RF(5) CANDY_RF(6) CANDY_RF(8)
+#undef CANDY_RF
+    return CANDY_HIP_ERR_UNSUPPORTED;
+}
+
+// A workgroup reads every activation, so this is for activations that a CU takes in (about 65 KB a us when all CUs read)
+// in less than the tiles of mmq_f16.hip lose to their barriers and to the launch that adds their K halves; and for weight
+// rows that give at least half of the CUs a workgroup.  us, tiles + split sum / this kernel: 786 KB (96 x 4096 values),
+// 11008 x 4096 Q4_K 24.0 + 4.6 / 22.7, Q8_0 35.8 + 4.6 / 25.9, 4096 x 4096 14.9 + 4.2 / 15.0 and 15.9 + 4.2 / 18.3; 1049 KB
+// (128 rows) 4096 x 4096 16.1 + 4.3 / 19.2 and 16.9 + 4.2 / 23.2; 4096 x 14336 at 77 rows 24.0 + 4.1 / 39.7.  Q6_K, whose blocks
+// are not staged, 5632 long: 540 KB 13.2 + 4.1 / 16.3, 720 KB 13.0 + 4.0 / 19.0.
+bool mmq_f16_rows_covers(const candy_hip_qtensor *w, int64_t m) {
+    const bool q6k = w->fmt == CANDY_HIP_Q6_K;
+    if (!q6k && ((uintptr_t)w->data & 15) != 0) return false;  // whole pieces
+    return m <= 128 && w->rows >= 2048 && (double)fragments(m) * 32.0 * (double)w->cols <= (q6k ? 700e3 : 800e3);
+}
+
+// CANDY_HIP_ERR_UNSUPPORTED: more rows than one round of workgroups takes
+int launch_mmq_f16_rows(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res) {
+    CANDY_REQUIRE(m >= 1 && m <= 128 && w->cols % 256 == 0, "internal: shape of the fp16 contraction");
+    switch (w->fmt) {
+    case CANDY_HIP_Q4_K: return launch_fmt<BigQ4K>(dev, w, xh, m, y, res);
+    case CANDY_HIP_Q5_K: return launch_fmt<BigQ5K>(dev, w, xh, m, y, res);
+    case CANDY_HIP_Q6_K: return launch_fmt<BigQ6K>(dev, w, xh, m, y, res);
+    case CANDY_HIP_Q8_0: return launch_fmt<BigQ8_0>(dev, w, xh, m, y, res);
+    case CANDY_HIP_Q4_0: return launch_fmt<BigQ4_0<false>>(dev, w, xh, m, y, res);
+    case CANDY_HIP_Q4_0_GGML: return launch_fmt<BigQ4_0<true>>(dev, w, xh, m, y, res);
+    default: return CANDY_HIP_ERR_UNSUPPORTED;
+    }
+}
+
+}  // namespace candy
