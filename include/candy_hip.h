@@ -123,7 +123,7 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *                                         0: a launch of its own sums them)
  *   "prefill.attention_valu"     0        comparison runs: prompt attention on the vector ALU
  *   "prefill.attention_groups"   0        comparison runs: matrix-core prompt attention with one (1) or two (2) groups of
- *                                         wavefronts per query tile that take alternate key tiles (0: two, of 32 or 64
+ *                                         wavefronts per query tile that take alternate key tiles (0: two, with 64 or 128
  *                                         queries by the size of the grid)
  * A decoder whose step has been captured into a graph notices a later candy_hip_set_option on its device and captures
  * the step again at its next decode call.
