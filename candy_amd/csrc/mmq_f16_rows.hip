@@ -191,14 +191,14 @@ static int launch_fmt(candy_hip_device *dev, const candy_hip_qtensor *w, const _
 
 // A workgroup reads every activation, so this is for activations that a CU takes in (about 65 KB a us when all CUs read)
 // in less than the tiles of mmq_f16.hip lose to their barriers and to the launch that adds their K halves; and for weight
-// rows that give at least half of the CUs a workgroup.  us, tiles + split sum / this kernel: 786 KB (96 x 4096 values),
-// 11008 x 4096 Q4_K 24.0 + 4.6 / 22.7, Q8_0 35.8 + 4.6 / 25.9, 4096 x 4096 14.9 + 4.2 / 15.0 and 15.9 + 4.2 / 18.3; 1049 KB
-// (128 rows) 4096 x 4096 16.1 + 4.3 / 19.2 and 16.9 + 4.2 / 23.2; 4096 x 14336 at 77 rows 24.0 + 4.1 / 39.7.  Q6_K, whose blocks
-// are not staged, 5632 long: 540 KB 13.2 + 4.1 / 16.3, 720 KB 13.0 + 4.0 / 19.0.
+// rows that give at least half of the CUs a workgroup.  us of a call, tiles / this kernel, 655 KB (80 x 4096 values): Q4_K
+// 4096 x 4096 19.6 / 14.6, 11008 x 4096 26.5 / 22.0, Q8_0 4096 x 4096 21.6 / 18.1; kernels alone at 786 KB: Q8_0 15.9 + 4.2 / 18.3,
+// at 1049 KB 16.9 + 4.2 / 23.2, 4096 x 14336 at 77 rows 24.0 + 4.1 / 39.7.  Q6_K, whose blocks are not staged: 393 KB 4096 x 4096
+// 18.6 / 14.7, 11008 x 4096 30.9 / 28.1; kernels alone at 524 KB 30.9 + 4.4 / 32.8, 5632 long at 540 KB 13.2 + 4.1 / 16.3.
 bool mmq_f16_rows_covers(const candy_hip_qtensor *w, int64_t m) {
     const bool q6k = w->fmt == CANDY_HIP_Q6_K;
     if (!q6k && ((uintptr_t)w->data & 15) != 0) return false;  // whole pieces
-    return m <= 128 && w->rows >= 2048 && (double)fragments(m) * 32.0 * (double)w->cols <= (q6k ? 700e3 : 800e3);
+    return m <= 128 && w->rows >= 2048 && (double)fragments(m) * 32.0 * (double)w->cols <= (q6k ? 450e3 : 700e3);
 }
 
 // CANDY_HIP_ERR_UNSUPPORTED: more rows than one round of workgroups takes
