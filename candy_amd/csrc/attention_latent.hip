@@ -1,9 +1,7 @@
 // Latent attention: a position's cache row is a normed latent c and a rotated key part shared by all heads (layout and
 // equations: include/candy_hip.h).
 //   k_latent_rows          projected rows -> normed query latents, normed latent and rotated key part into the cache
-//   k_latent_tiles         bfloat16 prompts on the matrix cores over expanded keys and values, 64 queries of a head per workgroup:
-//                          widths in whole 64s
-//   k_latent_prompt        the same for widths in between
+//   k_latent_prompt        bfloat16 prompts on the matrix cores over expanded keys and values, 64 queries of a head per workgroup
 //   k_latent_prompt_row    one wavefront per (query, head), vector ALU: f32 prompts, and heads too wide for the tiles
 //   k_latent_query         decode: queries contracted with Wuk, rotated part turned, the new cache row appended
 //   k_latent_decode        bfloat16 decode on the matrix cores: 16 heads against the cached rows, split over the positions
@@ -14,7 +12,6 @@
 #include <algorithm>
 #include <vector>
 
-#include "attention_tiles.h"
 #include "dense.h"
 
 namespace candy {
@@ -244,93 +241,6 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt(const LatentArgs a, co
     }
     if (h == a.H - 1)
         for (int i = a.H * a.vdim + g; i < a.out_cols; i += 4) out[(size_t)qi * a.ldo + i] = (bf16)0.0f;
-}
-
-// Widths that are multiples of 64 as they are: direct loads, two groups of wavefronts on alternate tiles of 32 keys, 32
-// queries per wavefront (attention_tiles.h).  us, 16 heads of 128 + 64 / 128, 2048 tokens: 94 -> 78.
-template <int DK, int DV>
-__global__ __launch_bounds__(256, DK + DV > 320 ? 1 : 2) void k_latent_tiles(const LatentArgs a, const Partial qp, const bf16 *__restrict__ cache,
-                                                         const bf16 *__restrict__ kv, int ldkv, bf16 *__restrict__ out, int n, int pos0, int q_tiles) {
-    typedef Bf16Tiles<DK, DV> Tiles;
-    __shared__ __align__(16) uint4 s[Tiles::LDS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
-    int h, tile;
-    attn_tile(blockIdx.x, a.H, q_tiles, h, tile);
-    const int i0 = tile * Tiles::QT, wi = i0 + 32 * (wave & 1), last = pos0 + min(i0 + Tiles::QT, n) - 1;
-    const bf16 *kh = kv + (size_t)h * a.dim, *vh = kv + (size_t)a.H * a.dim + (size_t)h * a.vdim, *kr = cache + a.kv_p - a.dim;
-    const float sign = a.scale < 0.0f ? -1.0f : 1.0f;
-    Tiles T;
-    const bool sink = a.sink && wave < 2;  // the sink is in the first group's state
-    for (int t = 0; t < 2; ++t) {
-        T.m[t] = sink ? a.sink[h] * LOG2E : LOW;
-        T.l[t] = sink && g == 0 ? 1.0f : 0.0f;
-    }
-    // The queries, projected in f32: every load of a thread is in flight before the first is used, the rotated part goes
-    // through LDS for its partners.
-    bf16x8 qf[2][DK / 32];
-    {
-        f32x4 x[2][DK / 32][2];
-        float *turn = (float *)s;  // rotated part of the workgroup's queries as projected
-        const int ldt = a.rot + 4;
-        for (int c = 0; c < qp.copies; ++c)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const float *src = qp.p + (size_t)c * qp.stride + (size_t)min(wi + 16 * t + r16, n - 1) * qp.ld + h * DK + g * 8;
-#pragma unroll
-                for (int ks = 0; ks < DK / 32; ++ks)
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const f32x4 p = *(const f32x4 *)(src + ks * 32 + 4 * e);
-                        x[t][ks][e] = c ? x[t][ks][e] + p : p;
-                    }
-            }
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int row = 32 * (wave & 1) + 16 * t + r16;
-#pragma unroll
-            for (int ks = 0; ks < DK / 32; ++ks)
-                if (ks * 32 >= a.dim && wave < 2)
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) *(f32x4 *)&turn[row * ldt + ks * 32 - a.dim + g * 8 + 4 * e] = x[t][ks][e];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int row = 32 * (wave & 1) + 16 * t + r16;
-            const size_t qpos = (size_t)(pos0 + min(wi + 16 * t + r16, n - 1)) * a.half;
-#pragma unroll
-            for (int ks = 0; ks < DK / 32; ++ks) {
-                if (ks * 32 >= a.dim) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int j = ks * 32 - a.dim + g * 8 + e, k = j < a.half ? j : j - a.half;
-                        if (j < 2 * a.half) {
-                            const float co = a.cos_t[qpos + k], si = a.sin_t[qpos + k], v = x[t][ks][e >> 2][e & 3];
-                            x[t][ks][e >> 2][e & 3] = j < a.half ? v * co - turn[row * ldt + j + a.half] * si : v * co + turn[row * ldt + k] * si;
-                        }
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) qf[t][ks][e] = (bf16)(x[t][ks][e >> 2][e & 3] * sign);
-            }
-        }
-        __syncthreads();
-    }
-    T.run(s, tid, pos0 + wi, 0, last, 1 << 30, qf,
-          [&](int p, int c) { return (c * 8 < a.dim ? kh + (size_t)p * ldkv : kr + (size_t)p * a.row) + c * 8; },
-          [&](int p, int c) { return vh + (size_t)p * ldkv + c * 8; }, [&](float z) { return z; },
-          tile_scale(a.scale * LOG2E), 0.0f);
-    if (wave >= 2) return;
-    for (int t = 0; t < 2; ++t) {
-        const int qi = wi + 16 * t + r16;
-        if (qi >= n) continue;
-        const float inv = 1.0f / T.l[t];
-        bf16 *dst = out + (size_t)qi * a.ldo + (size_t)h * a.vdim;
-#pragma unroll
-        for (int d = 0; d < DV / 16; ++d) *(bf16x4 *)(dst + d * 16 + 4 * g) = __builtin_convertvector(T.o[t][d] * inv, bf16x4);
-        if (h == a.H - 1)
-            for (int i = a.H * a.vdim + g; i < a.out_cols; i += 4) out[(size_t)qi * a.ldo + i] = (bf16)0.0f;
-    }
 }
 
 // ------------------------------------------------------------------ one wavefront per (query, head) or (head, split)
@@ -792,18 +702,6 @@ int launch_latent_prompt(candy_hip_device *dev, const LatentAttn &A, int n, int 
     CANDY_REQUIRE(A.q.ld % 4 == 0 && A.q.stride % 4 == 0 && ((uintptr_t)A.q.p & 15) == 0, "internal: unaligned queries");
     const int dk = a.dim + a.rot;
     bool done = false;
-    const dim3 tiles((unsigned)(a.H * ((n + 63) / 64)));
-    // direct loads place 16-byte pieces in eights, so these are the widths that need no padding (192 / 128, us: 94 in
-    // k_latent_prompt, 78 here); 256 / 256 would not fit LDS
-#define CANDY_LT(DK, DV)                                                                                                          \
-    if (dk == DK && a.vdim == DV) {                                                                                               \
-        hipLaunchKernelGGL((k_latent_tiles<DK, DV>), tiles, dim3(256), 0, dev->stream, a, A.q, (const bf16 *)A.cache,             \
-                           (const bf16 *)A.kv, (int)A.ukv->rows_pad, (bf16 *)A.out, n, pos0, (n + 63) / 64);                      \
-        CANDY_LAUNCH_CHECK();                                                                                                     \
-        return CANDY_HIP_OK;                                                                                                      \
-    }
-    CANDY_LT(64, 64) CANDY_LT(128, 64) CANDY_LT(128, 128) CANDY_LT(192, 64) CANDY_LT(192, 128) CANDY_LT(256, 128)
-#undef CANDY_LT
     if (dk <= 64) done = prompt_tiles<64>(dev, A, a, n, pos0);
     else if (dk <= 96) done = prompt_tiles<96>(dev, A, a, n, pos0);
     else if (dk <= 128) done = prompt_tiles<128>(dev, A, a, n, pos0);

@@ -104,6 +104,11 @@ struct DenseLaunch {
     int64_t n_store = 0;      // columns written per row: w->rows, or w->rows_pad (the padding comes out as zero)
     // NONE only, optional: the contraction may leave partial copies in the handle's split workspace instead of y
     Partial *partial = nullptr;
+    // with `partial`: as many copies as tiles of 128 x 128 would leave, whichever tile is taken, so that the order of every
+    // sum goes by the shape alone.  For a model that picks experts: at a near tie the last place of a sum picks another
+    // expert, and with it another result row (2048 tokens of 64 experts: on 3 of 40 inputs a value moved by 1 to 2 times the
+    // rows' root mean square when only the copies and the order of the attention's sums had changed).
+    bool steady = false;
     // block-diagonal weights: rows b * block_rows .. belong to block b, whose activations start at column b * w->ld
     // (a multiple of 128).  0: one block
     int block_rows = 0;

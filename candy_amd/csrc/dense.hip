@@ -676,17 +676,17 @@ constexpr BigTile BIG_TILES[] = {{256, 256, 1.52f}, {224, 256, 1.38f}, {192, 256
 // row_tiles(bm): tiles along the activation rows.  few: of the tiles with 128 or 256 weight rows only; even: whose weight
 // rows divide `rows`.
 template <class RowTiles>
-static MmPlan big_tile(const candy_hip_device *dev, int64_t rows, int64_t K, RowTiles row_tiles, int64_t out_bytes, int max_splits, bool few,
-                       bool even) {
+static MmPlan big_tile(const candy_hip_device *dev, int64_t rows, int64_t K, RowTiles row_tiles, int64_t out_bytes, int min_splits,
+                       int max_splits, bool few, bool even) {
     MmPlan best;
     best.big = true;
     float best_us = 1e30f;
     for (const BigTile &t : BIG_TILES) {
         if ((few && t.bn != 128 && t.bn != 256) || (even && rows % t.bn)) continue;
         const int64_t tiles = row_tiles(t.bm) * ((rows + t.bn - 1) / t.bn);
-        for (int sp = 1; sp <= max_splits; ++sp) {
+        for (int sp = min_splits; sp <= max_splits; ++sp) {
             const int64_t steps = (K / 64 + sp - 1) / sp;
-            if (sp > 1 && steps < 8) break;
+            if (sp > min_splits && steps < 8) break;
             const float us = (float)((tiles * sp + dev->num_cus - 1) / dev->num_cus * steps) * t.step +
                              (float)(sp - 1) * (float)out_bytes * 4e-7f;
             if (us < best_us) {
@@ -726,17 +726,20 @@ static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
     const int K = (int)L.w->ld;
     const int64_t rows = L.w->rows_pad;
     MmPlan p;
+    int copies = 1;
+    if (L.partial && (L.m <= 64 || L.steady)) {
+        // two workgroups (of 128 x 64 or 128 x 128) fit a CU; a slice keeps at least 512 values of K
+        const int bm = L.m <= 64 ? 64 : 128;
+        const int64_t room = 2 * (int64_t)dev->num_cus / ((L.m + bm - 1) / bm * ((rows + 127) / 128));
+        copies = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(room, 8), K / 512));
+    }
     if (L.m <= 64) {
-        if (L.partial) {
-            // two workgroups fit a CU; a slice keeps at least 512 values of K
-            const int64_t room = 2 * (int64_t)dev->num_cus / ((rows + 127) / 128);
-            p.splits = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(room, 8), K / 512));
-        }
+        p.splits = copies;
     } else {
         // block-diagonal: no tile may reach into a second block
         const int64_t blocks = L.block_rows ? rows / L.block_rows : 1;
-        p = big_tile(dev, rows / blocks, K, [&](int bm) { return (L.m + bm - 1) / bm * blocks; }, (int64_t)L.m * rows * 4, L.partial ? 8 : 1,
-                     L.epi != EPI_NONE && L.epi != EPI_RELU2, L.block_rows != 0);
+        p = big_tile(dev, rows / blocks, K, [&](int bm) { return (L.m + bm - 1) / bm * blocks; }, (int64_t)L.m * rows * 4, copies,
+                     L.partial && !L.steady ? 8 : copies, L.epi != EPI_NONE && L.epi != EPI_RELU2, L.block_rows != 0);
     }
     const int m_tiles = (L.m + p.bm - 1) / p.bm, n_tiles = (int)((rows + p.bn - 1) / p.bn);
     const int64_t tiles = (int64_t)m_tiles * n_tiles;

@@ -409,7 +409,7 @@ int launch_experts_prompt(candy_hip_device *dev, const ExpertLayer &A, int n) {
     S.ldy = S.n_store = A.w.shared_up->rows_pad;
     if (int rc = launch_dense(dev, S)) return rc;
     S.w = A.w.shared_down; S.x = A.shared_act; S.ldx = A.w.shared_down->ld; S.epi = CANDY_HIP_EPI_NONE; S.y = A.y; S.ldy = A.ldy;
-    S.n_store = A.w.shared_down->rows_pad; S.partial = A.shared;
+    S.n_store = A.w.shared_down->rows_pad; S.partial = A.shared; S.steady = true;
     return launch_dense(dev, S);
 }
 

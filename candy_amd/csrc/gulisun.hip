@@ -198,6 +198,7 @@ int candy_hip_gulisun::layers_forward(Buffers &B, int n, int pos0, const int *po
     auto linear = [&](const candy_hip_dense *w, const void *x, int64_t ldx, void *y, int64_t ldy, Partial *partial) {
         DenseLaunch D;
         D.w = w; D.x = x; D.ldx = ldx; D.f32 = f32; D.m = n; D.y = y; D.ldy = ldy; D.n_store = w->rows_pad; D.partial = partial;
+        D.steady = true;  // every result so far decides which experts a later layer picks
         return D;
     };
     for (const Layer &L : layers) {

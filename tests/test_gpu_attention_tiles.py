@@ -1,5 +1,5 @@
-"""Prompt attention in bfloat16 whose tiles go to LDS by direct loads, at the edges of its tiles: window attention with rows
-of 64 and 128 values, latent attention with keys and values of whole 64s."""
+"""Prompt attention in bfloat16 at the edges of its tiles: window attention with rows of 64 and 128 values, whose tiles go to
+LDS by direct loads, and latent attention with keys and values of whole 64s."""
 import numpy as np
 import pytest
 
@@ -44,7 +44,7 @@ def test_window(dev, heads, kv_heads, dim, window, scale, cap):
             assert rel(device_attention(dev, mx, q, k, s, hip.ACT_BF16, portions), want) < WINDOW_TOL, (s is None, portions)
 
 
-# heads, dim, rotated, values: every pair of widths that has its kernel (rotated parts of 32 and more, also ragged ones)
+# heads, dim, rotated, values: keys and values of whole 64s (rotated parts of 32 and more, also ragged ones)
 LATENT = [(8, 32, 32, 64), (3, 64, 64, 64), (2, 96, 18, 50), (16, 64, 40, 128), (5, 128, 64, 64), (8, 128, 64, 128), (1, 32, 150, 100),
           (4, 192, 64, 128), (2, 32, 224, 128), (2, 256, 0, 128)]
 
