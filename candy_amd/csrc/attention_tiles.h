@@ -73,7 +73,7 @@ struct Bf16Tiles {
     // qf: the wavefront's queries (16 + 16); key(p, c), value(p, c): address of piece c of position p's row; p_first: a multiple of
     // 64; positions up to `last`; wq0: first position of the wavefront's queries; reach: a query sees so many positions back,
     // itself included; the exponent of 2 is mul * raw(z) + add of the product z, with mul > 0, so that the maximum is
-    // taken before the one fma that it is subtracted in.  m and l hold the initial state (second group: none).
+    // taken before the one fma that it is subtracted in.  m (finite) and l hold the initial state (second group: none).
     template <class Key, class Value, class Raw>
     __device__ __forceinline__ void run(uint4 *s, int tid, int wq0, int p_first, int last, int reach, const v8 (&qf)[2][KS], Key key, Value value,
                                         Raw raw, float mul, float add) {

@@ -349,8 +349,11 @@ __global__ __launch_bounds__(256, 2) void k_window_attn_tiles(const WindowArgs a
     const bool turn = !CAP && a.scale < 0.0f;
     Tiles T;
     const bool sink = a.sink && wave < 2;  // the sink is in the first group's state
+    // A maximum starts finite: a query's first tile may be in front of its window altogether, and -infinity less -infinity is
+    // none.  (A sink below LOW has no weight beside any score; one that is no number stays so.)
+    const float at_sink = sink ? a.sink[h] * LOG2E : LOW, m0 = at_sink < LOW ? LOW : at_sink;
     for (int t = 0; t < 2; ++t) {
-        T.m[t] = sink ? a.sink[h] * LOG2E : LOW;
+        T.m[t] = m0;
         T.l[t] = sink && g == 0 ? 1.0f : 0.0f;
     }
     bf16x8 qf[2][Tiles::KS];

@@ -44,6 +44,23 @@ def test_window(dev, heads, kv_heads, dim, window, scale, cap):
             assert rel(device_attention(dev, mx, q, k, s, hip.ACT_BF16, portions), want) < WINDOW_TOL, (s is None, portions)
 
 
+# sinks of -infinity and of the type's lowest value (exp(sink) = 0: heads without one) where a query's first tile of 32 keys is
+# wholly in front of its window, the window within a tile, at its edge and longer
+@pytest.mark.parametrize("dim,window", [(64, 32), (128, 32), (64, 64), (128, 50), (64, 1)])
+def test_window_sink_of_no_weight(dev, dim, window):
+    n, heads = 195, 8
+    rng = np.random.default_rng(window)
+    q = (rng.standard_normal((n, heads, dim)) * 1.5).astype(np.float32)
+    k = (rng.standard_normal((n, 2, dim)) * 1.5).astype(np.float32)
+    sink = np.array([-np.inf, 0.5, -np.inf, -3.4e38, -1e30, -np.inf, -2.0, -3.4e38], np.float32)
+    for cap in (None, 20.0):
+        mx = sm.mixer(heads, 2, dim, window, 2 * (dim // 4), 1000.0, None, 0.1, cap)
+        want = oracle_attention(mx, q.astype(np.float64), k.astype(np.float64), sink, hip.ACT_BF16)
+        assert np.all(np.isfinite(want))
+        for portions in ([n], [31, 2, 32, 63, 67]):
+            assert rel(device_attention(dev, mx, q, k, sink, hip.ACT_BF16, portions), want) < WINDOW_TOL, (cap, portions)
+
+
 # heads, dim, rotated, values: keys and values of whole 64s (rotated parts of 32 and more, also ragged ones)
 LATENT = [(8, 32, 32, 64), (3, 64, 64, 64), (2, 96, 18, 50), (16, 64, 40, 128), (5, 128, 64, 64), (8, 128, 64, 128), (1, 32, 150, 100),
           (4, 192, 64, 128), (2, 32, 224, 128), (2, 256, 0, 128)]
