@@ -115,8 +115,9 @@ struct DenseLaunch {
     const GroupedRows *group = nullptr;  // NONE / SQUARED_RELU, m: rows over all experts
 };
 int launch_dense(candy_hip_device *dev, const DenseLaunch &L);
-// rows per tile (64 or 128) of a list of `slots` bfloat16 rows dealt to experts; widest_x: values between the widest rows read
-int grouped_tile_rows(int experts, int64_t slots, int64_t widest_x);
+// rows per tile (64 or 128) of a list of `slots` bfloat16 rows dealt to experts; widest: values between the widest rows of
+// activations and weights
+int grouped_tile_rows(int experts, int64_t slots, int64_t widest);
 
 // How a contraction of one row deals its weight rows to wavefronts.
 struct MvShape {

@@ -670,27 +670,32 @@ struct BigTile {
 constexpr BigTile BIG_TILES[] = {{256, 256, 1.52f}, {224, 256, 1.38f}, {192, 256, 1.24f}, {160, 256, 1.10f}, {128, 256, 0.92f},
                                  {256, 128, 0.89f}, {192, 128, 0.74f}, {128, 128, 0.57f}};
 
+// The large tiles' loads reach the rows of a tile through 32-bit byte offsets from its first one: all of them within 4 GB.  (Rows
+// of 8 million values and more go to k_dense_mm, whose addresses are pointers.)
+static bool tile_fits(int tile_rows, int64_t ld) { return tile_rows * ld * 2 <= 0xFFFFFFFFll; }
+
 // The tile and split with the shortest time by the steps a CU has to take one after the other: rounds of workgroups x
 // steps x the step's measured time, plus a pass over the copies of a split (written here, read by the launch behind).
 // Over twelve shapes of 300 .. 4096 rows this finds the fastest of the tiles measured or one within 3 % of it.
 // row_tiles(bm): tiles along the activation rows.  few: of the tiles with 128 or 256 weight rows only; even: whose weight
 // rows divide `rows`.
 template <class RowTiles>
-static MmPlan big_tile(const candy_hip_device *dev, int64_t rows, int64_t K, RowTiles row_tiles, int64_t out_bytes, int min_splits,
-                       int max_splits, bool few, bool even) {
+static MmPlan big_tile(int num_cus, int64_t rows, int64_t K, int64_t ldx, RowTiles row_tiles, int64_t out_bytes, int min_splits, int max_splits,
+                       bool few, bool even) {
     MmPlan best;
-    best.big = true;
+    best.splits = min_splits;
     float best_us = 1e30f;
     for (const BigTile &t : BIG_TILES) {
         if ((few && t.bn != 128 && t.bn != 256) || (even && rows % t.bn)) continue;
+        if (!tile_fits(t.bn, K) || !tile_fits(t.bm, ldx)) continue;
         const int64_t tiles = row_tiles(t.bm) * ((rows + t.bn - 1) / t.bn);
         for (int sp = min_splits; sp <= max_splits; ++sp) {
             const int64_t steps = (K / 64 + sp - 1) / sp;
             if (sp > min_splits && steps < 8) break;
-            const float us = (float)((tiles * sp + dev->num_cus - 1) / dev->num_cus * steps) * t.step +
-                             (float)(sp - 1) * (float)out_bytes * 4e-7f;
+            const float us = (float)((tiles * sp + num_cus - 1) / num_cus * steps) * t.step + (float)(sp - 1) * (float)out_bytes * 4e-7f;
             if (us < best_us) {
                 best_us = us;
+                best.big = true;
                 best.bn = t.bn;
                 best.bm = t.bm;
                 best.splits = sp;
@@ -698,6 +703,22 @@ static MmPlan big_tile(const candy_hip_device *dev, int64_t rows, int64_t K, Row
         }
     }
     return best;
+}
+
+// m rows of activations `ldx` apart against `rows` rows of K values
+static MmPlan mm_plan(int num_cus, int m, int64_t rows, int64_t K, int64_t ldx, bool partial, bool steady, bool few, int block_rows) {
+    MmPlan p;
+    if (partial && (m <= 64 || steady)) {
+        // two workgroups (of 128 x 64 or 128 x 128) fit a CU; a slice keeps at least 512 values of K
+        const int bm = m <= 64 ? 64 : 128;
+        const int64_t room = 2 * (int64_t)num_cus / ((m + bm - 1) / bm * ((rows + 127) / 128));
+        p.splits = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(room, 8), K / 512));
+    }
+    if (m <= 64) return p;
+    // block-diagonal: no tile may reach into a second block
+    const int64_t blocks = block_rows ? rows / block_rows : 1;
+    return big_tile(num_cus, rows / blocks, K, ldx, [&](int bm) { return (m + bm - 1) / bm * blocks; }, (int64_t)m * rows * 4, p.splits,
+                    partial && !steady ? 8 : p.splits, few, block_rows != 0);
 }
 
 template <int EPI, bool GROUPED, class... Args>
@@ -725,22 +746,8 @@ static void launch_big(const MmPlan &p, dim3 g, hipStream_t stream, Args... args
 static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
     const int K = (int)L.w->ld;
     const int64_t rows = L.w->rows_pad;
-    MmPlan p;
-    int copies = 1;
-    if (L.partial && (L.m <= 64 || L.steady)) {
-        // two workgroups (of 128 x 64 or 128 x 128) fit a CU; a slice keeps at least 512 values of K
-        const int bm = L.m <= 64 ? 64 : 128;
-        const int64_t room = 2 * (int64_t)dev->num_cus / ((L.m + bm - 1) / bm * ((rows + 127) / 128));
-        copies = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(room, 8), K / 512));
-    }
-    if (L.m <= 64) {
-        p.splits = copies;
-    } else {
-        // block-diagonal: no tile may reach into a second block
-        const int64_t blocks = L.block_rows ? rows / L.block_rows : 1;
-        p = big_tile(dev, rows / blocks, K, [&](int bm) { return (L.m + bm - 1) / bm * blocks; }, (int64_t)L.m * rows * 4, copies,
-                     L.partial && !L.steady ? 8 : copies, L.epi != EPI_NONE && L.epi != EPI_RELU2, L.block_rows != 0);
-    }
+    const MmPlan p = mm_plan(dev->num_cus, L.m, rows, K, L.ldx, L.partial != nullptr, L.steady, L.epi != EPI_NONE && L.epi != EPI_RELU2,
+                             L.block_rows);
     const int m_tiles = (L.m + p.bm - 1) / p.bm, n_tiles = (int)((rows + p.bn - 1) / p.bn);
     const int64_t tiles = (int64_t)m_tiles * n_tiles;
     CANDY_REQUIRE(tiles <= 0x7FFFFFFF, "matrix too large");
@@ -787,9 +794,9 @@ static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
 // reads every expert's weights either way: us, up / down, 128 x 128 tiles -> these, unevenly dealt rows: 64 experts of 1408 at
 // width 2048, 1024 tokens of 6 107 / 105 -> 107 / 102, 2048 134 / 149 -> 142 / 147; 16 of 2048 at 4096, 1024 tokens of 4
 // 144 / 128 -> 133 / 121, 2048 199 / 201 -> 194 / 196.  (256 rows: 127 / 114 and 220 / 194 in the second and last.)
-int grouped_tile_rows(int experts, int64_t slots, int64_t widest_x) {
-    // an activation row's place is a 32-bit offset in the large tiles' loads
-    return slots < 96 * (int64_t)experts || slots * widest_x * 2 > 0xFFFFFFFFll ? 64 : 128;
+int grouped_tile_rows(int experts, int64_t slots, int64_t widest) {
+    // an activation row's place is a 32-bit offset in the large tiles' loads, from the first of all rows, and so is a weight row's
+    return slots < 96 * (int64_t)experts || slots * widest * 2 > 0xFFFFFFFFll || !tile_fits(256, widest) ? 64 : 128;
 }
 
 // Rows dealt to experts: the grid has room for max_tiles row tiles, workgroups past the list's end leave at once.
@@ -1010,6 +1017,13 @@ int candy_hip_dense_matmul(candy_hip_device *dev, const candy_hip_dense *w, cons
     if (int rc = launch_dense(dev, L)) return rc;
     return launch_from_act(dev, f32, L.y, dev_y, m, w->rows, w->rows_pad);
 }
+
+// The rules that choose a tile, for their tests (no device needed): plan[0..3] = large tiles, weight rows, activation rows, splits.
+void candy_test_dense_plan(int num_cus, int m, int64_t rows, int64_t ld, int64_t ldx, int partial, int steady, int few, int block_rows, int *plan) {
+    const candy::MmPlan p = candy::mm_plan(num_cus, m, rows, ld, ldx, partial != 0, steady != 0, few != 0, block_rows);
+    plan[0] = p.big; plan[1] = p.bn; plan[2] = p.bm; plan[3] = p.splits;
+}
+int candy_test_grouped_tile_rows(int experts, int64_t slots, int64_t widest) { return candy::grouped_tile_rows(experts, slots, widest); }
 
 int candy_hip_dense_sweep(candy_hip_device *dev, const candy_hip_dense *const *ws, int n_ws, const float *dev_x, int64_t m,
                           int epilogue, int iters, float *elapsed_ms) {
