@@ -263,7 +263,9 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float *__restrict__ 
 // An f32 operand meets the matrix cores as a sum of parts, each part the rounding of what the parts before it leave:
 //   head_dim 128, f32 cache   two fp16 parts of q, K, V and the weights (22 bits), three products
 //   head_dim 64, f32 cache    three bfloat16 parts (24 bits and f32's range: what the vector ALU had), six products
-//   fp16 cache                K and V are their own single part; q in two fp16 parts (three for head_dim 64), the weights in two
+//   fp16 cache                K and V are their own single part; q and the weights in two fp16 parts, for head_dim 64 in three
+//                             (24 bits and f32's range: a query's row scaled to 2^13 .. 2^14, the weights by 2^15, so that what
+//                             falls below the last part's 2^-24 is 2^-38 of the row's largest value or the largest weight)
 // K and V parts lie in memory as rows like the cache's (k_kv_parts; a fp16 cache is read as it is), so that a tile goes
 // to LDS by direct loads and no workgroup converts what the others of its head convert as well.
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -302,10 +304,24 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
     const int wq0 = pos0 + i0 + 32 * qh;         // first position of this wavefront's 32 queries
 
     // q as the B operand (column = query, 8 consecutive d per lane), scaled for a softmax on powers of two
+    constexpr bool WIDE = KVP == 1 && QP == 3;  // fp16 parts that stand for 32 bits
     v8 qf[2][KS][QP];
+    float q_up[2], q_down[2];  // WIDE: a power of two on the query's row, and its inverse
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const float *qr = q + ((size_t)min(i0 + 32 * qh + 16 * t + r16, n - 1) * n_heads + head) * HD;
+        if (WIDE) {
+            float amax = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const float4 a = *(const float4 *)(qr + ks * 32 + g * 8), b = *(const float4 *)(qr + ks * 32 + g * 8 + 4);
+                amax = fmaxf(amax, fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
+                                         fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w)))));
+            }
+            const int up = min(14 - __builtin_amdgcn_frexp_expf(quad16_max(amax) * (scale * 1.44269504088896341f)), 120);
+            q_up[t] = ldexpf(1.0f, up);
+            q_down[t] = ldexpf(1.0f, -up);
+        }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const float4 a = *(const float4 *)(qr + ks * 32 + g * 8), b = *(const float4 *)(qr + ks * 32 + g * 8 + 4);
@@ -313,6 +329,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float rest = v[e] * (scale * 1.44269504088896341f);
+                if (WIDE) rest *= q_up[t];
 #pragma unroll
                 for (int p = 0; p < QP; ++p) {
                     qf[t][ks][p][e] = (T)rest;
@@ -390,7 +407,8 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
             }
             float mx = fmaxf(fmaxf(fmaxf(s[t][0][0], s[t][0][1]), fmaxf(s[t][0][2], s[t][0][3])),
                              fmaxf(fmaxf(s[t][1][0], s[t][1][1]), fmaxf(s[t][1][2], s[t][1][3])));
-            const float m_new = fmaxf(m_run[t], quad16_max(mx));
+            // WIDE: a maximum rounded up to a whole power of two, so that the weights' scale costs them no bit
+            const float m_new = fmaxf(m_run[t], WIDE ? ceilf(quad16_max(mx) * q_down[t]) : quad16_max(mx));
             const float m_at = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible yet: all weights are 2^-inf = 0
             const float corr = __builtin_amdgcn_exp2f(m_run[t] - m_at);
             m_run[t] = m_new;
@@ -399,7 +417,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    float w = __builtin_amdgcn_exp2f(s[t][kt][j] - m_at);
+                    float w = __builtin_amdgcn_exp2f(WIDE ? __builtin_fmaf(s[t][kt][j], q_down[t], 15.0f - m_at) : s[t][kt][j] - m_at);
                     sum += w;
 #pragma unroll
                     for (int p = 0; p < PP; ++p) {
@@ -612,7 +630,7 @@ int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cac
 #undef CANDY_VALU
     } else if (kv_f16) {
         if (head_dim == 64)
-            launch_attn_mfma<64, _Float16, 1, 3, 2>(dev, q, kh, vh, 0, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
+            launch_attn_mfma<64, _Float16, 1, 3, 3>(dev, q, kh, vh, 0, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
         else
             launch_attn_mfma<128, _Float16, 1, 2, 2>(dev, q, kh, vh, 0, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
     } else {

@@ -70,3 +70,71 @@ def test_tiles_edges_against_the_vector_kernel(dev, heads, kv_heads, head_dim, f
             # (below 256 rows and above it the projections round differently: fp16 operands, 3e-4 per contraction)
             mixed = n >= 256
             assert np.max(np.abs(got["cut"] - got[1][cut:])) <= (bar + 4e-3 if mixed else bar) * top, (n, cut)
+
+
+# ------------------------------------------------------------------ accuracy
+def mirror(dev, heads, kv_heads, head_dim, max_pos, q_std, k_std):
+    """One layer whose hidden rows are (but for x, a thousandth of them) the quantized attention itself: Wo is the identity.  q and k
+    are about q_std and k_std wide, v about 1."""
+    d, kd, f = heads * head_dim, kv_heads * head_dim, synth.Q8_0
+    model = hip.Llama(dev, n_layers=1, d_model=d, n_heads=heads, n_kv_heads=kv_heads, head_dim=head_dim, d_ffn=256, vocab=256, max_pos=max_pos,
+                      rms_eps=1e-12, rope_base=10000.0)
+
+    def matrix(rows, cols, seed, std):  # levels of +-127 / sqrt(3) rms
+        rng = np.random.default_rng(seed)
+        w = np.zeros((rows * cols // 32, 34), np.uint8)
+        w[:, :2] = np.full((len(w), 1), std / (127 / 3 ** 0.5 * cols ** 0.5), np.float16).view(np.uint8)
+        w[:, 2:] = rng.integers(-127, 128, (len(w), 32)).astype(np.int8).view(np.uint8)
+        return dev.qtensor(f, rows, cols, w.reshape(-1))
+
+    eye = np.zeros((d * d // 32, 34), np.uint8)
+    eye[:, :2] = np.full((len(eye), 1), 1 / 127, np.float16).view(np.uint8)
+    i = np.arange(d)
+    eye[i * (d // 32) + i // 32, 2 + i % 32] = 127
+    for kind, w in ((hip.W_Q, matrix(d, d, 1, q_std)), (hip.W_K, matrix(kd, d, 2, k_std)), (hip.W_V, matrix(kd, d, 3, 1.0)),
+                    (hip.W_O, dev.qtensor(f, d, d, eye.reshape(-1))), (hip.W_GATE, matrix(256, d, 4, 1.0)), (hip.W_UP, matrix(256, d, 5, 1.0)),
+                    (hip.W_DOWN, dev.qtensor(f, d, 256, np.zeros(synth.weight_nbytes(f, d, 256), np.uint8)))):
+        model.set_qweight(kind, 0, w)
+    model.set_qweight(hip.W_HEAD, -1, matrix(256, d, 6, 1.0))
+    model.set_qweight(hip.W_EMBED, -1, matrix(256, d, 7, 1e-3 * d ** 0.5))
+    for kind, layer in ((hip.W_ATTN_NORM, 0), (hip.W_FFN_NORM, 0), (hip.W_OUT_NORM, -1)):
+        model.set_norm(kind, layer, np.ones(d, np.float32))
+    return model
+
+
+def both(dev, model, tokens, pos0=0):
+    """Hidden rows by the vector-ALU kernel and by the matrix cores."""
+    got = []
+    try:
+        for valu in (1, 0):
+            dev.set_option("prefill.attention_valu", valu)
+            model.prefill(tokens, pos0, want_logits=False)
+            got.append(model.prompt_hidden(len(tokens)))
+    finally:
+        dev.set_option("prefill.attention_valu", 0)
+    return got
+
+
+# A level falls the other way where the two kernels' results, e of the block's largest value apart, lie on either side of its
+# edge: a share of 2 * 127 * e.  f32 sums and exponentials that round at 2^-24 to 2^-22 leave e of 2^-21 at most: 1.2e-4, and 2e-4
+# with room.  Weights of one 16-bit part (2^-12 each) are far past it.
+SHARE = 2e-4
+# (heads, kv heads, head_dim, f16 cache, q_std, k_std); queries past fp16's range, and keys near its end beside small queries:
+# head_dim 64, whose parts stand for 32 bits
+ACCURACY = [(8, 2, 64, False, 1.0, 1.0), (8, 2, 64, True, 1.0, 1.0), (6, 2, 128, False, 1.0, 1.0), (6, 2, 128, True, 1.0, 1.0),
+            (32, 4, 64, False, 1.5, 1.5), (32, 4, 64, True, 1.5, 1.5), (8, 2, 64, True, 3e5, 1e-4), (8, 2, 64, False, 3e5, 1e-4),
+            (8, 2, 64, True, 3e-4, 1e4), (8, 2, 64, False, 3e-4, 1e4)]
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,f16,q_std,k_std", ACCURACY)
+def test_levels_of_the_result(dev, heads, kv_heads, head_dim, f16, q_std, k_std):
+    model = mirror(dev, heads, kv_heads, head_dim, 1104, q_std, k_std)
+    if f16:
+        model.set_kv_f16(True)
+    rng = np.random.default_rng(head_dim)
+    for n in (70, 300) + ((1100,) if heads == 32 else ()):
+        want, got = both(dev, model, [int(t) for t in rng.integers(0, 256, n)])
+        assert np.all(np.isfinite(want)) and np.all(np.isfinite(got)), n
+        level = np.max(np.abs(want).reshape(n, -1, 32), axis=2, keepdims=True) / 127
+        moved = np.abs(got - want).reshape(n, -1, 32) > 0.5 * level
+        assert np.mean(moved) <= SHARE, n
