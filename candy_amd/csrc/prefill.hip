@@ -280,11 +280,36 @@ __device__ __forceinline__ float4v mfma16(half8 a, half8 b, float4v c) { return 
 __device__ __forceinline__ float4v mfma16(PartVec<__bf16>::v8 a, PartVec<__bf16>::v8 b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+// One query's attention by a wavefront on the vector ALU in f32, 64 keys at a time: lane d returns result d of 64.  For results
+// of the matrix cores that are no numbers: an infinity, or a value that rounds to one, becomes inf - inf in parts, where in
+// one piece it may only have been a weight of 0 or an infinite result.
+template <class KV>
+__device__ float attn_row_valu(const float *__restrict__ q, const KV *__restrict__ k, const KV *__restrict__ v, int n_keys, float scale, int lane) {
+    float m = -INFINITY, l = 0.0f, o = 0.0f;
+    for (int p0 = 0; p0 < n_keys; p0 += 64) {
+        const KV *row = k + (size_t)min(p0 + lane, n_keys - 1) * 64;
+        float s = 0.0f;
+        for (int d = 0; d < 64; d += 4) {
+            const float4 a = *(const float4 *)(q + d), b = kv_load4(row + d);
+            s += a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
+        }
+        s = p0 + lane < n_keys ? s * scale : -INFINITY;
+        const float m_new = fmaxf(m, wave_max(s));
+        const float m_at = m_new == -INFINITY ? 0.0f : m_new, corr = expf(m - m_at), w = expf(s - m_at);
+        m = m_new;
+        l = l * corr + wave_sum(w);
+        o *= corr;
+        for (int i = 0; i < min(64, n_keys - p0); ++i)
+            o += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i)) * (float)v[(size_t)(p0 + i) * 64 + lane];
+    }
+    return o * (1.0f / l);
+}
+
 template <int HD, class T, int KVP, int QP, int PP, int QH, int KG>
 __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * KG == 4 ? 1 : 2) void k_attn_prefill_mfma(const float *__restrict__ q, const T *__restrict__ kparts, const T *__restrict__ vparts,
                                                               int64_t part_stride, int64_t head_stride, float *__restrict__ out, int n, int pos0,
                                                               int n_heads, int group, int q_tiles, float scale,
-                                                              _Float16 *__restrict__ xh_out) {
+                                                              _Float16 *__restrict__ xh_out, const float *k_cache, const float *v_cache) {
     typedef typename PartVec<T>::v8 v8;
     typedef typename PartVec<T>::v4 v4;
     constexpr int THREADS = 64 * QH * KG, QT = 32 * QH, R = 32 * KG, C = HD / 8, KS = HD / 32, DT = HD / 16;
@@ -490,6 +515,32 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
         const float inv = 1.0f / l_run[t];
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[t][d] *= inv;
+        if constexpr (HD == 64) {
+            float all = 0.0f;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) all += (o[t][d][0] + o[t][d][1]) + (o[t][d][2] + o[t][d][3]);
+            unsigned long long lost = __ballot(all != all && i < n);
+            lost = (lost | lost >> 16 | lost >> 32 | lost >> 48) & 0xFFFF;  // by query
+            while (lost) {
+                const int r = __builtin_ctzll(lost), row = i0 + 32 * qh + 16 * t + r;
+                lost &= lost - 1;
+                const float *qr = q + ((size_t)row * n_heads + head) * HD;
+                float res;
+                if constexpr (KVP == 1) {
+                    res = attn_row_valu(qr, kh, vh, pos0 + row + 1, scale, lane);
+                } else {
+                    const size_t at = (size_t)(head / group) * head_stride;
+                    res = attn_row_valu(qr, k_cache + at, v_cache + at, pos0 + row + 1, scale, lane);
+                }
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float x = __shfl(res, 16 * d + 4 * g + j, 64);
+                        if (r16 == r) o[t][d][j] = x;
+                    }
+            }
+        }
         if (xh_out) {
             // The row leaves as the fp16 image of its Q8_0 quantization (what the o projection's fp16 tiles contract
             // with), the arithmetic of quantize_q8_lane4 + q8_lane4_to_half value by value: a 32-value block is
@@ -581,7 +632,8 @@ int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, cons
 
 template <int HD, class T, int KVP, int QP, int PP>
 static void launch_attn_mfma(candy_hip_device *dev, const float *q, const T *kparts, const T *vparts, int64_t part_stride, float *out, int n,
-                             int pos0, int n_heads, int n_kv_heads, int64_t cache_stride, float scale, _Float16 *xh_out) {
+                             int pos0, int n_heads, int n_kv_heads, int64_t cache_stride, float scale, _Float16 *xh_out,
+                             const float *k_cache = nullptr, const float *v_cache = nullptr) {
     // Two key groups per workgroup (64 queries, alternate tiles of 32 keys) where the launch lasts as long as its longest
     // walk; 128 queries and one group where there are workgroups enough to fill the chip twice over.
     // 64 queries per workgroup and two groups of wavefronts on alternate tiles of 32 keys, because a launch lasts as long
@@ -596,7 +648,7 @@ static void launch_attn_mfma(candy_hip_device *dev, const float *q, const T *kpa
         const int tiles = (n + 32 * QH - 1) / (32 * QH);                                                                              \
         hipLaunchKernelGGL((k_attn_prefill_mfma<HD, T, KVP, QP, PP, QH, KG>), dim3((unsigned)(n_heads * tiles)), dim3(64 * QH * KG),  \
                            0, dev->stream, q, kparts, vparts, part_stride, cache_stride, out, n, pos0, n_heads, n_heads / n_kv_heads, \
-                           tiles, scale, xh_out);                                                                                     \
+                           tiles, scale, xh_out, k_cache, v_cache);                                                                   \
     } while (0)
     if (form == 1) CANDY_ATTN(4, 1);
     else if (form == 2 || KVP == 1 || small <= 2 * (int64_t)dev->num_cus) CANDY_ATTN(2, 2);
@@ -641,7 +693,7 @@ int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cac
         const __bf16 *pb = (const __bf16 *)parts;
         const _Float16 *ph = (const _Float16 *)parts;
         if (head_dim == 64)
-            launch_attn_mfma<64, __bf16, 3, 3, 3>(dev, q, pb, pb + 3 * ps, ps, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
+            launch_attn_mfma<64, __bf16, 3, 3, 3>(dev, q, pb, pb + 3 * ps, ps, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out, kf, vf);
         else
             launch_attn_mfma<128, _Float16, 2, 2, 2>(dev, q, ph, ph + 2 * ps, ps, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
     }

@@ -138,3 +138,33 @@ def test_levels_of_the_result(dev, heads, kv_heads, head_dim, f16, q_std, k_std)
         level = np.max(np.abs(want).reshape(n, -1, 32), axis=2, keepdims=True) / 127
         moved = np.abs(got - want).reshape(n, -1, 32) > 0.5 * level
         assert np.mean(moved) <= SHARE, n
+
+
+# A key that is infinite, no number, or (f32) past what its first part can hold, among earlier positions and at the last of them.
+# A query whose scores of it are -infinity has a result (weight 0), which a sum of parts alone turns into inf - inf.
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, 3.4e38, np.nan])
+@pytest.mark.parametrize("cut,n", [(70, 75), (33, 40), (64, 700)])
+def test_keys_that_are_no_numbers(dev, f16, value, cut, n):
+    if f16 and value == 3.4e38:
+        pytest.skip("no such half")
+    heads, hd, max_pos = 4, 64, 800
+    model = mirror(dev, heads, heads, hd, max_pos, 1.0, 1.0)
+    if f16:
+        model.set_kv_f16(True)
+    tokens = [int(t) for t in np.random.default_rng(cut).integers(0, 256, cut + n)]
+    model.prefill(tokens[:cut], 0, want_logits=False)
+    dt = np.float16 if f16 else np.float32
+    k_ptr, _, _ = model.kv_cache()
+    for pos, d, x in ((5, 3, value), (cut - 1, 40, value)):
+        if pos == 5 and n == 75:
+            continue  # one alone
+        a = np.array([x], dt)
+        hip._check(hip.lib().candy_hip_h2d(dev.handle, k_ptr + ((2 * max_pos + pos) * hd + d) * a.itemsize, a.ctypes.data, a.nbytes))
+    want, got = both(dev, model, tokens[cut:], cut)
+    has = np.all(np.isfinite(want), axis=1)
+    assert np.isnan(value) or 0.1 < np.mean(has) < 0.9
+    assert np.all(np.isfinite(got[has]))
+    if np.any(has):
+        w, g = want[has].reshape(-1, 32), got[has].reshape(-1, 32)
+        assert np.mean(np.abs(g - w) > 0.5 * np.max(np.abs(w), axis=1, keepdims=True) / 127) <= 2 * SHARE
