@@ -548,9 +548,9 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
             const int K = n_heads * HD;
 #pragma unroll
             for (int b = 0; b < DT / 2; ++b) {
-                float amax = 0.0f;
+                float amax = fabsf(o[t][2 * b][0]);  // (not 0: a block without a number has no largest value, and stays so)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(o[t][2 * b + (e >> 2)][e & 3]));
+                for (int e = 1; e < 8; ++e) amax = fmaxf(amax, fabsf(o[t][2 * b + (e >> 2)][e & 3]));
                 amax = quad16_max(amax);
                 const float dq = amax / 127.0f, df = __half2float(__float2half_rn(dq));
 #pragma unroll

@@ -168,3 +168,21 @@ def test_keys_that_are_no_numbers(dev, f16, value, cut, n):
     if np.any(has):
         w, g = want[has].reshape(-1, 32), got[has].reshape(-1, 32)
         assert np.mean(np.abs(g - w) > 0.5 * np.max(np.abs(w), axis=1, keepdims=True) / 127) <= 2 * SHARE
+
+
+# The same behind a query that has no result: its row stays no number, also where the attention kernel quantizes it by itself
+# (from 256 rows on).
+@pytest.mark.parametrize("heads,head_dim", [(4, 64), (2, 128)])
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("n", [40, 300])
+def test_rows_without_a_number_stay_so(dev, heads, head_dim, f16, n):
+    max_pos = 400
+    model = mirror(dev, heads, heads, head_dim, max_pos, 1.0, 1.0)
+    if f16:
+        model.set_kv_f16(True)
+    tokens = [int(t) for t in np.random.default_rng(n).integers(0, 256, 64 + n)]
+    model.prefill(tokens[:64], 0, want_logits=False)
+    a = np.array([np.nan], np.float16 if f16 else np.float32)
+    hip._check(hip.lib().candy_hip_h2d(dev.handle, model.kv_cache()[0] + 5 * head_dim * a.itemsize, a.ctypes.data, a.nbytes))
+    for rows in both(dev, model, tokens[64:], 64):
+        assert not np.any(np.isfinite(rows[:, :head_dim]))
