@@ -511,36 +511,48 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int i = i0 + 32 * qh + 16 * t + r16;
         const float inv = 1.0f / l_run[t];
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[t][d] *= inv;
-        if constexpr (HD == 64) {
+    }
+    if constexpr (HD == 64) {
+        unsigned long long lost[2];  // the 16 queries each whose results are no numbers
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
             float all = 0.0f;
 #pragma unroll
             for (int d = 0; d < DT; ++d) all += (o[t][d][0] + o[t][d][1]) + (o[t][d][2] + o[t][d][3]);
-            unsigned long long lost = __ballot(all != all && i < n);
-            lost = (lost | lost >> 16 | lost >> 32 | lost >> 48) & 0xFFFF;  // by query
-            while (lost) {
-                const int r = __builtin_ctzll(lost), row = i0 + 32 * qh + 16 * t + r;
-                lost &= lost - 1;
-                const float *qr = q + ((size_t)row * n_heads + head) * HD;
-                float res;
-                if constexpr (KVP == 1) {
-                    res = attn_row_valu(qr, kh, vh, pos0 + row + 1, scale, lane);
-                } else {
-                    const size_t at = (size_t)(head / group) * head_stride;
-                    res = attn_row_valu(qr, k_cache + at, v_cache + at, pos0 + row + 1, scale, lane);
-                }
+            lost[t] = __ballot(all != all && i0 + 32 * qh + 16 * t + r16 < n);
+        }
+        if (__builtin_expect((lost[0] | lost[1]) != 0, 0)) {
 #pragma unroll
-                for (int d = 0; d < DT; ++d)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float x = __shfl(res, 16 * d + 4 * g + j, 64);
-                        if (r16 == r) o[t][d][j] = x;
+            for (int t = 0; t < 2; ++t) {
+                lost[t] = (lost[t] | lost[t] >> 16 | lost[t] >> 32 | lost[t] >> 48) & 0xFFFF;
+                while (lost[t]) {
+                    const int r = __builtin_ctzll(lost[t]), row = i0 + 32 * qh + 16 * t + r;
+                    lost[t] &= lost[t] - 1;
+                    const float *qr = q + ((size_t)row * n_heads + head) * HD;
+                    float res;
+                    if constexpr (KVP == 1) {
+                        res = attn_row_valu(qr, kh, vh, pos0 + row + 1, scale, lane);
+                    } else {
+                        const size_t at = (size_t)(head / group) * head_stride;
+                        res = attn_row_valu(qr, k_cache + at, v_cache + at, pos0 + row + 1, scale, lane);
                     }
+#pragma unroll
+                    for (int d = 0; d < DT; ++d)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float x = __shfl(res, 16 * d + 4 * g + j, 64);
+                            if (r16 == r) o[t][d][j] = x;
+                        }
+                }
             }
         }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int i = i0 + 32 * qh + 16 * t + r16;
         if (xh_out) {
             // The row leaves as the fp16 image of its Q8_0 quantization (what the o projection's fp16 tiles contract
             // with), the arithmetic of quantize_q8_lane4 + q8_lane4_to_half value by value: a 32-value block is
