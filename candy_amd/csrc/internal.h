@@ -69,6 +69,7 @@ struct Options {
     int prefill_fold_split_sums = 1; // prompt pass: split-K copies summed inside the launch that follows (norm, rope)
     int prefill_qkv_group = 1;       // prompt pass: q / k / v (and gate / up) on one grid each where they run on the fp16 tiles
     int prefill_attention_valu = 0;  // comparison runs: prompt attention on the vector ALU instead of the matrix cores
+    int kv_parts_mb = 0;             // MB at most for the 16-bit parts of a layer's f32 K and V (0: no limit); past it, the vector ALU
     int llama_graph = 1;         // decoders created afterwards replay a captured HIP graph (0: eager launches)
     int fused_wide = 1;          // decode step: one-workgroup-per-CU kernels for the big Q4_K shapes (0: the narrower ones)
     int wide_waves = 8;          // wavefronts per workgroup of those kernels: 8 (two workgroups per CU) or 16 (one)
@@ -319,11 +320,12 @@ int launch_contract(candy_hip_device *dev, const candy_hip_qtensor *w, const int
 int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, const float *v, const float *cos_t,
                            const float *sin_t, void *k_cache, void *v_cache, bool kv_f16, int n, int pos0, int n_heads,
                            int n_kv_heads, int head_dim, int64_t cache_stride, void *parts, const SplitPending *sp = nullptr);
-// parts: attn_prefill_parts_bytes() of scratch for an f32 cache (max_pos * head_dim = cache_stride), unused for fp16
+// parts: attn_prefill_parts_bytes() of scratch for an f32 cache (max_pos * head_dim = cache_stride), unused for fp16; without it the
+// attention of an f32 cache runs on the vector ALU
 size_t attn_prefill_parts_bytes(int n_kv_heads, int head_dim, int max_pos);
 int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cache, const void *v_cache, bool kv_f16, void *parts,
                         float *out, int n, int pos0, int n_heads, int n_kv_heads, int head_dim, int64_t cache_stride,
                         float scale, _Float16 *xh_out = nullptr);  // xh_out: the fp16 image of the quantized rows, not `out`
-bool attn_prefill_writes_half(const candy_hip_device *dev);
+bool attn_prefill_writes_half(const candy_hip_device *dev, bool half_operands);  // half_operands: fp16 cache, or parts
 
 }  // namespace candy

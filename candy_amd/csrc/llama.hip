@@ -356,8 +356,16 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
     int rc;
     P.k = P.q + (size_t)n * qd;  // q, k and v of this pass end to end, whatever the buffer's capacity
     P.v = P.k + (size_t)n * c.n_kv_heads * c.head_dim;
-    if (!m->kv_f16 && !kv_parts && (rc = decoder_alloc(m, &kv_parts, attn_prefill_parts_bytes(c.n_kv_heads, c.head_dim, c.max_pos))))
-        return rc;
+    uint8_t *parts = nullptr;
+    const size_t parts_bytes = attn_prefill_parts_bytes(c.n_kv_heads, c.head_dim, c.max_pos), parts_mb = (size_t)dev->opt.kv_parts_mb;
+    if (!m->kv_f16 && !dev->opt.prefill_attention_valu && (parts_mb == 0 || parts_bytes <= parts_mb << 20)) {
+        // no memory for them is no reason to refuse the prompt: the vector ALU reads the cache as it is
+        if (!kv_parts && (rc = decoder_alloc(m, &kv_parts, parts_bytes))) {
+            if (rc != CANDY_HIP_ERR_OOM) return rc;
+            (void)hipGetLastError();
+        }
+        parts = kv_parts;
+    }
     if ((rc = embed(prompt_ids, n, P.h))) return rc;
     // A projection that splits K leaves its partial copies for the launch that follows: the norm launch behind o / down
     // sums them, adds the residual and writes P.h before it normalizes, the rope launch behind q / k / v sums them on
@@ -402,11 +410,11 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
             if ((rc = launch_contract(dev, L.wv, P.xq, P.xs, n, P.v, xh_for(L.wv)))) return rc;
         }
         rc = launch_prefill_rope_kv(dev, P.q, P.k, P.v, m->cos_t, m->sin_t, kc, vc, m->kv_f16, n, pos0, c.n_heads,
-                                    c.n_kv_heads, c.head_dim, cache_stride, kv_parts, &pend);
+                                    c.n_kv_heads, c.head_dim, cache_stride, parts, &pend);
         pend.n_split = 0;
         if (rc) return rc;
-        _Float16 *att_xh = xh_for(L.wo) && mmq_fuses_residual(L.wo, n) && attn_prefill_writes_half(dev) ? P.xh : nullptr;
-        if ((rc = launch_attn_prefill(dev, P.q, kc, vc, m->kv_f16, kv_parts, P.att, n, pos0, c.n_heads, c.n_kv_heads, c.head_dim,
+        _Float16 *att_xh = xh_for(L.wo) && mmq_fuses_residual(L.wo, n) && attn_prefill_writes_half(dev, m->kv_f16 || parts) ? P.xh : nullptr;
+        if ((rc = launch_attn_prefill(dev, P.q, kc, vc, m->kv_f16, parts, P.att, n, pos0, c.n_heads, c.n_kv_heads, c.head_dim,
                                       cache_stride, scale, att_xh)))
             return rc;
         if (!att_xh && (rc = launch_quantize_q8(dev, P.att, n, qd, P.xq, P.xs, nullptr, xh_for(L.wo)))) return rc;

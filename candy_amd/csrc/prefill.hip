@@ -8,7 +8,7 @@
 //                       new k / v rows written into the f32 cache [kv_head][position][head_dim]
 //   k_kv_parts          cache rows of earlier positions as the sums of 16-bit parts the matrix cores contract
 //   k_attn_prefill_mfma causal attention of 64 or 128 queries of one head against the cache on the matrix cores
-//   k_attn_prefill      the same on the vector ALU (comparison runs)
+//   k_attn_prefill      the same on the vector ALU: where there is no memory for the parts (and in comparison runs)
 #include <cstdlib>
 
 #include "attention_tiles.h"
@@ -670,8 +670,8 @@ static void launch_attn_mfma(candy_hip_device *dev, const float *q, const T *kpa
 
 // The matrix-core kernel can leave its output as the fp16 image of the quantized rows instead of f32 (no separate
 // quantize launch in front of an o projection that runs on the fp16 tiles).
-bool attn_prefill_writes_half(const candy_hip_device *dev) {
-    return !dev->opt.prefill_attention_valu && dev->opt.prefill_fold_split_sums;
+bool attn_prefill_writes_half(const candy_hip_device *dev, bool half_operands) {
+    return half_operands && !dev->opt.prefill_attention_valu && dev->opt.prefill_fold_split_sums;
 }
 
 int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cache, const void *v_cache, bool kv_f16, void *parts,
@@ -679,10 +679,10 @@ int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cac
                         float scale, _Float16 *xh_out) {
     CANDY_REQUIRE(head_dim == 64 || head_dim == 128, "head_dim must be 64 or 128");
     CANDY_REQUIRE(n > 0 && pos0 >= 0 && n_heads % n_kv_heads == 0, "invalid attention shape");
-    CANDY_REQUIRE(!xh_out || attn_prefill_writes_half(dev), "internal: this attention kernel writes f32 only");
+    CANDY_REQUIRE(!xh_out || attn_prefill_writes_half(dev, kv_f16 || parts), "internal: this attention kernel writes f32 only");
     const float *kf = (const float *)k_cache, *vf = (const float *)v_cache;
     const _Float16 *kh = (const _Float16 *)k_cache, *vh = (const _Float16 *)v_cache;
-    if (dev->opt.prefill_attention_valu) {  // comparison runs
+    if (dev->opt.prefill_attention_valu || (!kv_f16 && !parts)) {
         const dim3 grid((unsigned)n_heads, (unsigned)((n + 31) / 32));
 #define CANDY_VALU(HD, KV, K, V)                                                                                              \
     hipLaunchKernelGGL((k_attn_prefill<HD, KV>), grid, dim3(256), 0, dev->stream, q, K, V, out, n, pos0, n_heads, n_kv_heads, \

@@ -361,6 +361,7 @@ const OptionKey OPTION_KEYS[] = {
     {"prefill.qkv_group", &candy::Options::prefill_qkv_group, 0, 1},
     {"prefill.fold_split_sums", &candy::Options::prefill_fold_split_sums, 0, 1},
     {"prefill.attention_valu", &candy::Options::prefill_attention_valu, 0, 1},
+    {"prefill.kv_parts_mb", &candy::Options::kv_parts_mb, 0, 1 << 20},
     {"llama.graph", &candy::Options::llama_graph, 0, 1},
     {"fused.wide", &candy::Options::fused_wide, 0, 1},
     {"fused.wide_waves", &candy::Options::wide_waves, 8, 16},

@@ -122,6 +122,9 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *                                         launch that follows (RMSNorm + quantize behind o / down, rope behind q / k / v;
  *                                         0: a launch of its own sums them)
  *   "prefill.attention_valu"     0        comparison runs: prompt attention on the vector ALU
+ *   "prefill.kv_parts_mb"        0        prompt attention on an f32 cache: MB at most for the 16-bit parts of a layer's K and
+ *                                         V that the matrix cores contract, 1 to 1.5 times one layer's cache for max_pos
+ *                                         (0: no limit).  Past the limit, and where the allocation fails, the vector ALU
  *   "prefill.attention_groups"   0        comparison runs: matrix-core prompt attention with one (1) or two (2) groups of
  *                                         wavefronts per query tile that take alternate key tiles (0: two, with 64 or 128
  *                                         queries by the size of the grid)

@@ -186,3 +186,30 @@ def test_rows_without_a_number_stay_so(dev, heads, head_dim, f16, n):
     hip._check(hip.lib().candy_hip_h2d(dev.handle, model.kv_cache()[0] + 5 * head_dim * a.itemsize, a.ctypes.data, a.nbytes))
     for rows in both(dev, model, tokens[64:], 64):
         assert not np.any(np.isfinite(rows[:, :head_dim]))
+
+
+# No memory for the parts of K and V: the prompt is taken all the same, by the vector kernel, and the next one with memory by the
+# matrix cores.  Positions in front that were cached either way serve both.
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("n", [40, 300])
+def test_prompt_without_memory_for_parts(dev, head_dim, n):
+    model = mirror(dev, 256 // head_dim, 256 // head_dim, head_dim, 4096, 1.0, 1.0)  # parts of 8 to 12 MB
+    tokens = [int(t) for t in np.random.default_rng(n).integers(0, 256, n)]
+
+    def rows(option, value, cut):
+        """Hidden rows of the last pass; the option is set for the first one."""
+        dev.set_option(option, value)
+        try:
+            model.prefill(tokens[:cut], 0, want_logits=False)
+        finally:
+            dev.set_option(option, 0)
+        if cut < n:
+            model.prefill(tokens[cut:], cut, want_logits=False)
+        return model.prompt_hidden(n if cut == n else n - cut)
+
+    for cut in (n, 33):
+        want = rows("prefill.attention_valu", 1, cut)
+        assert np.array_equal(rows("prefill.kv_parts_mb", 1, cut), want)
+        got = rows("prefill.kv_parts_mb", 0, cut)
+        level = np.max(np.abs(want).reshape(len(want), -1, 32), axis=2, keepdims=True) / 127
+        assert np.mean(np.abs(got - want).reshape(len(want), -1, 32) > 0.5 * level) <= SHARE, cut
