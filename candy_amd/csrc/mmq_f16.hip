@@ -672,10 +672,7 @@ static int launch_jobs(candy_hip_device *dev, const F16Job *jobs, int count, con
 // xh: fp16 activations [mmq_m_pad(m)][K], rows past m zero.
 int launch_mmq_f16_big(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y,
                        const float *res) {
-    if (mmq_f16_rows_covers(w, m) && dev->opt.f16_shape == 0 && dev->opt.f16_split == 0) {
-        const int rc = launch_mmq_f16_rows(dev, w, xh, m, y, res);
-        if (rc != CANDY_HIP_ERR_UNSUPPORTED) return rc;
-    }
+    if (mmq_f16_rows_covers(w, m) && dev->opt.f16_shape == 0 && dev->opt.f16_split == 0) return launch_mmq_f16_rows(dev, w, xh, m, y, res);
     const F16Job job{w, y, res};
     return launch_jobs(dev, &job, 1, xh, m);
 }

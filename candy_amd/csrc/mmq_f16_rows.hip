@@ -1,4 +1,4 @@
-// 33 to 128 activation rows of Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 on the fp16 matrix cores, K dealt to wavefronts:
+// 33 to 128 activation rows of Q4_K and Q6_K, 65 to 128 of Q5_K, Q8_0 and Q4_0, on the fp16 matrix cores, K dealt to wavefronts:
 // y[m, N] = x[m, K] . W^T with the operands of mmq_f16.hip.
 //
 // With so few rows a contraction should last as long as its weights take from memory, but in the role-split tiles of
@@ -11,7 +11,7 @@
 // rows, 11008 x 4096, before (with the split sum) -> now: Q4_K 22.8 + 4.5 -> 20.6, Q8_0 35.1 + 4.5 -> 24.0, Q4_0 33.4 + 4.5 ->
 // 21.2, Q5_K 31.5 + 4.5 -> 25.1; 2048 x 1024 Q8_0 13.0 + 4.1 -> 5.7.  What bounds it: the activations, which every CU reads
 // (655 KB here, 10 us), then the weights (48 MB of Q8_0, 8 us), half overlapped.
-#include <cstdlib>
+#include <type_traits>
 
 #include "f16_weights.h"
 #include "internal.h"
@@ -67,7 +67,11 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
                                              (__attribute__((address_space(3))) void *)(slice + it * 64), 16, 0, 0);
     };
     if (count > 0) {
-        typename F::Raw raw[STAGED ? 1 : 2][RF];
+        // Unstaged blocks are requested a super-block ahead, but three fragments of them twice over do not fit the registers: 41
+        // spilled at 64 rows, us, two sets / one: 11008 x 4096, 48 rows 28.1 / 26.1, x 2048, 40 rows 15.4 / 14.6.  (Two fragments
+        // and 128 rows spill 35, and come with one super-block per wavefront at most.)
+        constexpr int DEEP = STAGED || RF == 3 || RF * MF == 16 ? 1 : 2;
+        typename F::Raw raw[DEEP][RF];
         half8 xf[2][MF];
         auto load_w = [&](int sb, int u) __attribute__((always_inline)) {
 #pragma unroll
@@ -112,6 +116,14 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
                 if (k + 1 < count) request(sb + 8);
                 contract(sb, 0, k + 1 < count ? sb + 8 : sb);
             }
+        } else if constexpr (DEEP == 1) {
+            load_w(first, 0);
+            load_x(first * 4, 0);
+            for (int k = 0; k < count; ++k) {
+                const int sb = first + 8 * k;
+                contract(sb, 0, k + 1 < count ? sb + 8 : sb);
+                if (k + 1 < count) load_w(sb + 8, 0);
+            }
         } else {
             load_w(first, 0);
             if (count > 1) load_w(first + 8, 1);
@@ -154,13 +166,38 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
 
 static int fragments(int64_t m) { return m <= 48 ? 3 : m <= 64 ? 4 : m <= 80 ? 5 : m <= 96 ? 6 : 8; }
 
-// 16-row weight fragments per workgroup with which one round of workgroups serves every row, 0: none (a second round would
-// read the activations again; wider workgroups than these have no registers for their sums)
-template <class F>
-static int weight_fragments(const candy_hip_device *dev, int64_t rows, int mf) {
-    for (int rf = 1; rf <= 3 && (rf < 3 || mf <= (staged<F>() ? 6 : 4)) && rf * mf <= 18; ++rf)
-        if ((rows + 16 * rf - 1) / (16 * rf) <= dev->num_cus) return rf;
-    return 0;
+// 16-row weight fragments per workgroup with which one round of workgroups serves every row and this kernel is ahead of the tiles
+// of mmq_f16.hip; 0: none, the tiles.  A second round would read the activations again, and wider workgroups have no registers
+// for their sums.  Where the lines lie, us of a call, this kernel / tiles (1632 calls timed, sizes at and around each line):
+//   * weight rows for at least half of the CUs, from 2048
+//   * super-blocks for the wavefronts: with few of a cheap format the tiles' steps are short (11008 x 512, 80 rows, Q4_K 11.7 /
+//     10.8, Q5_K 13.3 / 12.4; x 1024 ahead; the others 256 long 10.2 / 9.7); no round of them that most wavefronts sit out
+//     (Q6_K 8200 x 2304, nine of them, 64 rows 21.6 / 19.9; x 2560 20.2 / 21.7)
+//   * a workgroup reads every activation, which a CU takes in at about 65 KB a us when all read: Q8_0 and Q4_0 700 KB (688 KB
+//     1.15 to 1.5 times as fast as the tiles); Q4_K and Q5_K, whose tiles cost less, 660 (4100 x 4096, 80 rows, 655 KB ahead, x 4352
+//     19.5 / 19.0 and 22.1 / 21.1); Q6_K, not staged, 450 for one fragment and 340 (8200 x 4096, 48 rows, 393 KB 25.8 / 26.1, x 4352
+//     31.3 / 25.6; 8200 x 3328, 64 rows, 426 KB 28.9 / 24.1, 328 KB 20.2 / 21.7)
+//   * Q4_K and Q5_K with many sums per wavefront: one round of super-blocks (8192 x 2304, 128 rows 24.7 / 17.8 and 22.8 / 20.4;
+//     96 rows 18.1 / 16.6 and 19.4 / 18.9); two fragments and 128 rows of Q4_K not at all (8192 x 1536 16.4 / 15.4)
+static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
+    const bool q6k = fmt == CANDY_HIP_Q6_K, cheap = fmt == CANDY_HIP_Q4_K || fmt == CANDY_HIP_Q5_K;
+    // up to 64 rows the other formats are on the exact tiles (mmq_f16_big_covers)
+    if (m > 128 || (m <= 64 && !q6k && fmt != CANDY_HIP_Q4_K) || rows < 2048 || cols % 256 != 0) return 0;
+    const int mf = fragments(m);
+    int rf = 1;
+    while ((rows + 16 * rf - 1) / (16 * rf) > num_cus)
+        if (++rf > 3) return 0;
+    if (rf == 3 && mf > (q6k ? 4 : 6)) return 0;
+    const int64_t blocks = cols / 256, rounds = (blocks + 7) / 8;
+    if (blocks < (cheap ? 4 : 2) || (rounds > 1 && 5 * blocks < 3 * 8 * rounds)) return 0;
+    if (cheap && (mf == 8 || (mf == 6 && rf == 2)) && rounds > 1) return 0;
+    if (fmt == CANDY_HIP_Q4_K && mf == 8 && rf == 2) return 0;
+    return mf * 32 * cols <= (q6k ? (rf == 1 ? 450000 : 340000) : cheap ? 660000 : 700000) ? rf : 0;
+}
+template <class F, int RF, int MF>
+constexpr bool reached() {
+    constexpr bool q4k = std::is_same<F, BigQ4K>::value, q6k = std::is_same<F, BigQ6K>::value;
+    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= (q6k ? 4 : 6)) && !(q4k && RF == 2 && MF == 8);
 }
 
 template <class F, int RF, int MF>
@@ -176,32 +213,26 @@ static int launch_rf(candy_hip_device *dev, const candy_hip_qtensor *w, const _F
 
 template <class F>
 static int launch_fmt(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res) {
-    const int mf = fragments(m), rf = weight_fragments<F>(dev, w->rows, mf);
-#define CANDY_RF(MF)                                                                      \
-    if (mf == MF) {                                                                       \
-        if (rf == 1) return launch_rf<F, 1, MF>(dev, w, xh, m, y, res);                   \
-        if (rf == 2) return launch_rf<F, 2, MF>(dev, w, xh, m, y, res);                   \
-        if constexpr (MF <= (staged<F>() ? 6 : 4))                                      \
-            if (rf == 3) return launch_rf<F, 3, MF>(dev, w, xh, m, y, res);               \
-    }
-    CANDY_RF(3) CANDY_RF(4) CANDY_RF(5) CANDY_RF(6) CANDY_RF(8)
+    const int mf = fragments(m), rf = rows_fragments(w->fmt, w->rows, w->cols, m, dev->num_cus);
+#define CANDY_RF(RF, MF)                    \
+    if constexpr (reached<F, RF, MF>())     \
+        if (rf == RF && mf == MF) return launch_rf<F, RF, MF>(dev, w, xh, m, y, res);
+#define CANDY_MF(MF) CANDY_RF(1, MF) CANDY_RF(2, MF) CANDY_RF(3, MF)
+    CANDY_MF(3) CANDY_MF(4) CANDY_MF(5) CANDY_MF(6) CANDY_MF(8)
+#undef CANDY_MF
 #undef CANDY_RF
-    return CANDY_HIP_ERR_UNSUPPORTED;
+    return fail(CANDY_HIP_ERR_INVALID, "internal: fp16 contraction of %lld rows", (long long)m);
 }
 
-// A workgroup reads every activation, so this is for activations that a CU takes in (about 65 KB a us when all CUs read)
-// in less than the tiles of mmq_f16.hip lose to their barriers and to the launch that adds their K halves; and for weight
-// rows that give at least half of the CUs a workgroup.  us of a call, tiles / this kernel, 655 KB (80 x 4096 values): Q4_K
-// 4096 x 4096 19.6 / 14.6, 11008 x 4096 26.5 / 22.0, Q8_0 4096 x 4096 21.6 / 18.1; kernels alone at 786 KB: Q8_0 15.9 + 4.2 / 18.3,
-// at 1049 KB 16.9 + 4.2 / 23.2, 4096 x 14336 at 77 rows 24.0 + 4.1 / 39.7.  Q6_K, whose blocks are not staged: 393 KB 4096 x 4096
-// 18.6 / 14.7, 11008 x 4096 30.9 / 28.1; kernels alone at 524 KB 30.9 + 4.4 / 32.8, 5632 long at 540 KB 13.2 + 4.1 / 16.3.
 bool mmq_f16_rows_covers(const candy_hip_qtensor *w, int64_t m) {
-    const bool q6k = w->fmt == CANDY_HIP_Q6_K;
-    if (!q6k && ((uintptr_t)w->data & 15) != 0) return false;  // whole pieces
-    return m <= 128 && w->rows >= 2048 && (double)fragments(m) * 32.0 * (double)w->cols <= (q6k ? 450e3 : 700e3);
+    if (w->fmt != CANDY_HIP_Q6_K && ((uintptr_t)w->data & 15) != 0) return false;  // whole pieces
+    switch (w->fmt) {
+    case CANDY_HIP_Q4_K: case CANDY_HIP_Q5_K: case CANDY_HIP_Q6_K: case CANDY_HIP_Q8_0: case CANDY_HIP_Q4_0: case CANDY_HIP_Q4_0_GGML:
+        return rows_fragments(w->fmt, w->rows, w->cols, m, w->dev->num_cus) > 0;
+    default: return false;
+    }
 }
 
-// CANDY_HIP_ERR_UNSUPPORTED: more rows than one round of workgroups takes
 int launch_mmq_f16_rows(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res) {
     CANDY_REQUIRE(m >= 1 && m <= 128 && w->cols % 256 == 0, "internal: shape of the fp16 contraction");
     switch (w->fmt) {
@@ -211,8 +242,13 @@ int launch_mmq_f16_rows(candy_hip_device *dev, const candy_hip_qtensor *w, const
     case CANDY_HIP_Q8_0: return launch_fmt<BigQ8_0>(dev, w, xh, m, y, res);
     case CANDY_HIP_Q4_0: return launch_fmt<BigQ4_0<false>>(dev, w, xh, m, y, res);
     case CANDY_HIP_Q4_0_GGML: return launch_fmt<BigQ4_0<true>>(dev, w, xh, m, y, res);
-    default: return CANDY_HIP_ERR_UNSUPPORTED;
+    default: return fail(CANDY_HIP_ERR_INVALID, "internal: format of the fp16 contraction");
     }
 }
 
 }  // namespace candy
+
+// The rule above, for its tests (no device needed).
+extern "C" int candy_test_rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
+    return candy::rows_fragments(fmt, rows, cols, m, num_cus);
+}

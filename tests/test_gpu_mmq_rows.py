@@ -1,12 +1,43 @@
 """fp16 contraction of up to 128 activation rows with K dealt to the wavefronts, against the 128 x 128 tiles on the same fp16
-operands and against the oracle."""
+operands and against the oracle: every kernel that the library's rule can choose."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from candy_amd import hip, synth
 from oracle import oracle as o
 
-pytestmark = pytest.mark.gpu
+FORMATS = [synth.Q4_K, synth.Q5_K, synth.Q6_K, synth.Q8_0, synth.Q4_0, synth.Q4_0_GGML]
+FRAGMENTS = {3: (33, 48), 4: (49, 64), 5: (65, 80), 6: (81, 96), 8: (97, 128)}  # of 16 activation rows: first and last count
+WEIGHT_ROWS = {1: (2048, 4096), 2: (4097, 8192), 3: (8193, 12288)}              # fragments of 16 weight rows on 256 CUs
+
+LIB = ctypes.CDLL(hip.LIB_PATH)
+LIB.candy_test_rows_fragments.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_int]
+
+
+def chosen(fmt, m, rows, cols, cus=256):
+    """Weight fragments per workgroup, 0: the tiles."""
+    return LIB.candy_test_rows_fragments(fmt, rows, cols, m, cus)
+
+
+def fragments(m):
+    return next(f for f, (_, last) in FRAGMENTS.items() if m <= last)
+
+
+def shapes():
+    """Per kernel: the fewest rows on either side with as many super-blocks as the rule allows of 4097 values, and the most rows (less one
+    weight row, a length not in fours) with few of them."""
+    for fmt in FORMATS:
+        for rf, (few, most) in WEIGHT_ROWS.items():
+            for mf, (low, high) in FRAGMENTS.items():
+                longest = max((c for c in range(256, 4097, 256) if chosen(fmt, low, few + 1, c) == rf), default=0)
+                if longest:
+                    yield fmt, rf, mf, low, few + 1, longest
+                    yield fmt, rf, mf, high, most - 1, 1024
+
+
+SHAPES = list(shapes())
 
 
 @pytest.fixture(scope="module")
@@ -16,16 +47,10 @@ def dev():
     d.close()
 
 
-# activation rows at the edges of their fragments (and 129: the tiles); weight rows that fill one, two and three fragments
-# per workgroup, one row over each, and one over what a round of workgroups takes; fewer super-blocks than wavefronts, as
-# many, and one more; a row length not in fours of weight rows
-SHAPES = [(65, 2048, 256), (80, 2049, 2304), (81, 4097, 512), (96, 8193, 768), (97, 2051, 2048), (128, 6000, 1024), (129, 2048, 512),
-          (77, 12288, 512), (70, 12289, 256), (66, 2050, 4096)]
-
-
-@pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q5_K, synth.Q6_K, synth.Q8_0, synth.Q4_0, synth.Q4_0_GGML])
-@pytest.mark.parametrize("m,rows,cols", SHAPES + [(33, 2048, 512), (48, 4100, 2048), (49, 2303, 768), (64, 2048, 1280)])
-def test_rows_against_tiles_and_oracle(dev, fmt, m, rows, cols):
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,rf,mf,m,rows,cols", SHAPES)
+def test_rows_against_tiles_and_oracle(dev, fmt, rf, mf, m, rows, cols):
+    assert chosen(fmt, m, rows, cols) == rf and fragments(m) == mf
     w = synth.random_weight(fmt, rows, cols, seed=rows + m)
     x = synth.random_activations(m, cols, seed=cols + m)
     q = dev.qtensor(fmt, rows, cols, w)
@@ -37,6 +62,7 @@ def test_rows_against_tiles_and_oracle(dev, fmt, m, rows, cols):
     finally:
         dev.set_option("mmq.f16_shape", 0)
     top = np.max(np.abs(tiles))
+    assert not np.array_equal(got, tiles)  # two kernels: another order of the sums
     # the same products in another order: K sums of f32, 2^-24 each of a partial sum no larger than the largest result's
     # order (random signs: sqrt(K) of them, 64 * 2^-24 = 4e-6 at K = 4096)
     assert np.max(np.abs(got - tiles)) <= 4e-6 * top
@@ -45,3 +71,31 @@ def test_rows_against_tiles_and_oracle(dev, fmt, m, rows, cols):
     want = o.qmatmul(fmt, w.reshape(rows, nb)[sub].reshape(-1), len(sub), cols, x)
     # fp16 operands: 2^-12 of each product, as for the tiles
     assert np.max(np.abs(got[:, sub] - want)) <= 5e-4 * np.max(np.abs(want))
+
+
+# ------------------------------------------------------------------ the rule, on the CPU
+def test_one_round_of_workgroups_and_bounded_activations():
+    rng = np.random.default_rng(5)
+    seen = set()
+    for _ in range(20000):
+        fmt, m = int(rng.choice(FORMATS)), int(rng.integers(1, 140))
+        rows, cols, cus = int(2 ** rng.uniform(8, 15)), 256 * int(2 ** rng.uniform(0, 6)), int(rng.choice([64, 256, 304]))
+        rf = chosen(fmt, m, rows, cols, cus)
+        assert 0 <= rf <= 3
+        if rf:
+            assert m <= 128 and rows >= 2048 and -(-rows // (16 * rf)) <= cus
+            assert m > 64 or fmt in (synth.Q4_K, synth.Q6_K)
+            assert fragments(m) * 32 * cols <= 700e3
+            seen.add((fmt, rf, fragments(m)))
+    assert seen == {s[:3] for s in SHAPES}  # no kernel but those tested above
+
+
+@pytest.mark.parametrize("fmt,m,rows,cols,rf", [
+    (synth.Q8_0, 77, 11008, 4096, 3), (synth.Q8_0, 128, 2048, 1024, 1), (synth.Q4_K, 80, 4096, 4096, 1), (synth.Q4_K, 33, 4096, 5632, 1),
+    (synth.Q6_K, 48, 11008, 3328, 3), (synth.Q6_K, 64, 8200, 2560, 3),
+    # where the tiles are ahead: long rows, too many of them, few super-blocks, a round that most wavefronts sit out
+    (synth.Q8_0, 77, 4096, 14336, 0), (synth.Q8_0, 77, 14336, 4096, 0), (synth.Q8_0, 129, 4096, 1024, 0), (synth.Q8_0, 64, 4096, 1024, 0),
+    (synth.Q4_K, 80, 11008, 512, 0), (synth.Q6_K, 64, 8200, 2304, 0), (synth.Q6_K, 64, 8200, 3328, 0), (synth.Q4_K, 128, 8192, 1536, 0),
+    (synth.Q5_K, 128, 8192, 2304, 0), (synth.Q4_K, 96, 8192, 2816, 0), (synth.Q4_K, 80, 4100, 4352, 0)])
+def test_where_the_lines_lie(fmt, m, rows, cols, rf):
+    assert chosen(fmt, m, rows, cols) == rf
