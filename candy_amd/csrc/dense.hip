@@ -790,13 +790,22 @@ static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
     return CANDY_HIP_OK;
 }
 
-// 64-row tiles while experts have few rows each.  From 96 on tiles of 256 x 128, the longer ones' share in a launch that
-// reads every expert's weights either way: us, up / down, 128 x 128 tiles -> these, unevenly dealt rows: 64 experts of 1408 at
-// width 2048, 1024 tokens of 6 107 / 105 -> 107 / 102, 2048 134 / 149 -> 142 / 147; 16 of 2048 at 4096, 1024 tokens of 4
-// 144 / 128 -> 133 / 121, 2048 199 / 201 -> 194 / 196.  (256 rows: 127 / 114 and 220 / 194 in the second and last.)
+// 64-row tiles (two workgroups per CU) while experts have few rows each, and for short contractions, whose few steps do not pay for
+// a large tile's first loads: us of a whole layer, 64 / 128 rows, 64 experts of 256 at width 512, 160 rows each 71.0 / 71.8, 256 85.6 /
+// 92.4; of 512 at 1024, 112 rows 96.0 / 107.1, 160 108.6 / 115.9, 192 121.9 / 119.8; of 1408 at 2048, 96 rows 293 / 265.
 int grouped_tile_rows(int experts, int64_t slots, int64_t widest) {
+    const bool few = slots < 96 * (int64_t)experts, brief = widest <= 768 || (widest <= 1024 && slots < 160 * (int64_t)experts);
     // an activation row's place is a 32-bit offset in the large tiles' loads, from the first of all rows, and so is a weight row's
-    return slots < 96 * (int64_t)experts || slots * widest * 2 > 0xFFFFFFFFll || !tile_fits(256, widest) ? 64 : 128;
+    return few || brief || slots * widest * 2 > 0xFFFFFFFFll || !tile_fits(256, widest) ? 64 : 128;
+}
+
+// Weight rows of the 128-row tiles: 256 for the longer share of a launch that reads every expert's weights either way, 128 where all
+// of these are on the chip at once (by the rows an expert has on average, and a few more).  us of a whole layer, 128 / 256: 64 experts
+// of 1408 at width 2048, 96 rows each 273 / 265, 192 396 / 362, 512 816 / 732; 16 of 2048 at 4096, 192 283 / 267; 8 of 4096 at
+// 4096, 96 rows (one round) 211 / 239, 128 rows (two) 264 / 245; 4 of 2048 at 1024, 256 rows 68 / 86; 8 of 4096 at 1024, 96 rows 82 / 107.
+static int grouped_weight_rows(int num_cus, int experts, int64_t slots, int expert_rows) {
+    const int64_t row_tiles = (slots / experts + 16 + 127) / 128 * experts;
+    return expert_rows <= 128 || row_tiles * ((expert_rows + 127) / 128) <= num_cus ? 128 : 256;
 }
 
 // Rows dealt to experts: the grid has room for max_tiles row tiles, workgroups past the list's end leave at once.
@@ -807,7 +816,7 @@ static int launch_mm_grouped(candy_hip_device *dev, const DenseLaunch &L) {
     if (gr.tile_rows > 64) {
         p.big = true;
         p.bm = 128;
-        p.bn = gr.expert_rows > 128 ? 256 : 128;
+        p.bn = grouped_weight_rows(dev->num_cus, (int)(L.w->rows / gr.expert_rows), L.m, gr.expert_rows);
     }
     const int n_tiles = (gr.expert_rows + p.bn - 1) / p.bn;
     const int64_t tiles = (int64_t)gr.max_tiles * n_tiles;
@@ -1024,6 +1033,9 @@ void candy_test_dense_plan(int num_cus, int m, int64_t rows, int64_t ld, int64_t
     plan[0] = p.big; plan[1] = p.bn; plan[2] = p.bm; plan[3] = p.splits;
 }
 int candy_test_grouped_tile_rows(int experts, int64_t slots, int64_t widest) { return candy::grouped_tile_rows(experts, slots, widest); }
+int candy_test_grouped_weight_rows(int num_cus, int experts, int64_t slots, int expert_rows) {
+    return candy::grouped_weight_rows(num_cus, experts, slots, expert_rows);
+}
 
 int candy_hip_dense_sweep(candy_hip_device *dev, const candy_hip_dense *const *ws, int n_ws, const float *dev_x, int64_t m,
                           int epilogue, int iters, float *elapsed_ms) {

@@ -12,6 +12,7 @@ LIB = ctypes.CDLL(hip.LIB_PATH)
 LIB.candy_test_dense_plan.argtypes = [ctypes.c_int] * 2 + [ctypes.c_int64] * 3 + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int)]
 LIB.candy_test_dense_plan.restype = None
 LIB.candy_test_grouped_tile_rows.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int64]
+LIB.candy_test_grouped_weight_rows.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int]
 LIMIT = 1 << 32
 TILES = {(256, 256), (224, 256), (192, 256), (160, 256), (128, 256), (256, 128), (192, 128), (128, 128)}
 
@@ -75,3 +76,14 @@ def test_grouped_tiles_fit_32_bits():
                 assert rows in (64, 128)
                 if rows == 128:  # 256 weight rows beside them
                     assert slots * widest * 2 <= LIMIT - 1 and 256 * widest * 2 <= LIMIT - 1
+
+
+# (experts, rows of each, width, rows of an expert's weight) -> rows of a tile, its weight rows: short contractions, few tiles, many
+@pytest.mark.parametrize("experts,rows,d,ff,tile,wide", [
+    (64, 95, 2048, 1408, 64, None), (64, 96, 2048, 1408, 128, 256), (64, 192, 2048, 1408, 128, 256), (64, 256, 512, 256, 64, None),
+    (64, 112, 1024, 512, 64, None), (64, 192, 1024, 512, 128, 256), (8, 96, 4096, 4096, 128, 128), (8, 128, 4096, 4096, 128, 256),
+    (4, 256, 1024, 2048, 128, 128), (16, 192, 4096, 2048, 128, 256), (200, 1000, 1088, 128, 128, 128)])
+def test_tiles_of_rows_dealt_to_experts(experts, rows, d, ff, tile, wide):
+    assert LIB.candy_test_grouped_tile_rows(experts, experts * rows, max(d, ff)) == tile
+    if wide:
+        assert LIB.candy_test_grouped_weight_rows(256, experts, experts * rows, ff) == wide

@@ -1,5 +1,7 @@
 """The large tiles of bfloat16 contractions at their edges: rows of the last tile (quarters of 32 and 64 rows), weight rows
 past the last tile, one stage of K and odd numbers of stages, every epilogue, rows dealt to experts."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -42,9 +44,7 @@ def test_tiles(dev, m, n, k):
     assert np.all(np.abs(got - 20 * np.tanh(want / 40)) <= bound + 1e-5)
 
 
-@pytest.mark.parametrize("tokens,skew", [(150, 0.0), (300, 0.0), (300, 3.0), (700, 1.0)])
-def test_rows_dealt_to_experts(dev, tokens, skew):
-    d, experts, top, ff = 192, 3, 2, 300
+def dealt(dev, tokens, skew, d, experts, top, ff):
     rng = np.random.default_rng(tokens)
     router = bf16(rng.standard_normal((experts, d)) * 0.3)
     router[0] += np.float32(skew * 0.0625)
@@ -54,7 +54,7 @@ def test_rows_dealt_to_experts(dev, tokens, skew):
     for e in range(experts):
         w[f"p.e{e}.up"], w[f"p.e{e}.down"] = up[e].astype(np.float64), down[e].astype(np.float64)
     want = ref.experts(x.astype(np.float64), w, "p", {"router": {"experts": experts, "top": top}})
-    padded = np.zeros((experts, 320, d), np.float32)
+    padded = np.zeros((experts, -(-ff // 64) * 64, d), np.float32)
     padded[:, :ff] = up
     weights = {"router": dev.dense(hip.bf16_bits(router)), "up": dev.dense(hip.bf16_bits(padded.reshape(-1, d))),
                "down": dev.dense(hip.bf16_bits(down.reshape(-1, ff)))}
@@ -64,3 +64,17 @@ def test_rows_dealt_to_experts(dev, tokens, skew):
     # the inner activations are rounded to bfloat16 once: 2^-9 of each, of random sign
     assert np.max(np.abs(got - want)) <= 2.0 ** -7 * np.max(np.abs(want))
     assert np.sqrt(np.mean((got - want) ** 2)) <= 2.0 ** -8 * np.sqrt(np.mean(want ** 2))
+
+
+@pytest.mark.parametrize("tokens,skew", [(150, 0.0), (300, 0.0), (300, 3.0), (700, 1.0)])
+def test_rows_dealt_to_experts(dev, tokens, skew):
+    dealt(dev, tokens, skew, 192, 3, 2, 300)
+
+
+# Contractions long enough for the large tiles: 128 weight rows each while all tiles are on the chip at once, 256 (up) beyond
+@pytest.mark.parametrize("tokens,skew,experts,ff", [(300, 0.0, 3, 800), (300, 3.0, 3, 800), (700, 1.0, 3, 1100), (1600, 0.0, 20, 830), (1700, 1.0, 20, 1100)])
+def test_rows_dealt_to_experts_large_tiles(dev, tokens, skew, experts, ff):
+    lib, padded = hip.lib(), -(-ff // 64) * 64
+    assert lib.candy_test_grouped_tile_rows(experts, ctypes.c_int64(2 * tokens), ctypes.c_int64(padded)) == 128
+    assert lib.candy_test_grouped_weight_rows(256, experts, ctypes.c_int64(2 * tokens), padded) == (256 if experts == 20 else 128)
+    dealt(dev, tokens, skew, 192, experts, 2, ff)
