@@ -84,31 +84,46 @@ __device__ __forceinline__ void store_parts(T *dst, int64_t part_stride, float4 
     }
 }
 
-// `count` cache rows of every kv head -> the parts k_attn_prefill_mfma reads, in rows like the cache's.
+// The first `count` cache rows of every kv head -> the parts k_attn_prefill_mfma reads, in rows like the cache's.
 template <class T, int P>
 __global__ __launch_bounds__(256) void k_kv_parts(const float *__restrict__ k_cache, const float *__restrict__ v_cache, int64_t cache_stride,
-                                                  T *__restrict__ kparts, T *__restrict__ vparts, int64_t part_stride, int lo, int count, int c4) {
+                                                  T *__restrict__ kparts, T *__restrict__ vparts, int64_t part_stride, int count, int c4) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (row, four values)
     if (idx >= (int64_t)count * c4) return;
-    const size_t at = (size_t)blockIdx.y * cache_stride + ((size_t)lo * c4 + idx) * 4;
+    const size_t at = (size_t)blockIdx.y * cache_stride + (size_t)idx * 4;
     store_parts<T, P>((blockIdx.z ? vparts : kparts) + at, part_stride, *(const float4 *)((blockIdx.z ? v_cache : k_cache) + at));
 }
 
 // The same four pairs per thread, for q, k and v rows that lie end to end in `src` ([n][q heads], [n][kv heads] twice),
 // optionally still as the n_split partial copies of a contraction split along K, `stride` floats apart, summed here in
 // the order of the separate split sum.  q is written to `q` (which may be `src`), k and v go to the cache and, with an
-// f32 cache (P > 0), as parts to the rows the attention kernel reads: a launch and a pass less than k_kv_parts behind it.
+// f32 cache (P > 0), as parts to the rows the attention kernel reads: a launch and a pass less than k_kv_parts behind it.  The
+// positions in front, whose parts may be another layer's, are workgroups of the same launch (`early_blocks` for each kv head of K, then
+// of V): us a layer of 20 tokens, 8B shape, behind 16 / 64 / 2000 positions, with a launch of their own 160 / 162 / 253, now 157 / 159 / 249.
 template <class KV, class T, int P>
 __global__ __launch_bounds__(256) void k_prefill_rope_kv4(float *q, const float *src, int n_split, size_t stride,
                                                           const float *__restrict__ cos_t,
                                                           const float *__restrict__ sin_t, KV *__restrict__ k_cache,
                                                           KV *__restrict__ v_cache, int n, int pos0, int n_heads,
                                                           int n_kv_heads, int head_dim, int64_t cache_stride,
-                                                          T *__restrict__ kparts, T *__restrict__ vparts, int64_t part_stride) {
+                                                          T *__restrict__ kparts, T *__restrict__ vparts, int64_t part_stride,
+                                                          unsigned early_blocks) {
     const int half = head_dim >> 1, hq = half >> 2;
     const int slots = n_heads + 2 * n_kv_heads;  // q heads, then k heads, then v heads
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t total = (int64_t)n * slots * hq;
+    if constexpr (P > 0) {
+        const unsigned blocks = (unsigned)((total + 255) >> 8);
+        if (blockIdx.x >= blocks) {
+            const unsigned b = blockIdx.x - blocks, h = b / early_blocks;
+            const int64_t e = (int64_t)(b - h * early_blocks) * 256 + threadIdx.x;
+            if (e >= (int64_t)pos0 * (head_dim >> 2)) return;
+            const bool is_v = h >= (unsigned)n_kv_heads;
+            const size_t at = (size_t)(is_v ? h - n_kv_heads : h) * cache_stride + (size_t)e * 4;
+            store_parts<T, P>((is_v ? vparts : kparts) + at, part_stride, *(const float4 *)((is_v ? v_cache : k_cache) + at));
+            return;
+        }
+    }
     if (idx >= total) return;
     const int j = (int)(idx % hq) * 4;
     const int slot = (int)((idx / hq) % slots);
@@ -587,16 +602,16 @@ size_t attn_prefill_parts_bytes(int n_kv_heads, int head_dim, int max_pos) {
     return (size_t)2 * (head_dim == 64 ? 3 : 2) * n_kv_heads * max_pos * head_dim * 2;
 }
 
-static int launch_kv_parts(candy_hip_device *dev, const float *k_cache, const float *v_cache, void *parts, int lo, int count, int n_kv_heads,
+static int launch_kv_parts(candy_hip_device *dev, const float *k_cache, const float *v_cache, void *parts, int count, int n_kv_heads,
                            int head_dim, int64_t cache_stride) {
     const int64_t part_stride = (int64_t)n_kv_heads * cache_stride;
     const dim3 grid((unsigned)(((int64_t)count * (head_dim / 4) + 255) / 256), (unsigned)n_kv_heads, 2);
     if (head_dim == 64)
         hipLaunchKernelGGL((k_kv_parts<__bf16, 3>), grid, dim3(256), 0, dev->stream, k_cache, v_cache, cache_stride, (__bf16 *)parts,
-                           (__bf16 *)parts + 3 * part_stride, part_stride, lo, count, head_dim / 4);
+                           (__bf16 *)parts + 3 * part_stride, part_stride, count, head_dim / 4);
     else
         hipLaunchKernelGGL((k_kv_parts<_Float16, 2>), grid, dim3(256), 0, dev->stream, k_cache, v_cache, cache_stride, (_Float16 *)parts,
-                           (_Float16 *)parts + 2 * part_stride, part_stride, lo, count, head_dim / 4);
+                           (_Float16 *)parts + 2 * part_stride, part_stride, count, head_dim / 4);
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }
@@ -611,14 +626,17 @@ int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, cons
     if (head_dim % 8 == 0 && k == q + q_count && v == k + kv_count && dev->opt.prefill_fold_split_sums) {
         // q, k and v end to end: four pairs per thread, and the partial copies of a split contraction summed on the way
         const int64_t total4 = (int64_t)n * (n_heads + 2 * n_kv_heads) * (head_dim / 8);
-        const dim3 grid4((unsigned)((total4 + 255) / 256));
+        const int64_t early = parts && !kv_f16 ? ((int64_t)pos0 * (head_dim / 4) + 255) / 256 : 0;
+        const int64_t blocks = (total4 + 255) / 256 + 2 * n_kv_heads * early;
+        CANDY_REQUIRE(blocks <= 0x7FFFFFFF, "prompt too long for one pass");
+        const dim3 grid4((unsigned)blocks);
         const float *src = pending ? sp->part : q;
         const int n_split = pending ? sp->n_split : 1;
         const size_t stride = pending ? sp->stride : 0;
 #define CANDY_ROPE4(KV, T, P)                                                                                                            \
     hipLaunchKernelGGL((k_prefill_rope_kv4<KV, T, P>), grid4, dim3(256), 0, dev->stream, q, src, n_split, stride, cos_t, sin_t,          \
                        (KV *)k_cache, (KV *)v_cache, n, pos0, n_heads, n_kv_heads, head_dim, cache_stride, (T *)parts,                   \
-                       (T *)parts + P * part_stride, part_stride)
+                       (T *)parts + P * part_stride, part_stride, (unsigned)early)
         if (kv_f16) CANDY_ROPE4(_Float16, _Float16, 0);
         else if (!parts) CANDY_ROPE4(float, _Float16, 0);
         else if (head_dim == 64) CANDY_ROPE4(float, __bf16, 3);
@@ -638,7 +656,7 @@ int launch_prefill_rope_kv(candy_hip_device *dev, float *q, const float *k, cons
         hipLaunchKernelGGL(k_prefill_rope_kv<float>, grid, dim3(256), 0, dev->stream, q, k, v, cos_t, sin_t,
                            (float *)k_cache, (float *)v_cache, n, pos0, n_heads, n_kv_heads, head_dim, cache_stride);
     CANDY_LAUNCH_CHECK();
-    return parts && !kv_f16 ? launch_kv_parts(dev, (const float *)k_cache, (const float *)v_cache, parts, pos0, n, n_kv_heads, head_dim, cache_stride)
+    return parts && !kv_f16 ? launch_kv_parts(dev, (const float *)k_cache, (const float *)v_cache, parts, pos0 + n, n_kv_heads, head_dim, cache_stride)
                             : CANDY_HIP_OK;
 }
 
@@ -698,9 +716,6 @@ int launch_attn_prefill(candy_hip_device *dev, const float *q, const void *k_cac
         else
             launch_attn_mfma<128, _Float16, 1, 2, 2>(dev, q, kh, vh, 0, out, n, pos0, n_heads, n_kv_heads, cache_stride, scale, xh_out);
     } else {
-        // the rope launch has left the new rows' parts; those of the positions in front may be another layer's
-        if (pos0 > 0)
-            if (int rc = launch_kv_parts(dev, kf, vf, parts, 0, pos0, n_kv_heads, head_dim, cache_stride)) return rc;
         const int64_t ps = (int64_t)n_kv_heads * cache_stride;
         const __bf16 *pb = (const __bf16 *)parts;
         const _Float16 *ph = (const _Float16 *)parts;
