@@ -751,8 +751,9 @@ int launch_window_prompt(candy_hip_device *dev, const WindowAttn &A, int n, int 
         hipLaunchKernelGGL((k_window_attn_prompt<DP>), g, b, 0, dev->stream, a, (const bf16 *)A.q, (const bf16 *)A.k_cache,        \
                            (const bf16 *)A.v_cache, (bf16 *)A.out, n, pos0);                                                      \
         break
-    // direct loads place 16-byte pieces in eights; the other widths keep the kernel that stages through registers (rows of
-    // 128, us: 112 there, 84 with direct loads)
+    // rows of 128, us: 112 in the kernel that stages through registers, 84 with direct loads.  Those place 16-byte pieces in eights,
+    // which rows of 32 and 96 are not; rows of 192 and 256 would be, but two of their tiles leave a CU room for one workgroup (98 and
+    // 131 KB of LDS): not tried
 #define CANDY_WT(DP)                                                                                                              \
     case DP:                                                                                                                      \
         if (a.cap > 0.0f)                                                                                                          \

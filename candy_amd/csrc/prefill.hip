@@ -664,8 +664,6 @@ template <int HD, class T, int KVP, int QP, int PP>
 static void launch_attn_mfma(candy_hip_device *dev, const float *q, const T *kparts, const T *vparts, int64_t part_stride, float *out, int n,
                              int pos0, int n_heads, int n_kv_heads, int64_t cache_stride, float scale, _Float16 *xh_out,
                              const float *k_cache = nullptr, const float *v_cache = nullptr) {
-    // Two key groups per workgroup (64 queries, alternate tiles of 32 keys) where the launch lasts as long as its longest
-    // walk; 128 queries and one group where there are workgroups enough to fill the chip twice over.
     // 64 queries per workgroup and two groups of wavefronts on alternate tiles of 32 keys, because a launch lasts as long
     // as its longest walk; 128 queries where the tiles of an f32 cache (96 or 128 KB for two steps) leave a CU room for
     // one workgroup and there are more than two of the small ones per CU.  us, 64 / 128 queries: head_dim 64, f32 cache,

@@ -88,6 +88,9 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *   "mmq.f16_api_min_m"          33       the same for one contraction through candy_hip_qmatmul / candy_hip_qmatmul_q8 (one
  *                                         matmul: 3e-4 < 1e-3): Q4_K and Q6_K from this many rows, the other formats from 65
  *                                         or this if larger
+ *   "prefill.kv_parts_mb"        0        prompt attention on an f32 cache: MB at most for the 16-bit parts of a layer's K and
+ *                                         V that the matrix cores contract, 1 to 1.5 times one layer's cache for max_pos
+ *                                         (0: no limit).  Past the limit, and where the allocation fails, the vector ALU
  *   -- comparison / test only --
  *   "matvec.span"                1        batch-1 kernel of 2-byte aligned formats fetches aligned 16-byte spans
  *   "matvec.small_batch_kernel"  1        2..8 rows on the one-workgroup-per-CU kernel (0: looping kernel)
@@ -122,9 +125,6 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *                                         launch that follows (RMSNorm + quantize behind o / down, rope behind q / k / v;
  *                                         0: a launch of its own sums them)
  *   "prefill.attention_valu"     0        comparison runs: prompt attention on the vector ALU
- *   "prefill.kv_parts_mb"        0        prompt attention on an f32 cache: MB at most for the 16-bit parts of a layer's K and
- *                                         V that the matrix cores contract, 1 to 1.5 times one layer's cache for max_pos
- *                                         (0: no limit).  Past the limit, and where the allocation fails, the vector ALU
  *   "prefill.attention_groups"   0        comparison runs: matrix-core prompt attention with one (1) or two (2) groups of
  *                                         wavefronts per query tile that take alternate key tiles (0: two, with 64 or 128
  *                                         queries by the size of the grid)

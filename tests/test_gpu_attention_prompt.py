@@ -213,3 +213,27 @@ def test_prompt_without_memory_for_parts(dev, head_dim, n):
         got = rows("prefill.kv_parts_mb", 0, cut)
         level = np.max(np.abs(want).reshape(len(want), -1, 32), axis=2, keepdims=True) / 127
         assert np.mean(np.abs(got - want).reshape(len(want), -1, 32) > 0.5 * level) <= SHARE, cut
+
+
+# The parts of earlier positions come out of the rope launch, or (split sums not folded) out of one of their own: the same bits.
+# Those positions are cached by decode steps here, so that the parts an earlier prompt left are another sequence's.
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(8, 2, 64), (4, 2, 128)])
+@pytest.mark.parametrize("cut,n", [(1, 2), (33, 40), (70, 3)])
+def test_parts_of_earlier_positions(dev, heads, kv_heads, head_dim, cut, n):
+    model = mirror(dev, heads, kv_heads, head_dim, 300, 1.0, 1.0)
+    tokens = [int(t) for t in np.random.default_rng(cut).integers(0, 256, cut + n)]
+    model.prefill(tokens[::-1], 0, want_logits=False)
+    for p in range(cut):
+        model.decode(tokens[p], p, want_logits=False)
+    want, got = both(dev, model, tokens[cut:], cut)
+    level = np.max(np.abs(want).reshape(n, -1, 32), axis=2, keepdims=True) / 127
+    assert np.mean(np.abs(got - want).reshape(n, -1, 32) > 0.5 * level) <= max(SHARE, 2 / want.size)
+    model.prefill(tokens[::-1], 0, want_logits=False)
+    for p in range(cut):
+        model.decode(tokens[p], p, want_logits=False)
+    dev.set_option("prefill.fold_split_sums", 0)
+    try:
+        model.prefill(tokens[cut:], cut, want_logits=False)
+        assert np.array_equal(model.prompt_hidden(n), got)
+    finally:
+        dev.set_option("prefill.fold_split_sums", 1)
