@@ -320,9 +320,9 @@ __global__ __launch_bounds__(256, 2) void k_dense_mm(const bf16 *__restrict__ W,
 
 // ------------------------------------------------------------------ prompt batches, bfloat16, large tiles
 // Tile: BN weight rows x BM activation rows, 64 values of K per stage, one workgroup of eight wavefronts (WN x WM) per CU;
-// a stage lies in LDS as in k_dense_mm.  What bounds it: the chip's power (the clock falls from 2.4 to 2.0 - 2.2 GHz) and, per
-// step of 256 x 256, 2 050 of 3 200 cycles of matrix instructions; without the loads the steps take 83 %, without the LDS
-// reads 91 % of the time.  Against two workgroups per CU of 128 x 128 tiles whose four wavefronts read all fragments of a
+// a stage lies in LDS as in k_dense_mm.  What bounds it: the chip's power (at 2000 rows the clock falls
+// from 2.4 to 2.0 GHz) and the matrix instructions, busy 50 - 61 % of a CU's cycles (a step of 256 x 256 is 2 048 cycles of them),
+// with fragment reads and the wait for a stage in between; no bank conflicts.  Against two workgroups per CU of 128 x 128 tiles whose four wavefronts read all fragments of a
 // half stage and then multiply: a wavefront's tile is up to twice as large, so that a fragment read meets more matrix
 // instructions (an eighth to a quarter fewer LDS reads); the fragments of the next half stage are read while this one is
 // multiplied; a stage's loads are requested when its place is free and have a step (two with three stages) to arrive.

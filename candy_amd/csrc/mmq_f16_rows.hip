@@ -11,6 +11,7 @@
 // rows, 11008 x 4096, before (with the split sum) -> now: Q4_K 22.8 + 4.5 -> 20.6, Q8_0 35.1 + 4.5 -> 24.0, Q4_0 33.4 + 4.5 ->
 // 21.2, Q5_K 31.5 + 4.5 -> 25.1; 2048 x 1024 Q8_0 13.0 + 4.1 -> 5.7.  What bounds it: the activations, which every CU reads
 // (655 KB here, 10 us), then the weights (48 MB of Q8_0, 8 us), half overlapped.
+#include <algorithm>
 #include <type_traits>
 
 #include "f16_weights.h"
@@ -69,8 +70,8 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
     if (count > 0) {
         // Unstaged blocks are requested a super-block ahead, but three fragments of them twice over do not fit the registers: 41
         // spilled at 64 rows, us, two sets / one: 11008 x 4096, 48 rows 28.1 / 26.1, x 2048, 40 rows 15.4 / 14.6.  (Two fragments
-        // and 128 rows spill 35, and come with one super-block per wavefront at most.)
-        constexpr int DEEP = STAGED || RF == 3 || RF * MF == 16 ? 1 : 2;
+        // and 128 rows spill 35 and are ahead with two sets all the same: 4200 x 1024 13.2 / 14.7, 8192 x 1536 18.1 / 18.1.)
+        constexpr int DEEP = STAGED || RF == 3 ? 1 : 2;
         typename F::Raw raw[DEEP][RF];
         half8 xf[2][MF];
         auto load_w = [&](int sb, int u) __attribute__((always_inline)) {
@@ -166,21 +167,33 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
 
 static int fragments(int64_t m) { return m <= 48 ? 3 : m <= 64 ? 4 : m <= 80 ? 5 : m <= 96 ? 6 : 8; }
 
-// 16-row weight fragments per workgroup with which one round of workgroups serves every row and this kernel is ahead of the tiles
-// of mmq_f16.hip; 0: none, the tiles.  A second round would read the activations again, and wider workgroups have no registers
-// for their sums.  Where the lines lie, us of a call, this kernel / tiles (1632 calls timed, sizes at and around each line):
-//   * weight rows for at least half of the CUs, from 2048
-//   * super-blocks for the wavefronts: with few of a cheap format the tiles' steps are short (11008 x 512, 80 rows, Q4_K 11.7 /
-//     10.8, Q5_K 13.3 / 12.4; x 1024 ahead; the others 256 long 10.2 / 9.7); no round of them that most wavefronts sit out
-//     (Q6_K 8200 x 2304, nine of them, 64 rows 21.6 / 19.9; x 2560 20.2 / 21.7)
-//   * a workgroup reads every activation, which a CU takes in at about 65 KB a us when all read: Q8_0 and Q4_0 700 KB (688 KB
-//     1.15 to 1.5 times as fast as the tiles); Q4_K and Q5_K, whose tiles cost less, 660 (4100 x 4096, 80 rows, 655 KB ahead, x 4352
-//     19.5 / 19.0 and 22.1 / 21.1); Q6_K, not staged, 450 for one fragment and 340 (8200 x 4096, 48 rows, 393 KB 25.8 / 26.1, x 4352
-//     31.3 / 25.6; 8200 x 3328, 64 rows, 426 KB 28.9 / 24.1, 328 KB 20.2 / 21.7)
-//   * Q4_K and Q5_K with many sums per wavefront: one round of super-blocks (8192 x 2304, 128 rows 24.7 / 17.8 and 22.8 / 20.4;
-//     96 rows 18.1 / 16.6 and 19.4 / 18.9); two fragments and 128 rows of Q4_K not at all (8192 x 1536 16.4 / 15.4)
+// What a call takes, us, here and on the 128 x 128 tiles of mmq_f16.hip: both fitted to 2940 calls (five formats, 2048 .. 12288 weight
+// rows, K 512 .. 6144, 48 .. 128 activation rows; the fits are 3 to 6 % off on average).  A line on any one size does not divide them:
+// a round of super-blocks that most wavefronts sit out, a split that leaves the tiles short, an odd number of 210-byte blocks (rows
+// 2 bytes off) each move it.
+struct RowsCost {
+    // a launch; a tile's super-block; a split's launch; MB of its copies; 1000 super-blocks of all tiles
+    float tile[5];
+    // a launch; a round of super-blocks: weight fragment, activation fragment; a super-block: activation fragment (read by every CU),
+    // weight fragment, the same of odd rows of Q6_K; the sums of a fragment pair; MB of results
+    float rows[8];
+};
+static const RowsCost &rows_cost(int fmt) {
+    static constexpr RowsCost Q4K{{8.03f, 1.13f, 3.39f, 0.25f, 2.82f}, {2.28f, 0.19f, 0.49f, 0.05f, 0.08f, 0.0f, 0.22f, 0.74f}},
+        Q5K{{8.50f, 1.73f, 3.73f, 0.19f, 4.33f}, {4.30f, 0.04f, 0.64f, 0.02f, 0.20f, 0.0f, 0.05f, 0.89f}},
+        Q6K{{9.42f, 1.45f, 3.36f, 0.21f, 4.00f}, {3.48f, 0.00f, 0.06f, 0.11f, 0.30f, 0.08f, 0.11f, 0.88f}},
+        Q80{{11.57f, 1.35f, 4.29f, 0.10f, 5.11f}, {3.12f, 0.41f, 0.16f, 0.11f, 0.09f, 0.0f, 0.00f, 1.39f}},
+        Q40{{11.50f, 0.95f, 5.15f, 0.05f, 6.95f}, {4.07f, 0.30f, 0.29f, 0.09f, 0.07f, 0.0f, 0.00f, 1.02f}};
+    return fmt == CANDY_HIP_Q4_K ? Q4K : fmt == CANDY_HIP_Q5_K ? Q5K : fmt == CANDY_HIP_Q6_K ? Q6K : fmt == CANDY_HIP_Q8_0 ? Q80 : Q40;
+}
+
+// 16-row weight fragments per workgroup with which one round of workgroups serves every row and this kernel is ahead of the tiles; 0:
+// none, the tiles.  A second round would read the activations again, wider workgroups have no registers for their sums; fewer than
+// 2048 weight rows leave half of the CUs idle.  Of the 2940 calls 26 take more than 2 % longer than on the tiles (16 % at most), and all together
+// 0.3 % more than the faster kernel for each.  us of a call, tiles / here: Q8_0 4096 x 2304, 80 rows 20.7 / 12.5, Q4_K 4096 x 2304, 48 rows
+// 15.2 / 9.7, Q6_K 8192 x 2048, 96 rows 19.3 / 17.0, 11008 x 4096, 48 rows 34.6 / 28.1, 8200 x 3840, 48 rows 25.4 / 28.9 (tiles).
 static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
-    const bool q6k = fmt == CANDY_HIP_Q6_K, cheap = fmt == CANDY_HIP_Q4_K || fmt == CANDY_HIP_Q5_K;
+    const bool q6k = fmt == CANDY_HIP_Q6_K;
     // up to 64 rows the other formats are on the exact tiles (mmq_f16_big_covers)
     if (m > 128 || (m <= 64 && !q6k && fmt != CANDY_HIP_Q4_K) || rows < 2048 || cols % 256 != 0) return 0;
     const int mf = fragments(m);
@@ -188,16 +201,24 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
     while ((rows + 16 * rf - 1) / (16 * rf) > num_cus)
         if (++rf > 3) return 0;
     if (rf == 3 && mf > (q6k ? 4 : 6)) return 0;
-    const int64_t blocks = cols / 256, rounds = (blocks + 7) / 8;
-    if (blocks < (cheap ? 4 : 2) || (rounds > 1 && 5 * blocks < 3 * 8 * rounds)) return 0;
-    if (cheap && (mf == 8 || (mf == 6 && rf == 2)) && rounds > 1) return 0;
-    if (fmt == CANDY_HIP_Q4_K && mf == 8 && rf == 2) return 0;
-    return mf * 32 * cols <= (q6k ? (rf == 1 ? 450000 : 340000) : cheap ? 660000 : 700000) ? rf : 0;
+    if (mf * 32 * cols > 1200000) return 0;  // not measured
+    const int64_t blocks = cols / 256, rounds = (blocks + 7) / 8, tiles = (rows + 127) / 128;
+    // as plan_split() deals K to the tiles' workgroups
+    int64_t splits = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(num_cus / tiles, blocks / 2), 16));
+    const int64_t per = (blocks + splits - 1) / splits;
+    splits = (blocks + per - 1) / per;
+    const RowsCost &c = rows_cost(fmt);
+    const float out = (float)(rows * m) * 4e-6f;
+    float tile = c.tile[0] + c.tile[1] * (float)per + c.tile[4] * 1e-3f * (float)(tiles * blocks);
+    if (splits > 1) tile += c.tile[2] + c.tile[3] * (float)(splits + 1) * out;
+    const float here = c.rows[0] + (float)rounds * (c.rows[1] * rf + c.rows[2] * mf) + (float)blocks * (c.rows[3] * mf + c.rows[4] * rf) +
+                       (blocks & 1 ? c.rows[5] * (float)(blocks * rf) : 0.0f) + c.rows[6] * (float)(rf * mf) + c.rows[7] * out;
+    return here < tile ? rf : 0;
 }
 template <class F, int RF, int MF>
 constexpr bool reached() {
     constexpr bool q4k = std::is_same<F, BigQ4K>::value, q6k = std::is_same<F, BigQ6K>::value;
-    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= (q6k ? 4 : 6)) && !(q4k && RF == 2 && MF == 8);
+    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= (q6k ? 4 : 6));
 }
 
 template <class F, int RF, int MF>

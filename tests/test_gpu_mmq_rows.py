@@ -27,14 +27,15 @@ def fragments(m):
 
 def shapes():
     """Per kernel: the fewest rows on either side with as many super-blocks as the rule allows of 4097 values, and the most rows (less one
-    weight row, a length not in fours) with few of them."""
+    weight row, a length not in fours) with as few of them."""
     for fmt in FORMATS:
         for rf, (few, most) in WEIGHT_ROWS.items():
             for mf, (low, high) in FRAGMENTS.items():
-                longest = max((c for c in range(256, 4097, 256) if chosen(fmt, low, few + 1, c) == rf), default=0)
-                if longest:
-                    yield fmt, rf, mf, low, few + 1, longest
-                    yield fmt, rf, mf, high, most - 1, 1024
+                lengths = range(256, 4097, 256)
+                for m, rows, pick in ((low, few + 1, max), (high, most - 1, min)):
+                    cols = pick((c for c in lengths if chosen(fmt, m, rows, c) == rf), default=0)
+                    if cols:
+                        yield fmt, rf, mf, m, rows, cols
 
 
 SHAPES = list(shapes())
@@ -62,7 +63,7 @@ def test_rows_against_tiles_and_oracle(dev, fmt, rf, mf, m, rows, cols):
     finally:
         dev.set_option("mmq.f16_shape", 0)
     top = np.max(np.abs(tiles))
-    assert not np.array_equal(got, tiles)  # two kernels: another order of the sums
+    assert cols == 256 or not np.array_equal(got, tiles)  # two kernels: another order of the sums (of a single super-block the same)
     # the same products in another order: K sums of f32, 2^-24 each of a partial sum no larger than the largest result's
     # order (random signs: sqrt(K) of them, 64 * 2^-24 = 4e-6 at K = 4096)
     assert np.max(np.abs(got - tiles)) <= 4e-6 * top
@@ -85,17 +86,18 @@ def test_one_round_of_workgroups_and_bounded_activations():
         if rf:
             assert m <= 128 and rows >= 2048 and -(-rows // (16 * rf)) <= cus
             assert m > 64 or fmt in (synth.Q4_K, synth.Q6_K)
-            assert fragments(m) * 32 * cols <= 700e3
+            assert fragments(m) * 32 * cols <= 1.2e6
             seen.add((fmt, rf, fragments(m)))
     assert seen == {s[:3] for s in SHAPES}  # no kernel but those tested above
 
 
 @pytest.mark.parametrize("fmt,m,rows,cols,rf", [
     (synth.Q8_0, 77, 11008, 4096, 3), (synth.Q8_0, 128, 2048, 1024, 1), (synth.Q4_K, 80, 4096, 4096, 1), (synth.Q4_K, 33, 4096, 5632, 1),
-    (synth.Q6_K, 48, 11008, 3328, 3), (synth.Q6_K, 64, 8200, 2560, 3),
-    # where the tiles are ahead: long rows, too many of them, few super-blocks, a round that most wavefronts sit out
+    (synth.Q6_K, 48, 11008, 4096, 3), (synth.Q6_K, 48, 8192, 4096, 2), (synth.Q6_K, 96, 8192, 2048, 2), (synth.Q6_K, 80, 4096, 2304, 1),
+    (synth.Q8_0, 96, 4096, 2304, 1), (synth.Q4_0, 80, 12288, 2304, 3), (synth.Q4_K, 48, 4096, 512, 1),
+    # where the tiles are ahead: long rows, too many of them, rounds that most wavefronts sit out, odd rows of Q6_K
     (synth.Q8_0, 77, 4096, 14336, 0), (synth.Q8_0, 77, 14336, 4096, 0), (synth.Q8_0, 129, 4096, 1024, 0), (synth.Q8_0, 64, 4096, 1024, 0),
-    (synth.Q4_K, 80, 11008, 512, 0), (synth.Q6_K, 64, 8200, 2304, 0), (synth.Q6_K, 64, 8200, 3328, 0), (synth.Q4_K, 128, 8192, 1536, 0),
-    (synth.Q5_K, 128, 8192, 2304, 0), (synth.Q4_K, 96, 8192, 2816, 0), (synth.Q4_K, 80, 4100, 4352, 0)])
+    (synth.Q6_K, 64, 8200, 3328, 0), (synth.Q6_K, 48, 8200, 3840, 0), (synth.Q5_K, 128, 8192, 2304, 0), (synth.Q4_K, 128, 8192, 2304, 0),
+    (synth.Q4_K, 80, 4200, 4352, 0)])
 def test_where_the_lines_lie(fmt, m, rows, cols, rf):
     assert chosen(fmt, m, rows, cols) == rf
