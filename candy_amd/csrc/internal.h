@@ -63,6 +63,7 @@ struct Options {
     int f16_split = 0;           // comparison runs: workgroups that share one fp16 tile's K (0: by grid size)
     int mmv_min_m = 3;           // f32 x Q4_K with this many .. mmv_max_m rows: the one-pass int8 kernel
     int mmv_max_m = 32;          //   (0: never; more than 16 rows only for rows of up to 4096 values)
+    int rows_i8 = 1;             // 3 .. 255 rows: the kernel that deals K to wavefronts, where it is ahead (0: never; nor with mmv.max_m 0)
     int mmv_variant = 0;         // comparison runs: 1 = one 16-row strip per wavefront, 2 = two
     int pair_rows = 0;           // fused gate/up: row pairs per workgroup, 32 / 16 / 8 (0: the most even split)
     int rms_rows = 0;            // fused RMSNorm prologue: rows per workgroup, 16 / 24 (0: the most even split)
@@ -227,10 +228,12 @@ bool mmq_f16_group_covers(const candy_hip_qtensor *const *ws, int count, int64_t
 int launch_mmq_f16_group(candy_hip_device *dev, const candy_hip_qtensor *const *ws, float *const *ys, int count,
                          const _Float16 *xh, int64_t m);
 // ops.hip: fused decode-step stages (all enqueue on dev->stream, no allocation, no sync).
+struct RowsImage;  // rows_i8.h: the image takes the place of qs, scales and xh
 int launch_rms_norm_quant(candy_hip_device *dev, const float *x, const float *alpha, float eps, int64_t rows,
-                          int64_t cols, float *xn_out, int8_t *qs, Q8Scale *scales, _Float16 *xh = nullptr);
+                          int64_t cols, float *xn_out, int8_t *qs, Q8Scale *scales, _Float16 *xh = nullptr,
+                          const RowsImage *image = nullptr);
 int launch_silu_mul_quant(candy_hip_device *dev, const float *gate, const float *up, int64_t rows, int64_t cols,
-                          float *act_out, int8_t *qs, Q8Scale *scales, _Float16 *xh = nullptr);
+                          float *act_out, int8_t *qs, Q8Scale *scales, _Float16 *xh = nullptr, const RowsImage *image = nullptr);
 // fused.hip: batch-1 contraction of one activation row with up to three weights, with optional
 // RMSNorm+quantize prologue (x != nullptr, else planar Q8_0 in xq/xs), residuals, or the
 // gate/up SiLU*Mul+quantize epilogue (pair). Returns CANDY_HIP_ERR_UNSUPPORTED when the shape
@@ -309,6 +312,7 @@ struct ActWorkspace {
     Q8Scale *scales;
     void *half_ws;
     void *mmv_ws = nullptr;  // operand-order activations for the small-batch int8 kernel (2 .. 32 rows)
+    void *rows_ws = nullptr; // the same for the kernel that deals K to wavefronts (3 .. 255 rows)
 };
 int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quants, ActWorkspace *out);
 // matvec.hip: y[m, rows] = x . W^T for any m from planar activations that live OUTSIDE the device

@@ -9,6 +9,7 @@
 
 #include "blocks.h"
 #include "decoder.h"
+#include "rows_i8.h"
 
 struct candy_hip_llama final : candy_hip_decoder {
     candy_hip_llama_config cfg{};
@@ -39,6 +40,7 @@ struct candy_hip_llama final : candy_hip_decoder {
         int8_t *xq = nullptr;
         candy::Q8Scale *xs = nullptr;
         _Float16 *xh = nullptr;  // the quantized activations as fp16 (d * q), for the fp16 tile kernels
+        uint8_t *image = nullptr;  // and as operands of the exact kernel for 3 to 255 rows
     } pf;
 
     int check_complete() const override;
@@ -341,6 +343,7 @@ int candy_hip_llama::reserve_prompt(int n) {
     if (!rc) rc = prompt_alloc(m, &P.xq, N * widest);
     if (!rc) rc = prompt_alloc(m, &P.xs, N * (widest / 32));
     if (!rc) rc = prompt_alloc(m, &P.xh, (size_t)mmq_m_pad(n) * widest);  // the tile kernel reads whole tiles of rows
+    if (!rc) rc = prompt_alloc(m, &P.image, rows_image_bytes(std::min(n, 255), (int64_t)widest));
     return rc;
 }
 
@@ -378,9 +381,47 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
         pend.n_split = 0;
         return e;
     };
+    // Weights that share their activations on one grid where they are of one format, else one after the other.
+    auto rows_linear = [&](const candy_hip_qtensor *const *ws, float *const *ys, const float *res, int count, const RowsImage &x) -> int {
+        bool one = true;
+        for (int i = 1; i < count; ++i) one = one && ws[i]->fmt == ws[0]->fmt;
+        for (int i = 0; i < count; i += one ? count : 1) {
+            RowsLaunch R;
+            R.n = one ? count : 1;
+            R.x = x;
+            for (int k = 0; k < R.n; ++k) { R.w[k] = ws[i + k]; R.y[k] = ys[i + k]; R.res[k] = res; }
+            if (int e = launch_rows_i8(dev, R, n)) return e;
+        }
+        return CANDY_HIP_OK;
+    };
     for (int l = 0; l < c.n_layers; ++l) {
         const candy_hip_llama::Layer &L = m->layers[l];
         void *kc = cache.k_of(l), *vc = cache.v_of(l);
+        // Every projection on the exact kernel for 3 to 255 rows: the launches in front write its operands, q / k / v and gate / up
+        // are a grid each, residuals ride in the epilogue, nothing is split: ten launches (24 tokens of the 1B shape: 22 before).
+        bool exact_rows = pend.n_split == 0;
+        for (const candy_hip_qtensor *w : {L.wq, L.wk, L.wv, L.wo, L.gate, L.up, L.down})
+            exact_rows = exact_rows && !mmq_f16_big_covers(w, n) && rows_i8_takes(w, n);
+        if (exact_rows) {
+            const RowsImage xd = rows_image(P.image, n, c.d_model), xq = rows_image(P.image, n, qd), xf = rows_image(P.image, n, c.d_ffn);
+            const candy_hip_qtensor *qkv[3] = {L.wq, L.wk, L.wv}, *gu[2] = {L.gate, L.up};
+            float *qkv_y[3] = {P.q, P.k, P.v}, *gu_y[2] = {P.gate, P.up};
+            if ((rc = launch_rms_norm_quant(dev, P.h, L.attn_norm, c.rms_eps, n, c.d_model, nullptr, nullptr, nullptr, nullptr, &xd))) return rc;
+            if ((rc = rows_linear(qkv, qkv_y, nullptr, 3, xd))) return rc;
+            if ((rc = launch_prefill_rope_kv(dev, P.q, P.k, P.v, m->cos_t, m->sin_t, kc, vc, m->kv_f16, n, pos0, c.n_heads, c.n_kv_heads,
+                                             c.head_dim, cache_stride, parts, &pend)))
+                return rc;
+            if ((rc = launch_attn_prefill(dev, P.q, kc, vc, m->kv_f16, parts, P.att, n, pos0, c.n_heads, c.n_kv_heads, c.head_dim, cache_stride,
+                                          scale, nullptr)))
+                return rc;
+            if ((rc = launch_rows_quantize(dev, P.att, n, qd, xq))) return rc;
+            if ((rc = rows_linear(&L.wo, &P.h, P.h, 1, xq))) return rc;  // h += Wo . att
+            if ((rc = launch_rms_norm_quant(dev, P.h, L.ffn_norm, c.rms_eps, n, c.d_model, nullptr, nullptr, nullptr, nullptr, &xd))) return rc;
+            if ((rc = rows_linear(gu, gu_y, nullptr, 2, xd))) return rc;
+            if ((rc = launch_silu_mul_quant(dev, P.gate, P.up, n, c.d_ffn, nullptr, nullptr, nullptr, nullptr, &xf))) return rc;
+            if ((rc = rows_linear(&L.down, &P.h, P.h, 1, xf))) return rc;  // h += Wdown . act
+            continue;
+        }
         // Where a projection runs on the fp16 tiles, the kernel that quantizes its input also writes the
         // fp16 expansion (one conversion for q/k/v, one for gate/up), and the residual add rides in the
         // projection's epilogue.

@@ -17,6 +17,7 @@
 
 #include "blocks.h"
 #include "internal.h"
+#include "rows_i8.h"
 #include "units.h"
 #include "formats_more.h"
 
@@ -767,12 +768,14 @@ int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quan
     const size_t s_bytes = need_quants ? (((size_t)(m * (cols >> 5)) * sizeof(Q8Scale) + 255) & ~(size_t)255) : 0;
     const size_t h_bytes = m >= 16 ? (size_t)(mmq_m_pad(m) * cols) * 2 : 0;
     const size_t v_bytes = need_quants && m >= 2 && m <= 32 && cols % 256 == 0 ? mmv_workspace_bytes(cols) : 0;
+    const size_t r_bytes = m >= 3 && m <= 255 && cols % 256 == 0 ? (rows_image_bytes(m, cols) + 255) & ~(size_t)255 : 0;
     void *ws = nullptr;
-    if (int rc = workspace(dev, q_bytes + s_bytes + h_bytes + v_bytes + 256, &ws)) return rc;
+    if (int rc = workspace(dev, q_bytes + s_bytes + h_bytes + r_bytes + v_bytes + 256, &ws)) return rc;
     out->qs = (int8_t *)ws;
     out->scales = (Q8Scale *)((uint8_t *)ws + q_bytes);
     out->half_ws = h_bytes ? (uint8_t *)ws + q_bytes + s_bytes : nullptr;
-    out->mmv_ws = v_bytes ? (uint8_t *)ws + q_bytes + s_bytes + h_bytes : nullptr;
+    out->rows_ws = r_bytes ? (uint8_t *)ws + q_bytes + s_bytes + h_bytes : nullptr;
+    out->mmv_ws = v_bytes ? (uint8_t *)ws + q_bytes + s_bytes + h_bytes + r_bytes : nullptr;
     return CANDY_HIP_OK;
 }
 
@@ -850,8 +853,21 @@ int noalloc_scratch_init(candy_hip_device *dev) {
 
 int mmq_min_m(const candy_hip_device *dev) { return dev->opt.mmq_min_m < 16 ? 16 : dev->opt.mmq_min_m; }
 
+static RowsLaunch rows_launch(const candy_hip_qtensor *w, int64_t m, float *y, const float *res, void *ws) {
+    RowsLaunch L;
+    L.n = 1; L.w[0] = w; L.y[0] = y; L.res[0] = res; L.x = rows_image(ws, m, w->cols);
+    return L;
+}
+
 int launch_contract(candy_hip_device *dev, const candy_hip_qtensor *w, const int8_t *qs, const Q8Scale *scales,
                     int64_t m, float *y, const _Float16 *xh_ready, const float *res) {
+    if (!xh_ready && !mmq_f16_big_covers(w, m) && rows_i8_picks(w, m, true)) {
+        ActWorkspace a;
+        if (int rc = act_workspace(dev, m, w->cols, false, &a)) return rc;
+        const RowsLaunch L = rows_launch(w, m, y, res, a.rows_ws);
+        if (int rc = launch_rows_pack_planar(dev, qs, scales, m, w->cols, L.x)) return rc;
+        return launch_rows_i8(dev, L, m);
+    }
     if (m < mmq_min_m(dev)) {
         CANDY_REQUIRE(res != y, "internal: in-place residual needs the fused epilogue");
         if (int rc = launch_matvec(dev, w, qs, scales, m, y)) return rc;
@@ -877,6 +893,11 @@ static int qmatmul_check(candy_hip_device *dev, const candy_hip_qtensor *w, int6
 }
 
 static int contract(candy_hip_device *dev, const candy_hip_qtensor *w, const ActWorkspace &a, int64_t m, float *y) {
+    if (a.rows_ws && rows_i8_picks(w, m, false)) {
+        const RowsLaunch L = rows_launch(w, m, y, nullptr, a.rows_ws);
+        if (int rc = launch_rows_pack_planar(dev, a.qs, a.scales, m, w->cols, L.x)) return rc;
+        return launch_rows_i8(dev, L, m);
+    }
     return m < mmq_min_m(dev) ? launch_matvec(dev, w, a.qs, a.scales, m, y)
                                : launch_mmq(dev, w, a.qs, a.scales, m, y, a.half_ws, nullptr, nullptr, dev->opt.f16_api_min_m);
 }
@@ -890,6 +911,11 @@ static int qmatmul_f32(candy_hip_device *dev, const candy_hip_qtensor *w, const 
         Wd.n = 1; Wd.w[0] = w; Wd.y[0] = dev_y; Wd.x = dev_x;
         const int rc = launch_matvec_wide(dev, Wd);
         if (rc != CANDY_HIP_ERR_UNSUPPORTED) return rc;
+    }
+    if (a.rows_ws && rows_i8_picks(w, m, false)) {
+        const RowsLaunch L = rows_launch(w, m, dev_y, nullptr, a.rows_ws);
+        if (int rc = launch_rows_quantize(dev, dev_x, m, w->cols, L.x)) return rc;
+        return launch_rows_i8(dev, L, m);
     }
     if (a.mmv_ws && mmv_covers(w, m) && !matvec_even_covers(w, m)) return launch_mmv(dev, w, dev_x, nullptr, m, dev_y, a.mmv_ws);
     if (a.half_ws && m >= mmq_min_m(dev) && !dev->opt.mmq_fp16_only && mmq_f16_big_covers(w, m, dev->opt.f16_api_min_m)) {
@@ -942,6 +968,11 @@ int candy_hip_qmatmul_q8(candy_hip_device *dev, const candy_hip_qtensor *w, cons
     if (int rc = use_device(dev)) return rc;
     ActWorkspace a;
     if (int rc = act_workspace(dev, m, w->cols, true, &a)) return rc;
+    if (a.rows_ws && rows_i8_picks(w, m, false)) {
+        const RowsLaunch L = rows_launch(w, m, dev_y, nullptr, a.rows_ws);
+        if (int rc = launch_rows_pack_blocks(dev, dev_x_q8_0, m, w->cols, L.x)) return rc;
+        return launch_rows_i8(dev, L, m);
+    }
     if (a.mmv_ws && mmv_covers(w, m) && !matvec_even_covers(w, m)) return launch_mmv(dev, w, nullptr, dev_x_q8_0, m, dev_y, a.mmv_ws);
     if (int rc = launch_q8_blocks_to_planar(dev, dev_x_q8_0, m * (w->cols >> 5), a.qs, a.scales)) return rc;
     return contract(dev, w, a, m, dev_y);

@@ -19,6 +19,7 @@
 //     operands are exactly what lane (row j, pair c) and lane (activation row j, pair c) already hold.
 #include "blocks.h"
 #include "internal.h"
+#include "rows_i8.h"
 
 namespace candy {
 
@@ -42,10 +43,6 @@ struct MmvOperands {
     float *xd, *xm;
     size_t frag_stride, scale_stride;  // bytes / floats from one tile to the next
 };
-__device__ __forceinline__ size_t mmv_frag_offset(int r, int k) {
-    const int sb = k >> 8, t = (k >> 5) & 7, c = (k >> 3) & 3;
-    return ((size_t)((sb * 4 + (t >> 1)) * 64 + c * 16 + r)) * 16 + (t & 1) * 8 + (k & 7);
-}
 
 // f32 [m, K] -> Q8_0 (quantize_q8_1 without its sum, quantized.cu:3521-3558; the same lane code as the quantize
 // kernel, hence the same quants and scales) written in operand order for 16 rows.
@@ -62,7 +59,7 @@ __global__ __launch_bounds__(256) void k_mmv_quantize_pack(const float4 *__restr
     __half h;
     int bsum;
     const uint32_t packed = quantize_q8_lane4(v, h, bsum);
-    *(uint32_t *)(o.xfrag + tile * o.frag_stride + mmv_frag_offset(r, k)) = packed;
+    *(uint32_t *)(o.xfrag + tile * o.frag_stride + rows_frag_offset(r, k)) = packed;
     if ((k & 31) == 0) {
         const float d = __half2float(h);
         const size_t at = tile * o.scale_stride + ((size_t)(k >> 8) * 16 + r) * 8 + ((k >> 5) & 7);
@@ -95,10 +92,10 @@ __global__ __launch_bounds__(256) void k_mmv_pack_blocks(const BlockQ8_0 *__rest
     s = dot4_i8(a.x, ones, s); s = dot4_i8(a.y, ones, s); s = dot4_i8(a.z, ones, s); s = dot4_i8(a.w, ones, s);
     s = dot4_i8(c.x, ones, s); s = dot4_i8(c.y, ones, s); s = dot4_i8(c.z, ones, s); s = dot4_i8(c.w, ones, s);
     // values 8 chunk .. 8 chunk + 7 of the block go to lane (r, chunk) of its pair
-    *(u32x2 *)(xfrag + mmv_frag_offset(r, k)) = u32x2{a.x, a.y};
-    *(u32x2 *)(xfrag + mmv_frag_offset(r, k + 8)) = u32x2{a.z, a.w};
-    *(u32x2 *)(xfrag + mmv_frag_offset(r, k + 16)) = u32x2{c.x, c.y};
-    *(u32x2 *)(xfrag + mmv_frag_offset(r, k + 24)) = u32x2{c.z, c.w};
+    *(u32x2 *)(xfrag + rows_frag_offset(r, k)) = u32x2{a.x, a.y};
+    *(u32x2 *)(xfrag + rows_frag_offset(r, k + 8)) = u32x2{a.z, a.w};
+    *(u32x2 *)(xfrag + rows_frag_offset(r, k + 16)) = u32x2{c.x, c.y};
+    *(u32x2 *)(xfrag + rows_frag_offset(r, k + 24)) = u32x2{c.z, c.w};
     const size_t at = ((size_t)(k >> 8) * 16 + r) * 8 + ((k >> 5) & 7);
     xd[at] = d;
     xm[at] = d * (float)s;
@@ -295,6 +292,46 @@ static int launch_mmv_cfg(candy_hip_device *dev, const candy_hip_qtensor *w, con
     hipLaunchKernelGGL(kern, dim3((unsigned)(N / (16 * STRIPS))), dim3(WAVES * 64), S::SMEM, dev->stream,
                        (const uint8_t *)w->data, (const uint8_t *)o.xfrag, (const float *)o.xd, (const float *)o.xm, y, N, M, K,
                        o.frag_stride, o.scale_stride);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+
+// Planar quants -> the same operand order; one lane per 16 values.
+__global__ __launch_bounds__(256) void k_rows_pack_planar(const u32x4 *__restrict__ qs, const Q8Scale *__restrict__ scales, int m, int K,
+                                                         RowsImage o) {
+    const int per_row = K >> 4;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)m * per_row) return;
+    const int row = (int)(i / per_row), k = (int)(i - (int64_t)row * per_row) * 16, tile = row >> 4, r = row & 15;
+    const u32x4 q = qs[i];
+    uint8_t *frag = o.frag + tile * o.frag_stride;
+    *(u32x2 *)(frag + rows_frag_offset(r, k)) = u32x2{q.x, q.y};
+    *(u32x2 *)(frag + rows_frag_offset(r, k + 8)) = u32x2{q.z, q.w};
+    if ((k & 31) == 0) {
+        const Q8Scale sc = scales[(size_t)row * (K >> 5) + (k >> 5)];
+        const size_t at = tile * o.scale_stride + ((size_t)(k >> 8) * 16 + r) * 8 + ((k >> 5) & 7);
+        o.d[at] = sc.d;
+        o.m[at] = sc.d * (float)sc.bsum;
+    }
+}
+
+int launch_rows_quantize(candy_hip_device *dev, const float *x, int64_t m, int64_t K, const RowsImage &o) {
+    hipLaunchKernelGGL(k_mmv_quantize_pack, dim3((unsigned)(16 * ((m + 15) / 16) * (K >> 2) / 256)), dim3(256), 0, dev->stream,
+                       (const float4 *)x, (int)m, (int)K, o.frag, o.d, o.m, o.frag_stride, o.scale_stride);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+int launch_rows_pack_blocks(candy_hip_device *dev, const void *blocks, int64_t m, int64_t K, const RowsImage &o) {
+    const MmvOperands p = {o.frag, o.d, o.m, o.frag_stride, o.scale_stride};
+    const int tiles = (int)((m + 15) / 16);
+    hipLaunchKernelGGL(k_mmv_pack_blocks, dim3((unsigned)((16 * (int64_t)tiles * (K >> 5) + 255) / 256)), dim3(256), 0, dev->stream,
+                       (const BlockQ8_0 *)blocks, (int)m, tiles, (int)K, p);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+int launch_rows_pack_planar(candy_hip_device *dev, const int8_t *qs, const Q8Scale *scales, int64_t m, int64_t K, const RowsImage &o) {
+    hipLaunchKernelGGL(k_rows_pack_planar, dim3((unsigned)((m * (K >> 4) + 255) / 256)), dim3(256), 0, dev->stream, (const u32x4 *)qs, scales,
+                       (int)m, (int)K, o);
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }

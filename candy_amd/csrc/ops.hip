@@ -4,6 +4,7 @@
 // sequential CPU loops by f32 rounding only.
 #include "blocks.h"
 #include "internal.h"
+#include "rows_i8.h"
 
 namespace candy {
 
@@ -291,7 +292,7 @@ __global__ __launch_bounds__(256) void k_matmul_f32_strided(const float *__restr
 __global__ __launch_bounds__(256) void k_rms_norm_quant(const float *__restrict__ x, const float *__restrict__ alpha,
                                                         float eps, int cols, float *__restrict__ xn_out,
                                                         uint32_t *__restrict__ qs, Q8Scale *__restrict__ scales,
-                                                        half4v *__restrict__ xh) {
+                                                        half4v *__restrict__ xh, const RowsImage image) {
     __shared__ float red[16];
     const float4 *xr = (const float4 *)(x + (size_t)blockIdx.x * cols);
     const int n4 = cols >> 2;
@@ -322,6 +323,10 @@ __global__ __launch_bounds__(256) void k_rms_norm_quant(const float *__restrict_
         if (!live) continue;
         const size_t i = (size_t)blockIdx.x * n4 + c;
         if (xn_out) ((float4 *)xn_out)[i] = v;
+        if (image.frag) {
+            rows_put(image, blockIdx.x, c, packed, h, bsum);
+            continue;
+        }
         qs[i] = packed;
         if (xh) xh[xh_index4(blockIdx.x, c, cols)] = q8_lane4_to_half(packed, h);
         if ((c & 7) == 0) {
@@ -340,7 +345,7 @@ template <int ITER>
 __global__ __launch_bounds__(256) void k_rms_norm_quant_row(const float *__restrict__ x, const float *__restrict__ alpha,
                                                             float eps, int cols, float *__restrict__ xn_out,
                                                             uint32_t *__restrict__ qs, Q8Scale *__restrict__ scales,
-                                                            half4v *__restrict__ xh) {
+                                                            half4v *__restrict__ xh, const RowsImage image) {
     __shared__ float red[16];
     const float4 *xr = (const float4 *)(x + (size_t)blockIdx.x * cols);
     const int n4 = cols >> 2;
@@ -374,6 +379,10 @@ __global__ __launch_bounds__(256) void k_rms_norm_quant_row(const float *__restr
         if (!live) continue;
         const size_t at = (size_t)blockIdx.x * n4 + c;
         if (xn_out) ((float4 *)xn_out)[at] = o;
+        if (image.frag) {
+            rows_put(image, blockIdx.x, c, packed, h, bsum);
+            continue;
+        }
         qs[at] = packed;
         if (xh) xh[xh_index4(blockIdx.x, c, cols)] = q8_lane4_to_half(packed, h);
         if ((c & 7) == 0) {
@@ -486,7 +495,7 @@ __global__ __launch_bounds__(256) void k_rms_norm_quant_regs(const float *res, c
 __global__ __launch_bounds__(256) void k_silu_mul_quant(const float4 *__restrict__ gate, const float4 *__restrict__ up,
                                                         int64_t n4, int64_t row_n4, float4 *__restrict__ act_out,
                                                         uint32_t *__restrict__ qs, Q8Scale *__restrict__ scales,
-                                                        half4v *__restrict__ xh) {
+                                                        half4v *__restrict__ xh, const RowsImage image) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool live = i < n4;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -499,6 +508,10 @@ __global__ __launch_bounds__(256) void k_silu_mul_quant(const float4 *__restrict
     const uint32_t packed = quantize_q8_lane4(v, h, bsum);
     if (!live) return;
     if (act_out) act_out[i] = v;
+    if (image.frag) {
+        rows_put(image, (int)(i / row_n4), (int)(i % row_n4), packed, h, bsum);
+        return;
+    }
     qs[i] = packed;
     if (xh) xh[xh_index4(i / row_n4, i % row_n4, 4 * row_n4)] = q8_lane4_to_half(packed, h);
     if ((i & 7) == 0) {
@@ -520,11 +533,11 @@ int launch_argmax_key(candy_hip_device *dev, const float *logits, int64_t cols, 
 }
 
 int launch_rms_norm_quant(candy_hip_device *dev, const float *x, const float *alpha, float eps, int64_t rows,
-                          int64_t cols, float *xn_out, int8_t *qs, Q8Scale *scales, _Float16 *xh) {
+                          int64_t cols, float *xn_out, int8_t *qs, Q8Scale *scales, _Float16 *xh, const RowsImage *image) {
     CANDY_REQUIRE(cols % 32 == 0 && cols > 0 && rows > 0 && cols <= 0x7FFFFFFF, "rms_norm_quant needs cols %% 32 == 0");
     auto kern = cols <= 4096 ? k_rms_norm_quant_row<4> : cols <= 8192 ? k_rms_norm_quant_row<8> : k_rms_norm_quant;
     hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(256), 0, dev->stream, x, alpha, eps, (int)cols, xn_out, (uint32_t *)qs,
-                       scales, (half4v *)xh);
+                       scales, (half4v *)xh, image ? *image : RowsImage{});
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }
@@ -550,12 +563,12 @@ int launch_split_rms_norm_quant(candy_hip_device *dev, const SplitPending &sp, c
 }
 
 int launch_silu_mul_quant(candy_hip_device *dev, const float *gate, const float *up, int64_t rows, int64_t cols,
-                          float *act_out, int8_t *qs, Q8Scale *scales, _Float16 *xh) {
+                          float *act_out, int8_t *qs, Q8Scale *scales, _Float16 *xh, const RowsImage *image) {
     CANDY_REQUIRE(cols % 32 == 0 && cols > 0 && rows > 0, "silu_mul_quant needs cols %% 32 == 0");
     const int64_t n4 = rows * cols >> 2;
     hipLaunchKernelGGL(k_silu_mul_quant, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, dev->stream,
                        (const float4 *)gate, (const float4 *)up, n4, cols >> 2, (float4 *)act_out, (uint32_t *)qs, scales,
-                       (half4v *)xh);
+                       (half4v *)xh, image ? *image : RowsImage{});
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }

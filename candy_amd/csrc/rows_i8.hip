@@ -1,0 +1,499 @@
+// 3 to 255 activation rows on the int8 matrix cores, K dealt to wavefronts: y[m, N] = x[m, K] . W^T, exact like the batch-1
+// matvec (integer dots of 32 values, scaled in f32; only the order of the f32 sums differs).
+//
+// The tile kernel of mmq_i8.hip shares activations over the wavefronts of a workgroup, with two barriers a super-block, and on
+// most shapes splits K over workgroups whose copies a second launch adds up.  Here nobody waits for anybody: a workgroup owns
+// 16 RF weight rows and 16 MT activation rows, each of its WAVES wavefronts takes every WAVES-th super-block of K: the blocks
+// of 16 weight rows by direct loads into a slot of its own in LDS, two slots, so that the next 16 rows (or the next
+// super-block) arrive while these are contracted; the activations straight into operand registers from an image in operand
+// order (rows_i8.h).  The wavefronts' sums meet in LDS at the end, in pairs (reproducible).
+//
+// What bounds it: up to 16 rows two launches and their first bytes, then the weights at 3.5 to 4.5 TB/s (a wavefront's chain of
+// LDS round trips between two waits); from about 48 rows the vector ALU (a conversion, a product and an fma per result and
+// sub-block).  us of a call, before (int8 tiles, mostly with a split of K) -> now:
+//   4096 x 14336, 6 rows   Q4_K 18.1 -> 11.4, Q5_K 17.9 -> 12.8, Q6_K 21.0 -> 16.3, Q8_0 24.4 -> 17.3, Q4_0 22.4 -> 14.2
+//   11008 x 4096, 32 rows  Q4_K 15.7 -> 14.0, Q5_K 27.7 -> 14.7, Q6_K 31.6 -> 22.0, Q8_0 41.6 -> 18.0, Q4_0 38.1 -> 14.9
+//   11008 x 4096, 64 rows  Q5_K 35.0 -> 20.7, Q8_0 44.6 -> 24.2, Q4_0 37.9 -> 23.4
+// and prompts of the quantized decoder (four layers and the head): 8B shape 16 / 48 / 160 tokens 603 / 885 / 1861 -> 419 / 617 /
+// 1195, 1B shape 435 / 544 / 786 -> 283 / 351 / 517.
+//
+// The running sums are pinned every few sub-blocks (empty asm statements): left alone the compiler moves the f32 part of a super-block
+// behind its last product, into the next basic block, and holds every product's result until then (300 bytes of scratch and more).
+#include <algorithm>
+#include <type_traits>
+
+#include "blocks.h"
+#include "internal.h"
+#include "rows_i8.h"
+
+namespace candy {
+
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void rows_lds_fence() {  // orders one wavefront's LDS traffic, which completes in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The activation side of one super-block: operands of sub-blocks 2p and 2p + 1 (8 values of row lane & 15 each), the row's
+// eight scales, and d * sum(q) of sub-blocks 2c and 2c + 1.
+template <int MT>
+struct RowsX {
+    u32x4 q[MT][4];
+    float4 d[MT][2];
+    float2 m[MT];
+};
+__device__ __forceinline__ float rows_d(const float4 (&d)[2], int t) {
+    const float4 v = d[t >> 2];
+    return (t & 3) == 0 ? v.x : (t & 3) == 1 ? v.y : (t & 3) == 2 ? v.z : v.w;
+}
+__device__ __forceinline__ long rows_b(const u32x4 (&q)[4], int t) {
+    const u32x4 v = q[t >> 1];
+    return t & 1 ? (long)(((uint64_t)v.w << 32) | v.z) : (long)(((uint64_t)v.y << 32) | v.x);
+}
+__device__ __forceinline__ long rows_pack(uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | lo); }
+
+// One policy per format.  A slot holds 16 rows of PIECES 16-byte pieces; lane (row j, chunk c) feeds 8 values of a sub-block.
+//   factors()  lane (j, c) unpacks its part of the row's factors into ex[GROUPS][16 rows] for the lanes that own the row in
+//              the C layout, and adds the minimum's (or offset's) products to acc
+//   operand()  8 values of sub-block t as int8
+
+// Q4_K, Q5_K: d * scale per sub-block, minus dmin * minimum times the activations' sum
+template <bool FIVE>
+struct RowsQ45K {
+    static constexpr int BLOCK = FIVE ? 176 : 144, PIECES = BLOCK / 16, GROUPS = 8;
+    static constexpr bool DIRECT = true, HALVES = false;
+    struct Row { u32x2 q[4], qh; };
+    template <int MT>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &x, float4v (&acc)[MT]) {
+        const u32x4 h = *(const u32x4 *)wl;
+        uint32_t sc2, m2;
+        q4k_scale_min_pair(h.y, h.z, h.w, c, sc2, m2);
+        const float d = half_bits_to_float((uint16_t)(h.x & 0xFFFF)), dmin = half_bits_to_float((uint16_t)(h.x >> 16));
+        ex[(2 * c) * 16 + j] = d * (float)(sc2 & 0xFF);
+        ex[(2 * c + 1) * 16 + j] = d * (float)(sc2 >> 8);
+        const float m_lo = -dmin * (float)(m2 & 0xFF), m_hi = -dmin * (float)(m2 >> 8);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(m_lo, x.m[t].x, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(m_hi, x.m[t].y, acc[t], 0, 0, 0);
+        }
+    }
+    static __device__ __forceinline__ void load(const uint8_t *wl, int c, Row &r) {
+        if (FIVE) r.qh = *(const u32x2 *)(wl + 16 + 8 * c);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) r.q[p] = *(const u32x2 *)(wl + (FIVE ? 48 : 16) + 32 * p + 8 * c);
+    }
+    static __device__ __forceinline__ long operand(const Row &r, int t, int) {
+        const u32x2 q = r.q[t >> 1];
+        const int sh = (t & 1) * 4;
+        uint32_t lo = (q.x >> sh) & 0x0F0F0F0Fu, hi = (q.y >> sh) & 0x0F0F0F0Fu;
+        if (FIVE) {
+            lo |= ((r.qh.x >> t) & 0x01010101u) << 4;
+            hi |= ((r.qh.y >> t) & 0x01010101u) << 4;
+        }
+        return rows_pack(lo, hi);
+    }
+};
+
+// Q8_0: eight 34-byte blocks; the operand is the block's quants as they lie
+struct RowsQ8_0 {
+    static constexpr int BLOCK = 272, PIECES = 17, GROUPS = 8;
+    static constexpr bool DIRECT = true, HALVES = false;
+    struct Row { u32x2 q[8]; };
+    template <int MT>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &, float4v (&)[MT]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) ex[(2 * c + h) * 16 + j] = half_bits_to_float(*(const uint16_t *)(wl + 34 * (2 * c + h)));
+    }
+    static __device__ __forceinline__ void load(const uint8_t *wl, int c, Row &r) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) r.q[t] = *(const u32x2_a2 *)(wl + 34 * t + 2 + 8 * c);
+    }
+    static __device__ __forceinline__ long operand(const Row &r, int t, int) { return rows_pack(r.q[t].x, r.q[t].y); }
+};
+
+// Q4_0: eight 18-byte blocks; the operand is 16 (level - 8): the nibble in the upper half of a byte, its top bit flipped
+template <bool GGML>
+struct RowsQ4_0 {
+    static constexpr int BLOCK = 144, PIECES = 9, GROUPS = 8;
+    static constexpr bool DIRECT = true, HALVES = false;
+    struct Row { u32x2 q[8]; };
+    template <int MT>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &, float4v (&)[MT]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) ex[(2 * c + h) * 16 + j] = 0.0625f * half_bits_to_float(*(const uint16_t *)(wl + 18 * (2 * c + h)));
+    }
+    static __device__ __forceinline__ void load(const uint8_t *wl, int c, Row &r) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            if (GGML) r.q[t] = *(const u32x2_a2 *)(wl + 18 * t + 2 + 8 * (c & 1));
+            else r.q[t].x = *(const u32_a2 *)(wl + 18 * t + 2 + 4 * c);
+        }
+    }
+    static __device__ __forceinline__ long operand(const Row &r, int t, int c) {
+        const uint32_t M = 0xF0F0F0F0u, TOP = 0x80808080u;
+        if (GGML) {
+            const int sh = c < 2 ? 4 : 0;
+            return rows_pack(((r.q[t].x << sh) & M) ^ TOP, ((r.q[t].y << sh) & M) ^ TOP);
+        }
+        const uint32_t l = ((r.q[t].x << 4) & M) ^ TOP, h = (r.q[t].x & M) ^ TOP;  // byte i: values 2i and 2i + 1
+        return rows_pack(__builtin_amdgcn_perm(h, l, 0x05010400u), __builtin_amdgcn_perm(h, l, 0x07030602u));
+    }
+};
+
+// Q6_K: blocks of 210 bytes start on any even address, which a direct load does not take: they come through registers, 14
+// pieces a row (the last one ends 14 bytes into the next block), 15 from row to row for the banks.  A sub-block's two groups of 16 have a
+// scale each: two products whose operand is zero in the other half.
+struct RowsQ6K {
+    static constexpr int BLOCK = 210, PIECES = 15, GROUPS = 17;
+    static constexpr bool DIRECT = false, HALVES = true;
+    struct Row { u32x2 ql[4], qh[2]; };
+    template <int MT>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &, float4v (&)[MT]) {
+        // the sixteen scales as integers, then d
+        const uint32_t sc = *(const uint32_t *)(wl + 192 + 4 * c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ((int *)ex)[(4 * c + i) * 16 + j] = (int)(sc << (24 - 8 * i)) >> 24;
+        if (c == 0) ex[16 * 16 + j] = half_bits_to_float(*(const uint16_t *)(wl + 208));
+    }
+    static __device__ __forceinline__ void load(const uint8_t *wl, int c, Row &r) {
+#pragma unroll
+        for (int ip = 0; ip < 2; ++ip) {
+            r.ql[2 * ip] = *(const u32x2 *)(wl + 64 * ip + 8 * c);
+            r.ql[2 * ip + 1] = *(const u32x2 *)(wl + 64 * ip + 32 + 8 * c);
+            r.qh[ip] = *(const u32x2 *)(wl + 128 + 32 * ip + 8 * c);
+        }
+    }
+    static __device__ __forceinline__ long operand(const Row &r, int t, int) {
+        const u32x2 ql = r.ql[2 * (t >> 2) + (t & 1)], qh = r.qh[t >> 2];
+        const int quarter = t & 3;
+        uint32_t w2[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t nib = (quarter & 2) ? (ql[e] >> 4) & 0x0F0F0F0Fu : ql[e] & 0x0F0F0F0Fu;
+            const uint32_t top = quarter == 0 ? (qh[e] << 4) : quarter == 1 ? (qh[e] << 2) : quarter == 2 ? qh[e] : (qh[e] >> 2);
+            // bytewise level - 32: bias by 128 so that no byte borrows, then flip the bias off
+            w2[e] = (((nib | (top & 0x30303030u)) | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
+        }
+        return rows_pack(w2[0], w2[1]);
+    }
+};
+
+template <class F, int RF, int MT, int WAVES>
+struct RowsLds {
+    static constexpr int LOADED = F::DIRECT ? F::PIECES : F::PIECES - 1;  // pieces of a row that are fetched
+    static constexpr int IT = (16 * LOADED + 63) / 64;          // loads per slot
+    static constexpr int SLOT = 16 * F::PIECES * 16;
+    static constexpr int EX = F::GROUPS * 16 * 4;
+    static constexpr int WAVE = (F::DIRECT ? 2 : 1) * SLOT + EX;
+    static constexpr int SUMS = WAVES * RF * MT * 1024;
+    static constexpr int BYTES = WAVES * WAVE > SUMS ? WAVES * WAVE : SUMS;
+};
+
+template <class F, int RF, int MT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 4 : 2) void k_rows_i8(
+    const uint8_t *__restrict__ xfrag, const float *__restrict__ xd, const float *__restrict__ xm, int K, int M, int frag_stride,
+    int scale_stride, const RowsJobs jobs) {
+    typedef RowsLds<F, RF, MT, WAVES> L;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, c = lane >> 4;
+    uint8_t *const mine = smem + wave * L::WAVE;
+    float *const ex = (float *)(mine + (F::DIRECT ? 2 : 1) * L::SLOT);
+    const int ji = (int)(blockIdx.x >= (unsigned)jobs.j[0].wg_end) + (int)(blockIdx.x >= (unsigned)jobs.j[1].wg_end);
+    const RowsJob job = jobs.j[ji];
+    const int wg = blockIdx.x - (ji > 0 ? jobs.j[ji - 1].wg_end : 0);
+    const int n0 = wg * (16 * RF), N = job.N, nsb = K >> 8;
+    const uint32_t rb = (uint32_t)nsb * F::BLOCK;
+    const int count = (nsb - wave + WAVES - 1) / WAVES;  // super-blocks wave, wave + WAVES, ... (may be none)
+    xfrag += (size_t)blockIdx.y * MT * frag_stride;
+    xd += (size_t)blockIdx.y * MT * scale_stride;
+    xm += (size_t)blockIdx.y * MT * scale_stride;
+
+    // a strip past the last row is moved back onto the rows that are there; its rows in front of n0 + 16 r are not stored
+    auto strip_row = [&](int r) __attribute__((always_inline)) { return min(n0 + 16 * r, N - 16); };
+    uint32_t from[L::IT];  // of a lane's piece, from the strip's first row and super-block
+#pragma unroll
+    for (int it = 0; it < L::IT; ++it) {
+        const int e = min(it * 64 + lane, 16 * L::LOADED - 1);
+        from[it] = (uint32_t)(e / L::LOADED) * rb + (uint32_t)(e % L::LOADED) * 16;
+    }
+    u32x4 held[F::DIRECT ? 1 : L::IT];
+    auto request = [&](int sb, int r, int slot) __attribute__((always_inline)) {
+        const uint8_t *base = job.W + (size_t)strip_row(r) * rb + (size_t)sb * F::BLOCK;
+#pragma unroll
+        for (int it = 0; it < L::IT; ++it) {
+            if constexpr (!F::DIRECT) {
+                held[it] = *(const u32x4_a2 *)(base + from[it]);
+            } else if ((it + 1) * 64 <= 16 * F::PIECES || it * 64 + lane < 16 * F::PIECES) {
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(base + from[it]),
+                                                 (__attribute__((address_space(3))) void *)(mine + slot * L::SLOT + it * 1024), 16, 0, 0);
+            }
+        }
+    };
+    auto park = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int it = 0; it < L::IT; ++it) {
+            const int e = min(it * 64 + lane, 16 * L::LOADED - 1);  // lanes past the last piece write it once more
+            *(u32x4 *)(mine + (e / L::LOADED) * (F::PIECES * 16) + (e % L::LOADED) * 16) = held[it];
+        }
+    };
+    RowsX<MT> x;
+    auto load_x = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const uint8_t *pf = xfrag + (size_t)t * frag_stride + (size_t)sb * 4096;
+            const float *pd = xd + (size_t)t * scale_stride + (size_t)sb * 128, *pm = xm + (size_t)t * scale_stride + (size_t)sb * 128;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) x.q[t][p] = *(const u32x4 *)(pf + p * 1024 + lane * 16);
+            x.d[t][0] = *(const float4 *)(pd + j * 8);
+            x.d[t][1] = *(const float4 *)(pd + j * 8 + 4);
+            x.m[t] = *(const float2 *)(pm + j * 8 + 2 * c);
+        }
+    };
+    float4v acc[RF][MT];
+#pragma unroll
+    for (int r = 0; r < RF; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[r][t] = float4v{0.f, 0.f, 0.f, 0.f};
+
+    if (count > 0) {
+        request(wave, 0, 0);
+        load_x(wave);
+        int slot = 0;
+        for (int k = 0; k < count; ++k) {
+            const int sb = wave + WAVES * k;
+#pragma unroll
+            for (int r = 0; r < RF; ++r) {
+                if constexpr (F::DIRECT) {
+                    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this slot has landed; the other one's reads are over
+                } else {
+                    park();
+                    rows_lds_fence();
+                }
+                if (r + 1 < RF) request(sb, r + 1, slot ^ 1);
+                else if (k + 1 < count) request(sb + WAVES, 0, slot ^ 1);
+                const uint8_t *wl = mine + slot * L::SLOT + j * (F::PIECES * 16);
+                F::template factors<MT>(wl, j, c, ex, x, acc[r]);
+                typename F::Row row;
+                F::load(wl, c, row);
+                rows_lds_fence();
+                float4v part[F::HALVES ? MT : 1];  // Q6_K: the super-block's sum in front of d
+                if constexpr (F::HALVES) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) part[mt] = float4v{0.f, 0.f, 0.f, 0.f};
+                }
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    constexpr int TOGETHER = MT == 1 ? (F::HALVES ? 2 : 4) : MT == 2 && !F::HALVES ? 2 : 1;
+                    if (t % TOGETHER == 0) {  // the sums so far are made here, not all behind the last product
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) {
+                            if constexpr (F::HALVES) asm volatile("" : "+v"(part[mt]));
+                            else asm volatile("" : "+v"(acc[r][mt]));
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    const long a = F::operand(row, t, c);
+                    if constexpr (F::HALVES) {
+                        const long a_lo = c < 2 ? a : 0, a_hi = c < 2 ? 0 : a;
+                        const int4v fl = *(const int4v *)&ex[(2 * t) * 16 + 4 * c], fh = *(const int4v *)&ex[(2 * t + 1) * 16 + 4 * c];
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) {
+                            const long b = rows_b(x.q[mt], t);
+                            const int4v dl = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_lo, b, int4v{0, 0, 0, 0}, 0, 0, 0);
+                            const int4v dh = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, b, int4v{0, 0, 0, 0}, 0, 0, 0);
+                            const float dx = rows_d(x.d[mt], t);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)  // |dot| <= 2^16, |scale| <= 2^7: exact
+                                part[mt][i] += dx * (float)(__mul24(dh[i], fh[i]) + __mul24(dl[i], fl[i]));
+                        }
+                    } else {
+                        const float4v f = *(const float4v *)&ex[t * 16 + 4 * c];
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) {
+                            const int4v d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, rows_b(x.q[mt], t), int4v{0, 0, 0, 0}, 0, 0, 0);
+                            const float dx = rows_d(x.d[mt], t);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[r][mt][i] += (f[i] * dx) * (float)d[i];  // fp16 scales: their product is exact
+                        }
+                    }
+                }
+                if constexpr (F::HALVES) {
+                    const float4v d = *(const float4v *)&ex[16 * 16 + 4 * c];
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) acc[r][mt] += d * part[mt];
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[r][mt]));
+                rows_lds_fence();  // the factors' place is rewritten next
+                __builtin_amdgcn_sched_barrier(0);
+                if (F::DIRECT) slot ^= 1;
+            }
+            if (k + 1 < count) load_x(sb + WAVES);
+        }
+    }
+    __syncthreads();  // the slots are consumed
+    float4v *const sums = (float4v *)smem;  // [wave][RF][MT][lane]
+#pragma unroll
+    for (int r = 0; r < RF; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sums[((wave * RF + r) * MT + t) * 64 + lane] = acc[r][t];
+    __syncthreads();
+    for (int f = wave; f < RF * MT; f += WAVES) {
+        const int r = f / MT, t = f - r * MT;
+        float4v p[WAVES];
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) p[w] = sums[(w * RF * MT + f) * 64 + lane];
+#pragma unroll
+        for (int d = 1; d < WAVES; d *= 2)  // neighbours first: a shorter chain of roundings
+#pragma unroll
+            for (int w = 0; w < WAVES; w += 2 * d) p[w] += p[w + d];
+        float4v s = p[0];
+        const int m = (blockIdx.y * MT + t) * 16 + j, own = n0 + 16 * r, n = strip_row(r) + 4 * c;  // weight rows n .. n + 3
+        if (m >= M) continue;
+        float *dst = job.y + (size_t)m * N + n;
+        const float *res = job.res ? job.res + (size_t)m * N + n : nullptr;  // may be y: read before the store
+        if (n >= own && (N & 3) == 0) {
+            if (res) s = *(const float4v *)res + s;
+            *(float4v *)dst = s;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i >= own) dst[i] = res ? res[i] + s[i] : s[i];
+        }
+    }
+}
+
+template <class F, int RF, int MT, int WAVES>
+static int launch_rows_cfg(candy_hip_device *dev, const RowsLaunch &L, int64_t m) {
+    typedef RowsLds<F, RF, MT, WAVES> S;
+    static_assert(S::BYTES <= 160 * 1024, "LDS");
+    RowsJobs jobs{};
+    int total = 0;
+    for (int i = 0; i < 3; ++i) {
+        if (i < L.n) {
+            jobs.j[i].W = (const uint8_t *)L.w[i]->data;
+            jobs.j[i].y = L.y[i];
+            jobs.j[i].res = L.res[i];
+            jobs.j[i].N = (int)L.w[i]->rows;
+            total += (jobs.j[i].N + 16 * RF - 1) / (16 * RF);
+        }
+        jobs.j[i].wg_end = total;
+    }
+    const int K = (int)L.w[0]->cols;
+    auto kern = k_rows_i8<F, RF, MT, WAVES>;
+    if (S::BYTES > 48 * 1024)
+        CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::BYTES));
+    hipLaunchKernelGGL(kern, dim3((unsigned)total, (unsigned)((m + 16 * MT - 1) / (16 * MT))), dim3(WAVES * 64), S::BYTES, dev->stream,
+                       L.x.frag, L.x.d, L.x.m, K, (int)m, (int)L.x.frag_stride, (int)L.x.scale_stride, jobs);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+
+template <class F>
+static int launch_rows_fmt(candy_hip_device *dev, const RowsLaunch &L, int64_t m, int rf, int mt, int waves) {
+#define CANDY_ROWS(RF, MT, WAVES) \
+    if (rf == RF && mt == MT && waves == WAVES) return launch_rows_cfg<F, RF, MT, WAVES>(dev, L, m);
+    CANDY_ROWS(1, 1, 16) CANDY_ROWS(1, 1, 8)
+    if constexpr (std::is_same<F, RowsQ6K>::value) {
+        CANDY_ROWS(2, 1, 8)
+    } else {
+        CANDY_ROWS(4, 1, 8)
+    }
+    CANDY_ROWS(1, 2, 8) CANDY_ROWS(1, 3, 8) CANDY_ROWS(2, 3, 8)
+    if constexpr (std::is_same<F, RowsQ6K>::value) {
+        CANDY_ROWS(1, 4, 8) CANDY_ROWS(2, 4, 8)
+    } else {
+        CANDY_ROWS(1, 2, 16) CANDY_ROWS(2, 2, 16) CANDY_ROWS(2, 2, 8)
+    }
+#undef CANDY_ROWS
+    return fail(CANDY_HIP_ERR_INVALID, "internal: shape of the row contraction");
+}
+
+bool rows_i8_covers(const candy_hip_qtensor *w) {
+    if (w->cols % 256 != 0 || w->cols > (1 << 20) || w->rows < 16 || w->rows > 0x7FFFFFF || ((uintptr_t)w->data & (w->fmt == CANDY_HIP_Q6_K ? 1 : 15)) != 0)
+        return false;
+    switch (w->fmt) {
+    case CANDY_HIP_Q4_K: case CANDY_HIP_Q5_K: case CANDY_HIP_Q8_0: case CANDY_HIP_Q4_0: case CANDY_HIP_Q4_0_GGML: return true;
+    case CANDY_HIP_Q6_K: return w->padded;  // the last piece of a row ends up to 14 bytes behind it
+    default: return false;
+    }
+}
+
+bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
+    const Options &o = w->dev->opt;
+    return o.rows_i8 && o.mmv_max_m != 0 && !o.mmq_fp16_only && m >= 3 && m <= 255 && rows_i8_covers(w);
+}
+
+// Where the other kernels are ahead or level, us of a call, there / here:
+//   Q4_K up to 16 (8192 or fewer weight rows: 32) activation rows of 4096 or fewer values, the one-shot kernel of mmv_i8.hip:
+//     4096 x 4096, 16 rows 7.1 / 7.2, 14336 x 4096 11.2 / 12.1, 8192 x 2048, 32 rows 7.7 / 8.0 (but 32000 x 4096 19.6 / 17.8, 14336 x
+//     4096, 32 rows 16.4 / 15.1, 4096 x 11008, 16 rows 11.1 / 9.7)
+//   three and four rows, the vector kernels: small weights (1024 x 4096, Q5_K 7.2 / 7.2, Q8_0 7.3 / 7.6), and Q8_0 and Q4_0 where a
+//     workgroup's few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0; 4096 x 4096 8.4 / 7.7)
+//   the fp16 kernels, whose scales are in the operands, where a call may take them: Q4_K and Q6_K from 33 rows (11008 x 4096, 48 rows
+//     16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 / 35.8)
+// Weights under a million values are launches and nothing else whatever the kernel.
+bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
+    const Options &o = w->dev->opt;
+    const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16;
+    if (!rows_i8_takes(w, m) || values < 1 << 20 || m < o.i8_min_m || o.small_batch_kernel == 0) return false;
+    const bool q4k = w->fmt == CANDY_HIP_Q4_K, q6k = w->fmt == CANDY_HIP_Q6_K;
+    if (q4k && w->cols <= 4096 && mmv_covers(w, m) && w->rows <= (m <= 16 ? 64 * cus : 32 * cus)) return false;
+    if (m <= 4 && values <= 1 << 22) return false;
+    if (m <= 4 && !q4k && !q6k && w->fmt != CANDY_HIP_Q5_K && w->cols <= 4096 && strips > 2 * cus && strips <= 4 * cus) return false;
+    return exact || m <= (q4k || q6k ? 32 : 64);
+}
+
+// Tile and wavefronts.  One activation tile per workgroup where the strips alone leave half of the CUs idle (weights read
+// again come from L2), else the tiles that the registers hold.  Sixteen wavefronts where there is one workgroup per CU, eight (two
+// workgroups) otherwise; two or four strips of weight rows per workgroup where a launch would otherwise be more than four
+// (17 to 32 rows: three) rounds.  us: Q8_0 2048 x 8192, 32 rows, tiles of 16 / 32 rows 10.6 / 12.1, 4096 x 14336 25.1 / 20.3; 32000 x 4096,
+// 16 rows, 1 / 2 / 4 strips 32.7 / 29.5 / 28.0; Q4_K 4096 x 14336, 6 rows, 16 / 8 wavefronts 11.7 / 13.5, 11008 x 4096 12.1 / 9.8.
+int launch_rows_i8(candy_hip_device *dev, const RowsLaunch &L, int64_t m) {
+    int64_t strips = 0;  // of 16 weight rows
+    for (int i = 0; i < L.n; ++i) strips += (L.w[i]->rows + 15) / 16;
+    const bool q6k = L.w[0]->fmt == CANDY_HIP_Q6_K;
+    const int64_t cus = dev->num_cus, tiles = (m + 15) / 16;
+    int rf, mt, waves;
+    if (tiles == 1 || (strips <= cus / 2 && strips * tiles <= 2 * cus)) {
+        mt = 1;
+        rf = strips <= 4 * cus ? 1 : q6k ? 2 : 4;
+        waves = strips * tiles <= cus ? 16 : 8;
+    } else if (m <= 32 && q6k) {  // two tiles are 148 registers: eight wavefronts a CU, less than the weights' stream needs past 1024 strips
+        mt = strips <= 4 * cus ? 2 : 1;
+        rf = strips <= 4 * cus ? 1 : 2;
+        waves = 8;
+    } else if (m <= 32) {
+        mt = 2;
+        rf = strips <= 3 * cus ? 1 : 2;
+        waves = strips <= cus ? 16 : 8;
+    } else if (m <= 48) {
+        mt = 3;
+        rf = strips <= 4 * cus ? 1 : 2;
+        waves = 8;
+    } else if (q6k) {
+        mt = 4;
+        rf = m <= 64 && strips <= cus ? 1 : 2;
+        waves = 8;
+    } else {
+        mt = 2;
+        rf = 2;
+        waves = strips * ((m + 31) / 32) <= 2 * cus ? 16 : 8;
+    }
+    CANDY_REQUIRE((m + 16 * mt - 1) / (16 * mt) * mt <= rows_tiles(m), "internal: tiles of the row contraction");
+    switch (L.w[0]->fmt) {
+    case CANDY_HIP_Q4_K: return launch_rows_fmt<RowsQ45K<false>>(dev, L, m, rf, mt, waves);
+    case CANDY_HIP_Q5_K: return launch_rows_fmt<RowsQ45K<true>>(dev, L, m, rf, mt, waves);
+    case CANDY_HIP_Q6_K: return launch_rows_fmt<RowsQ6K>(dev, L, m, rf, mt, waves);
+    case CANDY_HIP_Q8_0: return launch_rows_fmt<RowsQ8_0>(dev, L, m, rf, mt, waves);
+    case CANDY_HIP_Q4_0: return launch_rows_fmt<RowsQ4_0<false>>(dev, L, m, rf, mt, waves);
+    case CANDY_HIP_Q4_0_GGML: return launch_rows_fmt<RowsQ4_0<true>>(dev, L, m, rf, mt, waves);
+    default: return fail(CANDY_HIP_ERR_INVALID, "internal: format of the row contraction");
+    }
+}
+
+}  // namespace candy
