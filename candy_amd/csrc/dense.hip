@@ -517,6 +517,95 @@ __global__ __launch_bounds__(512, 2) void k_dense_big(const bf16 *__restrict__ W
     }
 }
 
+// ------------------------------------------------------------------ prompt batches, bfloat16, few tiles
+// Tile: 32 weight rows x BM = 32 or 64 activation rows, four wavefronts, K whole: for contractions whose epilogue does not let K be
+// split and whose large tiles leave most of the chip idle.  There a workgroup's walk along K is a chain of stage latencies
+// (0.8 us each, 64 values); here up to five stages are in flight, and four times as many workgroups walk.  What bounds it: the
+// activations, which every workgroup reads.  A value's sum goes along K in the order of the other tiles: the same bits.
+// us of a call with two conversions around it (6 us), before -> now: 2816 x 2048, 16 / 64 / 200 rows 20.9 / 22.1 / 23.2 -> 11.6 / 13.5 /
+// 16.9; 6144 x 4096, 40 / 100 rows 39.0 / 35.4 -> 20.8 / 26.9; 14336 x 4096, 16 / 64 rows 40.3 / 44.5 -> 31.0 / 35.6.
+constexpr int NARROW_BN = 32;
+template <int EPI, int BM>
+__global__ __launch_bounds__(256, 2) void k_dense_narrow(const bf16 *__restrict__ W, const bf16 *__restrict__ X, void *__restrict__ yv, int M,
+                                                         int Np, int ld, int ldx, int64_t ldy, int n_store, int m_tiles, const EpiArgs ea) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+    constexpr int BN = NARROW_BN, BK = 64, ROWS = BN + BM, PIECES = ROWS / 8, LOADS = PIECES / 4, STAGES = 6, TM = BM / 32;
+    static_assert(PIECES % 4 == 0, "every wavefront has as many loads");
+    __shared__ __align__(16) u32x4v s[STAGES * ROWS * 8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = blockIdx.x / m_tiles * BN, m0 = blockIdx.x % m_tiles * BM;
+    const int n_it = ld / BK;
+    f32x4 acc[TM];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int r16 = lane & 15, g = lane >> 4, sw = (r16 >> 1) & 7;
+    const int wn = (wave >> 1) * 16, wm = BN + (wave & 1) * (BM / 2);
+    auto describe = [](const bf16 *p, int64_t values) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, values >= 1ll << 31 ? -1 : (int)(uint32_t)(values * 2), 0x00027000);
+    };
+    const __amdgpu_buffer_rsrc_t rw = describe(W + (size_t)n0 * ld, (int64_t)(Np - n0) * ld),
+                                 rx = describe(X + (size_t)m0 * ldx, (int64_t)(M - m0 - 1) * ldx + ld);
+    uint32_t off[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int r = (wave + 4 * i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        // activation rows past the last one repeat it
+        off[i] = (r < BN ? (uint32_t)r * (uint32_t)ld : (uint32_t)min(r - BN, M - m0 - 1) * (uint32_t)ldx) * 2 + c * 16;
+    }
+    int k_off = 0;
+    auto load = [&](int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            auto *to = (__attribute__((address_space(3))) void *)(s + stage * ROWS * 8 + (wave + 4 * i) * 64);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(4 * i < BN / 8 ? rw : rx, to, 16, off[i], k_off, 0, 0);  // pieces 0 .. 3 are W's
+        }
+        k_off += BK * 2;
+    };
+    auto compute = [&](int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const u32x4v *p = s + stage * ROWS * 8 + r16 * 8 + ((kk * 4 + g) ^ sw);
+            const bf16x8 a = __builtin_bit_cast(bf16x8, p[wn * 8]);
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, p[(wm + j * 16) * 8]), acc[j], 0, 0, 0);
+        }
+    };
+    // stages in flight behind the one waited for: STAGES - 2, none once the last one is requested
+    constexpr int ARRIVED = 0x0070, BEHIND = LOADS * (STAGES - 2), ARRIVED_BUT = 0x0070 | (BEHIND & 15) | (BEHIND >> 4) << 14;
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i)
+        if (i < n_it) load(i);
+    int cur = 0;
+    for (int it = 0; it < n_it; ++it) {
+        if (it + STAGES - 1 <= n_it) __builtin_amdgcn_s_waitcnt(ARRIVED_BUT);
+        else __builtin_amdgcn_s_waitcnt(ARRIVED);
+        __builtin_amdgcn_s_barrier();  // this stage is there for every wavefront, and the one in front of it is consumed
+        asm volatile("" ::: "memory");
+        if (it + STAGES - 1 < n_it) load(cur == 0 ? STAGES - 1 : cur - 1);
+        compute(cur);
+        cur = cur + 1 == STAGES ? 0 : cur + 1;
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        const int m = m0 + wm - BN + j * 16 + r16, n = n0 + wn + 4 * g;
+        if (m >= M) continue;
+        f32x4 z = acc[j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[e] = epilogue<EPI>(z[e], ea);
+        if (to_act(EPI)) {
+            if (n < n_store) *(bf16x4 *)((bf16 *)yv + (size_t)m * ldy + n) = __builtin_convertvector(z, bf16x4);
+        } else {
+            float *y = (float *)yv + (size_t)m * ldy + n;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < n_store) y[e] = z[e];
+        }
+    }
+#endif
+}
+
 // ------------------------------------------------------------------ prompt batches, f32 activations
 template <int EPI, bool GROUPED>
 __global__ __launch_bounds__(256) void k_dense_mm_f32(const bf16 *__restrict__ W, const float *__restrict__ X, float *__restrict__ yv,
@@ -743,11 +832,34 @@ static void launch_big(const MmPlan &p, dim3 g, hipStream_t stream, Args... args
 #undef CANDY_BIG
 }
 
+// Where the narrow tiles are at most two workgroups per CU: past that the activations they read again cost more than the shorter
+// walk saves (us as above, large tiles / narrow ones: 6144 x 4096, 200 rows 38.1 / 46.3, 11008 x 4096, 100 rows 36.3 / 45.4; at 512
+// workgroups, 8192 x 2048, 100 rows 22.5 / 20.8).
+static bool narrow_covers(int num_cus, const DenseLaunch &L) {
+    if (L.f32 || L.partial || L.block_rows || L.group || !to_act(L.epi)) return false;
+    const int64_t m_tiles = L.m <= 32 ? 1 : (L.m + 63) / 64, tiles = m_tiles * (L.w->rows_pad / NARROW_BN);
+    return tiles <= 2 * (int64_t)num_cus && tile_fits(NARROW_BN, L.w->ld) && tile_fits(64, L.ldx);
+}
+static int launch_narrow(candy_hip_device *dev, const DenseLaunch &L) {
+    const int K = (int)L.w->ld, rows = (int)L.w->rows_pad, bm = L.m <= 32 ? 32 : 64, m_tiles = (L.m + bm - 1) / bm;
+    const dim3 g((unsigned)(m_tiles * (rows / NARROW_BN))), b(256);
+    const EpiArgs ea{L.scale, L.cap};
+    const bf16 *W = (const bf16 *)L.w->data, *X = (const bf16 *)L.x;
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, g, b, 0, dev->stream, W, X, L.y, L.m, rows, K, (int)L.ldx, L.ldy, (int)L.n_store, m_tiles, ea);
+    };
+    if (L.epi == EPI_RELU2) bm == 32 ? launch(k_dense_narrow<EPI_RELU2, 32>) : launch(k_dense_narrow<EPI_RELU2, 64>);
+    else bm == 32 ? launch(k_dense_narrow<EPI_ACT, 32>) : launch(k_dense_narrow<EPI_ACT, 64>);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+
 static int launch_mm(candy_hip_device *dev, const DenseLaunch &L) {
     const int K = (int)L.w->ld;
     const int64_t rows = L.w->rows_pad;
     const MmPlan p = mm_plan(dev->num_cus, L.m, rows, K, L.ldx, L.partial != nullptr, L.steady, L.epi != EPI_NONE && L.epi != EPI_RELU2,
                              L.block_rows);
+    if (narrow_covers(dev->num_cus, L)) return launch_narrow(dev, L);
     const int m_tiles = (L.m + p.bm - 1) / p.bm, n_tiles = (int)((rows + p.bn - 1) / p.bn);
     const int64_t tiles = (int64_t)m_tiles * n_tiles;
     CANDY_REQUIRE(tiles <= 0x7FFFFFFF, "matrix too large");

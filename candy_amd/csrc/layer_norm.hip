@@ -5,6 +5,7 @@
 // One workgroup per row, the row in registers; mean and variance in two passes over them.
 // (The reference path this library stands behind normalizes in front of its sublayers only, reduce.go:3071-3092.)
 #include <algorithm>
+#include <type_traits>
 
 #include "dense.h"
 
@@ -25,8 +26,11 @@ struct NormKernelArgs {
     float mult, eps;
 };
 
-// V: float4 per thread; columns past `cols` (inside the padding) hold zeros and stay zero
-template <class AT, int V>
+// V: float4 per thread; columns past `cols` (inside the padding) hold zeros and stay zero.  BATCH: copies and slots of y are
+// requested in batches of eight, four and two and added in order, a round trip for each batch and not for each row: for launches of so
+// few rows that a workgroup waits alone (us, 16 rows of 4096, eight copies 11.9 -> 7.7).  The registers for it cost a large launch
+// its occupancy (1500 rows, one or two copies 21.3 -> 24.6), which adds them one by one.
+template <class AT, int V, bool BATCH>
 __global__ __launch_bounds__(256) void k_norm_chain(const NormKernelArgs a) {
     __shared__ float red[4];
     const int tid = threadIdx.x;
@@ -41,7 +45,16 @@ __global__ __launch_bounds__(256) void k_norm_chain(const NormKernelArgs a) {
         for (int i = 0; i < V; ++i) d[i] = col(i) < padded ? *(const f32x4 *)(p + col(i)) : f32x4{0.f, 0.f, 0.f, 0.f};
     };
     // in place: d <- (d - mean) * rstd * w + b inside `cols`, 0 outside (RMS: mean and b are 0)
-    auto normalize = [&](f32x4 (&d)[V], const float *w, const float *b) {
+    // BATCH: weights and biases of both norms are requested with the row, not behind its sums
+    f32x4 held[BATCH ? 4 : 1][V];
+    if constexpr (BATCH) {
+        load_row(a.x + src * a.ldx, x);
+        load_row(a.post_w, held[0]);
+        if (a.post_b) load_row(a.post_b, held[1]);
+        if (a.out && a.pre_w) load_row(a.pre_w, held[2]);
+        if (a.out && a.pre_b) load_row(a.pre_b, held[3]);
+    }
+    auto normalize = [&](f32x4 (&d)[V], const float *w, const float *b, const f32x4 (&hw)[V], const f32x4 (&hb)[V]) {
         float mean = 0.0f;
         if (!a.rms) {
             float s = 0.0f;
@@ -61,31 +74,45 @@ __global__ __launch_bounds__(256) void k_norm_chain(const NormKernelArgs a) {
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             if (col(i) >= padded) continue;
-            const f32x4 wv = *(const f32x4 *)(w + col(i));  // zero in the padding, like b
-            const f32x4 bv = b ? *(const f32x4 *)(b + col(i)) : f32x4{0.f, 0.f, 0.f, 0.f};
+            const f32x4 wv = BATCH ? hw[i] : *(const f32x4 *)(w + col(i));  // zero in the padding, like b
+            const f32x4 bv = !b ? f32x4{0.f, 0.f, 0.f, 0.f} : BATCH ? hb[i] : *(const f32x4 *)(b + col(i));
 #pragma unroll
             for (int j = 0; j < 4; ++j) d[i][j] = d[i][j] * rstd * wv[j] + bv[j];
         }
     };
-    load_row(a.x + src * a.ldx, x);
+    if constexpr (!BATCH) load_row(a.x + src * a.ldx, x);
     if (a.y || a.slots) {
 #pragma unroll
         for (int i = 0; i < V; ++i) y[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int c = 0; a.y && c < a.y_copies; ++c) {
-            f32x4 t[V];
-            load_row(a.y + src * a.ldy + (size_t)c * a.y_stride, t);
+        auto add_rows = [&](auto rows_c, int first, auto row_of, auto weight_of) __attribute__((always_inline)) {
+            constexpr int R = decltype(rows_c)::value;
+            f32x4 t[R][V];
+            float g[R];
 #pragma unroll
-            for (int i = 0; i < V; ++i) y[i] += t[i];
-        }
-        for (int k = 0; a.slots && k < a.top; ++k) {
-            const size_t slot = src * a.top + k;
-            const float g = a.slot_weight[slot];
-            f32x4 t[V];
-            load_row(a.slots + slot * a.slot_ld, t);
+            for (int k = 0; k < R; ++k) {
+                g[k] = weight_of(first + k);
+                load_row(row_of(first + k), t[k]);
+            }
 #pragma unroll
-            for (int i = 0; i < V; ++i) y[i] += g * t[i];
-        }
-        normalize(y, a.post_w, a.post_b);
+            for (int k = 0; k < R; ++k)
+#pragma unroll
+                for (int i = 0; i < V; ++i) y[i] += g[k] * t[k][i];
+        };
+        auto add_all = [&](int count, auto row_of, auto weight_of) __attribute__((always_inline)) {
+            int c = 0;
+            if constexpr (BATCH && V <= 2)
+                for (; c + 8 <= count; c += 8) add_rows(std::integral_constant<int, 8>{}, c, row_of, weight_of);
+            if constexpr (BATCH && V <= 4)
+                for (; c + 4 <= count; c += 4) add_rows(std::integral_constant<int, 4>{}, c, row_of, weight_of);
+            if constexpr (BATCH)
+                for (; c + 2 <= count; c += 2) add_rows(std::integral_constant<int, 2>{}, c, row_of, weight_of);
+            for (; c < count; ++c) add_rows(std::integral_constant<int, 1>{}, c, row_of, weight_of);
+        };
+        if (a.y)
+            add_all(a.y_copies, [&](int c) { return a.y + src * a.ldy + (size_t)c * a.y_stride; }, [](int) { return 1.0f; });
+        if (a.slots)
+            add_all(a.top, [&](int k) { return a.slots + (src * a.top + k) * a.slot_ld; }, [&](int k) { return a.slot_weight[src * a.top + k]; });
+        normalize(y, a.post_w, a.post_b, held[0], held[BATCH ? 1 : 0]);
 #pragma unroll
         for (int i = 0; i < V; ++i) x[i] += a.mult * y[i];
     }
@@ -100,7 +127,7 @@ __global__ __launch_bounds__(256) void k_norm_chain(const NormKernelArgs a) {
             if (col(i) < padded) *(f32x4 *)(a.x_out + row * a.ldx + col(i)) = x[i];
     }
     if (a.out) {
-        if (a.pre_w) normalize(x, a.pre_w, a.pre_b);
+        if (a.pre_w) normalize(x, a.pre_w, a.pre_b, held[BATCH ? 2 : 0], held[BATCH ? 3 : 0]);
         AT *o = (AT *)a.out + row * a.ldo;
         typedef AT at4 __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -116,17 +143,24 @@ int launch_norm_chain(candy_hip_device *dev, const NormArgs &A) {
                      A.eps};
     const int v = (int)((pad64(A.cols) + 1023) / 1024);
     const dim3 g((unsigned)A.rows), b(256);
-#define CANDY_NORM(AT)                                                                         \
-    do {                                                                                       \
-        if (v <= 1) hipLaunchKernelGGL((k_norm_chain<AT, 1>), g, b, 0, dev->stream, k);        \
-        else if (v <= 2) hipLaunchKernelGGL((k_norm_chain<AT, 2>), g, b, 0, dev->stream, k);   \
-        else if (v <= 4) hipLaunchKernelGGL((k_norm_chain<AT, 4>), g, b, 0, dev->stream, k);   \
-        else if (v <= 8) hipLaunchKernelGGL((k_norm_chain<AT, 8>), g, b, 0, dev->stream, k);   \
-        else hipLaunchKernelGGL((k_norm_chain<AT, 16>), g, b, 0, dev->stream, k);              \
+    const bool batch = A.rows <= 2 * dev->num_cus && v <= 4 && (A.y.copies > 1 || A.slots);
+#define CANDY_NORM_V(AT, V)                                                                                          \
+    do {                                                                                                             \
+        if (batch && V <= 4) hipLaunchKernelGGL((k_norm_chain<AT, V, (V <= 4)>), g, b, 0, dev->stream, k);           \
+        else hipLaunchKernelGGL((k_norm_chain<AT, V, false>), g, b, 0, dev->stream, k);                              \
+    } while (0)
+#define CANDY_NORM(AT)                          \
+    do {                                        \
+        if (v <= 1) CANDY_NORM_V(AT, 1);        \
+        else if (v <= 2) CANDY_NORM_V(AT, 2);   \
+        else if (v <= 4) CANDY_NORM_V(AT, 4);   \
+        else if (v <= 8) CANDY_NORM_V(AT, 8);   \
+        else CANDY_NORM_V(AT, 16);              \
     } while (0)
     if (A.f32) CANDY_NORM(float);
     else CANDY_NORM(bf16);
 #undef CANDY_NORM
+#undef CANDY_NORM_V
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }
