@@ -655,6 +655,15 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     if (single) return launch_big<F, 128, 256, 2, 4>(dev, jobs, count, xh, m);
     if constexpr (std::is_same<F, BigQ4K>::value)
         if (narrow(256)) return launch_big<F, 112, 256, 2, 4, true>(dev, jobs, count, xh, m);
+    // A grid of 128 x 256 tiles that fills the chip, where the 128 x 128 tiles take no more rounds of workgroups: the
+    // wide grid's last round is then at most a third full and its last column of tiles half empty, and a round of the
+    // narrower tiles is the shorter one (about 0.7).  us on 128 x 256 / 128 x 128 tiles, two rounds either way: 11008 x
+    // 4096 at 513..640 rows (258 and 430 tiles) Q4_K 109 / 80, Q5_K 125 / 105, Q6_K 125 / 98, Q8_0 144 / 110, Q4_0
+    // 138 / 116; 21760 x 2048 at 300 rows (340 and 510, the fullest grids that the rule takes) 60 / 47, 70 / 60, 69 / 59,
+    // 80 / 64, 77 / 65; 9300 x 1024 at 890 rows 40 / 34, 45 / 41, 45 / 40, 52 / 44, 49 / 43.  Where it costs a round
+    // more the wider tiles win: 32000 x 4096 at 300 rows, two against three, Q5_K and Q4_0 0.86x on the narrow ones.
+    auto rounds = [&](int bm) { return (n128 * ((m + bm - 1) / bm) + dev->num_cus - 1) / dev->num_cus; };
+    if (shape == 0 && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256)) return small_tiles();
     return launch_big<F, 128, 256, 2, 4, true>(dev, jobs, count, xh, m);
 }
 
