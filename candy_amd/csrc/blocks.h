@@ -144,6 +144,9 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 
 
+// unary.go:3353-3366: x / (1 + exp(-x))
+__device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
+
 // 1 / sqrt(v) as reduce.go:3083-3085 evaluates it for RMSNorm: 1 / float32(math.Sqrt(float64(v))).  The square root
 // of an f32 taken in f64 and rounded back is the correctly rounded f32 square root (53 bits >= 2 * 24 + 2), which is
 // what sqrtf is here (hipcc rounds f32 sqrt and division correctly by default), so no f64 instruction is needed.

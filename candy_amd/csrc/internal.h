@@ -69,6 +69,7 @@ struct Options {
     int rms_rows = 0;            // fused RMSNorm prologue: rows per workgroup, 16 / 24 (0: the most even split)
     int prefill_fold_split_sums = 1; // prompt pass: split-K copies summed inside the launch that follows (norm, rope)
     int prefill_qkv_group = 1;       // prompt pass: q / k / v (and gate / up) on one grid each where they run on the fp16 tiles
+    int prefill_fold_silu = 1;       // prompt pass: silu(gate) * up and its quantization in the epilogue of their fp16 tiles
     int prefill_attention_valu = 0;  // comparison runs: prompt attention on the vector ALU instead of the matrix cores
     int kv_parts_mb = 0;             // MB at most for the 16-bit parts of a layer's f32 K and V (0: no limit); past it, the vector ALU
     int llama_graph = 1;         // decoders created afterwards replay a captured HIP graph (0: eager launches)
@@ -227,6 +228,10 @@ int launch_mmq_f16_rows(candy_hip_device *dev, const candy_hip_qtensor *w, const
 bool mmq_f16_group_covers(const candy_hip_qtensor *const *ws, int count, int64_t m);
 int launch_mmq_f16_group(candy_hip_device *dev, const candy_hip_qtensor *const *ws, float *const *ys, int count,
                          const _Float16 *xh, int64_t m);
+// silu(gate) * up of the same activations, quantized to Q8_0, as the fp16 image `act` [mmq_m_pad(m)][rows] in one launch.
+bool mmq_f16_silu_covers(const candy_hip_qtensor *gate, const candy_hip_qtensor *up, int64_t m);
+int launch_mmq_f16_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, const candy_hip_qtensor *up, const _Float16 *xh, int64_t m,
+                        _Float16 *act);
 // ops.hip: fused decode-step stages (all enqueue on dev->stream, no allocation, no sync).
 struct RowsImage;  // rows_i8.h: the image takes the place of qs, scales and xh
 int launch_rms_norm_quant(candy_hip_device *dev, const float *x, const float *alpha, float eps, int64_t rows,

@@ -426,10 +426,10 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
         // fp16 expansion (one conversion for q/k/v, one for gate/up), and the residual add rides in the
         // projection's epilogue.
         auto xh_for = [&](const candy_hip_qtensor *w) { return mmq_f16_big_covers(w, n) ? P.xh : nullptr; };
-        auto add_linear = [&](const candy_hip_qtensor *w) -> int {  // P.h += (quantized activations) . w^T
+        auto add_linear = [&](const candy_hip_qtensor *w, const _Float16 *image = nullptr) -> int {  // P.h += (quantized activations) . w^T
             if (mmq_fuses_residual(w, n)) {
                 dev->defer_split = &pend;
-                const int e = launch_contract(dev, w, P.xq, P.xs, n, P.h, xh_for(w), P.h);
+                const int e = launch_contract(dev, w, P.xq, P.xs, n, P.h, image ? image : xh_for(w), P.h);
                 dev->defer_split = nullptr;
                 return e;
             }
@@ -462,6 +462,13 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
         if ((rc = add_linear(L.wo))) return rc;  // h += Wo . att
         xh = (xh_for(L.gate) || xh_for(L.up)) ? P.xh : nullptr;
         if ((rc = norm_quant(L.ffn_norm, xh))) return rc;
+        if (xh && mmq_fuses_residual(L.down, n) && mmq_f16_silu_covers(L.gate, L.up, n)) {
+            // mmq_m_pad(n) rows of 2-byte values fit in gate's n > 128 rows of 4-byte ones
+            _Float16 *act = (_Float16 *)P.gate;
+            if ((rc = launch_mmq_f16_silu(dev, L.gate, L.up, xh, n, act))) return rc;
+            if ((rc = add_linear(L.down, act))) return rc;
+            continue;
+        }
         const candy_hip_qtensor *gu_w[2] = {L.gate, L.up};
         float *gu_y[2] = {P.gate, P.up};
         if (xh && mmq_f16_group_covers(gu_w, 2, n)) {  // the second projection's tiles fill the first one's last round

@@ -30,6 +30,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "attention_tiles.h"
 #include "f16_weights.h"
 #include "internal.h"
 
@@ -72,6 +73,7 @@ struct F16Seg {
 struct F16Group {
     F16Seg seg[3];
     int count;
+    _Float16 *act;  // EPI_SILU: the fp16 image that takes the place of both outputs
     __device__ __forceinline__ F16Seg pick(int nt) const {
         F16Seg s = seg[0];
         if (count > 1 && nt >= seg[1].tile0) s = seg[1];
@@ -263,7 +265,22 @@ __global__ __launch_bounds__(WN * WM * 64) void k_mmq_f16(const F16Group grp, co
 // row counts that are a multiple of 7 * 16 and not of 256 * 128: 14336 = 128 * 112 rows are 128 tiles, one or two per
 // CU, where 112 tiles of 128 rows leave an eighth of the chip idle or wait for a short last round.  The LDS buffers
 // keep room for 128 rows; the producer wavefront whose second task would fall on rows 112 .. 127 repeats its first.
-template <class F, int BN, int BM, bool RES>
+// EPI_SILU: one grid for gate (segment 0) and up (segment 1), 64 rows of each per tile in turns of 32, so that a lane
+// ends with gate and up of the same eight values of a Q8_0 block and the four lanes that share an activation row hold
+// the block: silu(gate) * up leaves as the fp16 image of its quantization, which the down projection reads.  Neither
+// product is written or read as f32.  us per layer, its own launch / this one: Llama-3.2-1B shape 300 rows 157 / 151, 1500
+// rows 368 / 348; Llama-3-8B shape (whose two tensors alone would take tiles of 112 rows) 300 rows 331 / 324, 512 rows 356 /
+// 342, 2048 rows 1124 / 1052; Llama-2-7B shape 300 rows 311 / 308, 1400 rows 847 / 824.  A CU holds one such workgroup, so
+// the epilogue's vector instructions are exposed: with q8_level's branch asked value by value and the full division in
+// silu_f half of the gain was lost (1.035 against 1.058 at 1500 rows).
+enum { EPI_PLAIN, EPI_RES, EPI_SILU };
+// silu_f with the quotient corrected once by its own residual: the same bits for 13 million values from -80 to 100, and 0
+// below -87.3, where the reciprocal is too small for a normal number
+__device__ __forceinline__ float silu_once(float x) {
+    const float den = 1.0f + expf(-x), r = __builtin_amdgcn_rcpf(den), q = x * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-den, q, x), r, q), den, x);
+}
+template <class F, int BN, int BM, int EPI>
 __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _Float16 *__restrict__ xh, int M, int K,
                                                     int n_tiles, int m_tiles, int sb_per, size_t split_stride) {
     constexpr int PT = 256, BNB = 128;  // BNB: weight rows an LDS buffer has room for
@@ -288,9 +305,10 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
     int v = blockIdx.x - split * total;
     if ((total & 7) == 0) v = (v & 7) * (total >> 3) + (v >> 3);
     const int mt = v / n_tiles, nt = v - mt * n_tiles;
-    const F16Seg seg = grp.pick(nt);
+    static_assert(EPI != EPI_SILU || BN == 128, "64 rows of gate and of up");
+    const F16Seg seg = EPI == EPI_SILU ? grp.seg[wave >> 1 & 1] : grp.pick(nt);  // producers 0, 1 gate and 2, 3 up
     const int N = seg.N;
-    const int n0 = (nt - seg.tile0) * BN, m0 = mt * BM;
+    const int n0 = EPI == EPI_SILU ? nt * (BN / 2) : (nt - seg.tile0) * BN, m0 = mt * BM;
 
     const size_t rb = (size_t)(K >> 8) * F::BLOCK;
     const int sb0 = split * sb_per;
@@ -308,10 +326,11 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
         // neighbouring lanes take neighbouring quarters of a row; a half-wavefront takes rows {x, x+4, x+8, x+12}
         const int a_c = lane & 3, a_row = 16 * wave + 4 * ((lane >> 2) & 3) + (lane >> 4);   // + a_step i
         const int a_step = BN == 112 && wave == 3 ? 0 : 64;
+        const int w_row = EPI == EPI_SILU ? a_row & 31 : a_row, w_step = EPI == EPI_SILU ? 32 : a_step;  // in the tensor
         auto gload_a = [&](int sb, int slot) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < ATK; ++i)
-                F::load(W + (size_t)min(n0 + a_row + a_step * i, N - 1) * rb + (size_t)sb * F::BLOCK, a_c, raw[slot][i]);
+                F::load(W + (size_t)min(n0 + w_row + w_step * i, N - 1) * rb + (size_t)sb * F::BLOCK, a_c, raw[slot][i]);
         };
         auto stage = [&](int g, int aslot, int buf) __attribute__((always_inline)) {
             _Float16 *a = sA + buf * BNB * BIG_BK;
@@ -430,6 +449,54 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
         }
     }
 
+    if constexpr (EPI == EPI_SILU) {
+        // the arithmetic of k_silu_mul_quant (quantize_q8_lane4 + q8_lane4_to_half) value by value
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+            const int m = m0 + cw * (BM / 4) + tm * 16 + (lane & 15);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                float z[2][4], amax = 0.0f;
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                    for (int l = 0; l < 4; ++l) {
+                        z[hf][l] = silu_once(acc[4 * b + hf][tm][l]) * acc[4 * b + 2 + hf][tm][l];
+                        amax = hf + l ? fmaxf(amax, fabsf(z[hf][l])) : fabsf(z[hf][l]);
+                    }
+                amax = quad16_max(amax);
+                const float d = amax / 127.0f, df = __half2float(__float2half_rn(d)), inv = __builtin_amdgcn_rcpf(d);
+                // q8_level: the rounded product is the level unless it lies within 6.1e-5 of a half (or is no number: an
+                // empty block, a scale or a value that is not finite), asked once for the eight values
+                float level[2][4];
+                bool unsure = false;
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                    for (int l = 0; l < 4; ++l) {
+                        const float t = z[hf][l] * inv;
+                        level[hf][l] = rintf(t);
+                        unsure |= !(fabsf(t - level[hf][l]) < 0.5f - 6.1e-5f);
+                    }
+                if (__builtin_expect(unsure, 0)) {
+#pragma unroll
+                    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                        for (int l = 0; l < 4; ++l) level[hf][l] = (float)(int8_t)(amax != 0.0f ? q8_level(z[hf][l], d) : 0);
+                }
+                const int n = n0 + 32 * b + 4 * (lane >> 4);
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf) {
+                    half4v h;
+#pragma unroll
+                    for (int l = 0; l < 4; ++l) h[l] = (_Float16)(df * level[hf][l]);
+                    if (m < M && n < N) *(half4v *)(grp.act + xh_index4(m, (n + 16 * hf) >> 2, N) * 4) = h;
+                }
+            }
+        }
+        return;
+    }
+
     // C layout of a 16x16 tile: lane holds activation row (lane & 15) and weight rows 4*(lane>>4)..+3
 #pragma unroll
     for (int tn = 0; tn < TNF; ++tn)
@@ -439,7 +506,7 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
             const int n = n0 + tn * 16 + 4 * (lane >> 4);
             if (m >= M) continue;
             float *dst = out + (size_t)m * N + n;
-            const float *r = RES && res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
+            const float *r = EPI == EPI_RES && res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
             if (n + 3 < N && (N & 3) == 0) {
                 float4 o = make_float4(acc[tn][tm][0], acc[tn][tm][1], acc[tn][tm][2], acc[tn][tm][3]);
                 if (r) {
@@ -549,7 +616,7 @@ static int launch_big(candy_hip_device *dev, const F16Job *jobs, int count, cons
     constexpr size_t smem = (size_t)(PC ? 3 * 128 : 2 * (BN + BM)) * BIG_BK * sizeof(_Float16);  // role-split: weight tiles only
     const bool epi_res = any_res && n_split == 1;
     void (*kern)(const F16Group, const _Float16 *, int, int, int, int, int, size_t);
-    if constexpr (PC) kern = epi_res ? k_mmq_f16_pc<F, BN, BM, true> : k_mmq_f16_pc<F, BN, BM, false>;
+    if constexpr (PC) kern = epi_res ? k_mmq_f16_pc<F, BN, BM, EPI_RES> : k_mmq_f16_pc<F, BN, BM, EPI_PLAIN>;
     else kern = epi_res ? k_mmq_f16<F, BN, BM, WN, WM, true> : k_mmq_f16<F, BN, BM, WN, WM, false>;
     CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * n_split)), dim3(WN * WM * 64), smem, dev->stream, grp, xh, (int)m, K,
@@ -703,6 +770,55 @@ int launch_mmq_f16_group(candy_hip_device *dev, const candy_hip_qtensor *const *
     F16Job jobs[3];
     for (int s = 0; s < count; ++s) jobs[s] = F16Job{ws[s], ys[s], nullptr};
     return launch_jobs(dev, jobs, count, xh, m);
+}
+
+// Gate, up and silu(gate) * up in one launch (EPI_SILU), where a tile's sums are whole: the grid of 128 x 256 tiles has to
+// fill the chip without a split of K.
+static bool silu_fills(const candy_hip_device *dev, int64_t rows, int64_t m) {
+    return (rows / 64) * ((m + 255) / 256) >= (3 * (int64_t)dev->num_cus) / 4;
+}
+
+bool mmq_f16_silu_covers(const candy_hip_qtensor *gate, const candy_hip_qtensor *up, int64_t m) {
+    const candy_hip_qtensor *const ws[2] = {gate, up};
+    const Options &opt = gate->dev->opt;
+    return opt.prefill_fold_silu && opt.f16_shape == 0 && opt.f16_split == 0 && m > 128 && gate->rows == up->rows && gate->rows % 64 == 0 &&
+           mmq_f16_group_covers(ws, 2, m) && silu_fills(gate->dev, gate->rows, m);
+}
+
+template <class F, int BM>
+static int launch_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, const candy_hip_qtensor *up, const _Float16 *xh, int64_t m,
+                       _Float16 *act) {
+    const int N = (int)gate->rows, K = (int)gate->cols, n_tiles = N / 64, m_tiles = (int)((m + BM - 1) / BM);
+    F16Group grp{};
+    grp.count = 2;
+    grp.act = act;
+    grp.seg[0] = F16Seg{(const uint8_t *)gate->data, nullptr, nullptr, N, 0};
+    grp.seg[1] = F16Seg{(const uint8_t *)up->data, nullptr, nullptr, N, 0};
+    constexpr size_t smem = (size_t)3 * 128 * BIG_BK * sizeof(_Float16);
+    void (*kern)(const F16Group, const _Float16 *, int, int, int, int, int, size_t) = k_mmq_f16_pc<F, 128, BM, EPI_SILU>;
+    CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n_tiles * m_tiles)), dim3(512), smem, dev->stream, grp, xh, (int)m, K, n_tiles, m_tiles,
+                       K >> 8, (size_t)0);
+    CANDY_LAUNCH_CHECK();
+    return CANDY_HIP_OK;
+}
+
+int launch_mmq_f16_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, const candy_hip_qtensor *up, const _Float16 *xh, int64_t m,
+                        _Float16 *act) {
+    CANDY_REQUIRE(mmq_f16_silu_covers(gate, up, m), "internal: gate and up cannot share tiles");
+    // the narrower tiles where they take no more rounds of workgroups, as in launch_shapes
+    auto rounds = [&](int bm) { return (gate->rows / 64 * ((m + bm - 1) / bm) + dev->num_cus - 1) / dev->num_cus; };
+    const bool narrow = rounds(128) <= rounds(256);
+#define CANDY_SILU(F) return narrow ? launch_silu<F, 128>(dev, gate, up, xh, m, act) : launch_silu<F, 256>(dev, gate, up, xh, m, act)
+    switch (gate->fmt) {
+    case CANDY_HIP_Q6_K: CANDY_SILU(BigQ6K);
+    case CANDY_HIP_Q5_K: CANDY_SILU(BigQ5K);
+    case CANDY_HIP_Q8_0: CANDY_SILU(BigQ8_0);
+    case CANDY_HIP_Q4_0: CANDY_SILU(BigQ4_0<false>);
+    case CANDY_HIP_Q4_0_GGML: CANDY_SILU(BigQ4_0<true>);
+    default: CANDY_SILU(BigQ4K);
+    }
+#undef CANDY_SILU
 }
 
 }  // namespace candy

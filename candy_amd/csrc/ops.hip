@@ -108,9 +108,6 @@ __global__ __launch_bounds__(256) void k_softmax(const float *__restrict__ src, 
     for (int c = threadIdx.x; c < cols; c += blockDim.x) orow[c] *= inv;
 }
 
-// unary.go:3353-3366: x / (1 + exp(-x))
-__device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
-
 enum { EW_SILU = 0, EW_ADD = 1, EW_MUL = 2, EW_SILU_MUL = 3 };
 template <int OP>
 __global__ __launch_bounds__(256) void k_elementwise(const float *__restrict__ a, const float *__restrict__ b,

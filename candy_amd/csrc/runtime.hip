@@ -360,6 +360,7 @@ const OptionKey OPTION_KEYS[] = {
     {"fused.pair_rows", &candy::Options::pair_rows, 0, 32},
     {"fused.rms_rows", &candy::Options::rms_rows, 0, 24},
     {"prefill.qkv_group", &candy::Options::prefill_qkv_group, 0, 1},
+    {"prefill.fold_silu", &candy::Options::prefill_fold_silu, 0, 1},
     {"prefill.fold_split_sums", &candy::Options::prefill_fold_split_sums, 0, 1},
     {"prefill.attention_valu", &candy::Options::prefill_attention_valu, 0, 1},
     {"prefill.kv_parts_mb", &candy::Options::kv_parts_mb, 0, 1 << 20},

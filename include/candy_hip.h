@@ -123,6 +123,8 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *                                         workgroups per kv head (latent attention: per 16 heads), 1..64 (0: by shape); read when a decoder is created
  *   "prefill.qkv_group"          1        prompt pass: projections that share their input (q / k / v; gate / up) as one
  *                                         grid each where all of them run on the fp16 tiles (0: one launch each)
+ *   "prefill.fold_silu"          1        prompt pass: silu(gate) * up and its quantization in the epilogue of the launch that
+ *                                         contracts gate and up on shared fp16 tiles, where those fill the chip (0: a launch of its own)
  *   "prefill.fold_split_sums"    1        prompt pass: the partial copies a projection split along K leaves are summed by the
  *                                         launch that follows (RMSNorm + quantize behind o / down, rope behind q / k / v;
  *                                         0: a launch of its own sums them)
