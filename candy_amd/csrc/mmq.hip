@@ -313,7 +313,8 @@ static int launch_fmt(candy_hip_device *dev, const candy_hip_qtensor *w, const _
     return launch_tile<F, 128, 128, 64>(dev, w, xh, m, y);
 }
 
-int64_t mmq_m_pad(int64_t m) { return (m + 255) / 256 * 256; }  // a multiple of every tile height
+// whole tiles of 256 (128) and of 192 rows
+int64_t mmq_m_pad(int64_t m) { return std::max((m + 255) / 256 * 256, (m + 191) / 192 * 192); }
 
 static int mmq_dispatch(candy_hip_device *dev, const candy_hip_qtensor *w, const int8_t *qs, const Q8Scale *scales,
                         int64_t m, float *y, void *half_ws, const _Float16 *xh_ready, const float *res, bool *res_done,

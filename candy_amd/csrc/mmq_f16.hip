@@ -13,7 +13,7 @@
 // Both roundings are 2^-12 relative per element; the result stays a few 1e-4 (max-norm) from the
 // CPU contraction, inside the 1e-3 bar.
 //
-// Tiling: a workgroup owns 128 weight rows x 256 (or 128) activation rows and walks K in steps of 64.
+// Tiling: a workgroup owns 128 weight rows x 256 (192, 128) activation rows and walks K in steps of 64.
 //   k_mmq_f16_pc (what runs): four producer wavefronts dequantize 16 weights per thread and step into an LDS tile
 //     (two or three buffers, one barrier per step); four consumer wavefronts read the weight fragments from LDS,
 //     load their activation fragments straight from memory into operand registers (the fp16 image is stored
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(WN * WM * 64) void k_mmq_f16(const F16Group grp, co
 }
 
 // ------------------------------------------------------------------ the same tile with the work split by role
-// 128 weight rows x BM (256 or 128) activation rows, 8 wavefronts: wavefronts 0-3 (one per SIMD) are producers, 4-7
+// 128 weight rows x BM (256, 192 or 128) activation rows, 8 wavefronts: wavefronts 0-3 (one per SIMD) are producers, 4-7
 // consumers.
 // Producers request weights, dequantize them and fill the LDS weight buffer of step s + 1 (two buffers) while the
 // consumers contract step s; one workgroup barrier per step hands a buffer over.  The activations never touch LDS:
@@ -288,12 +288,12 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
     constexpr int TNF = BN / 16;        // 16-row weight fragments of the tile
     static_assert(BN == 128 || BN == 112, "weight rows per tile");
     constexpr int TM = BM / 64;       // 16-row activation fragments of a consumer's sub-tile (its rows: BM / 4)
-    static_assert(BM == 256 || BM == 128, "activation rows per tile");
-    // BM = 256: the producers work two steps ahead into the third of three weight buffers, and a consumer reads the
+    static_assert(BM == 256 || BM == 192 || BM == 128, "activation rows per tile");
+    // BM = 256, 192: the producers work two steps ahead into the third of three weight buffers, and a consumer reads the
     // first weight fragments of step s + 1 during the last matrix instructions of step s (16 per phase cover the
     // read).  BM = 128 (8 matrix instructions per phase) is faster one step ahead with two buffers: 33.8 against
     // 35.2 us at 14336 x 4096 x 128.
-    constexpr int LEAD = BM == 256 ? 2 : 1, NB = LEAD + 1;
+    constexpr int LEAD = BM > 128 ? 2 : 1, NB = LEAD + 1;
     extern __shared__ __align__(16) uint8_t smem_raw[];
     _Float16 *sA = (_Float16 *)smem_raw;               // [NB][BNB / 16][2] fragments
 
@@ -432,8 +432,8 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
 #pragma unroll
             for (int p = 0; p < PH; ++p) {
 #pragma unroll
-                for (int t = 0; t < 2 * TM / PH; ++t) {
-                    const int l = p * (2 * TM / PH) + t, kk = l / TM, tm = l % TM;
+                for (int l = 2 * TM * p / PH; l < 2 * TM * (p + 1) / PH; ++l) {
+                    const int kk = l / TM, tm = l % TM;
                     bf[(g + BD) & (NS - 1)][kk][tm] = *(const half8 *)(xfrag + ((size_t)tm * (K >> 5) + (size_t)ksn * 2 + kk) * 512);
                 }
                 // the next phase's weight fragments - after the last phase: the next step's first, whose buffer has
@@ -581,7 +581,7 @@ static int plan_split(const candy_hip_device *dev, int tiles, int n_sb) {
 
 template <class F, int BN, int BM, int WN, int WM, bool PC = false>
 static int launch_big(candy_hip_device *dev, const F16Job *jobs, int count, const _Float16 *xh, int64_t m) {
-    static_assert(!PC || ((BN == 128 || BN == 112) && (BM == 256 || BM == 128) && WN * WM == 8), "the role-split kernel's tiles");
+    static_assert(!PC || ((BN == 128 || BN == 112) && (BM == 256 || BM == 192 || BM == 128) && WN * WM == 8), "the role-split kernel's tiles");
     const int K = (int)jobs[0].w->cols;
     F16Group grp{};
     grp.count = count;
@@ -672,7 +672,7 @@ bool mmq_f16_big_covers(const candy_hip_qtensor *w, int64_t m, int min_m) {
     return false;
 }
 
-// Tile shape by batch and grid.  Every format: 128 x 128 tiles up to 128 activation rows, 128 x 256 above.  Q4_K, whose
+// Tile shape by batch and grid.  Every format: 128 x 128 tiles up to 128 activation rows, 128 x 256 or 128 x 192 above.  Q4_K, whose
 // dequantization is the cheapest, also takes the narrower tiles on some grids above 128 rows (with the heavier formats
 // the producers then set the pace: Q6_K 14336 x 4096 at 192 rows 58.3 us on 128 x 128 tiles against 53.8, Q8_0 68.5
 // against 58.6), and tiles of 112 weight rows.
@@ -680,24 +680,26 @@ template <class F>
 static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, const _Float16 *xh, int64_t m) {
     const int shape = dev->opt.f16_shape;  // comparison runs
     const bool single = shape == 3;        // every wavefront in both roles
+    // What the busiest CU does: rounds of workgroups x weight rows per tile x super-blocks per workgroup, x 8 (a step of 192
+    // activation rows: 7, of 256: 8; measured 0.84 to 0.88, the producers' share being the same).  0: not for these rows.
+    auto cost = [&](int bn, int bm) -> int64_t {
+        const int n_sb = (int)(jobs[0].w->cols >> 8), m_tiles = (int)((m + bm - 1) / bm);
+        int64_t tiles = 0;
+        for (int s = 0; s < count; ++s) {
+            if (bn == 112 && jobs[s].w->rows % 112 != 0) return 0;
+            tiles += (jobs[s].w->rows + bn - 1) / bn;
+        }
+        const int ns = plan_split(dev, (int)(tiles * m_tiles), n_sb), sb_per = (n_sb + ns - 1) / ns;
+        const int64_t wgs = tiles * m_tiles * ((n_sb + sb_per - 1) / sb_per);
+        return ((wgs + dev->num_cus - 1) / dev->num_cus) * bn * sb_per * (bm == 192 ? 7 : 8);
+    };
     // Tiles of 112 weight rows where every tensor's rows divide by 112 and the grid then takes fewer row-steps of its
-    // busiest CU: rounds of workgroups x rows per tile x super-blocks per workgroup (14336 rows: 128 tiles instead of
-    // 112, so 256 instead of 224 workgroups at 512 activation rows, 512 instead of 448 for a gate / up pair).
+    // busiest CU (14336 rows: 128 tiles instead of 112, so 256 instead of 224 workgroups at 512 activation rows, 512
+    // instead of 448 for a gate / up pair).
     auto narrow = [&](int bm) {
         if (!std::is_same<F, BigQ4K>::value || single || shape == 4) return false;
-        const int n_sb = (int)(jobs[0].w->cols >> 8), m_tiles = (int)((m + bm - 1) / bm);
-        int64_t t112 = 0, t128 = 0;
-        for (int s = 0; s < count; ++s) {
-            if (jobs[s].w->rows % 112 != 0) return false;
-            t112 += jobs[s].w->rows / 112;
-            t128 += (jobs[s].w->rows + 127) / 128;
-        }
-        auto cost = [&](int64_t tiles, int bn) {
-            const int ns = plan_split(dev, (int)(tiles * m_tiles), n_sb), sb_per = (n_sb + ns - 1) / ns;
-            const int64_t wgs = tiles * m_tiles * ((n_sb + sb_per - 1) / sb_per);
-            return ((wgs + dev->num_cus - 1) / dev->num_cus) * bn * sb_per;
-        };
-        return cost(t112, 112) < cost(t128, 128);
+        const int64_t c112 = cost(112, bm);
+        return c112 > 0 && c112 < cost(128, bm);
     };
     auto small_tiles = [&]() {
         if (single) return launch_big<F, 128, 128, 2, 4>(dev, jobs, count, xh, m);
@@ -720,8 +722,6 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     if (q4k && shape == 0 && jobs[0].w->cols <= 4096 && n128 * ((m + 255) / 256) < fill && n128 * ((m + 127) / 128) <= dev->num_cus)
         return small_tiles();
     if (single) return launch_big<F, 128, 256, 2, 4>(dev, jobs, count, xh, m);
-    if constexpr (std::is_same<F, BigQ4K>::value)
-        if (narrow(256)) return launch_big<F, 112, 256, 2, 4, true>(dev, jobs, count, xh, m);
     // A grid of 128 x 256 tiles that fills the chip, where the 128 x 128 tiles take no more rounds of workgroups: the
     // wide grid's last round is then at most a third full and its last column of tiles half empty, and a round of the
     // narrower tiles is the shorter one (about 0.7).  us on 128 x 256 / 128 x 128 tiles, two rounds either way: 11008 x
@@ -730,7 +730,19 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     // 80 / 64, 77 / 65; 9300 x 1024 at 890 rows 40 / 34, 45 / 41, 45 / 40, 52 / 44, 49 / 43.  Where it costs a round
     // more the wider tiles win: 32000 x 4096 at 300 rows, two against three, Q5_K and Q4_0 0.86x on the narrow ones.
     auto rounds = [&](int bm) { return (n128 * ((m + bm - 1) / bm) + dev->num_cus - 1) / dev->num_cus; };
-    if (shape == 0 && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256)) return small_tiles();
+    if (shape == 0 && !narrow(256) && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256)) return small_tiles();
+    // Tiles of 192 activation rows where they leave the busiest CU less to do: a last column of tiles that would be mostly
+    // empty (300 rows are 2 x 192 as they are 2 x 256), or a grid that fills the rounds better (1300 rows against 4096
+    // weight rows: 224 workgroups instead of 192).  Over thirteen weight shapes and seventeen row counts from 140 to 2048,
+    // five formats, the rule takes them at 4 points of 10, 1.09x on the geometric mean there, 0.996x to 1.225x.  us before /
+    // with them: Q4_K 14336 x 4096 at 300 rows 60.6 / 51.0, 4096 x 14336 at 560 rows 101 / 87.5; Q5_K 32000 x 4096 at 560
+    // rows 199 / 179; Q8_0 11008 x 4096 at 300 rows 77 / 70; Q6_K 4096 x 4096 at 1300 rows 69.9 / 63.4.
+    const bool rows192 = shape == 0 && (narrow(192) ? cost(112, 192) : cost(128, 192)) < (narrow(256) ? cost(112, 256) : cost(128, 256));
+    if constexpr (std::is_same<F, BigQ4K>::value) {
+        if (rows192 && narrow(192)) return launch_big<F, 112, 192, 2, 4, true>(dev, jobs, count, xh, m);
+        if (!rows192 && narrow(256)) return launch_big<F, 112, 256, 2, 4, true>(dev, jobs, count, xh, m);
+    }
+    if (rows192) return launch_big<F, 128, 192, 2, 4, true>(dev, jobs, count, xh, m);
     return launch_big<F, 128, 256, 2, 4, true>(dev, jobs, count, xh, m);
 }
 
@@ -806,10 +818,12 @@ static int launch_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, con
 int launch_mmq_f16_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, const candy_hip_qtensor *up, const _Float16 *xh, int64_t m,
                         _Float16 *act) {
     CANDY_REQUIRE(mmq_f16_silu_covers(gate, up, m), "internal: gate and up cannot share tiles");
-    // the narrower tiles where they take no more rounds of workgroups, as in launch_shapes
+    // the tiles of fewer activation rows by the rules of launch_shapes
     auto rounds = [&](int bm) { return (gate->rows / 64 * ((m + bm - 1) / bm) + dev->num_cus - 1) / dev->num_cus; };
-    const bool narrow = rounds(128) <= rounds(256);
-#define CANDY_SILU(F) return narrow ? launch_silu<F, 128>(dev, gate, up, xh, m, act) : launch_silu<F, 256>(dev, gate, up, xh, m, act)
+    const int bm = rounds(128) <= rounds(256) ? 128 : 7 * rounds(192) < 8 * rounds(256) ? 192 : 256;
+#define CANDY_SILU(F)                                                                                                     \
+    return bm == 128 ? launch_silu<F, 128>(dev, gate, up, xh, m, act)                                                     \
+                     : bm == 192 ? launch_silu<F, 192>(dev, gate, up, xh, m, act) : launch_silu<F, 256>(dev, gate, up, xh, m, act)
     switch (gate->fmt) {
     case CANDY_HIP_Q6_K: CANDY_SILU(BigQ6K);
     case CANDY_HIP_Q5_K: CANDY_SILU(BigQ5K);

@@ -29,8 +29,8 @@ def model(dev, fmt, d_ffn, gain, max_pos):
     return m
 
 
-# 128 x 256 tiles (whole, and one row into the second column of tiles); 128 x 128 tiles where they need no more rounds (three, five
-# columns of tiles, the last of 1 and 128 rows); products that fp16 scales, and f32, cannot hold
+# 128 x 256 tiles (whole, and a ragged second column); 128 x 192 (one row past 256, and 300); 128 x 128 where they need no more
+# rounds (three, five columns of tiles, the last of 1 and 128 rows); products that fp16 scales, and f32, cannot hold
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q5_K, synth.Q6_K, synth.Q8_0, synth.Q4_0, synth.Q4_0_GGML])
 @pytest.mark.parametrize("n,d_ffn,gain", [(256, 12288, 1), (257, 6144, 1), (500, 6400, 0.01), (257, 9472, 1), (640, 5632, 1), (300, 6144, 30),
