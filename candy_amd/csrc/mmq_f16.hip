@@ -274,11 +274,12 @@ __global__ __launch_bounds__(WN * WM * 64) void k_mmq_f16(const F16Group grp, co
 // the epilogue's vector instructions are exposed: with q8_level's branch asked value by value and the full division in
 // silu_f half of the gain was lost (1.035 against 1.058 at 1500 rows).
 enum { EPI_PLAIN, EPI_RES, EPI_SILU };
-// silu_f with the quotient corrected once by its own residual: the same bits for 13 million values from -80 to 100, and 0
-// below -87.3, where the reciprocal is too small for a normal number
+// silu_f with the quotient corrected once by its own residual: the same bits for every f32.  Below -87.3 the divisor's reciprocal
+// is too small for a normal number: there both sides of the division are taken at a quarter (x near -88: exact).
 __device__ __forceinline__ float silu_once(float x) {
-    const float den = 1.0f + expf(-x), r = __builtin_amdgcn_rcpf(den), q = x * r;
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-den, q, x), r, q), den, x);
+    const float den = 1.0f + expf(-x), part = den >= 0x1p126f ? 0.25f : 1.0f, dp = den * part, xp = x * part;
+    const float r = __builtin_amdgcn_rcpf(dp), q = xp * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-dp, q, xp), r, q), den, x);
 }
 template <class F, int BN, int BM, int EPI>
 __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _Float16 *__restrict__ xh, int M, int K,
