@@ -211,6 +211,7 @@ bool mmq_i8_covers(const candy_hip_qtensor *w, const int8_t *qs);
 // mmv_i8.hip: 2 .. 32 activation rows against a Q4_K weight, one pass over the weights on the int8 matrix cores
 size_t mmv_workspace_bytes(int64_t K);
 bool mmv_covers(const candy_hip_qtensor *w, int64_t m);
+bool matvec_row_fits(int64_t cols);  // whether the vector kernels (fewer than 16 activation rows) hold rows of this length
 bool matvec_even_covers(const candy_hip_qtensor *w, int64_t m);  // the even-split vector kernel takes this batch
 int launch_mmv(candy_hip_device *dev, const candy_hip_qtensor *w, const float *x, const void *q8_blocks, int64_t m,
                float *y, void *ws);

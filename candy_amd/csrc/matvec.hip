@@ -656,12 +656,16 @@ static int launch_even(candy_hip_device *dev, const candy_hip_qtensor *w, const 
     return launch_even_cfg<U, 4, 1, 2>(dev, w, qs, scales, m, y, grid);
 }
 
+// LDS bytes of one activation row's image in the vector kernels (planar quants, 16 bytes apart every 256, and scales), and whether
+// such rows can be taken at all.
+static size_t matvec_row_bytes(int64_t K) { return (size_t)K + (((size_t)K >> 8) << 4) + (size_t)(K >> 5) * sizeof(Q8Scale); }
+bool matvec_row_fits(int64_t K) { return matvec_row_bytes(K) <= 64 * 1024; }
+
 template <class U, int NB, int R, int WAVES>
 static int launch_one(candy_hip_device *dev, const candy_hip_qtensor *w, const int8_t *qs, const Q8Scale *scales,
                       float *y, int m = NB) {
     const int N = (int)w->rows, K = (int)w->cols;
-    const size_t q_bytes = (size_t)K + (((size_t)K >> 8) << 4);
-    const size_t smem = NB * (q_bytes + (size_t)(K >> 5) * sizeof(Q8Scale));
+    const size_t smem = NB * matvec_row_bytes(K);
     CANDY_REQUIRE(smem <= 64 * 1024, "contraction dim %d too large for the matvec kernel (%zu bytes of LDS)", K, smem);
     const int rows_per_wg = R * WAVES;
     const unsigned grid = (unsigned)((N + rows_per_wg - 1) / rows_per_wg);

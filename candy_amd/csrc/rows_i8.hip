@@ -423,8 +423,11 @@ bool rows_i8_covers(const candy_hip_qtensor *w) {
     }
 }
 
+// Below 16 activation rows the length of the weight rows is limited by the vector kernels, whichever kernel is ahead: a batch that
+// one row more or less would have refused is not taken here either (matvec.hip takes it where its tiles do).
 bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
     const Options &o = w->dev->opt;
+    if (m < 16 && !matvec_row_fits(w->cols)) return false;
     return o.rows_i8 && o.mmv_max_m != 0 && !o.mmq_fp16_only && m >= 3 && m <= 255 && rows_i8_covers(w);
 }
 
@@ -497,3 +500,16 @@ int launch_rows_i8(candy_hip_device *dev, const RowsLaunch &L, int64_t m) {
 }
 
 }  // namespace candy
+
+// The rules above, for their tests (no device needed): bit 0 whether a single contraction goes here, bit 1 whether a prompt does.
+extern "C" int candy_test_rows_i8(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus, int exact, int f16_api_min_m, int i8_min_m,
+                                  int small_batch_kernel) {
+    candy_hip_device dev;
+    dev.num_cus = num_cus;
+    dev.opt.f16_api_min_m = f16_api_min_m;
+    dev.opt.i8_min_m = i8_min_m;
+    dev.opt.small_batch_kernel = small_batch_kernel;
+    candy_hip_qtensor w;
+    w.dev = &dev; w.fmt = fmt; w.rows = rows; w.cols = cols; w.padded = true;
+    return (candy::rows_i8_picks(&w, m, exact != 0) ? 1 : 0) | (candy::rows_i8_takes(&w, m) ? 2 : 0);
+}

@@ -307,6 +307,17 @@ def test_rows_past_the_small_batch_limit_are_an_error_not_a_fault(dev):
     q.free()
 
 
+# Formats and sizes that the matrix-core kernels for few rows would take: what the vector kernels refuse is refused here too
+@pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q8_0])
+def test_three_and_four_rows_past_the_limit_are_refused(dev, fmt):
+    rows, cols = 80, 65536  # more than 4 M values
+    q = dev.qtensor(fmt, rows, cols, synth.random_weight(fmt, rows, cols, seed=3))
+    for m in (3, 4):
+        with pytest.raises(hip.CandyHipError, match="too large for the matvec kernel"):
+            dev.qmatmul(q, synth.random_activations(m, cols, seed=m))
+    dev.synchronize()
+
+
 def test_qmatmul_from_prequantized_blocks(dev):
     rows, cols, m = 64, 1024, 3
     w = synth.random_weight(synth.Q4_K, rows, cols, seed=1)
