@@ -437,8 +437,8 @@ bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
 //     4096, 32 rows 16.4 / 15.1, 4096 x 11008, 16 rows 11.1 / 9.7)
 //   three and four rows, the vector kernels: small weights (1024 x 4096, Q5_K 7.2 / 7.2, Q8_0 7.3 / 7.6), and Q8_0 and Q4_0 where a
 //     workgroup's few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0; 4096 x 4096 8.4 / 7.7)
-//   the fp16 kernels, whose scales are in the operands, where a call may take them: Q4_K and Q6_K from 33 rows (11008 x 4096, 48 rows
-//     16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 / 35.8)
+//   the fp16 kernels, whose scales are in the operands, where a call may take them (mmq.f16_api_min_m): Q4_K and Q6_K from 33 rows
+//     (11008 x 4096, 48 rows 16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 / 35.8)
 // Weights under a million values are launches and nothing else whatever the kernel.
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     const Options &o = w->dev->opt;
@@ -448,7 +448,7 @@ bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     if (q4k && w->cols <= 4096 && mmv_covers(w, m) && w->rows <= (m <= 16 ? 64 * cus : 32 * cus)) return false;
     if (m <= 4 && values <= 1 << 22) return false;
     if (m <= 4 && !q4k && !q6k && w->fmt != CANDY_HIP_Q5_K && w->cols <= 4096 && strips > 2 * cus && strips <= 4 * cus) return false;
-    return exact || m <= (q4k || q6k ? 32 : 64);
+    return exact || !mmq_f16_big_covers(w, m, o.f16_api_min_m);
 }
 
 // Tile and wavefronts.  One activation tile per workgroup where the strips alone leave half of the CUs idle (weights read

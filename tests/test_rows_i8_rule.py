@@ -30,3 +30,13 @@ def test_rows_too_long_for_the_vector_kernels(fmt):
             assert not single(fmt, 4096, 196 * 256, m, exact) and not prompt(fmt, 4096, 196 * 256, m)
     assert prompt(fmt, 4096, 195 * 256, 15) and single(fmt, 4096, 195 * 256, 15)
     assert prompt(fmt, 4096, 196 * 256, 16) and single(fmt, 4096, 65536, 16)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_single_contractions_leave_the_batches_that_take_fp16_tiles(fmt):
+    k46 = fmt in (synth.Q4_K, synth.Q6_K)
+    for option in (16, 20, 33, 64, 65, 100, 1 << 30):
+        first = option if k46 else max(option, 65)  # candy_hip.h: the other formats from 65 or this if larger
+        for m in (17, 19, 20, 32, 33, 63, 64, 65, 99, 100, 200, 255):
+            assert single(fmt, 11000, 4096, m, f16_api_min_m=option) == (m < first), (option, m)
+            assert single(fmt, 11000, 4096, m, exact=1, f16_api_min_m=option) and prompt(fmt, 11000, 4096, m, f16_api_min_m=option)
