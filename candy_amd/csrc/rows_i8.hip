@@ -428,6 +428,7 @@ bool rows_i8_covers(const candy_hip_qtensor *w) {
 bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
     const Options &o = w->dev->opt;
     if (m < 16 && !matvec_row_fits(w->cols)) return false;
+    if (m < o.i8_min_m || o.small_batch_kernel == 0) return false;  // comparison runs that ask for the vector kernels
     return o.rows_i8 && o.mmv_max_m != 0 && !o.mmq_fp16_only && m >= 3 && m <= 255 && rows_i8_covers(w);
 }
 
@@ -443,7 +444,7 @@ bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     const Options &o = w->dev->opt;
     const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16;
-    if (!rows_i8_takes(w, m) || values < 1 << 20 || m < o.i8_min_m || o.small_batch_kernel == 0) return false;
+    if (!rows_i8_takes(w, m) || values < 1 << 20) return false;
     const bool q4k = w->fmt == CANDY_HIP_Q4_K, q6k = w->fmt == CANDY_HIP_Q6_K;
     if (q4k && w->cols <= 4096 && mmv_covers(w, m) && w->rows <= (m <= 16 ? 64 * cus : 32 * cus)) return false;
     if (m <= 4 && values <= 1 << 22) return false;

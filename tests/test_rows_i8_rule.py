@@ -40,3 +40,11 @@ def test_single_contractions_leave_the_batches_that_take_fp16_tiles(fmt):
         for m in (17, 19, 20, 32, 33, 63, 64, 65, 99, 100, 200, 255):
             assert single(fmt, 11000, 4096, m, f16_api_min_m=option) == (m < first), (option, m)
             assert single(fmt, 11000, 4096, m, exact=1, f16_api_min_m=option) and prompt(fmt, 11000, 4096, m, f16_api_min_m=option)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_comparison_runs_on_the_vector_kernels(fmt):
+    for m in (5, 12, 40):
+        assert prompt(fmt, 11000, 4096, m) and prompt(fmt, 11000, 4096, m, i8_min_m=2)
+        for kw in (dict(i8_min_m=99), dict(small_batch_kernel=0)):
+            assert not prompt(fmt, 11000, 4096, m, **kw) and not single(fmt, 11000, 4096, m, **kw)
