@@ -432,10 +432,21 @@ bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
     return o.rows_i8 && o.mmv_max_m != 0 && !o.mmq_fp16_only && m >= 3 && m <= 255 && rows_i8_covers(w);
 }
 
+// Whether launches of four strips of weight rows per workgroup leave a tenth or more of the chip's two slots a CU idle: just past a
+// whole round (1025 to 1840 strips, 2049 to 2560).
+static bool four_strips_idle(int64_t strips, int64_t cus) {
+    const int64_t wgs = (strips + 3) / 4, slots = 2 * cus;
+    return strips > 4 * cus && strips <= 10 * cus && 10 * wgs < 9 * slots * ((wgs + slots - 1) / slots);
+}
+
 // Where the other kernels are ahead or level, us of a call, there / here:
 //   Q4_K up to 16 (8192 or fewer weight rows: 32) activation rows of 4096 or fewer values, the one-shot kernel of mmv_i8.hip:
 //     4096 x 4096, 16 rows 7.1 / 7.2, 14336 x 4096 11.2 / 12.1, 8192 x 2048, 32 rows 7.7 / 8.0 (but 32000 x 4096 19.6 / 17.8, 14336 x
-//     4096, 32 rows 16.4 / 15.1, 4096 x 11008, 16 rows 11.1 / 9.7)
+//     4096, 32 rows 16.4 / 15.1, 4096 x 11008, 16 rows 11.1 / 9.7).  Further on only where this kernel's grid leaves slots idle
+//     (16400 x 4096, 3 rows 0.81 of that kernel's speed, 20000 x 2048, 16 rows 0.79, 24576 x 4096 0.95), at seven and eight super-blocks,
+//     a step of its wavefronts (64000 x 2048, 3 / 8 / 16 rows 0.93, 0.98, 1.02; 12000 x 2048, 32 rows 0.95), and of 29 to 32
+//     super-blocks, two for each of its wavefronts, where a strip a CU is all there is: 2048 x 8192, 3 / 8 / 16 rows 7.7 / 8.3, 7.8 / 8.8,
+//     7.8 / 8.2 (but 28 super-blocks level, 33 10.2 / 8.0, 5120 x 8192, 16 rows 11.2 / 10.2).  Planar quants do not go there.
 //   three and four rows, the vector kernels: small weights (1024 x 4096, Q5_K 7.2 / 7.2, Q8_0 7.3 / 7.6), and Q8_0 and Q4_0 where a
 //     workgroup's few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0; 4096 x 4096 8.4 / 7.7)
 //   the fp16 kernels, whose scales are in the operands, where a call may take them (mmq.f16_api_min_m): Q4_K and Q6_K from 33 rows
@@ -443,10 +454,16 @@ bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
 // Weights under a million values are launches and nothing else whatever the kernel.
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     const Options &o = w->dev->opt;
-    const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16;
+    const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16, nsb = w->cols >> 8;
     if (!rows_i8_takes(w, m) || values < 1 << 20) return false;
     const bool q4k = w->fmt == CANDY_HIP_Q4_K, q6k = w->fmt == CANDY_HIP_Q6_K;
-    if (q4k && w->cols <= 4096 && mmv_covers(w, m) && w->rows <= (m <= 16 ? 64 * cus : 32 * cus)) return false;
+    if (q4k && mmv_covers(w, m)) {
+        const bool eight = nsb == 7 || nsb == 8;
+        if (nsb <= 16 && w->rows <= (m <= 16 ? 64 * cus : 32 * cus)) return false;
+        if (!exact && nsb > 2 && nsb <= 16 && m <= 16 && (four_strips_idle(strips, cus) || (eight && m <= 8))) return false;
+        if (!exact && m > 16 && nsb > 4 && nsb <= 8 && w->rows <= 48 * cus) return false;
+        if (!exact && nsb > 28 && nsb <= 32 && strips <= cus) return false;
+    }
     if (m <= 4 && values <= 1 << 22) return false;
     if (m <= 4 && !q4k && !q6k && w->fmt != CANDY_HIP_Q5_K && w->cols <= 4096 && strips > 2 * cus && strips <= 4 * cus) return false;
     return exact || !mmq_f16_big_covers(w, m, o.f16_api_min_m);

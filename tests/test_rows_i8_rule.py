@@ -48,3 +48,24 @@ def test_comparison_runs_on_the_vector_kernels(fmt):
         assert prompt(fmt, 11000, 4096, m) and prompt(fmt, 11000, 4096, m, i8_min_m=2)
         for kw in (dict(i8_min_m=99), dict(small_batch_kernel=0)):
             assert not prompt(fmt, 11000, 4096, m, **kw) and not single(fmt, 11000, 4096, m, **kw)
+
+
+def test_q4_k_stays_on_its_one_pass_kernel_up_to_32_super_blocks_a_strip_a_cu():
+    for m in (3, 5, 16):
+        for rows in (1024, 2048, 4096):
+            for blocks, here in ((20, True), (28, True), (29, False), (32, False), (33, True), (43, True)):
+                assert single(synth.Q4_K, rows, 256 * blocks, m) == here, (rows, blocks, m)
+            assert single(synth.Q4_K, rows - 1, 8192, m)  # rows that kernel does not take
+        assert single(synth.Q4_K, 4112, 8192, m) and single(synth.Q5_K, 2048, 8192, m)
+    assert single(synth.Q4_K, 2048, 8192, 17) and prompt(synth.Q4_K, 2048, 8192, 16) and single(synth.Q4_K, 2048, 8192, 16, exact=1)
+
+
+def test_q4_k_stays_on_its_one_pass_kernel_where_the_grid_leaves_slots_idle():
+    for m in (3, 8, 16):
+        for rows, here in ((16384, False), (16400, False), (24576, False), (30720, True), (32000, True), (40000, False), (48000, True)):
+            for cols in (1024, 1536, 4096):
+                assert single(synth.Q4_K, rows, cols, m) == here, (rows, cols, m)
+            assert single(synth.Q4_K, rows, 4352, m) and single(synth.Q4_K, rows, 512, m) == (rows > 16384)
+            assert single(synth.Q4_K, rows, 4096, m, exact=1) == (rows > 16384)
+        assert single(synth.Q4_K, 64000, 2048, m) == (m > 8)
+    assert [single(synth.Q4_K, rows, 2048, 32) for rows in (8192, 12288, 12304, 20000)] == [False, False, True, True]
