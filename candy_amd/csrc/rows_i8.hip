@@ -447,8 +447,10 @@ static bool four_strips_idle(int64_t strips, int64_t cus) {
 //     a step of its wavefronts (64000 x 2048, 3 / 8 / 16 rows 0.93, 0.98, 1.02; 12000 x 2048, 32 rows 0.95), and of 29 to 32
 //     super-blocks, two for each of its wavefronts, where a strip a CU is all there is: 2048 x 8192, 3 / 8 / 16 rows 7.7 / 8.3, 7.8 / 8.8,
 //     7.8 / 8.2 (but 28 super-blocks level, 33 10.2 / 8.0, 5120 x 8192, 16 rows 11.2 / 10.2).  Planar quants do not go there.
-//   three and four rows, the vector kernels: small weights (1024 x 4096, Q5_K 7.2 / 7.2, Q8_0 7.3 / 7.6), and Q8_0 and Q4_0 where a
-//     workgroup's few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0; 4096 x 4096 8.4 / 7.7)
+//   three and four rows, the vector kernels: small weights (1024 x 4096, Q5_K 7.2 / 7.2, Q8_0 7.3 / 7.6), and Q8_0 and Q4_0 in two rounds
+//     of workgroups whose few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0, 8208 x 5120 0.89 of the vector kernels'
+//     speed, 8208 x 8192 1.01; 4096 x 4096 8.4 / 7.7), where four strips a workgroup leave slots idle (16400 x 4096 0.73 and 0.75, 24576 x
+//     8192 0.88 and 0.82, 32000 x 4096 1.01 and 1.05), and Q4_0, three rows of 2304 to 5120 values, in less than one round (5000 x 4096 0.88)
 //   the fp16 kernels, whose scales are in the operands, where a call may take them (mmq.f16_api_min_m): Q4_K and Q6_K from 33 rows
 //     (11008 x 4096, 48 rows 16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 / 35.8)
 // Weights under a million values are launches and nothing else whatever the kernel.
@@ -465,7 +467,11 @@ bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
         if (!exact && nsb > 28 && nsb <= 32 && strips <= cus) return false;
     }
     if (m <= 4 && values <= 1 << 22) return false;
-    if (m <= 4 && !q4k && !q6k && w->fmt != CANDY_HIP_Q5_K && w->cols <= 4096 && strips > 2 * cus && strips <= 4 * cus) return false;
+    if (m <= 4 && !q4k && !q6k && w->fmt != CANDY_HIP_Q5_K) {  // Q8_0, Q4_0
+        if (nsb <= 24 && strips > 2 * cus && strips <= 4 * cus) return false;
+        if (nsb > 5 && four_strips_idle(strips, cus)) return false;
+        if (w->fmt != CANDY_HIP_Q8_0 && m == 3 && nsb > 8 && nsb <= 20 && strips > cus && strips < 2 * cus) return false;
+    }
     return exact || !mmq_f16_big_covers(w, m, o.f16_api_min_m);
 }
 

@@ -69,3 +69,15 @@ def test_q4_k_stays_on_its_one_pass_kernel_where_the_grid_leaves_slots_idle():
             assert single(synth.Q4_K, rows, 4096, m, exact=1) == (rows > 16384)
         assert single(synth.Q4_K, 64000, 2048, m) == (m > 8)
     assert [single(synth.Q4_K, rows, 2048, 32) for rows in (8192, 12288, 12304, 20000)] == [False, False, True, True]
+
+
+@pytest.mark.parametrize("fmt", [synth.Q8_0, synth.Q4_0, synth.Q4_0_GGML])
+def test_three_and_four_rows_of_the_32_value_formats(fmt):
+    for m in (3, 4):
+        for rows, cols, here in ((8192, 6144, True), (8208, 6144, False), (16384, 6144, False), (12288, 6400, True),  # two rounds
+                                 (16400, 1536, False), (24576, 8192, False), (16400, 14336, False), (40000, 4096, False),  # idle slots
+                                 (16400, 1280, True), (30720, 4096, True), (32000, 8192, True), (48000, 4096, True)):
+            assert single(fmt, rows, cols, m) == here, (rows, cols, m)
+        assert single(fmt, 5000, 4096, m) == (fmt == synth.Q8_0 or m == 4)
+        assert single(fmt, 5000, 2048, m) and single(fmt, 5000, 5376, m)
+    assert single(fmt, 16400, 4096, 5) and single(synth.Q5_K, 16400, 4096, 3)
