@@ -63,7 +63,7 @@ struct Options {
     int f16_split = 0;           // comparison runs: workgroups that share one fp16 tile's K (0: by grid size)
     int mmv_min_m = 3;           // f32 x Q4_K with this many .. mmv_max_m rows: the one-pass int8 kernel
     int mmv_max_m = 32;          //   (0: never; more than 16 rows only for rows of up to 4096 values)
-    int rows_i8 = 1;             // 3 .. 255 rows: the kernel that deals K to wavefronts, where it is ahead (0: never; nor with mmv.max_m 0)
+    int rows_i8 = 1;             // 3 .. 255 rows: the kernel that deals K to wavefronts, where it is ahead (0: never; nor with mmv.max_m 0; 2: wherever it can)
     int mmv_variant = 0;         // comparison runs: 1 = one 16-row strip per wavefront, 2 = two
     int pair_rows = 0;           // fused gate/up: row pairs per workgroup, 32 / 16 / 8 (0: the most even split)
     int rms_rows = 0;            // fused RMSNorm prologue: rows per workgroup, 16 / 24 (0: the most even split)

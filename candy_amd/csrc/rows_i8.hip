@@ -423,13 +423,34 @@ bool rows_i8_covers(const candy_hip_qtensor *w) {
     }
 }
 
+// Super-blocks that a weight row must have for the kernel to be ahead.  With fewer than eight, wavefronts have none and only meet the
+// others at the end; past a round or two of workgroups that is most of the time.  Speed of the kernels that were there / this one:
+//   Q5_K 16000 x 256, 33 rows 0.57, 32000 x 512, 5 / 17 / 33 rows 0.81, 0.82, 0.55, 32000 x 768 1.00, 1.01, 0.69, 64000 x 1536 1.07, 1.28, 0.91
+//   Q6_K 12000 x 512, 5 / 17 rows 2.2, 0.74, 16000 x 1280 1.01, 0.81, 32000 x 1024 0.92, 0.94, 64000 x 1536 0.98, 0.96
+//   Q8_0 16000 x 256, 8 / 17 / 33 rows 1.9, 0.84, 0.62, 24000 x 512 2.4, 1.02, 0.85, 32000 x 1024 2.2, 1.61, 1.02 (Q4_0 2.7, 1.5, 0.90)
+// Up to eight rows of Q8_0 and Q4_0, and three and four rows at all, the alternative is the looping vector kernel, far behind there.
+static int64_t least_blocks(const candy_hip_qtensor *w, int64_t m) {
+    const int64_t cus = w->dev->num_cus, strips = (w->rows + 15) / 16;
+    const bool q5 = w->fmt == CANDY_HIP_Q5_K, q6 = w->fmt == CANDY_HIP_Q6_K, q8 = w->fmt == CANDY_HIP_Q8_0;
+    if (w->fmt == CANDY_HIP_Q4_K) return 1;  // its one-pass kernel is asked first
+    if (m <= 4) return !(q5 || q6) || strips <= 10 * cus ? 1 : strips <= 20 * cus ? 3 : 6;
+    if (m <= 8 && !q5 && !q6) return 1;
+    if (strips <= 2 * cus) return m > 8 ? 2 : 1;
+    if (strips <= 4 * cus) return m > 16 ? (q6 ? 7 : q5 ? 3 : 2) : m > 8 || strips > 3 * cus ? 2 : 1;
+    if (m <= 16) return q6 && strips > 7 * cus ? 6 : q5 || q6 ? 4 : 3;
+    if (m <= 32) return q6 ? 7 : q5 ? 3 : 2;
+    const bool far = strips > 7 * cus;
+    return q5 || q6 ? (far ? 7 : 4) : q8 ? (far ? 4 : 3) : far ? 6 : 4;
+}
+
 // Below 16 activation rows the length of the weight rows is limited by the vector kernels, whichever kernel is ahead: a batch that
 // one row more or less would have refused is not taken here either (matvec.hip takes it where its tiles do).
 bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m) {
     const Options &o = w->dev->opt;
     if (m < 16 && !matvec_row_fits(w->cols)) return false;
     if (m < o.i8_min_m || o.small_batch_kernel == 0) return false;  // comparison runs that ask for the vector kernels
-    return o.rows_i8 && o.mmv_max_m != 0 && !o.mmq_fp16_only && m >= 3 && m <= 255 && rows_i8_covers(w);
+    if (!o.rows_i8 || o.mmv_max_m == 0 || o.mmq_fp16_only || m < 3 || m > 255 || !rows_i8_covers(w)) return false;
+    return o.rows_i8 == 2 || (w->cols >> 8) >= least_blocks(w, m);
 }
 
 // Whether launches of four strips of weight rows per workgroup leave a tenth or more of the chip's two slots a CU idle: just past a
@@ -457,7 +478,9 @@ static bool four_strips_idle(int64_t strips, int64_t cus) {
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     const Options &o = w->dev->opt;
     const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16, nsb = w->cols >> 8;
-    if (!rows_i8_takes(w, m) || values < 1 << 20) return false;
+    if (!rows_i8_takes(w, m)) return false;
+    if (o.rows_i8 == 2) return true;
+    if (values < 1 << 20) return false;
     const bool q4k = w->fmt == CANDY_HIP_Q4_K, q6k = w->fmt == CANDY_HIP_Q6_K;
     if (q4k && mmv_covers(w, m)) {
         const bool eight = nsb == 7 || nsb == 8;

@@ -355,7 +355,7 @@ const OptionKey OPTION_KEYS[] = {
     {"mmq.f16_split", &candy::Options::f16_split, 0, 16},
     {"mmv.min_m", &candy::Options::mmv_min_m, 2, 32},
     {"mmv.max_m", &candy::Options::mmv_max_m, 0, 32},
-    {"rows.i8", &candy::Options::rows_i8, 0, 1},
+    {"rows.i8", &candy::Options::rows_i8, 0, 2},
     {"mmv.variant", &candy::Options::mmv_variant, 0, 2},
     {"fused.pair_rows", &candy::Options::pair_rows, 0, 32},
     {"fused.rms_rows", &candy::Options::rms_rows, 0, 24},

@@ -109,7 +109,7 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *   "mmv.min_m"                  3        candy_hip_qmatmul on Q4_K: batches of this many .. "mmv.max_m" rows take the
  *   "mmv.max_m"                  32         one-pass int8 matrix-core kernel (max 0: never)
  *   "rows.i8"                    1        3 .. 255 activation rows: the exact kernel that deals K to wavefronts, where it is ahead (0:
- *                                         never; with mmv.max_m 0 neither)
+ *                                         never; with mmv.max_m 0 neither; 2: wherever it can, also past the thresholds above)
  *   "mmv.variant"                0        that kernel with one (1) or two (2) 16-row strips per wavefront (0: by shape)
  *   "fused.pair_rows"            0        fused gate/up: row pairs per workgroup 32 / 16 / 8 (0: most even split)
  *   "fused.rms_rows"             0        fused RMSNorm prologue: rows per workgroup 16 / 24 (0: most even split)

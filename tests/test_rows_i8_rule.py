@@ -81,3 +81,25 @@ def test_three_and_four_rows_of_the_32_value_formats(fmt):
         assert single(fmt, 5000, 4096, m) == (fmt == synth.Q8_0 or m == 4)
         assert single(fmt, 5000, 2048, m) and single(fmt, 5000, 5376, m)
     assert single(fmt, 16400, 4096, 5) and single(synth.Q5_K, 16400, 4096, 3)
+
+
+# weight rows x values, activation rows: (with one super-block less, with this many)
+LEAST = [(synth.Q5_K, 16000, 33, 3), (synth.Q5_K, 32000, 5, 4), (synth.Q5_K, 32000, 33, 7), (synth.Q5_K, 12000, 17, 3), (synth.Q5_K, 8192, 17, 2),
+         (synth.Q6_K, 12000, 17, 7), (synth.Q6_K, 20000, 8, 4), (synth.Q6_K, 32000, 8, 6), (synth.Q6_K, 64000, 17, 7), (synth.Q6_K, 64000, 3, 3), (synth.Q6_K, 128000, 4, 6),
+         (synth.Q8_0, 8192, 9, 2), (synth.Q8_0, 16000, 17, 2), (synth.Q8_0, 24000, 9, 3), (synth.Q8_0, 24000, 33, 3), (synth.Q4_0, 24000, 33, 4),
+         (synth.Q8_0, 32000, 33, 4), (synth.Q4_0, 32000, 33, 6), (synth.Q5_K, 24000, 33, 4)]
+
+
+@pytest.mark.parametrize("fmt,rows,m,least", LEAST)
+def test_rows_of_few_super_blocks(fmt, rows, m, least):
+    assert not single(fmt, rows, 256 * (least - 1), m, exact=1) and not prompt(fmt, rows, 256 * (least - 1), m)
+    assert single(fmt, rows, 256 * least, m, exact=1) and prompt(fmt, rows, 256 * least, m)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_eight_super_blocks_are_enough_and_few_rows_have_no_better_kernel(fmt):
+    for rows in (4096, 12000, 64000):
+        for m in (3, 5, 12, 20, 60):
+            assert prompt(fmt, rows, 2048, m)
+    if fmt in (synth.Q8_0, synth.Q4_0, synth.Q4_0_GGML):
+        assert single(fmt, 32000, 256, 8) and single(fmt, 32000, 256, 3)
