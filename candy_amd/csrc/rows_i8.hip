@@ -460,6 +460,22 @@ static bool four_strips_idle(int64_t strips, int64_t cus) {
     return strips > 4 * cus && strips <= 10 * cus && 10 * wgs < 9 * slots * ((wgs + slots - 1) / slots);
 }
 
+// Quants that are planar already (candy_hip_qmatmul_qact) take a launch more here, which orders them, and none on the vector kernels and
+// the tiles.  Speed of those / this one, 3 / 5 rows where there are two: Q8_0 4096 x 4096 0.70, 1.04, 2048 x 4096 0.58, 0.91, Q5_K 11008 x 4096
+// 0.85, 1.50, 4096 x 8192 1.27, 1.29, 24576 x 2048 1.26, Q6_K 4096 x 4096 0.94, 1.21, 16384 x 2048 0.95, 0.98, 11008 x 4096 1.10, Q4_K 4096 x 11008 0.90, 1.45, 4096 x
+// 14336 1.38, 1.35, 24576 x 2048 1.37; 10 rows of 1024 x 2048 0.84 (launches only), of 24576 x 1024, short rows, 0.82 to 0.87.
+static bool planar_behind(const candy_hip_qtensor *w, int64_t m) {
+    const int64_t values = w->rows * w->cols, cols = w->cols, cus = w->dev->num_cus;
+    const bool q4k = w->fmt == CANDY_HIP_Q4_K, q6k = w->fmt == CANDY_HIP_Q6_K, k_quant = q4k || q6k || w->fmt == CANDY_HIP_Q5_K;
+    if (m <= 4) {
+        if (!k_quant || (values < 1 << 24 && cols <= 12288)) return true;
+        return q6k ? values < 40000000 && cols <= 4096 : values < 100000000 && w->rows < 20000 && cols <= (q4k ? 12288 : 5632);
+    }
+    if (m <= 16 && k_quant && cols < 2048 && w->rows > (q6k ? 32 : q4k && m <= 8 ? 120 : 48) * cus) return true;
+    if (m <= 8) return !k_quant && values <= 1 << 23 && cols <= 4096 && w->rows <= 4096;
+    return m <= 16 && values <= 1 << 22 && cols <= 2560;
+}
+
 // Where the other kernels are ahead or level, us of a call, there / here:
 //   Q4_K up to 16 (8192 or fewer weight rows: 32) activation rows of 4096 or fewer values, the one-shot kernel of mmv_i8.hip:
 //     4096 x 4096, 16 rows 7.1 / 7.2, 14336 x 4096 11.2 / 12.1, 8192 x 2048, 32 rows 7.7 / 8.0 (but 32000 x 4096 19.6 / 17.8, 14336 x
@@ -489,6 +505,7 @@ bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
         if (!exact && m > 16 && nsb > 4 && nsb <= 8 && w->rows <= 48 * cus) return false;
         if (!exact && nsb > 28 && nsb <= 32 && strips <= cus) return false;
     }
+    if (exact && planar_behind(w, m)) return false;
     if (m <= 4 && values <= 1 << 22) return false;
     if (m <= 4 && !q4k && !q6k && w->fmt != CANDY_HIP_Q5_K) {  // Q8_0, Q4_0
         if (nsb <= 24 && strips > 2 * cus && strips <= 4 * cus) return false;

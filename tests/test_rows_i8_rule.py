@@ -66,7 +66,7 @@ def test_q4_k_stays_on_its_one_pass_kernel_where_the_grid_leaves_slots_idle():
             for cols in (1024, 1536, 4096):
                 assert single(synth.Q4_K, rows, cols, m) == here, (rows, cols, m)
             assert single(synth.Q4_K, rows, 4352, m) and single(synth.Q4_K, rows, 512, m) == (rows > 16384)
-            assert single(synth.Q4_K, rows, 4096, m, exact=1) == (rows > 16384)
+            assert single(synth.Q4_K, rows, 4096, m, exact=1) == (rows > (16384 if m > 4 else 20000))
         assert single(synth.Q4_K, 64000, 2048, m) == (m > 8)
     assert [single(synth.Q4_K, rows, 2048, 32) for rows in (8192, 12288, 12304, 20000)] == [False, False, True, True]
 
@@ -93,7 +93,7 @@ LEAST = [(synth.Q5_K, 16000, 33, 3), (synth.Q5_K, 32000, 5, 4), (synth.Q5_K, 320
 @pytest.mark.parametrize("fmt,rows,m,least", LEAST)
 def test_rows_of_few_super_blocks(fmt, rows, m, least):
     assert not single(fmt, rows, 256 * (least - 1), m, exact=1) and not prompt(fmt, rows, 256 * (least - 1), m)
-    assert single(fmt, rows, 256 * least, m, exact=1) and prompt(fmt, rows, 256 * least, m)
+    assert prompt(fmt, rows, 256 * least, m) and single(fmt, rows, 256 * least, m, f16_api_min_m=99)
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
@@ -103,3 +103,19 @@ def test_eight_super_blocks_are_enough_and_few_rows_have_no_better_kernel(fmt):
             assert prompt(fmt, rows, 2048, m)
     if fmt in (synth.Q8_0, synth.Q4_0, synth.Q4_0_GGML):
         assert single(fmt, 32000, 256, 8) and single(fmt, 32000, 256, 3)
+
+
+# format, weight rows, values, activation rows: planar quants there, f32 and Q8_0 blocks elsewhere or not
+PLANAR = [(synth.Q8_0, 4112, 14336, 3, False), (synth.Q4_0, 4112, 14336, 4, False), (synth.Q8_0, 2048, 4096, 8, False),
+          (synth.Q8_0, 4112, 4096, 5, True), (synth.Q8_0, 1024, 8192, 5, True), (synth.Q5_K, 11008, 4096, 3, False),
+          (synth.Q5_K, 11008, 4096, 5, True), (synth.Q5_K, 4096, 8192, 3, True), (synth.Q5_K, 1024, 8192, 3, False),
+          (synth.Q5_K, 24576, 2048, 3, True), (synth.Q6_K, 4096, 4096, 4, False), (synth.Q6_K, 16384, 2048, 4, False),
+          (synth.Q6_K, 11008, 4096, 4, True),
+          (synth.Q4_K, 4096, 11008, 3, False), (synth.Q4_K, 4096, 11008, 5, True), (synth.Q4_K, 4096, 14336, 3, True),
+          (synth.Q6_K, 11008, 1024, 10, False), (synth.Q5_K, 24576, 1024, 10, False), (synth.Q5_K, 11008, 1024, 10, True),
+          (synth.Q5_K, 1024, 2048, 10, False), (synth.Q5_K, 1024, 4096, 10, True)]
+
+
+@pytest.mark.parametrize("fmt,rows,cols,m,here", PLANAR)
+def test_planar_quants_where_a_launch_more_pays(fmt, rows, cols, m, here):
+    assert single(fmt, rows, cols, m) and single(fmt, rows, cols, m, exact=1) == here
