@@ -119,3 +119,17 @@ PLANAR = [(synth.Q8_0, 4112, 14336, 3, False), (synth.Q4_0, 4112, 14336, 4, Fals
 @pytest.mark.parametrize("fmt,rows,cols,m,here", PLANAR)
 def test_planar_quants_where_a_launch_more_pays(fmt, rows, cols, m, here):
     assert single(fmt, rows, cols, m) and single(fmt, rows, cols, m, exact=1) == here
+
+
+def test_q6_k_tiles_of_more_than_48_rows():
+    def shape(rows, m):
+        return divmod(LIB.candy_test_rows_q6k_shape(ctypes.c_int64(rows), ctypes.c_int64(m), 256), 100)
+
+    for rows in (16, 1000, 1024, 1536, 2048, 2560, 3072, 5000, 14336, 128256):
+        for m in range(49, 256):
+            rf, mt = shape(rows, m)
+            tiles = -(-m // (16 * mt)) * mt
+            assert (rf, mt) in ((2, 4), (1, 4), (1, 3), (1, 2), (1, 1)) and tiles <= (m + 63) // 64 * 4  # the image's tiles
+    # a grid that two strips and four tiles would leave half empty takes smaller ones; a full one does not
+    assert shape(2048, 100) == (1, 4) and shape(1536, 80) == (1, 1) and shape(3072, 192) == (1, 3)
+    assert shape(14336, 255) == (2, 4) and shape(8192, 128) == (2, 4)
