@@ -834,11 +834,16 @@ static void launch_big(const MmPlan &p, dim3 g, hipStream_t stream, Args... args
 
 // Where the narrow tiles are at most two workgroups per CU: past that the activations they read again cost more than the shorter
 // walk saves (us as above, large tiles / narrow ones: 6144 x 4096, 200 rows 38.1 / 46.3, 11008 x 4096, 100 rows 36.3 / 45.4; at 512
-// workgroups, 8192 x 2048, 100 rows 22.5 / 20.8).
+// workgroups, 8192 x 2048, 100 rows 22.5 / 20.8).  Where two a CU are nearly all there, a second column of tiles that is not even half full
+// is too dear: 8192 x 8192, 65 / 96 / 97 rows 53.5 / 62.0, 55.0 / 59.5, 62.0 / 59.3, 8192 x 4096 30.9 / 31.9, 32.2 / 32.6, 36.0 / 32.7 (but 7168 x 8192,
+// 65 rows 53.3 / 53.7, 6144 x 4096 30.6 / 26.3, and short K, 8192 x 1536 16.9 / 16.4).
+static bool narrow_pays(int num_cus, int64_t m, int64_t rows, int64_t ld) {
+    const int64_t m_tiles = m <= 32 ? 1 : (m + 63) / 64, tiles = m_tiles * (rows / NARROW_BN);
+    return tiles <= 2 * (int64_t)num_cus && (4 * tiles <= 7 * (int64_t)num_cus || m <= 64 || ld < 2048 || m % 64 == 0 || m % 64 > 32);
+}
 static bool narrow_covers(int num_cus, const DenseLaunch &L) {
     if (L.f32 || L.partial || L.block_rows || L.group || !to_act(L.epi)) return false;
-    const int64_t m_tiles = L.m <= 32 ? 1 : (L.m + 63) / 64, tiles = m_tiles * (L.w->rows_pad / NARROW_BN);
-    return tiles <= 2 * (int64_t)num_cus && tile_fits(NARROW_BN, L.w->ld) && tile_fits(64, L.ldx);
+    return narrow_pays(num_cus, L.m, L.w->rows_pad, L.w->ld) && tile_fits(NARROW_BN, L.w->ld) && tile_fits(64, L.ldx);
 }
 static int launch_narrow(candy_hip_device *dev, const DenseLaunch &L) {
     const int K = (int)L.w->ld, rows = (int)L.w->rows_pad, bm = L.m <= 32 ? 32 : 64, m_tiles = (L.m + bm - 1) / bm;
@@ -1144,6 +1149,7 @@ void candy_test_dense_plan(int num_cus, int m, int64_t rows, int64_t ld, int64_t
     const candy::MmPlan p = candy::mm_plan(num_cus, m, rows, ld, ldx, partial != 0, steady != 0, few != 0, block_rows);
     plan[0] = p.big; plan[1] = p.bn; plan[2] = p.bm; plan[3] = p.splits;
 }
+int candy_test_narrow_pays(int num_cus, int64_t m, int64_t rows, int64_t ld) { return candy::narrow_pays(num_cus, m, rows, ld); }
 int candy_test_grouped_tile_rows(int experts, int64_t slots, int64_t widest) { return candy::grouped_tile_rows(experts, slots, widest); }
 int candy_test_grouped_weight_rows(int num_cus, int experts, int64_t slots, int expert_rows) {
     return candy::grouped_weight_rows(num_cus, experts, slots, expert_rows);

@@ -87,3 +87,14 @@ def test_tiles_of_rows_dealt_to_experts(experts, rows, d, ff, tile, wide):
     assert LIB.candy_test_grouped_tile_rows(experts, experts * rows, max(d, ff)) == tile
     if wide:
         assert LIB.candy_test_grouped_weight_rows(256, experts, experts * rows, ff) == wide
+
+
+def test_narrow_tiles_where_their_last_column_is_half_full():
+    def pays(m, rows, ld):
+        return bool(LIB.candy_test_narrow_pays(256, *(ctypes.c_int64(v) for v in (m, rows, ld))))
+
+    for m in (2, 32, 33, 64):
+        assert pays(m, 8192, 8192) and pays(m, 16384, 8192) and not pays(m, 16448, 8192)
+    assert [m for m in range(65, 129) if pays(m, 8192, 8192)] == list(range(97, 129))  # two columns: 512 workgroups
+    assert all(pays(m, 8192, 1536) for m in range(65, 129)) and all(pays(m, 7168, 8192) for m in range(65, 129))
+    assert not any(pays(m, 8256, 1536) for m in range(65, 129))
