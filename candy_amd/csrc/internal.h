@@ -115,6 +115,7 @@ struct candy_hip_device {
     candy::SplitPending *defer_split = nullptr;
     // This GPU's copy of the library's file-scope scratch array (matvec.hip), resolved when the handle is opened.
     void *noalloc_scratch = nullptr;
+    int fail_alloc = 0;  // tests: the allocation that many requests from now is refused (0: none)
 };
 
 struct candy_hip_qtensor {
@@ -158,6 +159,7 @@ int use_device(const candy_hip_device *dev);
 // out-of-range index (the word is cleared), CANDY_HIP_OK otherwise.
 int check_fault(candy_hip_device *dev);
 // Returns a workspace of at least `bytes` bytes (256-byte aligned).
+int device_malloc(candy_hip_device *dev, void **p, size_t bytes);
 int workspace(candy_hip_device *dev, size_t bytes, void **out);
 // Second buffer, for the split-K partial sums (lives beside the activation workspace).
 int splitk_workspace(candy_hip_device *dev, size_t bytes, void **out);

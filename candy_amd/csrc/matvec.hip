@@ -867,10 +867,15 @@ int launch_contract(candy_hip_device *dev, const candy_hip_qtensor *w, const int
                     int64_t m, float *y, const _Float16 *xh_ready, const float *res) {
     if (!xh_ready && !mmq_f16_big_covers(w, m) && rows_i8_picks(w, m, true)) {
         ActWorkspace a;
-        if (int rc = act_workspace(dev, m, w->cols, false, &a)) return rc;
-        const RowsLaunch L = rows_launch(w, m, y, res, a.rows_ws);
-        if (int rc = launch_rows_pack_planar(dev, qs, scales, m, w->cols, L.x)) return rc;
-        return launch_rows_i8(dev, L, m);
+        const int rc = act_workspace(dev, m, w->cols, false, &a);
+        if (!rc) {
+            const RowsLaunch L = rows_launch(w, m, y, res, a.rows_ws);
+            if (int e = launch_rows_pack_planar(dev, qs, scales, m, w->cols, L.x)) return e;
+            return launch_rows_i8(dev, L, m);
+        }
+        // fewer than 16 rows need no memory in the kernels below: none for the image is no reason to refuse them
+        if (rc != CANDY_HIP_ERR_OOM || m >= mmq_min_m(dev)) return rc;
+        (void)hipGetLastError();
     }
     if (m < mmq_min_m(dev)) {
         CANDY_REQUIRE(res != y, "internal: in-place residual needs the fused epilogue");

@@ -63,6 +63,12 @@ int check_fault(candy_hip_device *dev) {
     return CANDY_HIP_OK;
 }
 
+int device_malloc(candy_hip_device *dev, void **p, size_t bytes) {
+    if (dev->fail_alloc && --dev->fail_alloc == 0) return fail(CANDY_HIP_ERR_OOM, "%zu bytes refused (asked for by a test)", bytes);
+    CANDY_HIP_TRY(hipMalloc(p, bytes));
+    return CANDY_HIP_OK;
+}
+
 int workspace(candy_hip_device *dev, size_t bytes, void **out) {
     if (bytes > dev->ws_bytes) {
         // Work already enqueued may still read the old buffer.
@@ -71,7 +77,7 @@ int workspace(candy_hip_device *dev, size_t bytes, void **out) {
         dev->ws = nullptr;
         dev->ws_bytes = 0;
         size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-        CANDY_HIP_TRY(hipMalloc(&dev->ws, want));
+        if (int rc = device_malloc(dev, &dev->ws, want)) return rc;
         dev->ws_bytes = want;
     }
     *out = dev->ws;
@@ -85,7 +91,7 @@ int splitk_workspace(candy_hip_device *dev, size_t bytes, void **out) {
         dev->ws_split = nullptr;
         dev->ws_split_bytes = 0;
         size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-        CANDY_HIP_TRY(hipMalloc(&dev->ws_split, want));
+        if (int rc = device_malloc(dev, &dev->ws_split, want)) return rc;
         dev->ws_split_bytes = want;
     }
     *out = dev->ws_split;
@@ -205,9 +211,11 @@ int candy_hip_alloc(candy_hip_device *dev, size_t bytes, void **dptr) {
     *dptr = nullptr;
     if (int rc = use_device(dev)) return rc;
     if (bytes == 0) bytes = 1;  // a zero-length storage still gets a distinct address
-    CANDY_HIP_TRY(hipMalloc(dptr, bytes));
-    return CANDY_HIP_OK;
+    return device_malloc(dev, dptr, bytes);
 }
+
+// What a call does when there is no memory, for tests: the nth request from now is refused.
+void candy_test_fail_alloc(candy_hip_device *dev, int nth) { dev->fail_alloc = nth; }
 
 int candy_hip_free(candy_hip_device *dev, void *dptr) {
     if (!dptr) return CANDY_HIP_OK;
