@@ -343,7 +343,13 @@ int candy_hip_llama::reserve_prompt(int n) {
     if (!rc) rc = prompt_alloc(m, &P.xq, N * widest);
     if (!rc) rc = prompt_alloc(m, &P.xs, N * (widest / 32));
     if (!rc) rc = prompt_alloc(m, &P.xh, (size_t)mmq_m_pad(n) * widest);  // the tile kernel reads whole tiles of rows
-    if (!rc) rc = prompt_alloc(m, &P.image, rows_image_bytes(std::min(n, 255), (int64_t)widest));
+    if (!rc && (rc = prompt_alloc(m, &P.image, rows_image_bytes(std::min(n, 255), (int64_t)widest)))) {
+        // no memory for it is no reason to refuse the prompt: the int8 tiles read planar quants
+        if (rc != CANDY_HIP_ERR_OOM) return rc;
+        (void)hipGetLastError();
+        P.image = nullptr;
+        rc = CANDY_HIP_OK;
+    }
     return rc;
 }
 
@@ -399,7 +405,7 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
         void *kc = cache.k_of(l), *vc = cache.v_of(l);
         // Every projection on the exact kernel for 3 to 255 rows: the launches in front write its operands, q / k / v and gate / up
         // are a grid each, residuals ride in the epilogue, nothing is split: ten launches (24 tokens of the 1B shape: 22 before).
-        bool exact_rows = pend.n_split == 0;
+        bool exact_rows = P.image && pend.n_split == 0;
         for (const candy_hip_qtensor *w : {L.wq, L.wk, L.wv, L.wo, L.gate, L.up, L.down})
             exact_rows = exact_rows && !mmq_f16_big_covers(w, n) && rows_i8_takes(w, n);
         if (exact_rows) {
