@@ -322,7 +322,7 @@ struct ActWorkspace {
     void *mmv_ws = nullptr;  // operand-order activations for the small-batch int8 kernel (2 .. 32 rows)
     void *rows_ws = nullptr; // the same for the kernel that deals K to wavefronts (3 .. 255 rows)
 };
-int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quants, ActWorkspace *out);
+int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quants, ActWorkspace *out, bool rows = false);
 // matvec.hip: y[m, rows] = x . W^T for any m from planar activations that live OUTSIDE the device
 // workspace (the tile kernel may carve its fp16 scratch from it).
 int mmq_min_m(const candy_hip_device *dev);

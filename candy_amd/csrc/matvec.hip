@@ -767,12 +767,12 @@ int launch_matvec_multi(candy_hip_device *dev, const candy_hip_qtensor *const *w
     return CANDY_HIP_OK;
 }
 
-int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quants, ActWorkspace *out) {
+int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quants, ActWorkspace *out, bool rows) {
     const size_t q_bytes = need_quants ? (((size_t)(m * cols) + 255) & ~(size_t)255) : 0;
     const size_t s_bytes = need_quants ? (((size_t)(m * (cols >> 5)) * sizeof(Q8Scale) + 255) & ~(size_t)255) : 0;
     const size_t h_bytes = m >= 16 ? (size_t)(mmq_m_pad(m) * cols) * 2 : 0;
     const size_t v_bytes = need_quants && m >= 2 && m <= 32 && cols % 256 == 0 ? mmv_workspace_bytes(cols) : 0;
-    const size_t r_bytes = m >= 3 && m <= 255 && cols % 256 == 0 ? (rows_image_bytes(m, cols) + 255) & ~(size_t)255 : 0;
+    const size_t r_bytes = rows && m >= 3 && m <= 255 && cols % 256 == 0 ? (rows_image_bytes(m, cols) + 255) & ~(size_t)255 : 0;
     void *ws = nullptr;
     if (int rc = workspace(dev, q_bytes + s_bytes + h_bytes + r_bytes + v_bytes + 256, &ws)) return rc;
     out->qs = (int8_t *)ws;
@@ -857,21 +857,27 @@ int noalloc_scratch_init(candy_hip_device *dev) {
 
 int mmq_min_m(const candy_hip_device *dev) { return dev->opt.mmq_min_m < 16 ? 16 : dev->opt.mmq_min_m; }
 
-static RowsLaunch rows_launch(const candy_hip_qtensor *w, int64_t m, float *y, const float *res, void *ws) {
+static RowsLaunch rows_launch(const candy_hip_qtensor *w, float *y, const float *res, const RowsImage &x) {
     RowsLaunch L;
-    L.n = 1; L.w[0] = w; L.y[0] = y; L.res[0] = res; L.x = rows_image(ws, m, w->cols);
+    L.n = 1; L.w[0] = w; L.y[0] = y; L.res[0] = res; L.x = x;
     return L;
+}
+// The image of m rows as all that the workspace holds: a call that goes to the row kernel needs nothing else of it.
+static int rows_workspace(candy_hip_device *dev, int64_t m, int64_t cols, RowsImage *out) {
+    void *ws = nullptr;
+    if (int rc = workspace(dev, rows_image_bytes(m, cols), &ws)) return rc;
+    *out = rows_image(ws, m, cols);
+    return CANDY_HIP_OK;
 }
 
 int launch_contract(candy_hip_device *dev, const candy_hip_qtensor *w, const int8_t *qs, const Q8Scale *scales,
                     int64_t m, float *y, const _Float16 *xh_ready, const float *res) {
     if (!xh_ready && !mmq_f16_big_covers(w, m) && rows_i8_picks(w, m, true)) {
-        ActWorkspace a;
-        const int rc = act_workspace(dev, m, w->cols, false, &a);
+        RowsImage x;
+        const int rc = rows_workspace(dev, m, w->cols, &x);
         if (!rc) {
-            const RowsLaunch L = rows_launch(w, m, y, res, a.rows_ws);
-            if (int e = launch_rows_pack_planar(dev, qs, scales, m, w->cols, L.x)) return e;
-            return launch_rows_i8(dev, L, m);
+            if (int e = launch_rows_pack_planar(dev, qs, scales, m, w->cols, x)) return e;
+            return launch_rows_i8(dev, rows_launch(w, y, res, x), m);
         }
         // fewer than 16 rows need no memory in the kernels below: none for the image is no reason to refuse them
         if (rc != CANDY_HIP_ERR_OOM || m >= mmq_min_m(dev)) return rc;
@@ -902,10 +908,10 @@ static int qmatmul_check(candy_hip_device *dev, const candy_hip_qtensor *w, int6
 }
 
 static int contract(candy_hip_device *dev, const candy_hip_qtensor *w, const ActWorkspace &a, int64_t m, float *y) {
-    if (a.rows_ws && rows_i8_picks(w, m, false)) {
-        const RowsLaunch L = rows_launch(w, m, y, nullptr, a.rows_ws);
-        if (int rc = launch_rows_pack_planar(dev, a.qs, a.scales, m, w->cols, L.x)) return rc;
-        return launch_rows_i8(dev, L, m);
+    if (a.rows_ws && rows_i8_picks(w, m, false)) {  // the sweep only: calls do not come here with what goes to the row kernel
+        const RowsImage x = rows_image(a.rows_ws, m, w->cols);
+        if (int rc = launch_rows_pack_planar(dev, a.qs, a.scales, m, w->cols, x)) return rc;
+        return launch_rows_i8(dev, rows_launch(w, y, nullptr, x), m);
     }
     return m < mmq_min_m(dev) ? launch_matvec(dev, w, a.qs, a.scales, m, y)
                                : launch_mmq(dev, w, a.qs, a.scales, m, y, a.half_ws, nullptr, nullptr, dev->opt.f16_api_min_m);
@@ -922,9 +928,9 @@ static int qmatmul_f32(candy_hip_device *dev, const candy_hip_qtensor *w, const 
         if (rc != CANDY_HIP_ERR_UNSUPPORTED) return rc;
     }
     if (a.rows_ws && rows_i8_picks(w, m, false)) {
-        const RowsLaunch L = rows_launch(w, m, dev_y, nullptr, a.rows_ws);
-        if (int rc = launch_rows_quantize(dev, dev_x, m, w->cols, L.x)) return rc;
-        return launch_rows_i8(dev, L, m);
+        const RowsImage x = rows_image(a.rows_ws, m, w->cols);
+        if (int rc = launch_rows_quantize(dev, dev_x, m, w->cols, x)) return rc;
+        return launch_rows_i8(dev, rows_launch(w, dev_y, nullptr, x), m);
     }
     if (a.mmv_ws && mmv_covers(w, m) && !matvec_even_covers(w, m)) return launch_mmv(dev, w, dev_x, nullptr, m, dev_y, a.mmv_ws);
     if (a.half_ws && m >= mmq_min_m(dev) && !dev->opt.mmq_fp16_only && mmq_f16_big_covers(w, m, dev->opt.f16_api_min_m)) {
@@ -943,6 +949,12 @@ int candy_hip_qmatmul(candy_hip_device *dev, const candy_hip_qtensor *w, const f
     CANDY_REQUIRE(dev_x, "lhs is nil");
     CANDY_REQUIRE(((uintptr_t)dev_x & 15) == 0, "lhs must be 16-byte aligned");
     if (int rc = use_device(dev)) return rc;
+    if (rows_i8_picks(w, m, false)) {
+        RowsImage x;
+        if (int rc = rows_workspace(dev, m, w->cols, &x)) return rc;
+        if (int rc = launch_rows_quantize(dev, dev_x, m, w->cols, x)) return rc;
+        return launch_rows_i8(dev, rows_launch(w, dev_y, nullptr, x), m);
+    }
     ActWorkspace a;
     if (int rc = act_workspace(dev, m, w->cols, true, &a)) return rc;
     return qmatmul_f32(dev, w, dev_x, m, dev_y, a);
@@ -975,13 +987,14 @@ int candy_hip_qmatmul_q8(candy_hip_device *dev, const candy_hip_qtensor *w, cons
     CANDY_REQUIRE(dev_x_q8_0, "lhs is nil");
     CANDY_REQUIRE(((uintptr_t)dev_x_q8_0 & 1) == 0, "lhs blocks must be 2-byte aligned");
     if (int rc = use_device(dev)) return rc;
+    if (rows_i8_picks(w, m, false)) {
+        RowsImage x;
+        if (int rc = rows_workspace(dev, m, w->cols, &x)) return rc;
+        if (int rc = launch_rows_pack_blocks(dev, dev_x_q8_0, m, w->cols, x)) return rc;
+        return launch_rows_i8(dev, rows_launch(w, dev_y, nullptr, x), m);
+    }
     ActWorkspace a;
     if (int rc = act_workspace(dev, m, w->cols, true, &a)) return rc;
-    if (a.rows_ws && rows_i8_picks(w, m, false)) {
-        const RowsLaunch L = rows_launch(w, m, dev_y, nullptr, a.rows_ws);
-        if (int rc = launch_rows_pack_blocks(dev, dev_x_q8_0, m, w->cols, L.x)) return rc;
-        return launch_rows_i8(dev, L, m);
-    }
     if (a.mmv_ws && mmv_covers(w, m) && !matvec_even_covers(w, m)) return launch_mmv(dev, w, nullptr, dev_x_q8_0, m, dev_y, a.mmv_ws);
     if (int rc = launch_q8_blocks_to_planar(dev, dev_x_q8_0, m * (w->cols >> 5), a.qs, a.scales)) return rc;
     return contract(dev, w, a, m, dev_y);
@@ -1055,7 +1068,7 @@ int candy_hip_qmatmul_sweep(candy_hip_device *dev, const candy_hip_qtensor *cons
     if (int rc = use_device(dev)) return rc;
     const int64_t K = ws[0]->cols;
     ActWorkspace a;
-    if (int rc = act_workspace(dev, m, K, true, &a)) return rc;
+    if (int rc = act_workspace(dev, m, K, true, &a, true)) return rc;
     if (int rc = launch_quantize_q8(dev, dev_x, m, K, a.qs, a.scales, nullptr)) return rc;
     CANDY_HIP_TRY(hipEventRecord(dev->ev_start, dev->stream));
     for (int i = 0; i < iters; ++i) {

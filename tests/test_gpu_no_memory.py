@@ -88,3 +88,12 @@ def test_prompt_without_memory_for_its_operands(dev):
     answered = [nth for nth, g in enumerate(got) if g and not same(g, exact)]
     assert len(answered) == 1 and same(got[answered[0]], tiles)
     assert got[0] is None and same(got[-1], exact)
+
+
+@pytest.mark.parametrize("fmt,rows,m,mib", [(synth.Q4_1, 64, 100, 5), (synth.Q4_K, 512, 8, 1), (synth.Q8_0, 4096, 40, 1)])
+def test_the_workspace_holds_what_the_call_uses(dev, fmt, rows, m, mib):
+    """Quants, their fp16 image and operands only where the kernel that runs reads them (8192 values a row, in whole MiB)."""
+    cols = 8192
+    w = dev.qtensor(fmt, rows, cols, synth.random_weight(fmt, rows, cols, seed=fmt))
+    dev.qmatmul(w, synth.random_activations(m, cols, seed=m))
+    assert dev.get_option("runtime.workspace_bytes") == mib << 20
