@@ -240,4 +240,17 @@ int candy_hip_add_rms_norm(candy_hip_device *dev, float *x, const float *y, cons
     return norm_op(dev, x, y, w, nullptr, eps, mult, nullptr, rows, cols, x, true);
 }
 
+// The chain with everything that a decoder gives it, for its tests.  p: x, y, slots, slot_weight, post_w, post_b, step, x_out, pre_w,
+// pre_b, out, row_ids; n: ldx, y's row stride, copies and their stride, slot_ld, top, ldo, f32, rms, rows, cols.
+int candy_test_norm_chain(candy_hip_device *dev, void *const *p, const int64_t *n, float mult, float eps) {
+    NormArgs A;
+    A.x = (const float *)p[0]; A.y.p = (float *)p[1]; A.slots = (const float *)p[2]; A.slot_weight = (const float *)p[3];
+    A.post_w = (const float *)p[4]; A.post_b = (const float *)p[5]; A.step = (const float *)p[6]; A.x_out = (float *)p[7];
+    A.pre_w = (const float *)p[8]; A.pre_b = (const float *)p[9]; A.out = p[10]; A.row_ids = (const int *)p[11];
+    A.ldx = n[0]; A.y.ld = (int)n[1]; A.y.copies = (int)n[2]; A.y.stride = (size_t)n[3]; A.slot_ld = n[4]; A.top = (int)n[5]; A.ldo = n[6];
+    A.f32 = n[7] != 0; A.rms = n[8] != 0; A.rows = (int)n[9]; A.cols = (int)n[10]; A.mult = mult; A.eps = eps;
+    if (int rc = use_device(dev)) return rc;
+    return launch_norm_chain(dev, A);
+}
+
 }  // extern "C"

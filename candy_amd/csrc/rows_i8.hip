@@ -597,3 +597,29 @@ extern "C" int candy_test_rows_q6k_shape(int64_t weight_rows, int64_t m, int num
     candy::rows_q6k_shape((weight_rows + 15) / 16, m, num_cus, &rf, &mt);
     return rf * 100 + mt;
 }
+
+// Weights that share a launch, with residuals, for their tests: f32 rows x against n of them.
+extern "C" int candy_test_rows_launch(candy_hip_device *dev, int n, const candy_hip_qtensor *const *ws, float *const *ys,
+                                      const float *const *res, const float *x, int64_t m) {
+    void *ws_p = nullptr;
+    if (int rc = candy::use_device(dev)) return rc;
+    if (int rc = candy::workspace(dev, candy::rows_image_bytes(m, ws[0]->cols), &ws_p)) return rc;
+    candy::RowsLaunch L;
+    L.n = n;
+    L.x = candy::rows_image(ws_p, m, ws[0]->cols);
+    for (int i = 0; i < n; ++i) { L.w[i] = ws[i]; L.y[i] = ys[i]; L.res[i] = res[i]; }
+    if (int rc = candy::launch_rows_quantize(dev, x, m, ws[0]->cols, L.x)) return rc;
+    return candy::launch_rows_i8(dev, L, m);
+}
+
+// The image as the norm (b: its weights) or the SiLU launch (b: up) writes it, and the planar quants of the same launch.
+extern "C" int candy_test_rows_image(candy_hip_device *dev, int silu, const float *a, const float *b, int64_t m, int64_t cols, void *image,
+                                     int8_t *qs, candy::Q8Scale *scales) {
+    if (int rc = candy::use_device(dev)) return rc;
+    const candy::RowsImage x = candy::rows_image(image, m, cols);
+    for (const candy::RowsImage *to : {&x, (const candy::RowsImage *)nullptr})
+        if (int rc = silu ? candy::launch_silu_mul_quant(dev, a, b, m, cols, nullptr, to ? nullptr : qs, to ? nullptr : scales, nullptr, to)
+                          : candy::launch_rms_norm_quant(dev, a, b, 1e-5f, m, cols, nullptr, to ? nullptr : qs, to ? nullptr : scales, nullptr, to))
+            return rc;
+    return CANDY_HIP_OK;
+}

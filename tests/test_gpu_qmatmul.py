@@ -103,11 +103,17 @@ def test_two_rows_even_split_kernel(dev, rows, cols):
     assert rel_err(got[:, sub], o.qmatmul(synth.Q4_K, wsub, len(sub), cols, x)) <= 2e-5
 
 
+def without_row_kernel(request, dev):
+    dev.set_option("rows.i8", 0)
+    request.addfinalizer(lambda: dev.set_option("rows.i8", 1))
+
+
 @pytest.mark.parametrize("fmt", [synth.Q8_0, synth.Q4_0, synth.Q5_1])
-def test_five_to_eight_rows_on_a_big_weight_take_the_tile_kernel(dev, fmt):
-    # 32-value formats, weights of 40 M values and more: 5 .. 8 rows run on the int8 tile kernel (integer-exact, like
-    # the vector kernels they replace there: the two differ by f32 summation order only)
+def test_five_to_eight_rows_on_a_big_weight_take_the_tile_kernel(request, dev, fmt):
+    # 32-value formats, weights of 40 M values and more, without the row kernel (which has no Q5_1): 5 .. 8 rows run on the
+    # int8 tile kernel (integer-exact, like the vector kernels they replace there: the two differ by f32 summation order only)
     rows, cols = 4096, 11008
+    without_row_kernel(request, dev)
     w = synth.random_weight(fmt, rows, cols, seed=fmt + 50)
     q = dev.qtensor(fmt, rows, cols, w)
     sub = np.arange(3, rows, 61)
@@ -126,9 +132,10 @@ def test_five_to_eight_rows_on_a_big_weight_take_the_tile_kernel(dev, fmt):
 
 
 @pytest.mark.parametrize("fmt", [synth.Q6_K, synth.Q5_K])
-def test_three_and_four_rows_on_long_weight_rows_take_the_tile_kernel(dev, fmt):
+def test_three_and_four_rows_on_long_weight_rows_take_the_tile_kernel(request, dev, fmt):
     # Q6_K / Q5_K with weight rows so long that the looping kernel holds one or two activation rows per launch:
-    # 3 and 4 rows run as one 16-row int8 tile; on 4096-long weight rows the vector kernel keeps them
+    # 3 and 4 rows run as one 16-row int8 tile; on 4096-long weight rows the vector kernel keeps them (without the row kernel)
+    without_row_kernel(request, dev)
     for rows, cols, tiles in ((4096, 14336, True), (1024, 4096, False)):
         w = synth.random_weight(fmt, rows, cols, seed=fmt + 70)
         q = dev.qtensor(fmt, rows, cols, w)
