@@ -204,9 +204,8 @@ int candy_hip_quantize(candy_hip_device *dev, int fmt, const float *dev_x, int64
 /* y[m, rows] = x[m, cols] . W^T, activations quantized to Q8_0 on the device first.
  * m < 16 runs the bandwidth-bound matvec family (QCU:2787-2871 mul_mat_vec_q and its entry
  * points :2874, :2906, :2930, :2946); m >= 16 the MFMA tile kernel (QCU:455-578 mul_mat_q).
- * Q4_K with 3 <= m <= 16, rows % 16 == 0 and cols <= 12288 (m <= 32 for cols <= 4096): one pass over
- * the weights with the batch on the 16-wide side of the int8 matrix instruction (same integer dots,
- * same scales).
+ * 3 <= m <= 255 of Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0, and 3 <= m <= 32 of Q4_K, take kernels with the batch on the 16-wide side of
+ * the int8 matrix instruction where those are ahead ("rows.i8", "mmv.max_m"): same integer dots, same scales.
  * y is row-major [m, rows] (candy's result layout, tensor/ops.go:1264). */
 int candy_hip_qmatmul(candy_hip_device *dev, const candy_hip_qtensor *w, const float *dev_x,
                       int64_t m, float *dev_y);
@@ -220,8 +219,8 @@ int candy_hip_dmmv(candy_hip_device *dev, const candy_hip_qtensor *w, const floa
 
 /* candy_hip_qmatmul for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): no counterpart in the reference.  Same result as candy_hip_qmatmul,
- * 1 <= m <= 15 activation rows (the matvec family; the vector kernels answer every batch, so from 5 rows on the
- * bits may differ from candy_hip_qmatmul's tile kernel by f32 summation order).  The quantized activations live
+ * 1 <= m <= 15 activation rows (the matvec family; the vector kernels answer every batch, so from 3 rows on the
+ * bits may differ from those of candy_hip_qmatmul's matrix-core kernels by f32 summation order).  The quantized activations live
  * in a 1 MiB array inside the library that every call on a GPU shares: a call whose m * cols * 1.25 bytes (plus
  * rounding to 256) exceed it fails with CANDY_HIP_ERR_INVALID, and calls that overlap on one GPU (two handles,
  * two threads) race on it.  Calls no hipMalloc / hipFree. */

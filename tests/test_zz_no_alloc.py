@@ -53,6 +53,18 @@ def test_two_calls_in_a_row_second_smaller(dev, fmt):
             assert err <= 2e-6, (fmt, m, err)  # the bar is 1e-3; two evaluations of the same exact dots stay far inside it
 
 
+@pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q5_K, synth.Q8_0, synth.Q6_K, synth.Q4_0])
+def test_up_to_four_rows_of_a_big_weight(dev, fmt):
+    # 4.5 M values and rows that are whole strips of 16: candy_hip_qmatmul has other kernels from three rows on (the int8 matrix cores),
+    # the same exact dots in another order of f32 sums
+    rows, cols = 1040, 4352
+    w = dev.qtensor(fmt, rows, cols, synth.random_weight(fmt, rows, cols, seed=903 + fmt))
+    for m in (1, 2, 3, 4):
+        ref, got = both(dev, w, synth.random_activations(m, cols, seed=m))
+        err = float(np.max(np.abs(got.astype(np.float64) - ref)) / np.max(np.abs(ref)))
+        assert err == 0 if m <= 2 else err <= 2e-6, (m, err)
+
+
 @pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q8_0, synth.Q6_K, synth.Q4_0])
 def test_against_the_cpu_oracle_on_a_handle_that_never_allocated(fmt):
     # A fresh device handle whose FIRST contraction is the allocation-free one: the handle's grow-only workspaces
