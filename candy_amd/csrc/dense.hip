@@ -526,11 +526,11 @@ __global__ __launch_bounds__(512, 2) void k_dense_big(const bf16 *__restrict__ W
 // 16.9; 6144 x 4096, 40 / 100 rows 39.0 / 35.4 -> 20.8 / 26.9; 14336 x 4096, 16 / 64 rows 40.3 / 44.5 -> 31.0 / 35.6.
 constexpr int NARROW_BN = 32;
 template <int EPI, int BM>
-__global__ __launch_bounds__(256, 2) void k_dense_narrow(const bf16 *__restrict__ W, const bf16 *__restrict__ X, void *__restrict__ yv, int M,
+__global__ __launch_bounds__(256, 2) void k_dense_narrow(const bf16 *__restrict__ W, const bf16 *__restrict__ X, bf16 *__restrict__ y, int M,
                                                          int Np, int ld, int ldx, int64_t ldy, int n_store, int m_tiles, const EpiArgs ea) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
     constexpr int BN = NARROW_BN, BK = 64, ROWS = BN + BM, PIECES = ROWS / 8, LOADS = PIECES / 4, STAGES = 6, TM = BM / 32;
-    static_assert(PIECES % 4 == 0, "every wavefront has as many loads");
+    static_assert(PIECES % 4 == 0 && to_act(EPI), "every wavefront has as many loads; results are activations");
     __shared__ __align__(16) u32x4v s[STAGES * ROWS * 8];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -594,14 +594,7 @@ __global__ __launch_bounds__(256, 2) void k_dense_narrow(const bf16 *__restrict_
         f32x4 z = acc[j];
 #pragma unroll
         for (int e = 0; e < 4; ++e) z[e] = epilogue<EPI>(z[e], ea);
-        if (to_act(EPI)) {
-            if (n < n_store) *(bf16x4 *)((bf16 *)yv + (size_t)m * ldy + n) = __builtin_convertvector(z, bf16x4);
-        } else {
-            float *y = (float *)yv + (size_t)m * ldy + n;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < n_store) y[e] = z[e];
-        }
+        if (n < n_store) *(bf16x4 *)(y + (size_t)m * ldy + n) = __builtin_convertvector(z, bf16x4);
     }
 #endif
 }
@@ -851,7 +844,7 @@ static int launch_narrow(candy_hip_device *dev, const DenseLaunch &L) {
     const EpiArgs ea{L.scale, L.cap};
     const bf16 *W = (const bf16 *)L.w->data, *X = (const bf16 *)L.x;
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, g, b, 0, dev->stream, W, X, L.y, L.m, rows, K, (int)L.ldx, L.ldy, (int)L.n_store, m_tiles, ea);
+        hipLaunchKernelGGL(kern, g, b, 0, dev->stream, W, X, (bf16 *)L.y, L.m, rows, K, (int)L.ldx, L.ldy, (int)L.n_store, m_tiles, ea);
     };
     if (L.epi == EPI_RELU2) bm == 32 ? launch(k_dense_narrow<EPI_RELU2, 32>) : launch(k_dense_narrow<EPI_RELU2, 64>);
     else bm == 32 ? launch(k_dense_narrow<EPI_ACT, 32>) : launch(k_dense_narrow<EPI_ACT, 64>);

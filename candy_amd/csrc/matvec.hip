@@ -786,6 +786,7 @@ int act_workspace(candy_hip_device *dev, int64_t m, int64_t cols, bool need_quan
 int launch_matvec(candy_hip_device *dev, const candy_hip_qtensor *w, const int8_t *qs, const Q8Scale *scales,
                   int64_t m, float *y, bool vector_only) {
     CANDY_REQUIRE(w->rows <= 0x7FFFFFFF && w->cols <= 0x7FFFFFFF, "matrix too large");
+    // (From three rows on Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 come here with what the row kernel leaves: rows_i8_picks.)
     // the 32-value formats: the vector kernels match the tile kernel up to 8 rows (one pass) on small weights; from 9
     // rows on they need two passes, and on weights of 40 M values and more the tile kernel is level or ahead from 5 rows
     // (us per call, 5-8 rows on the vector kernels / 9 rows on the tiles: Q8_0 32000 x 4096 50.5-51.4 / 46.3, 4096 x 11008

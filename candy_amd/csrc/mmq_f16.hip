@@ -758,7 +758,8 @@ static int launch_jobs(candy_hip_device *dev, const F16Job *jobs, int count, con
     }
 }
 
-// xh: fp16 activations [mmq_m_pad(m)][K], rows past m zero.
+// xh: fp16 activations [mmq_m_pad(m)][K]; rows past m may hold anything (EPI_SILU leaves what was there): a row reaches its own
+// results only.
 int launch_mmq_f16_big(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y,
                        const float *res) {
     if (mmq_f16_rows_covers(w, m) && dev->opt.f16_shape == 0 && dev->opt.f16_split == 0) return launch_mmq_f16_rows(dev, w, xh, m, y, res);

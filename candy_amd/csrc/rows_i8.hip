@@ -317,7 +317,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
                             const int4v d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, rows_b(x.q[mt], t), int4v{0, 0, 0, 0}, 0, 0, 0);
                             const float dx = rows_d(x.d[mt], t);
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) acc[r][mt][i] += (f[i] * dx) * (float)d[i];  // fp16 scales: their product is exact
+                            for (int i = 0; i < 4; ++i) acc[r][mt][i] += (f[i] * dx) * (float)d[i];  // Q8_0, Q4_0: f * dx is exact
                         }
                     }
                 }
@@ -491,6 +491,9 @@ static bool planar_behind(const candy_hip_qtensor *w, int64_t m) {
 //   the fp16 kernels, whose scales are in the operands, where a call may take them (mmq.f16_api_min_m): Q4_K and Q6_K from 33 rows
 //     (11008 x 4096, 48 rows 16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 / 35.8)
 // Weights under a million values are launches and nothing else whatever the kernel.
+// Not left to a faster kernel: Q8_0 and Q4_0 whose results come to four million and more (planar quants and prompts of up to 255 rows, single
+// calls of up to 64 against 44000 weight rows), which the fp16 tiles of mmq.hip took before (32000 x 4096, 200 rows 119 us there, 176 here; 100
+// rows 109 and 105).  Below the fp16 thresholds every product is exact, and this is the fastest kernel that is.
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     const Options &o = w->dev->opt;
     const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16, nsb = w->cols >> 8;
