@@ -113,7 +113,8 @@ PLANAR = [(synth.Q8_0, 4112, 14336, 3, False), (synth.Q4_0, 4112, 14336, 4, Fals
           (synth.Q6_K, 11008, 4096, 4, True),
           (synth.Q4_K, 4096, 11008, 3, False), (synth.Q4_K, 4096, 11008, 5, True), (synth.Q4_K, 4096, 14336, 3, True),
           (synth.Q6_K, 11008, 1024, 10, False), (synth.Q5_K, 24576, 1024, 10, False), (synth.Q5_K, 11008, 1024, 10, True),
-          (synth.Q5_K, 1024, 2048, 10, False), (synth.Q5_K, 1024, 4096, 10, True)]
+          (synth.Q5_K, 1024, 2048, 10, False), (synth.Q5_K, 1024, 4096, 10, True), (synth.Q5_K, 2048, 4096, 5, False),
+          (synth.Q5_K, 1024, 5120, 5, True), (synth.Q5_K, 4112, 1024, 5, True)]
 
 
 @pytest.mark.parametrize("fmt,rows,cols,m,here", PLANAR)
