@@ -66,7 +66,8 @@ struct RowsLaunch {
 };
 bool rows_i8_covers(const candy_hip_qtensor *w);  // whether the kernel takes the weight
 bool rows_i8_takes(const candy_hip_qtensor *w, int64_t m);  // the same with the batch and the options
-// whether a single contraction of m rows goes there; exact: the alternatives are the exact kernels only (fp16 operands otherwise)
+// whether a single contraction of m rows goes there; exact: its quants are planar already and the alternatives are the exact kernels only
+// (else f32 rows or Q8_0 blocks, and kernels with fp16 operands as well)
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact);
 int launch_rows_i8(candy_hip_device *dev, const RowsLaunch &L, int64_t m);
 // f32 rows, Q8_0 blocks or planar quants -> the image

@@ -461,9 +461,10 @@ static bool four_strips_idle(int64_t strips, int64_t cus) {
 }
 
 // Quants that are planar already (candy_hip_qmatmul_qact) take a launch more here, which orders them, and none on the vector kernels and
-// the tiles.  Speed of those / this one, 3 / 5 rows where there are two: Q8_0 4096 x 4096 0.70, 1.04, 2048 x 4096 0.58, 0.91, Q5_K 11008 x 4096
-// 0.85, 1.50, 4096 x 8192 1.27, 1.29, 24576 x 2048 1.26, 2048 x 4096, 5 rows 0.91, Q6_K 4096 x 4096 0.94, 1.21, 16384 x 2048 0.95, 0.98, 11008 x 4096 1.10, Q4_K 4096 x 11008 0.90, 1.45, 4096 x
-// 14336 1.38, 1.35, 24576 x 2048 1.37; 10 rows of 1024 x 2048 0.84 (launches only), of 24576 x 1024, short rows, 0.82 to 0.87.
+// the tiles.  Speed of those / this one, 3 / 5 rows where there are two: Q8_0 4096 x 4096 0.70, 1.04, 2048 x 4096 0.58, 0.91; Q5_K 11008 x
+// 4096 0.85, 1.50, 4096 x 8192 1.27, 1.29, 24576 x 2048 1.26, 2048 x 4096, 5 rows 0.91; Q6_K 4096 x 4096 0.94, 1.21, 16384 x 2048 0.95, 0.98,
+// 11008 x 4096 1.10; Q4_K 4096 x 11008 0.90, 1.45, 4096 x 14336 1.38, 1.35, 24576 x 2048 1.37; 10 rows of 1024 x 2048 0.84 (launches only), of
+// 24576 x 1024, short rows, 0.82 to 0.87.
 static bool planar_behind(const candy_hip_qtensor *w, int64_t m) {
     const int64_t values = w->rows * w->cols, cols = w->cols, cus = w->dev->num_cus;
     const bool q4k = w->fmt == CANDY_HIP_Q4_K, q6k = w->fmt == CANDY_HIP_Q6_K, k_quant = q4k || q6k || w->fmt == CANDY_HIP_Q5_K;
