@@ -9,8 +9,15 @@
 // matrix operands in registers, activation fragments straight from their image, each loaded by one wavefront of the
 // workgroup.  The wavefronts' sums meet in LDS at the end, in the order of the wavefronts (reproducible).  Kernel us, 77
 // rows, 11008 x 4096, before (with the split sum) -> now: Q4_K 22.8 + 4.5 -> 20.6, Q8_0 35.1 + 4.5 -> 24.0, Q4_0 33.4 + 4.5 ->
-// 21.2, Q5_K 31.5 + 4.5 -> 25.1; 2048 x 1024 Q8_0 13.0 + 4.1 -> 5.7.  What bounds it: the activations, which every CU reads
-// (655 KB here, 10 us), then the weights (48 MB of Q8_0, 8 us), half overlapped.
+// 21.2, Q5_K 31.5 + 4.5 -> 25.1; 2048 x 1024 Q8_0 13.0 + 4.1 -> 5.7.
+// A step's second half of activations is requested in front of its dequantization, and held there: left alone the compiler
+// dequantizes several steps in advance and requests the activations behind that, where nothing hides them.  A wavefront's loads are
+// the same in number at every step, with weights to fetch or not (request()).  us of a call, without / with both: 11008 x 4096, 77
+// rows Q8_0 24.9 / 22.7, Q4_0 21.9 / 19.7, Q5_K 25.1 / 21.9, Q4_K 20.2 / 17.7; 3000 x 2560 Q5_K 14.9 / 10.9; 8192 x 2048, 100 rows
+// Q4_K 16.3 / 13.4, Q6_K 19.9 / 18.6 (4096 x 4096, 77 rows Q4_K 14.0 / 14.2).  Fences behind the first half's loads too, or the loads
+// three halves ahead: 3 and 7 % slower.  What bounds it: without any weights or activations fetched the Q8_0 call takes 17.6 (a
+// launch of the quantizer 2.5, dequantization and products of two wavefronts a SIMD, the sums), the activations, which every CU
+// reads (655 KB), add 2 to 3, the weights (48 MB of Q8_0) the rest.
 #include <algorithm>
 #include <type_traits>
 
@@ -31,6 +38,7 @@ constexpr size_t lds_bytes() {
 template <class F, int RF, int MF>
 __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restrict__ W, const _Float16 *__restrict__ xh, float *y,
                                                          const float *res, int M, int N, int K) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
     constexpr bool STAGED = staged<F>();
     extern __shared__ __align__(16) uint8_t smem_raw[];
     float4v *sums = (float4v *)smem_raw;  // [wave][RF][MF][lane]
@@ -61,11 +69,15 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
         }
     }
     const uint8_t *w0 = W + (size_t)n0 * rb;
-    auto request = [&](int sb) __attribute__((always_inline)) {
+    // any false: the same loads from a matrix of no bytes, so that as many are in flight at every step: behind a branch around them
+    // the compiler waits for the activations by the smaller count, which is a wait for the weights too
+    auto request = [&](int sb, bool any) __attribute__((always_inline)) {
+        const int at = any ? sb * F::BLOCK : 0;  // (a scalar offset past an empty matrix would count as inside)
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)w0, 0, any ? (int)(RF * 16 * rb) : 0, 0x00027000);
 #pragma unroll
         for (int it = 0; it < IT; ++it)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(w0 + (size_t)sb * F::BLOCK + from[it]),
-                                             (__attribute__((address_space(3))) void *)(slice + it * 64), 16, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(slice + it * 64), 16, from[it],
+                                                     at, 0, 0);
     };
     if (count > 0) {
         // Unstaged blocks are requested a super-block ahead, but three fragments of them twice over do not fit the registers: 41
@@ -89,6 +101,7 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 load_x(sb * 4 + g, 1);
+                __builtin_amdgcn_sched_barrier(0);  // and the loads are out
                 half8 a[RF][2];
 #pragma unroll
                 for (int i = 0; i < RF; ++i) {
@@ -107,14 +120,14 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
             }
         };
         if constexpr (STAGED) {
-            request(first);
+            request(first, true);
             load_x(first * 4, 0);
             for (int k = 0; k < count; ++k) {
                 const int sb = first + 8 * k;
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the slice has landed
                 load_w(sb, 0);
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and is in registers
-                if (k + 1 < count) request(sb + 8);
+                request(sb + 8, k + 1 < count);
                 contract(sb, 0, k + 1 < count ? sb + 8 : sb);
             }
         } else if constexpr (DEEP == 1) {
@@ -163,6 +176,7 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
                 if (n + j < N) dst[j] = r ? r[j] + s[j] : s[j];
         }
     }
+#endif
 }
 
 static int fragments(int64_t m) { return m <= 48 ? 3 : m <= 64 ? 4 : m <= 80 ? 5 : m <= 96 ? 6 : 8; }
