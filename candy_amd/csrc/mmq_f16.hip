@@ -282,6 +282,17 @@ __device__ __forceinline__ float silu_once(float x) {
     const float den = 1.0f + expf(-x), r = __builtin_amdgcn_rcpf(den), q = x * r;
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-den, q, x), r, q), den, x);
 }
+// STAGED: a producer's blocks come into a slice of LDS of its own, 16-byte pieces in the order they lie in memory, and from there
+// to its lanes.  For Q8_0, whose lanes would ask for eight runs of 16 bytes and eight scales 34 bytes apart in every super-block:
+// that many lines per load bound the tiles, not the dequantization.  us of a call, loads of single lanes / staged: 11008 x 4096, 140
+// rows 44.3 / 39.7, 1400 rows 200.8 / 177.6; 4096 x 14336, 1400 rows 227 / 211; 4096 x 4096, 400 rows 37.7 / 35.6.  The other formats'
+// blocks are fewer loads, and a slice is a wait for LDS once a super-block: Q4_0 level, Q5_K and Q4_K 3 to 5 % slower, Q6_K (14
+// pieces from the one its even address lies in) 7 to 13 %.
+template <class F>
+constexpr bool f16_staged() { return std::is_same<F, BigQ8_0>::value; }
+template <class F>
+constexpr int f16_slice_loads() { return (32 * F::BLOCK / 16 + 63) / 64; }  // of 1 KB, for a producer's 32 rows
+
 template <class F, int BN, int BM, int EPI>
 __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _Float16 *__restrict__ xh, int M, int K,
                                                     int n_tiles, int m_tiles, int sb_per, size_t split_stride) {
@@ -323,8 +334,10 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
 
     if (wave < 4) {
         // ---------------- producers: the weight tile of step t + LEAD (buffer (t + LEAD) % NB) while step t is contracted
-        typename F::Raw raw[2][ATK];
-        typename F16Pre<F>::type pre[2][ATK];
+        constexpr bool STAGED = f16_staged<F>();
+        constexpr int SLOTS = STAGED ? 1 : 2;
+        typename F::Raw raw[SLOTS][ATK];
+        typename F16Pre<F>::type pre[SLOTS][ATK];
         // neighbouring lanes take neighbouring quarters of a row; a half-wavefront takes rows {x, x+4, x+8, x+12}
         const int a_c = lane & 3, a_row = 16 * wave + 4 * ((lane >> 2) & 3) + (lane >> 4);   // + a_step i
         const int a_step = BN == 112 && wave == 3 ? 0 : 64;
@@ -350,24 +363,83 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
                 *(half8 *)&a[frag_off(a_row + a_step * i, k1)] = o1;
             }
         };
-        gload_a(0, 0);
-        gload_a(min(1, n_sb - 1), 1);
-        stage(0, 0, 0);
-        if (LEAD == 2) stage(1, 0, 1);
-        __syncthreads();
-        // Iteration t = 8 j + u stages step t + LEAD (past the end: a clamped super-block, into a buffer nobody
-        // reads): super-blocks alternate between the two raw slots, so u fixes group and slot of the staged step.
-        int buf = LEAD % NB;
-        for (int t8 = 0; t8 < steps; t8 += 8) {
+        if constexpr (STAGED) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+            constexpr int P = F::BLOCK / 16, IT = f16_slice_loads<F>();
+            static_assert(F::BLOCK % 16 == 0, "whole pieces");
+            uint8_t *const slice = smem_raw + 3 * BNB * BIG_BK * 2 + wave * (IT * 1024);
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)n0 * rb), 0, -1, 0x00027000);
+            const int row0 = EPI == EPI_SILU ? 16 * wave & 31 : 16 * wave;
+            uint32_t from[IT];  // of a lane's piece, from the tile's first row and super-block
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int t = t8 + u;
-                if ((u & 3) == 0 && t >= steps) break;  // steps is a multiple of 4
-                const int g = (u + LEAD) & 3, slot = ((u + LEAD) >> 2) & 1;
-                stage(g, slot, NB == 2 ? ((u + LEAD) & 1) : buf);  // two buffers: a constant of the unrolled body
-                buf = buf == NB - 1 ? 0 : buf + 1;
-                if (g == 3) gload_a(min(((t + LEAD) >> 2) + 2, n_sb - 1), slot);
-                __syncthreads();
+            for (int it = 0; it < IT; ++it) {
+                const int e = min(it * 64 + lane, 32 * P - 1), r = e / P;  // lanes past the last piece fetch it once more
+                from[it] = (uint32_t)(min(n0 + row0 + (r & 15) + (r >> 4) * w_step, N - 1) - n0) * (uint32_t)rb + (uint32_t)(e - r * P) * 16;
+            }
+            auto request = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+                for (int it = 0; it < IT; ++it)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(slice + it * 1024), 16, from[it],
+                                                             sb * F::BLOCK, 0, 0);
+            };
+            auto take = [&]() __attribute__((always_inline)) {
+                __builtin_amdgcn_s_waitcnt(0x0070);  // the slice has landed
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int i = 0; i < ATK; ++i) F::load(slice + ((a_row & 15) + 16 * i) * F::BLOCK, a_c, raw[0][i]);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(0x0070);  // and is in registers
+            };
+            auto meet = [&]() __attribute__((always_inline)) {  // __syncthreads() without a wait for the slice
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            };
+            request(0);
+            take();
+            request(min(1, n_sb - 1));
+            stage(0, 0, 0);
+            if (LEAD == 2) stage(1, 0, 1);
+            meet();
+            int buf = LEAD % NB;
+            for (int t4 = 0; t4 < steps; t4 += 4) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int g = (u + LEAD) & 3, sb = (t4 + u + LEAD) >> 2;
+                    if (g == 0) {
+                        take();
+                        request(min(sb + 1, n_sb - 1));
+                    }
+                    stage(g, 0, NB == 2 ? ((u + LEAD) & 1) : buf);
+                    buf = buf == NB - 1 ? 0 : buf + 1;
+                    meet();
+                }
+            }
+            __builtin_amdgcn_s_waitcnt(0x0070);  // the last request writes LDS that is still this workgroup's
+#endif
+            return;
+        }
+        if constexpr (!STAGED) {
+            gload_a(0, 0);
+            gload_a(min(1, n_sb - 1), 1);
+            stage(0, 0, 0);
+            if (LEAD == 2) stage(1, 0, 1);
+            __syncthreads();
+            // Iteration t = 8 j + u stages step t + LEAD (past the end: a clamped super-block, into a buffer nobody
+            // reads): super-blocks alternate between the two raw slots, so u fixes group and slot of the staged step.
+            int buf = LEAD % NB;
+            for (int t8 = 0; t8 < steps; t8 += 8) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int t = t8 + u;
+                    if ((u & 3) == 0 && t >= steps) break;  // steps is a multiple of 4
+                    const int g = (u + LEAD) & 3, slot = ((u + LEAD) >> 2) & 1;
+                    stage(g, slot, NB == 2 ? ((u + LEAD) & 1) : buf);  // two buffers: a constant of the unrolled body
+                    buf = buf == NB - 1 ? 0 : buf + 1;
+                    if (g == 3) gload_a(min(((t + LEAD) >> 2) + 2, n_sb - 1), slot);
+                    __syncthreads();
+                }
             }
         }
         return;
@@ -591,6 +663,10 @@ static int plan_split(const candy_hip_device *dev, int tiles, int n_sb) {
     return n_split;
 }
 
+// LDS of the role-split kernel: weight tiles, and the producers' slices
+template <class F>
+constexpr size_t pc_lds() { return (size_t)3 * 128 * BIG_BK * sizeof(_Float16) + (f16_staged<F>() ? (size_t)4 * 1024 * f16_slice_loads<F>() : 0); }
+
 template <class F, int BN, int BM, int WN, int WM, bool PC = false>
 static int launch_big(candy_hip_device *dev, const F16Job *jobs, int count, const _Float16 *xh, int64_t m) {
     static_assert(!PC || ((BN == 128 || BN == 112) && (BM == 256 || BM == 192 || BM == 128) && WN * WM == 8), "the role-split kernel's tiles");
@@ -625,7 +701,7 @@ static int launch_big(candy_hip_device *dev, const F16Job *jobs, int count, cons
             off += (size_t)m * (size_t)jobs[s].w->rows;
         }
     }
-    constexpr size_t smem = (size_t)(PC ? 3 * 128 : 2 * (BN + BM)) * BIG_BK * sizeof(_Float16);  // role-split: weight tiles only
+    constexpr size_t smem = PC ? pc_lds<F>() : (size_t)2 * (BN + BM) * BIG_BK * sizeof(_Float16);
     const bool epi_res = any_res && n_split == 1;
     void (*kern)(const F16Group, const _Float16 *, int, int, int, int, int, size_t);
     if constexpr (PC) kern = epi_res ? k_mmq_f16_pc<F, BN, BM, EPI_RES> : k_mmq_f16_pc<F, BN, BM, EPI_PLAIN>;
@@ -678,8 +754,8 @@ bool mmq_f16_big_covers(const candy_hip_qtensor *w, int64_t m, int min_m) {
     if (min_m <= 0) min_m = w->dev->opt.f16_big_min_m;
     else if (w->fmt != CANDY_HIP_Q4_K && w->fmt != CANDY_HIP_Q6_K) min_m = std::max(min_m, 65);
     if (m < min_m || w->cols % 256 != 0) return false;
-    if (w->fmt == CANDY_HIP_Q4_K || w->fmt == CANDY_HIP_Q5_K) return ((uintptr_t)w->data & 15) == 0;
-    if (w->fmt == CANDY_HIP_Q6_K || w->fmt == CANDY_HIP_Q8_0 || w->fmt == CANDY_HIP_Q4_0 || w->fmt == CANDY_HIP_Q4_0_GGML)
+    if (w->fmt == CANDY_HIP_Q4_K || w->fmt == CANDY_HIP_Q5_K || w->fmt == CANDY_HIP_Q8_0) return ((uintptr_t)w->data & 15) == 0;
+    if (w->fmt == CANDY_HIP_Q6_K || w->fmt == CANDY_HIP_Q4_0 || w->fmt == CANDY_HIP_Q4_0_GGML)
         return ((uintptr_t)w->data & 1) == 0;
     return false;
 }
@@ -819,7 +895,7 @@ static int launch_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, con
     grp.act = act;
     grp.seg[0] = F16Seg{(const uint8_t *)gate->data, nullptr, nullptr, N, 0};
     grp.seg[1] = F16Seg{(const uint8_t *)up->data, nullptr, nullptr, N, 0};
-    constexpr size_t smem = (size_t)3 * 128 * BIG_BK * sizeof(_Float16);
+    constexpr size_t smem = pc_lds<F>();
     void (*kern)(const F16Group, const _Float16 *, int, int, int, int, int, size_t) = k_mmq_f16_pc<F, 128, BM, EPI_SILU>;
     CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3((unsigned)(n_tiles * m_tiles)), dim3(512), smem, dev->stream, grp, xh, (int)m, K, n_tiles, m_tiles,
