@@ -165,6 +165,23 @@ __device__ __forceinline__ int q8_level(float x, float d) {
     return (int)roundf(t);
 }
 
+// The levels of eight values of a block at once, 0 where the block is empty: q8_level() for each, whose question whether the
+// product decides (by 6.1e-5 away from a half, and a number) is asked once for all of them.
+__device__ __forceinline__ void q8_levels8(const float (&x)[8], float amax, float d, float (&level)[8]) {
+    const float inv = __builtin_amdgcn_rcpf(d);
+    bool unsure = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float t = x[e] * inv;
+        level[e] = rintf(t);
+        unsure |= !(fabsf(t - level[e]) < 0.5f - 6.1e-5f);
+    }
+    if (__builtin_expect(unsure, 0)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) level[e] = (float)(amax != 0.0f ? q8_level(x[e], d) : 0);
+    }
+}
+
 // Q8_0 quantization of 4 consecutive values held by one lane; the 8 lanes that share a 32-value
 // block must be consecutive lanes of one wavefront (lane % 8 == position in the block) and all
 // active.  quantize_q8_1 (quantized.cu:3521-3558) without its `sum`: amax over the block,

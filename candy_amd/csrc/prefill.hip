@@ -331,7 +331,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
     constexpr int ARR = R * C, STEP = 2 * KVP * ARR;  // 16-byte pieces of one part of K or V, and of everything a step stages
     constexpr int IT = ARR / THREADS;
     static_assert(ARR % THREADS == 0 && (HD == 64 || HD == 128), "whole pieces per thread");
-    constexpr int MERGE = KG == 1 ? 0 : (4 + 2 * 4 * DT) * 16 * QH;  // the second key group's state at the end
+    constexpr int MERGE = KG == 1 ? 0 : (2 + 4 * DT) * 32 * QH;  // half of either key group's state at the end
     __shared__ __align__(16) uint4 s_all[2 * STEP > MERGE ? 2 * STEP : MERGE];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -495,56 +495,69 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) l_run[t] = quad16_sum(l_run[t]);
-    if constexpr (KG == 2) {  // value k of thread t of the second group at k * 64 QH + t
+    // The two key groups share the end as well: group 0 takes the first 16 queries of each 32, group 1 the others; what the other
+    // group needs goes through LDS, value k of thread t of group kg at (2 k + kg) * 64 QH + t.  With one group merging, dividing
+    // and quantizing both halves, level by level, what is not the walk along the keys was 17 of 31 us at 512 tokens.  Kernel us, so / now:
+    // head_dim 128, 512 tokens 31.5 / 27.4, fp16 cache 24.8 / 19.9, 2000 tokens 129 / 119; head_dim 64, 1500 tokens 78 / 73.
+    constexpr int NT = KG == 2 ? 1 : 2;  // 16 queries each
+    const int t_own = KG == 2 ? kg : 0;
+    if constexpr (KG == 2) {
+        constexpr int GROUP = 64 * QH;
         float *st = (float *)s_all;
-        const int at = tid & (64 * QH - 1);
-        __syncthreads();
-        if (kg == 1) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                st[t * 64 * QH + at] = m_run[t];
-                st[(2 + t) * 64 * QH + at] = l_run[t];
-#pragma unroll
-                for (int d = 0; d < DT; ++d)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) st[(4 + (t * DT + d) * 4 + j) * 64 * QH + at] = o[t][d][j];
-            }
-        }
-        __syncthreads();
-        if (kg == 1) return;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const float m1 = st[t * 64 * QH + at], l1 = st[(2 + t) * 64 * QH + at];
-            const float m = fmaxf(m_run[t], m1);  // finite: position 0 is in the first group
-            const float f0 = __builtin_amdgcn_exp2f(m_run[t] - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
-            l_run[t] = l_run[t] * f0 + l1 * f1;
+        const int at = tid & (GROUP - 1);
+        auto give = [&](int t) __attribute__((always_inline)) {
+            float *to = st + kg * GROUP + at;
+            to[0] = m_run[t];
+            to[2 * GROUP] = l_run[t];
 #pragma unroll
             for (int d = 0; d < DT; ++d)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) o[t][d][j] = o[t][d][j] * f0 + st[(4 + (t * DT + d) * 4 + j) * 64 * QH + at] * f1;
-        }
+                for (int j = 0; j < 4; ++j) to[(4 + 8 * d + 2 * j) * GROUP] = o[t][d][j];
+        };
+        auto merge = [&](int t) __attribute__((always_inline)) {
+            const float *from = st + (1 - kg) * GROUP + at;
+            const float m_its = from[0], l_its = from[2 * GROUP];
+            const float m = fmaxf(m_run[t], m_its);  // finite: position 0 is in the first group
+            const float f_own = __builtin_amdgcn_exp2f(m_run[t] - m), f_its = __builtin_amdgcn_exp2f(m_its - m);
+            // the sums in the order of the groups
+            const float f0 = t == 0 ? f_own : f_its, f1 = t == 0 ? f_its : f_own;
+            l_run[0] = __builtin_fmaf(t == 0 ? l_run[t] : l_its, f0, (t == 0 ? l_its : l_run[t]) * f1);
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float its = from[(4 + 8 * d + 2 * j) * GROUP], own = o[t][d][j];
+                    o[0][d][j] = __builtin_fmaf(t == 0 ? own : its, f0, (t == 0 ? its : own) * f1);
+                }
+        };
+        __syncthreads();
+        if (kg == 0) give(1);
+        else give(0);
+        __syncthreads();
+        if (kg == 0) merge(0);
+        else merge(1);
     }
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < NT; ++t) {
         const float inv = 1.0f / l_run[t];
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[t][d] *= inv;
     }
     if constexpr (HD == 64) {
-        unsigned long long lost[2];  // the 16 queries each whose results are no numbers
+        unsigned long long lost[2] = {0, 0};  // the 16 queries each whose results are no numbers
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < NT; ++t) {
             float all = 0.0f;
 #pragma unroll
             for (int d = 0; d < DT; ++d) all += (o[t][d][0] + o[t][d][1]) + (o[t][d][2] + o[t][d][3]);
-            lost[t] = __ballot(all != all && i0 + 32 * qh + 16 * t + r16 < n);
+            lost[t] = __ballot(all != all && i0 + 32 * qh + 16 * (t + t_own) + r16 < n);
         }
         if (__builtin_expect((lost[0] | lost[1]) != 0, 0)) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+            for (int t = 0; t < NT; ++t) {
                 lost[t] = (lost[t] | lost[t] >> 16 | lost[t] >> 32 | lost[t] >> 48) & 0xFFFF;
                 while (lost[t]) {
-                    const int r = __builtin_ctzll(lost[t]), row = i0 + 32 * qh + 16 * t + r;
+                    const int r = __builtin_ctzll(lost[t]), row = i0 + 32 * qh + 16 * (t + t_own) + r;
                     lost[t] &= lost[t] - 1;
                     const float *qr = q + ((size_t)row * n_heads + head) * HD;
                     float res;
@@ -566,8 +579,8 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
         }
     }
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int i = i0 + 32 * qh + 16 * t + r16;
+    for (int t = 0; t < NT; ++t) {
+        const int i = i0 + 32 * qh + 16 * (t + t_own) + r16;
         if (xh_out) {
             // The row leaves as the fp16 image of its Q8_0 quantization (what the o projection's fp16 tiles contract
             // with), the arithmetic of quantize_q8_lane4 + q8_lane4_to_half value by value: a 32-value block is
@@ -575,16 +588,20 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
             const int K = n_heads * HD;
 #pragma unroll
             for (int b = 0; b < DT / 2; ++b) {
-                float amax = fabsf(o[t][2 * b][0]);  // (not 0: a block without a number has no largest value, and stays so)
+                float x[8], level[8];
 #pragma unroll
-                for (int e = 1; e < 8; ++e) amax = fmaxf(amax, fabsf(o[t][2 * b + (e >> 2)][e & 3]));
+                for (int e = 0; e < 8; ++e) x[e] = o[t][2 * b + (e >> 2)][e & 3];
+                float amax = fabsf(x[0]);  // (not 0: a block without a number has no largest value, and stays so)
+#pragma unroll
+                for (int e = 1; e < 8; ++e) amax = fmaxf(amax, fabsf(x[e]));
                 amax = quad16_max(amax);
                 const float dq = amax / 127.0f, df = __half2float(__float2half_rn(dq));
+                q8_levels8(x, amax, dq, level);
 #pragma unroll
                 for (int hf = 0; hf < 2; ++hf) {
                     half4h w;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) w[j] = (_Float16)(df * (float)(amax != 0.0f ? q8_level(o[t][2 * b + hf][j], dq) : 0));
+                    for (int j = 0; j < 4; ++j) w[j] = (_Float16)(df * level[4 * hf + j]);
                     const int col = head * HD + 32 * b + 16 * hf + 4 * g;
                     if (i < n) *(half4h *)(xh_out + xh_index4(i, col >> 2, K) * 4) = w;
                 }
