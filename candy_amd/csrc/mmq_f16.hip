@@ -807,7 +807,12 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     // short K (at most 16 super-blocks) on a grid that 128 x 256 tiles would have to split: 128 x 128 tiles halve the
     // split as long as they still fit one round (Q4_K 4096 x 4096 at 512 rows 35.5 against 36.8 us, at 1024 rows 50.9
     // against 54.2; 6144 x 4096 at 512 rows 44.8 against 47.1; with K = 14336 the split is cheap and the wider tile wins)
-    if (q4k && shape == 0 && jobs[0].w->cols <= 4096 && n128 * ((m + 255) / 256) < fill && n128 * ((m + 127) / 128) <= dev->num_cus)
+    // Not where the launch behind sums the copies anyway (the decoder's prompts: the norm, the rotation) and two are all that the
+    // wide tiles leave: us of an 8B-shaped prompt (four layers and the head), narrow / wide tiles for q / k / v: 300 tokens 1170 / 1131,
+    // 512 1368 / 1349, 700 1878 / 1834; for o, 1B shape, 1500 tokens 1426 / 1404, 7B 600 1664 / 1624.  (With four copies level: 8B
+    // 512 tokens, o as well 1360, 256 tokens 894 / 915.)
+    const bool cheap = dev->defer_split && plan_split(dev, (int)(n128 * ((m + 255) / 256)), (int)(jobs[0].w->cols >> 8)) <= 2;
+    if (q4k && !cheap && shape == 0 && jobs[0].w->cols <= 4096 && n128 * ((m + 255) / 256) < fill && n128 * ((m + 127) / 128) <= dev->num_cus)
         return small_tiles();
     if (single) return launch_big<F, 128, 256, 2, 4>(dev, jobs, count, xh, m);
     // A grid of 128 x 256 tiles that fills the chip, where the 128 x 128 tiles take no more rounds of workgroups: the
