@@ -8,9 +8,16 @@
 // super-block) arrive while these are contracted; the activations straight into operand registers from an image in operand
 // order (rows_i8.h).  The wavefronts' sums meet in LDS at the end, in pairs (reproducible).
 //
-// What bounds it: up to 16 rows two launches and their first bytes, then the weights at 3.5 to 4.5 TB/s (a wavefront's chain of
-// LDS round trips between two waits); from about 48 rows the vector ALU (a conversion, a product and an fma per result and
-// sub-block).  us of a call, before (int8 tiles, mostly with a split of K) -> now:
+// Up to eight rows the 16 columns of a product are two groups of eight (PAIRS): one takes the even, the other the odd sub-blocks (Q6_K: the
+// first and the second 16 values of each), the other's values being zero in its operand, so that a result register stands for two
+// dots and its conversion, product and fma are half as many.  A column's sums meet its twin's at the end.  Vector instructions of a
+// super-block and wavefront: Q6_K 250 -> 180, Q4_0 144 -> 112; us of a call, 16 columns / two groups, 6 rows: 4096 x 14336 Q6_K 16.4 / 14.6, Q4_K
+// 11.6 / 10.7, Q5_K 12.8 / 12.3, Q8_0 17.5 / 17.0, Q4_0 14.2 / 13.5; 32000 x 4096 Q6_K 26.4 / 23.0, Q4_K 17.7 / 16.2, Q4_0 25.5 / 23.9.
+// The distance from 64 bits is smaller than with 16 columns for every format (Q6_K 8.6e-8 -> 8.2e-8, Q4_K 2.2e-7 -> 1.7e-7).
+//
+// What bounds it: up to 16 rows two launches and their first bytes, then the vector ALU (without any weights or activations fetched
+// the Q6_K call of 6 rows took 13.8 of its 16.3 us) beside the weights at 3.5 to 4.5 TB/s; from about 48 rows the vector ALU alone (a
+// conversion, a product and an fma per result and sub-block).  us of a call, before (int8 tiles, mostly with a split of K) -> now:
 //   4096 x 14336, 6 rows   Q4_K 18.1 -> 11.4, Q5_K 17.9 -> 12.8, Q6_K 21.0 -> 16.3, Q8_0 24.4 -> 17.3, Q4_0 22.4 -> 14.2
 //   11008 x 4096, 32 rows  Q4_K 15.7 -> 14.0, Q5_K 27.7 -> 14.7, Q6_K 31.6 -> 22.0, Q8_0 41.6 -> 18.0, Q4_0 38.1 -> 14.9
 //   11008 x 4096, 64 rows  Q5_K 35.0 -> 20.7, Q8_0 44.6 -> 24.2, Q4_0 37.9 -> 23.4
@@ -45,6 +52,16 @@ struct RowsX {
     float4 d[MT][2];
     float2 m[MT];
 };
+// The same of up to eight rows, whose 16 columns of a product are two groups of eight: a column belongs to row j & 7 and takes one
+// half of what is scaled apart, sub-blocks 2p + (j >> 3), or for Q6_K (halves) 16 values of every sub-block.  What a
+// column does not take is zero in its operand.
+template <bool HALVES>
+struct RowsPairs {
+    u32x4 q[HALVES ? 4 : 1];            // Q6_K: as above
+    u32x2 even[4], odd[4];              // sub-blocks 2p and 2p + 1
+    float d[HALVES ? 8 : 4];
+    float2 m[1];
+};
 __device__ __forceinline__ float rows_d(const float4 (&d)[2], int t) {
     const float4 v = d[t >> 2];
     return (t & 3) == 0 ? v.x : (t & 3) == 1 ? v.y : (t & 3) == 2 ? v.z : v.w;
@@ -66,8 +83,8 @@ struct RowsQ45K {
     static constexpr int BLOCK = FIVE ? 176 : 144, PIECES = BLOCK / 16, GROUPS = 8;
     static constexpr bool DIRECT = true, HALVES = false;
     struct Row { u32x2 q[4], qh; };
-    template <int MT>
-    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &x, float4v (&acc)[MT]) {
+    template <int MT, class X>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const X &x, float4v (&acc)[MT]) {
         const u32x4 h = *(const u32x4 *)wl;
         uint32_t sc2, m2;
         q4k_scale_min_pair(h.y, h.z, h.w, c, sc2, m2);
@@ -103,8 +120,8 @@ struct RowsQ8_0 {
     static constexpr int BLOCK = 272, PIECES = 17, GROUPS = 8;
     static constexpr bool DIRECT = true, HALVES = false;
     struct Row { u32x2 q[8]; };
-    template <int MT>
-    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &, float4v (&)[MT]) {
+    template <int MT, class X>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const X &, float4v (&)[MT]) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) ex[(2 * c + h) * 16 + j] = half_bits_to_float(*(const uint16_t *)(wl + 34 * (2 * c + h)));
     }
@@ -121,8 +138,8 @@ struct RowsQ4_0 {
     static constexpr int BLOCK = 144, PIECES = 9, GROUPS = 8;
     static constexpr bool DIRECT = true, HALVES = false;
     struct Row { u32x2 q[8]; };
-    template <int MT>
-    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &, float4v (&)[MT]) {
+    template <int MT, class X>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const X &, float4v (&)[MT]) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) ex[(2 * c + h) * 16 + j] = 0.0625f * half_bits_to_float(*(const uint16_t *)(wl + 18 * (2 * c + h)));
     }
@@ -151,13 +168,13 @@ struct RowsQ6K {
     static constexpr int BLOCK = 210, PIECES = 15, GROUPS = 17;
     static constexpr bool DIRECT = false, HALVES = true;
     struct Row { u32x2 ql[4], qh[2]; };
-    template <int MT>
-    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const RowsX<MT> &, float4v (&)[MT]) {
+    template <int MT, class X>
+    static __device__ __forceinline__ void factors(const uint8_t *wl, int j, int c, float *ex, const X &, float4v (&)[MT]) {
         // the sixteen scales as integers, then d
         const uint32_t sc = *(const uint32_t *)(wl + 192 + 4 * c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) ((int *)ex)[(4 * c + i) * 16 + j] = (int)(sc << (24 - 8 * i)) >> 24;
-        if (c == 0) ex[16 * 16 + j] = half_bits_to_float(*(const uint16_t *)(wl + 208));
+        if (c == 0) ex[16 * 16 + j] = 0.25f * half_bits_to_float(*(const uint16_t *)(wl + 208));
     }
     static __device__ __forceinline__ void load(const uint8_t *wl, int c, Row &r) {
 #pragma unroll
@@ -173,10 +190,9 @@ struct RowsQ6K {
         uint32_t w2[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const uint32_t nib = (quarter & 2) ? (ql[e] >> 4) & 0x0F0F0F0Fu : ql[e] & 0x0F0F0F0Fu;
-            const uint32_t top = quarter == 0 ? (qh[e] << 4) : quarter == 1 ? (qh[e] << 2) : quarter == 2 ? qh[e] : (qh[e] >> 2);
-            // bytewise level - 32: bias by 128 so that no byte borrows, then flip the bias off
-            w2[e] = (((nib | (top & 0x30303030u)) | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
+            // 4 (level - 32): the level in the upper six bits of a byte, its top bit flipped
+            const uint32_t nib = quarter & 2 ? (ql[e] >> 2) & 0x3C3C3C3Cu : (ql[e] << 2) & 0x3C3C3C3Cu;
+            w2[e] = (nib | ((qh[e] << (6 - 2 * quarter)) & 0xC0C0C0C0u)) ^ 0x80808080u;
         }
         return rows_pack(w2[0], w2[1]);
     }
@@ -193,10 +209,12 @@ struct RowsLds {
     static constexpr int BYTES = WAVES * WAVE > SUMS ? WAVES * WAVE : SUMS;
 };
 
-template <class F, int RF, int MT, int WAVES>
+template <class F, int RF, int MT, int WAVES, bool PAIRS>
 __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 4 : 2) void k_rows_i8(
     const uint8_t *__restrict__ xfrag, const float *__restrict__ xd, const float *__restrict__ xm, int K, int M, int frag_stride,
     int scale_stride, const RowsJobs jobs) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+    static_assert(!PAIRS || MT == 1, "eight rows");
     typedef RowsLds<F, RF, MT, WAVES> L;
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, c = lane >> 4;
@@ -240,8 +258,35 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
             *(u32x4 *)(mine + (e / L::LOADED) * (F::PIECES * 16) + (e % L::LOADED) * 16) = held[it];
         }
     };
-    RowsX<MT> x;
+    std::conditional_t<PAIRS, RowsPairs<F::HALVES>, RowsX<MT>> x;
+    const int group = j >> 3;  // PAIRS: of columns
+    // PAIRS: what a column does not take is asked for past the image's end, and comes as zero
+    constexpr uint32_t NOTHING = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)xfrag, 0, frag_stride, 0x00027000);
+    const uint32_t mine_at = ((uint32_t)(j & 7) + 16 * c) * 16;
+    const uint32_t at_half = c >> 1 == group ? mine_at : NOTHING;
     auto load_x = [&](int sb) __attribute__((always_inline)) {
+        if constexpr (PAIRS) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                if constexpr (F::HALVES) {
+                    x.q[p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, at_half + p * 1024, sb * 4096, 0));
+                } else {
+                    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, mine_at + p * 1024, sb * 4096, 0));
+                    x.even[p] = group == 0 ? u32x2{v.x, v.y} : u32x2{0, 0};
+                    x.odd[p] = group == 1 ? u32x2{v.z, v.w} : u32x2{0, 0};
+                }
+            }
+            const float *pd = xd + (size_t)sb * 128 + (j & 7) * 8, *pm = xm + (size_t)sb * 128 + (j & 7) * 8 + 2 * c;
+            const float4 a = *(const float4 *)pd, b = *(const float4 *)(pd + 4);
+            if constexpr (F::HALVES) {
+                x.d[0] = a.x; x.d[1] = a.y; x.d[2] = a.z; x.d[3] = a.w; x.d[4] = b.x; x.d[5] = b.y; x.d[6] = b.z; x.d[7] = b.w;
+            } else {
+                x.d[0] = group ? a.y : a.x; x.d[1] = group ? a.w : a.z; x.d[2] = group ? b.y : b.x; x.d[3] = group ? b.w : b.z;
+            }
+            const float2 v = *(const float2 *)pm;
+            x.m[0] = group == 0 ? float2{v.x, 0.0f} : float2{0.0f, v.y};  // with the products that it is taken off
+        } else
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const uint8_t *pf = xfrag + (size_t)t * frag_stride + (size_t)sb * 4096;
@@ -276,15 +321,47 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
                 if (r + 1 < RF) request(sb, r + 1, slot ^ 1);
                 else if (k + 1 < count) request(sb + WAVES, 0, slot ^ 1);
                 const uint8_t *wl = mine + slot * L::SLOT + j * (F::PIECES * 16);
-                F::template factors<MT>(wl, j, c, ex, x, acc[r]);
+                F::template factors<MT, decltype(x)>(wl, j, c, ex, x, acc[r]);
                 typename F::Row row;
                 F::load(wl, c, row);
                 rows_lds_fence();
-                float4v part[F::HALVES ? MT : 1];  // Q6_K: the super-block's sum in front of d
+                // Q6_K: the super-block's sum in front of d (PAIRS: of every second sub-block, for a shorter chain of roundings: the
+                // columns' sums meet in one rounding more)
+                constexpr int PARTS = F::HALVES ? (PAIRS ? 2 : MT) : 1;
+                float4v part[PARTS];
                 if constexpr (F::HALVES) {
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) part[mt] = float4v{0.f, 0.f, 0.f, 0.f};
+                    for (int mt = 0; mt < PARTS; ++mt) part[mt] = float4v{0.f, 0.f, 0.f, 0.f};
                 }
+                if constexpr (PAIRS && F::HALVES) {
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        if (t % 2 == 0) {
+                            asm volatile("" : "+v"(part[0]), "+v"(part[PARTS - 1]));
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        const u32x4 v = x.q[t >> 1];
+                        const long b = t & 1 ? rows_pack(v.z, v.w) : rows_pack(v.x, v.y);
+                        const int4v d = __builtin_amdgcn_mfma_i32_16x16x32_i8(F::operand(row, t, c), b, int4v{0, 0, 0, 0}, 0, 0, 0);
+                        const int4v f = *(const int4v *)&ex[(2 * t + group) * 16 + 4 * c];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) part[t & 1][i] += x.d[t] * (float)__mul24(d[i], f[i]);
+                    }
+                } else if constexpr (PAIRS) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        if (p % 2 == 0) {
+                            asm volatile("" : "+v"(acc[r][0]));
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        int4v d = __builtin_amdgcn_mfma_i32_16x16x32_i8(F::operand(row, 2 * p, c), rows_pack(x.even[p].x, x.even[p].y),
+                                                                        int4v{0, 0, 0, 0}, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_i32_16x16x32_i8(F::operand(row, 2 * p + 1, c), rows_pack(x.odd[p].x, x.odd[p].y), d, 0, 0, 0);
+                        const float4v f = *(const float4v *)&ex[(2 * p + group) * 16 + 4 * c];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[r][0][i] += (f[i] * x.d[p]) * (float)d[i];
+                    }
+                } else
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
                     constexpr int TOGETHER = MT == 1 ? (F::HALVES ? 2 : 4) : MT == 2 && !F::HALVES ? 2 : 1;
@@ -307,7 +384,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
                             const int4v dh = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_hi, b, int4v{0, 0, 0, 0}, 0, 0, 0);
                             const float dx = rows_d(x.d[mt], t);
 #pragma unroll
-                            for (int i = 0; i < 4; ++i)  // |dot| <= 2^16, |scale| <= 2^7: exact
+                            for (int i = 0; i < 4; ++i)  // |dot| <= 2^18, in fours, |scale| <= 2^7: exact
                                 part[mt][i] += dx * (float)(__mul24(dh[i], fh[i]) + __mul24(dl[i], fl[i]));
                         }
                     } else {
@@ -321,6 +398,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
                         }
                     }
                 }
+                if constexpr (PAIRS && F::HALVES) part[0] += part[PARTS - 1];
                 if constexpr (F::HALVES) {
                     const float4v d = *(const float4v *)&ex[16 * 16 + 4 * c];
 #pragma unroll
@@ -348,10 +426,24 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) p[w] = sums[(w * RF * MT + f) * 64 + lane];
 #pragma unroll
-        for (int d = 1; d < WAVES; d *= 2)  // neighbours first: a shorter chain of roundings
+        for (int d = 1; d < (PAIRS && F::HALVES ? WAVES / 2 : WAVES); d *= 2)  // neighbours first: a shorter chain of roundings
 #pragma unroll
             for (int w = 0; w < WAVES; w += 2 * d) p[w] += p[w + d];
         float4v s = p[0];
+        // PAIRS: and the same of the row's other column (row_ror:8).  Q6_K: the last two sums and theirs in one rounding, against the
+        // rounding more that sums from twice the columns have (the others' chains of a super-block are half as long)
+        if constexpr (PAIRS && F::HALVES) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double v = (double)p[0][i] + (double)p[WAVES / 2][i];
+                const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+                const uint32_t lo = (uint32_t)dpp_move_i<0x128>((int)(uint32_t)bits), hi = (uint32_t)dpp_move_i<0x128>((int)(uint32_t)(bits >> 32));
+                s[i] = (float)(v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo));
+            }
+        } else if constexpr (PAIRS) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += dpp_move<0x128>(s[i]);
+        }
         const int m = (blockIdx.y * MT + t) * 16 + j, own = n0 + 16 * r, n = strip_row(r) + 4 * c;  // weight rows n .. n + 3
         if (m >= M) continue;
         float *dst = job.y + (size_t)m * N + n;
@@ -365,9 +457,10 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES == 16 || MT + F::HALVES <= 2) ? 
                 if (n + i >= own) dst[i] = res ? res[i] + s[i] : s[i];
         }
     }
+#endif
 }
 
-template <class F, int RF, int MT, int WAVES>
+template <class F, int RF, int MT, int WAVES, bool PAIRS = false>
 static int launch_rows_cfg(candy_hip_device *dev, const RowsLaunch &L, int64_t m) {
     typedef RowsLds<F, RF, MT, WAVES> S;
     static_assert(S::BYTES <= 160 * 1024, "LDS");
@@ -384,7 +477,7 @@ static int launch_rows_cfg(candy_hip_device *dev, const RowsLaunch &L, int64_t m
         jobs.j[i].wg_end = total;
     }
     const int K = (int)L.w[0]->cols;
-    auto kern = k_rows_i8<F, RF, MT, WAVES>;
+    auto kern = k_rows_i8<F, RF, MT, WAVES, PAIRS>;
     if (S::BYTES > 48 * 1024)
         CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::BYTES));
     hipLaunchKernelGGL(kern, dim3((unsigned)total, (unsigned)((m + 16 * MT - 1) / (16 * MT))), dim3(WAVES * 64), S::BYTES, dev->stream,
@@ -395,8 +488,12 @@ static int launch_rows_cfg(candy_hip_device *dev, const RowsLaunch &L, int64_t m
 
 template <class F>
 static int launch_rows_fmt(candy_hip_device *dev, const RowsLaunch &L, int64_t m, int rf, int mt, int waves) {
-#define CANDY_ROWS(RF, MT, WAVES) \
-    if (rf == RF && mt == MT && waves == WAVES) return launch_rows_cfg<F, RF, MT, WAVES>(dev, L, m);
+#define CANDY_ROWS(RF, MT, WAVES)                                                                                  \
+    if (rf == RF && mt == MT && waves == WAVES) {                                                                  \
+        if constexpr (MT == 1)                                                                                     \
+            if (m <= 8) return launch_rows_cfg<F, RF, MT, WAVES, true>(dev, L, m);                                 \
+        return launch_rows_cfg<F, RF, MT, WAVES>(dev, L, m);                                                       \
+    }
     CANDY_ROWS(1, 1, 16) CANDY_ROWS(1, 1, 8)
     if constexpr (std::is_same<F, RowsQ6K>::value) {
         CANDY_ROWS(2, 1, 8)

@@ -109,3 +109,17 @@ def test_a_prompt_sees_its_own_rows_only(dev, fmt):
     want, m = hidden(model(), tokens), model()
     assert np.isfinite(want).all() and not np.isfinite(hidden(m, tokens + [255] * 10)[5:]).any()
     assert np.array_equal(hidden(m, tokens).view(np.uint32), want.view(np.uint32))
+
+
+# Up to eight rows share the columns of a product in two groups: as many strips per workgroup and wavefronts as there are, the last
+# column and the first row count past it, against the same rows in a batch of 16 columns.
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("rows,cols", [(16, 256), (1030, 4352), (4099, 512), (8200, 256), (16500, 768)])
+def test_two_groups_of_columns(dev, fmt, rows, cols):
+    w = synth.random_weight(fmt, rows, cols, seed=rows + fmt)
+    x = synth.random_activations(16, cols, seed=cols)
+    q = dev.qtensor(fmt, rows, cols, w)
+    whole = exact(dev, q, x)
+    for m in (3, 7, 8, 9):
+        assert rel_err(exact(dev, q, x[:m]), whole[:m]) <= 2e-6  # two orders of f32 sums, as above
