@@ -101,3 +101,14 @@ def test_one_round_of_workgroups_and_bounded_activations():
     (synth.Q4_K, 80, 4200, 4352, 0)])
 def test_where_the_lines_lie(fmt, m, rows, cols, rf):
     assert chosen(fmt, m, rows, cols) == rf
+
+
+@pytest.mark.parametrize("fmt,m,rows,cols,rf", [
+    # ahead of the tiles since a step's loads stand in front of its arithmetic (14.5 / 20.9 us, 7.8 / 11.1, 21.2 / 24.6, 24.1 / 26.7)
+    (synth.Q4_K, 96, 8200, 2560, 3), (synth.Q5_K, 128, 4096, 512, 1), (synth.Q4_0, 128, 4096, 4096, 1), (synth.Q8_0, 128, 6144, 4096, 2),
+    # one super-block in the last round: the tiles at eight fragments, and at five while few CUs are at work
+    (synth.Q5_K, 128, 4352, 4352, 0), (synth.Q4_K, 80, 4576, 4352, 0), (synth.Q4_K, 80, 4577, 4352, 2), (synth.Q4_K, 64, 4200, 4352, 2),
+    # long rows of few weight rows and Q4_0 from 65 rows
+    (synth.Q8_0, 96, 2816, 5632, 0), (synth.Q4_0, 66, 4096, 4096, 1)])
+def test_where_the_fitted_costs_cross(fmt, m, rows, cols, rf):
+    assert chosen(fmt, m, rows, cols) == rf
