@@ -14,7 +14,7 @@
 // dequantizes several steps in advance and requests the activations behind that, where nothing hides them.  A wavefront's loads are
 // the same in number at every step, with weights to fetch or not (request()).  us of a call, without / with both: 11008 x 4096, 77
 // rows Q8_0 24.9 / 22.7, Q4_0 21.9 / 19.7, Q5_K 25.1 / 21.9, Q4_K 20.2 / 17.7; 3000 x 2560 Q5_K 14.9 / 10.9; 8192 x 2048, 100 rows
-// Q4_K 16.3 / 13.4, Q6_K 19.9 / 18.6 (4096 x 4096, 77 rows Q4_K 14.0 / 14.2).  Fences behind the first half's loads too, or the loads
+// Q4_K 16.3 / 13.4 (4096 x 4096, 77 rows Q4_K 14.0 / 14.2).  Fences behind the first half's loads too, or the loads
 // three halves ahead: 3 and 7 % slower.  What bounds it: without any weights or activations fetched the Q8_0 call takes 17.6 (a
 // launch of the quantizer 2.5, dequantization and products of two wavefronts a SIMD, the sums), the activations, which every CU
 // reads (655 KB), add 2 to 3, the weights (48 MB of Q8_0) the rest.
@@ -26,12 +26,13 @@
 
 namespace candy {
 
+// 16-byte pieces that hold a super-block wherever it starts (Q6_K: 210 bytes, up to 14 behind the start of a piece)
 template <class F>
-constexpr bool staged() { return F::BLOCK % 16 == 0; }
+constexpr int pieces() { return F::BLOCK % 16 == 0 ? F::BLOCK / 16 : (F::BLOCK + 14) / 16; }
 
 template <class F, int RF, int MF>
 constexpr size_t lds_bytes() {
-    const size_t sums = (size_t)8 * RF * MF * 1024, slices = staged<F>() ? (size_t)8 * 1024 * ((RF * F::BLOCK / 16 + 3) / 4) : 0;
+    const size_t sums = (size_t)8 * RF * MF * 1024, slices = (size_t)8 * 1024 * ((RF * pieces<F>() + 3) / 4);
     return sums > slices ? sums : slices;
 }
 
@@ -39,7 +40,7 @@ template <class F, int RF, int MF>
 __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restrict__ W, const _Float16 *__restrict__ xh, float *y,
                                                          const float *res, int M, int N, int K) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
-    constexpr bool STAGED = staged<F>();
+    constexpr bool WHOLE = F::BLOCK % 16 == 0;  // pieces
     extern __shared__ __align__(16) uint8_t smem_raw[];
     float4v *sums = (float4v *)smem_raw;  // [wave][RF][MF][lane]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, c = lane >> 4;
@@ -57,47 +58,46 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
     // A super-block of the workgroup's rows comes into the wavefront's own slice of LDS, 16-byte pieces in the order they
     // lie in memory (requests of a lane for its own few bytes of a row cost the cache a line each: Q8_0 9 us per 16 rows of
     // 4096 and CU, against 3 for the bytes themselves); from there to registers, which frees the slice for the next one.
-    // Q6_K blocks (210 bytes) are not whole pieces: their requests go straight to registers.
-    constexpr int PIECES = F::BLOCK / 16, IT = (RF * 16 * PIECES + 63) / 64;
+    // A Q6_K block (210 bytes) starts anywhere in its first piece: 14 pieces hold it wherever that is.  us of a call, nine requests of a lane
+    // for its own bytes / staged: 4096 x 4096, 64 rows 15.9 / 12.7, 11008 x 4096, 48 rows 25.1 / 17.1, 8192 x 4096, 40 rows 18.8 / 12.8.
+    constexpr int PIECES = pieces<F>(), IT = (RF * 16 * PIECES + 63) / 64;
     uint4 *slice = (uint4 *)smem_raw + wave * (IT * 64);
-    uint32_t from[STAGED ? IT : 1];
-    if constexpr (STAGED) {
+    uint32_t from[IT];
 #pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int e = it * 64 + lane, row = min(e / PIECES, RF * 16 - 1);
-            from[it] = (uint32_t)(min(n0 + row, N - 1) - n0) * (uint32_t)rb + (uint32_t)(e % PIECES) * 16;
-        }
+    for (int it = 0; it < IT; ++it) {
+        const int e = it * 64 + lane, row = min(e / PIECES, RF * 16 - 1);
+        from[it] = (uint32_t)(min(n0 + row, N - 1) - n0) * (uint32_t)rb + (uint32_t)(e % PIECES) * 16;
     }
     const uint8_t *w0 = W + (size_t)n0 * rb;
     // any false: the same loads from a matrix of no bytes, so that as many are in flight at every step: behind a branch around them
     // the compiler waits for the activations by the smaller count, which is a wait for the weights too
     auto request = [&](int sb, bool any) __attribute__((always_inline)) {
         const int at = any ? sb * F::BLOCK : 0;  // (a scalar offset past an empty matrix would count as inside)
-        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)w0, 0, any ? (int)(RF * 16 * rb) : 0, 0x00027000);
+        // pieces past the last block of a Q6_K matrix: no bytes; its end lies in an aligned word, which counts as a whole
+        const int size = WHOLE ? (int)(RF * 16 * rb) : ((int)(min(RF * 16, N - n0) * rb) + 3) & ~3;
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)w0, 0, any ? size : 0, 0x00027000);
 #pragma unroll
         for (int it = 0; it < IT; ++it)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(slice + it * 64), 16, from[it],
-                                                     at, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(slice + it * 64), 16,
+                                                     WHOLE ? from[it] : (from[it] + (uint32_t)at) & ~15u, WHOLE ? at : 0, 0, 0);
     };
     if (count > 0) {
-        // Unstaged blocks are requested a super-block ahead, but three fragments of them twice over do not fit the registers: 41
-        // spilled at 64 rows, us, two sets / one: 11008 x 4096, 48 rows 28.1 / 26.1, x 2048, 40 rows 15.4 / 14.6.  (Two fragments
-        // and 128 rows spill 35 and are ahead with two sets all the same: 4200 x 1024 13.2 / 14.7, 8192 x 1536 18.1 / 18.1.)
-        constexpr int DEEP = STAGED || RF == 3 ? 1 : 2;
-        typename F::Raw raw[DEEP][RF];
+        typename F::Raw raw[RF];
         half8 xf[2][MF];
-        auto load_w = [&](int sb, int u) __attribute__((always_inline)) {
+        auto load_w = [&](int sb) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < RF; ++i)
-                F::load(STAGED ? (const uint8_t *)slice + (16 * i + r16) * F::BLOCK
-                               : W + (size_t)min(n0 + 16 * i + r16, N - 1) * rb + (size_t)sb * F::BLOCK, c, raw[u][i]);
+            for (int i = 0; i < RF; ++i) {
+                const int row = 16 * i + r16;
+                const uint32_t behind = WHOLE ? 0 : ((uint32_t)(min(n0 + row, N - 1) - n0) * (uint32_t)rb + (uint32_t)(sb * F::BLOCK)) & 15;
+                F::load((const uint8_t *)slice + row * (16 * PIECES) + behind, c, raw[i]);
+            }
         };
         auto load_x = [&](int step, int h) __attribute__((always_inline)) {  // step: in 64s along K
             const _Float16 *p = xl + (size_t)step * 1024 + h * HALF;
 #pragma unroll
             for (int t = 0; t < MF; ++t) xf[h][t] = *(const half8 *)(p + t * xrow);
         };
-        auto contract = [&](int sb, int u, int sb_next) __attribute__((always_inline)) {
+        auto contract = [&](int sb, int sb_next) __attribute__((always_inline)) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 load_x(sb * 4 + g, 1);
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
 #pragma unroll
                 for (int i = 0; i < RF; ++i) {
                     int k0, k1;
-                    F::dequant(raw[u][i], g, c, a[i][0], a[i][1], k0, k1);
+                    F::dequant(raw[i], g, c, a[i][0], a[i][1], k0, k1);
                 }
 #pragma unroll
                 for (int t = 0; t < MF; ++t)
@@ -119,38 +119,15 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
                     for (int i = 0; i < RF; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][1], xf[1][t], acc[i][t], 0, 0, 0);
             }
         };
-        if constexpr (STAGED) {
-            request(first, true);
-            load_x(first * 4, 0);
-            for (int k = 0; k < count; ++k) {
-                const int sb = first + 8 * k;
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the slice has landed
-                load_w(sb, 0);
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and is in registers
-                request(sb + 8, k + 1 < count);
-                contract(sb, 0, k + 1 < count ? sb + 8 : sb);
-            }
-        } else if constexpr (DEEP == 1) {
-            load_w(first, 0);
-            load_x(first * 4, 0);
-            for (int k = 0; k < count; ++k) {
-                const int sb = first + 8 * k;
-                contract(sb, 0, k + 1 < count ? sb + 8 : sb);
-                if (k + 1 < count) load_w(sb + 8, 0);
-            }
-        } else {
-            load_w(first, 0);
-            if (count > 1) load_w(first + 8, 1);
-            load_x(first * 4, 0);
-            for (int k = 0; k < count; k += 2) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    if (k + u >= count) break;
-                    const int sb = first + 8 * (k + u);
-                    contract(sb, u, k + u + 1 < count ? sb + 8 : sb);
-                    if (k + u + 2 < count) load_w(sb + 16, u);
-                }
-            }
+        request(first, true);
+        load_x(first * 4, 0);
+        for (int k = 0; k < count; ++k) {
+            const int sb = first + 8 * k;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the slice has landed
+            load_w(sb);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and is in registers
+            request(sb + 8, k + 1 < count);
+            contract(sb, k + 1 < count ? sb + 8 : sb);
         }
     }
     __syncthreads();  // the slices are consumed
@@ -267,7 +244,7 @@ static int launch_fmt(candy_hip_device *dev, const candy_hip_qtensor *w, const _
 }
 
 bool mmq_f16_rows_covers(const candy_hip_qtensor *w, int64_t m) {
-    if (w->fmt != CANDY_HIP_Q6_K && ((uintptr_t)w->data & 15) != 0) return false;  // whole pieces
+    if (((uintptr_t)w->data & 15) != 0) return false;  // whole pieces
     switch (w->fmt) {
     case CANDY_HIP_Q4_K: case CANDY_HIP_Q5_K: case CANDY_HIP_Q6_K: case CANDY_HIP_Q8_0: case CANDY_HIP_Q4_0: case CANDY_HIP_Q4_0_GGML:
         return rows_fragments(w->fmt, w->rows, w->cols, m, w->dev->num_cus) > 0;

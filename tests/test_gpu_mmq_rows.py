@@ -112,3 +112,18 @@ def test_where_the_lines_lie(fmt, m, rows, cols, rf):
     (synth.Q8_0, 96, 2816, 5632, 0), (synth.Q4_0, 66, 4096, 4096, 1)])
 def test_where_the_fitted_costs_cross(fmt, m, rows, cols, rf):
     assert chosen(fmt, m, rows, cols) == rf
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,m", [(2049, 2304, 48), (2063, 256, 80), (4099, 2304, 64), (4111, 2048, 48), (8209, 1280, 48)])
+def test_q6_k_blocks_behind_the_start_of_a_piece(dev, rows, cols, m):
+    # odd rows of odd blocks start 2 .. 14 bytes into a piece, and the matrix ends in the middle of a word
+    assert chosen(synth.Q6_K, m, rows, cols)
+    w = synth.random_weight(synth.Q6_K, rows, cols, seed=rows)
+    x = synth.random_activations(m, cols, seed=cols)
+    got = dev.qmatmul(dev.qtensor(synth.Q6_K, rows, cols, w), x)
+    nb = synth.weight_nbytes(synth.Q6_K, 1, cols)
+    sub = np.r_[0:9, rows - 17:rows]
+    want = o.qmatmul(synth.Q6_K, w.reshape(rows, nb)[sub].reshape(-1), len(sub), cols, x)
+    # fp16 operands: 2^-12 of each product
+    assert np.max(np.abs(got[:, sub] - want)) <= 5e-4 * np.max(np.abs(want))
