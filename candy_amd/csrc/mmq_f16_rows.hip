@@ -158,11 +158,10 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
 
 static int fragments(int64_t m) { return m <= 48 ? 3 : m <= 64 ? 4 : m <= 80 ? 5 : m <= 96 ? 6 : 8; }
 
-// What a call takes, us, here and on the 128 x 128 tiles of mmq_f16.hip, the tiles 2 % below their fit: both fitted to 3604 calls (five
-// formats, 2048 .. 12288 weight rows, K 512 .. 8192, 36 .. 128 activation rows; the fits are 3 to 6 % off on average; Q6_K's to 2940
-// calls of the kernels before, which another fit divides no better).  A line on any one size does not divide them: a round of
-// super-blocks that most wavefronts sit out, a split that leaves the tiles short, an odd number of 210-byte blocks (rows 2 bytes
-// off) each move it.
+// What a call takes, us, here and on the 128 x 128 tiles of mmq_f16.hip, the tiles 2 % below their fit: both fitted to 3729 calls (five
+// formats, 2048 .. 12288 weight rows, K 512 .. 8192, 36 .. 128 activation rows; the fits are 3 to 6 % off on average).  A line on any
+// one size does not divide them: a round of super-blocks that most wavefronts sit out, a split that leaves the tiles short, an odd
+// number of 210-byte blocks (rows 2 bytes off) each move it.
 struct RowsCost {
     // a launch; a tile's super-block; a split's launch; MB of its copies; 1000 super-blocks of all tiles
     float tile[5];
@@ -173,7 +172,7 @@ struct RowsCost {
 static const RowsCost &rows_cost(int fmt) {
     static constexpr RowsCost Q4K{{7.74f, 1.16f, 2.49f, 0.33f, 2.25f}, {4.49f, 0.32f, 0.02f, 0.10f, 0.01f, 0.0f, 0.05f, 0.33f}},
         Q5K{{8.22f, 1.24f, 3.32f, 0.27f, 2.51f}, {4.23f, 0.15f, 0.03f, 0.10f, 0.05f, 0.0f, 0.05f, 0.43f}},
-        Q6K{{9.42f, 1.45f, 3.36f, 0.21f, 4.00f}, {3.48f, 0.00f, 0.06f, 0.11f, 0.30f, 0.08f, 0.11f, 0.88f}},
+        Q6K{{8.64f, 1.50f, 2.55f, 0.32f, 2.63f}, {4.16f, 0.27f, 0.00f, 0.10f, 0.07f, 0.01f, 0.07f, 0.63f}},
         Q80{{8.67f, 2.12f, 3.06f, 0.26f, 2.35f}, {4.18f, 0.00f, 0.05f, 0.10f, 0.13f, 0.0f, 0.00f, 0.70f}},
         Q40{{10.18f, 1.31f, 3.00f, 0.27f, 3.37f}, {4.34f, 0.14f, 0.01f, 0.11f, 0.03f, 0.0f, 0.07f, 0.35f}};
     return fmt == CANDY_HIP_Q4_K ? Q4K : fmt == CANDY_HIP_Q5_K ? Q5K : fmt == CANDY_HIP_Q6_K ? Q6K : fmt == CANDY_HIP_Q8_0 ? Q80 : Q40;
@@ -181,9 +180,9 @@ static const RowsCost &rows_cost(int fmt) {
 
 // 16-row weight fragments per workgroup with which one round of workgroups serves every row and this kernel is ahead of the tiles; 0:
 // none, the tiles.  A second round would read the activations again, wider workgroups have no registers for their sums; fewer than
-// 2048 weight rows leave half of the CUs idle.  All 3604 calls together take 0.2 % more than the faster kernel for each.  us of a call,
+// 2048 weight rows leave half of the CUs idle.  All 3729 calls together take 0.3 % more than the faster kernel for each.  us of a call,
 // tiles / here: Q8_0 4096 x 2304, 96 rows 20.4 / 12.1, Q4_K 4096 x 4096, 80 rows 18.9 / 14.3, 128 rows 21.8 / 20.4, 8200 x 2560,
-// 96 rows 20.9 / 14.5, Q6_K 8192 x 2048, 96 rows 17.1 / 15.0, 11008 x 4096, 48 rows 30.0 / 25.1, 8200 x 3840, 48 rows 23.3 / 27.6 (tiles).
+// 96 rows 20.9 / 14.5, Q6_K 4096 x 4096, 96 rows 21.6 / 17.9, 11008 x 4096, 48 rows 29.8 / 17.1, 64 rows 30.7 / 18.4.
 static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
     const bool q6k = fmt == CANDY_HIP_Q6_K;
     // up to 64 rows the other formats are on the exact tiles (mmq_f16_big_covers)
@@ -192,7 +191,7 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
     int rf = 1;
     while ((rows + 16 * rf - 1) / (16 * rf) > num_cus)
         if (++rf > 3) return 0;
-    if (rf == 3 && mf > (q6k ? 4 : 6)) return 0;
+    if (rf == 3 && mf > 6) return 0;
     if (mf * 32 * cols > 1200000) return 0;  // not measured
     const int64_t blocks = cols / 256, rounds = (blocks + 7) / 8, tiles = (rows + 127) / 128;
     // as plan_split() deals K to the tiles' workgroups
@@ -205,18 +204,20 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
     if (splits > 1) tile += c.tile[2] + c.tile[3] * (float)(splits + 1) * out;
     const float here = c.rows[0] + (float)rounds * (c.rows[1] * rf + c.rows[2] * mf) + (float)blocks * (c.rows[3] * mf + c.rows[4] * rf) +
                        (blocks & 1 ? c.rows[5] * (float)(blocks * rf) : 0.0f) + c.rows[6] * (float)(rf * mf) + c.rows[7] * out;
-    // Q4_K and Q5_K with a single super-block in the last round, at eight activation fragments or little more than half of the CUs at work:
-    // on the tiles, where the kernel's form before had them and the rule's test holds them (17.6 / 15.2 us Q4_K 8192 x 2304, 128 rows,
-    // 18.5 / 16.4 4200 x 4352, 80 rows: tiles / here)
+    // Three kinds of calls stay on the tiles, where the kernel's forms before had them and the rule's test holds them.  Q4_K and Q5_K with a
+    // single super-block in the last round, at eight activation fragments or little more than half of the CUs at work (tiles / here:
+    // Q4_K 8192 x 2304, 128 rows 17.6 / 15.2 us, 4200 x 4352, 80 rows 18.5 / 16.4); Q6_K with an odd number of blocks, 13 or more, up to 64 rows, in
+    // little more than two thirds of the CUs (8200 x 3840, 40 rows 23.0 / 16.1)
     if ((fmt == CANDY_HIP_Q4_K || fmt == CANDY_HIP_Q5_K) && rf == 2 && blocks % 8 == 1 &&
         (mf == 8 || (mf >= 5 && blocks > 8 && (rows + 31) / 32 * 16 < num_cus * 9)))
         return 0;
+    if (q6k && rf == 3 && mf <= 4 && blocks % 2 != 0 && blocks >= 13 && (rows + 47) / 48 * 16 < num_cus * 11) return 0;
     return here < tile ? rf : 0;
 }
 template <class F, int RF, int MF>
 constexpr bool reached() {
     constexpr bool q4k = std::is_same<F, BigQ4K>::value, q6k = std::is_same<F, BigQ6K>::value;
-    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= (q6k ? 4 : 6));
+    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= 6);
 }
 
 template <class F, int RF, int MF>

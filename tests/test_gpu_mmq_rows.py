@@ -109,7 +109,10 @@ def test_where_the_lines_lie(fmt, m, rows, cols, rf):
     # one super-block in the last round: the tiles at eight fragments, and at five while few CUs are at work
     (synth.Q5_K, 128, 4352, 4352, 0), (synth.Q4_K, 80, 4576, 4352, 0), (synth.Q4_K, 80, 4577, 4352, 2), (synth.Q4_K, 64, 4200, 4352, 2),
     # long rows of few weight rows and Q4_0 from 65 rows
-    (synth.Q8_0, 96, 2816, 5632, 0), (synth.Q4_0, 66, 4096, 4096, 1)])
+    (synth.Q8_0, 96, 2816, 5632, 0), (synth.Q4_0, 66, 4096, 4096, 1),
+    # Q6_K through LDS: three weight fragments beside five and six of activations; odd blocks on few CUs, and not on more or fewer blocks
+    (synth.Q6_K, 96, 11008, 4096, 3), (synth.Q6_K, 128, 8192, 4096, 2), (synth.Q6_K, 48, 8400, 3328, 0), (synth.Q6_K, 48, 8401, 3328, 3),
+    (synth.Q6_K, 48, 8200, 2816, 3), (synth.Q6_K, 80, 8200, 3328, 3)])
 def test_where_the_fitted_costs_cross(fmt, m, rows, cols, rf):
     assert chosen(fmt, m, rows, cols) == rf
 
