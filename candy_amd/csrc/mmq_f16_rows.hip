@@ -7,9 +7,9 @@
 // Here nobody waits for anybody: a workgroup owns 16, 32 or 48 weight rows and all activation rows, and each of its eight
 // wavefronts takes every eighth super-block of K: weight blocks by direct loads into its own slice of LDS, dequantized into
 // matrix operands in registers, activation fragments straight from their image, each loaded by one wavefront of the
-// workgroup.  The wavefronts' sums meet in LDS at the end, in the order of the wavefronts (reproducible).  Kernel us, 77
-// rows, 11008 x 4096, before (with the split sum) -> now: Q4_K 22.8 + 4.5 -> 20.6, Q8_0 35.1 + 4.5 -> 24.0, Q4_0 33.4 + 4.5 ->
-// 21.2, Q5_K 31.5 + 4.5 -> 25.1; 2048 x 1024 Q8_0 13.0 + 4.1 -> 5.7.
+// workgroup.  The wavefronts' sums meet in LDS at the end, in the order of the wavefronts (reproducible).  us of a call, 77
+// rows, 11008 x 4096, tiles -> here: Q4_K 28.1 -> 18.7, Q5_K 35.6 -> 19.1, Q6_K 31.4 -> 21.7, Q8_0 40.0 -> 22.7, Q4_0 38.2 -> 18.2; 2048 x
+// 1024 Q8_0, the kernels with the split sum 17.1 -> 5.7.
 // A step's second half of activations is requested in front of its dequantization, and held there: left alone the compiler
 // dequantizes several steps in advance and requests the activations behind that, where nothing hides them.  A wavefront's loads are
 // the same in number at every step, with weights to fetch or not (request()).  us of a call, without / with both: 11008 x 4096, 77

@@ -16,9 +16,10 @@
 // The distance from 64 bits is smaller than with 16 columns for every format (Q6_K 8.6e-8 -> 8.2e-8, Q4_K 2.2e-7 -> 1.7e-7).
 //
 // What bounds it: up to 16 rows two launches and their first bytes, then the vector ALU (without any weights or activations fetched
-// the Q6_K call of 6 rows took 13.8 of its 16.3 us) beside the weights at 3.5 to 4.5 TB/s; from about 48 rows the vector ALU alone (a
-// conversion, a product and an fma per result and sub-block).  us of a call, before (int8 tiles, mostly with a split of K) -> now:
-//   4096 x 14336, 6 rows   Q4_K 18.1 -> 11.4, Q5_K 17.9 -> 12.8, Q6_K 21.0 -> 16.3, Q8_0 24.4 -> 17.3, Q4_0 22.4 -> 14.2
+// the Q6_K call of 6 rows took 13.8 of the 16.3 us it took with 16 columns) beside the weights at 3.5 to 4.5 TB/s; from about 48 rows
+// the vector ALU alone (a conversion, a product and an fma per result and sub-block).  us of a call, before (int8 tiles, mostly with a
+// split of K) -> now:
+//   4096 x 14336, 6 rows   Q4_K 18.1 -> 10.6, Q5_K 17.9 -> 12.4, Q6_K 21.0 -> 14.4, Q8_0 24.4 -> 16.8, Q4_0 22.4 -> 13.5
 //   11008 x 4096, 32 rows  Q4_K 15.7 -> 14.0, Q5_K 27.7 -> 14.7, Q6_K 31.6 -> 22.0, Q8_0 41.6 -> 18.0, Q4_0 38.1 -> 14.9
 //   11008 x 4096, 64 rows  Q5_K 35.0 -> 20.7, Q8_0 44.6 -> 24.2, Q4_0 37.9 -> 23.4
 // and prompts of the quantized decoder (four layers and the head): 8B shape 16 / 48 / 160 tokens 603 / 885 / 1861 -> 419 / 617 /
