@@ -764,18 +764,21 @@ bool mmq_f16_big_covers(const candy_hip_qtensor *w, int64_t m, int min_m) {
 // dequantization is the cheapest, also takes the narrower tiles on some grids above 128 rows (with the heavier formats
 // the producers then set the pace: Q6_K 14336 x 4096 at 192 rows 58.3 us on 128 x 128 tiles against 53.8, Q8_0 68.5
 // against 58.6), and tiles of 112 weight rows.
-template <class F>
-static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, const _Float16 *xh, int64_t m) {
+struct F16Tile {
+    int bn, bm;  // weight rows, activation rows
+};
+static F16Tile pick_tile(const candy_hip_device *dev, bool q4k, const int64_t *rows, int count, int64_t cols, int64_t m) {
     const int shape = dev->opt.f16_shape;  // comparison runs
     const bool single = shape == 3;        // every wavefront in both roles
+    const int n_sb = (int)(cols >> 8);
     // What the busiest CU does: rounds of workgroups x weight rows per tile x super-blocks per workgroup, x 8 (a step of 192
     // activation rows: 7, of 256: 8; measured 0.84 to 0.88, the producers' share being the same).  0: not for these rows.
     auto cost = [&](int bn, int bm) -> int64_t {
-        const int n_sb = (int)(jobs[0].w->cols >> 8), m_tiles = (int)((m + bm - 1) / bm);
+        const int m_tiles = (int)((m + bm - 1) / bm);
         int64_t tiles = 0;
         for (int s = 0; s < count; ++s) {
-            if (bn == 112 && jobs[s].w->rows % 112 != 0) return 0;
-            tiles += (jobs[s].w->rows + bn - 1) / bn;
+            if (bn == 112 && rows[s] % 112 != 0) return 0;
+            tiles += (rows[s] + bn - 1) / bn;
         }
         const int ns = plan_split(dev, (int)(tiles * m_tiles), n_sb), sb_per = (n_sb + ns - 1) / ns;
         const int64_t wgs = tiles * m_tiles * ((n_sb + sb_per - 1) / sb_per);
@@ -785,36 +788,31 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     // busiest CU (14336 rows: 128 tiles instead of 112, so 256 instead of 224 workgroups at 512 activation rows, 512
     // instead of 448 for a gate / up pair).
     auto narrow = [&](int bm) {
-        if (!std::is_same<F, BigQ4K>::value || single || shape == 4) return false;
+        if (!q4k || single || shape == 4) return false;
         const int64_t c112 = cost(112, bm);
         return c112 > 0 && c112 < cost(128, bm);
     };
-    auto small_tiles = [&]() {
-        if (single) return launch_big<F, 128, 128, 2, 4>(dev, jobs, count, xh, m);
-        if constexpr (std::is_same<F, BigQ4K>::value)
-            if (narrow(128)) return launch_big<F, 112, 128, 2, 4, true>(dev, jobs, count, xh, m);
-        return launch_big<F, 128, 128, 2, 4, true>(dev, jobs, count, xh, m);
-    };
+    auto tile = [&](int bm) { return F16Tile{narrow(bm) ? 112 : 128, bm}; };
     // up to 128 activation rows: 128 x 128 tiles, K split over workgroups to fill the chip
-    if (shape == 2 || m <= 128) return small_tiles();
-    constexpr bool q4k = std::is_same<F, BigQ4K>::value;
+    if (shape == 2 || m <= 128) return tile(128);
     // up to 256 rows where the 128 x 128 tiles fill the chip and the 128 x 256 tiles would have to split K
     // (Q4_K 14336 x 4096 at 256 rows: 70.7 us against 80.3)
     int64_t n128 = 0;
-    for (int s = 0; s < count; ++s) n128 += (jobs[s].w->rows + 127) / 128;
+    for (int s = 0; s < count; ++s) n128 += (rows[s] + 127) / 128;
     const int64_t fill = (3 * (int64_t)dev->num_cus) / 4;
-    if (q4k && m <= 256 && n128 * ((m + 127) / 128) >= fill && n128 * ((m + 255) / 256) < fill) return small_tiles();
+    if (q4k && m <= 256 && n128 * ((m + 127) / 128) >= fill && n128 * ((m + 255) / 256) < fill) return tile(128);
     // short K (at most 16 super-blocks) on a grid that 128 x 256 tiles would have to split: 128 x 128 tiles halve the
     // split as long as they still fit one round (Q4_K 4096 x 4096 at 512 rows 35.5 against 36.8 us, at 1024 rows 50.9
     // against 54.2; 6144 x 4096 at 512 rows 44.8 against 47.1; with K = 14336 the split is cheap and the wider tile wins)
-    // Not where the launch behind sums the copies anyway (the decoder's prompts: the norm, the rotation) and two are all that the
-    // wide tiles leave: us of an 8B-shaped prompt (four layers and the head), narrow / wide tiles for q / k / v: 300 tokens 1170 / 1131,
-    // 512 1368 / 1349, 700 1878 / 1834; for o, 1B shape, 1500 tokens 1426 / 1404, 7B 600 1664 / 1624.  (With four copies level: 8B
-    // 512 tokens, o as well 1360, 256 tokens 894 / 915.)
-    const bool cheap = dev->defer_split && plan_split(dev, (int)(n128 * ((m + 255) / 256)), (int)(jobs[0].w->cols >> 8)) <= 2;
-    if (q4k && !cheap && shape == 0 && jobs[0].w->cols <= 4096 && n128 * ((m + 255) / 256) < fill && n128 * ((m + 127) / 128) <= dev->num_cus)
-        return small_tiles();
-    if (single) return launch_big<F, 128, 256, 2, 4>(dev, jobs, count, xh, m);
+    // Not where the launch behind sums the copies anyway (the decoder's prompts: the norm, the rotation) and the wide tiles leave it
+    // two: us of a prompt (four layers and the head), narrow / wide tiles: q / k / v of the 8B shape 300 tokens 1179 / 1143, 512 1381 /
+    // 1366; o 700 tokens 1891 / 1852, 1B shape 1300 tokens 1327 / 1303, 7B 600 1700 / 1658.  (With four copies level: 8B 512 tokens, o as well
+    // 1360, 256 tokens 894 / 915.)  Where the wide tiles are not split either there is nothing to sum, and the fuller round of narrow ones
+    // is ahead: q / k / v of the 8B shape, 240 workgroups of 256, 520 tokens narrow / wide 1608 / 1621, 640 1815 / 1836.
+    const bool cheap = dev->defer_split && plan_split(dev, (int)(n128 * ((m + 255) / 256)), n_sb) == 2;
+    if (q4k && !cheap && shape == 0 && cols <= 4096 && n128 * ((m + 255) / 256) < fill && n128 * ((m + 127) / 128) <= dev->num_cus)
+        return tile(128);
+    if (single) return F16Tile{128, 256};
     // A grid of 128 x 256 tiles that fills the chip, where the 128 x 128 tiles take no more rounds of workgroups: the
     // wide grid's last round is then at most a third full and its last column of tiles half empty, and a round of the
     // narrower tiles is the shorter one (about 0.7).  us on 128 x 256 / 128 x 128 tiles, two rounds either way: 11008 x
@@ -823,7 +821,7 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     // 80 / 64, 77 / 65; 9300 x 1024 at 890 rows 40 / 34, 45 / 41, 45 / 40, 52 / 44, 49 / 43.  Where it costs a round
     // more the wider tiles win: 32000 x 4096 at 300 rows, two against three, Q5_K and Q4_0 0.86x on the narrow ones.
     auto rounds = [&](int bm) { return (n128 * ((m + bm - 1) / bm) + dev->num_cus - 1) / dev->num_cus; };
-    if (shape == 0 && !narrow(256) && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256)) return small_tiles();
+    if (shape == 0 && !narrow(256) && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256)) return tile(128);
     // Tiles of 192 activation rows where they leave the busiest CU less to do: a last column of tiles that would be mostly
     // empty (300 rows are 2 x 192 as they are 2 x 256), or a grid that fills the rounds better (1300 rows against 4096
     // weight rows: 224 workgroups instead of 192).  Over thirteen weight shapes and seventeen row counts from 140 to 2048,
@@ -831,11 +829,24 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     // with them: Q4_K 14336 x 4096 at 300 rows 60.6 / 51.0, 4096 x 14336 at 560 rows 101 / 87.5; Q5_K 32000 x 4096 at 560
     // rows 199 / 179; Q8_0 11008 x 4096 at 300 rows 77 / 70; Q6_K 4096 x 4096 at 1300 rows 69.9 / 63.4.
     const bool rows192 = shape == 0 && (narrow(192) ? cost(112, 192) : cost(128, 192)) < (narrow(256) ? cost(112, 256) : cost(128, 256));
-    if constexpr (std::is_same<F, BigQ4K>::value) {
-        if (rows192 && narrow(192)) return launch_big<F, 112, 192, 2, 4, true>(dev, jobs, count, xh, m);
-        if (!rows192 && narrow(256)) return launch_big<F, 112, 256, 2, 4, true>(dev, jobs, count, xh, m);
+    return tile(rows192 ? 192 : 256);
+}
+
+template <class F>
+static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, const _Float16 *xh, int64_t m) {
+    constexpr bool q4k = std::is_same<F, BigQ4K>::value;
+    int64_t rows[3];
+    for (int s = 0; s < count; ++s) rows[s] = jobs[s].w->rows;
+    const F16Tile t = pick_tile(dev, q4k, rows, count, jobs[0].w->cols, m);
+    if (dev->opt.f16_shape == 3)
+        return t.bm == 128 ? launch_big<F, 128, 128, 2, 4>(dev, jobs, count, xh, m) : launch_big<F, 128, 256, 2, 4>(dev, jobs, count, xh, m);
+    if constexpr (q4k) {
+        if (t.bn == 112 && t.bm == 128) return launch_big<F, 112, 128, 2, 4, true>(dev, jobs, count, xh, m);
+        if (t.bn == 112 && t.bm == 192) return launch_big<F, 112, 192, 2, 4, true>(dev, jobs, count, xh, m);
+        if (t.bn == 112) return launch_big<F, 112, 256, 2, 4, true>(dev, jobs, count, xh, m);
     }
-    if (rows192) return launch_big<F, 128, 192, 2, 4, true>(dev, jobs, count, xh, m);
+    if (t.bm == 128) return launch_big<F, 128, 128, 2, 4, true>(dev, jobs, count, xh, m);
+    if (t.bm == 192) return launch_big<F, 128, 192, 2, 4, true>(dev, jobs, count, xh, m);
     return launch_big<F, 128, 256, 2, 4, true>(dev, jobs, count, xh, m);
 }
 
@@ -930,3 +941,13 @@ int launch_mmq_f16_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, co
 }
 
 }  // namespace candy
+
+// The rule above, for its tests (no device needed): weight rows * 1000 + activation rows of a tile.
+extern "C" int candy_test_f16_tile(int q4k, const int64_t *rows, int count, int64_t cols, int64_t m, int num_cus, int deferred) {
+    candy_hip_device dev;
+    candy::SplitPending pend;
+    dev.num_cus = num_cus;
+    if (deferred) dev.defer_split = &pend;
+    const candy::F16Tile t = candy::pick_tile(&dev, q4k != 0, rows, count, cols, m);
+    return t.bn * 1000 + t.bm;
+}
