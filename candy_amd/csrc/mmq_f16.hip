@@ -292,6 +292,11 @@ template <class F>
 constexpr bool f16_staged() { return std::is_same<F, BigQ8_0>::value; }
 template <class F>
 constexpr int f16_slice_loads() { return (32 * F::BLOCK / 16 + 63) / 64; }  // of 1 KB, for a producer's 32 rows
+// A staged piece is found by a 32-bit offset from the tile's first row: the tile's rows within 4 GB (128 rows of Q8_0: 31.5 million
+// values each).  Longer ones take the tiles whose lanes load their own runs, through pointers.
+static bool f16_roles_fit(int fmt, int64_t tile_rows, int64_t cols) {
+    return fmt != CANDY_HIP_Q8_0 || tile_rows * (cols / 256 * BigQ8_0::BLOCK) <= 0xFFFFFFFFll;
+}
 
 template <class F, int BN, int BM, int EPI>
 __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _Float16 *__restrict__ xh, int M, int K,
@@ -765,11 +770,13 @@ bool mmq_f16_big_covers(const candy_hip_qtensor *w, int64_t m, int min_m) {
 // the producers then set the pace: Q6_K 14336 x 4096 at 192 rows 58.3 us on 128 x 128 tiles against 53.8, Q8_0 68.5
 // against 58.6), and tiles of 112 weight rows.
 struct F16Tile {
-    int bn, bm;  // weight rows, activation rows
+    int bn, bm;   // weight rows, activation rows
+    bool single;  // every wavefront in both roles
 };
-static F16Tile pick_tile(const candy_hip_device *dev, bool q4k, const int64_t *rows, int count, int64_t cols, int64_t m) {
+static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *rows, int count, int64_t cols, int64_t m) {
+    const bool q4k = fmt == CANDY_HIP_Q4_K;
     const int shape = dev->opt.f16_shape;  // comparison runs
-    const bool single = shape == 3;        // every wavefront in both roles
+    const bool single = shape == 3 || !f16_roles_fit(fmt, std::min<int64_t>(128, *std::max_element(rows, rows + count)), cols);
     const int n_sb = (int)(cols >> 8);
     // What the busiest CU does: rounds of workgroups x weight rows per tile x super-blocks per workgroup, x 8 (a step of 192
     // activation rows: 7, of 256: 8; measured 0.84 to 0.88, the producers' share being the same).  0: not for these rows.
@@ -792,7 +799,7 @@ static F16Tile pick_tile(const candy_hip_device *dev, bool q4k, const int64_t *r
         const int64_t c112 = cost(112, bm);
         return c112 > 0 && c112 < cost(128, bm);
     };
-    auto tile = [&](int bm) { return F16Tile{narrow(bm) ? 112 : 128, bm}; };
+    auto tile = [&](int bm) { return F16Tile{narrow(bm) ? 112 : 128, bm, single}; };
     // up to 128 activation rows: 128 x 128 tiles, K split over workgroups to fill the chip
     if (shape == 2 || m <= 128) return tile(128);
     // up to 256 rows where the 128 x 128 tiles fill the chip and the 128 x 256 tiles would have to split K
@@ -812,7 +819,7 @@ static F16Tile pick_tile(const candy_hip_device *dev, bool q4k, const int64_t *r
     const bool cheap = dev->defer_split && plan_split(dev, (int)(n128 * ((m + 255) / 256)), n_sb) == 2;
     if (q4k && !cheap && shape == 0 && cols <= 4096 && n128 * ((m + 255) / 256) < fill && n128 * ((m + 127) / 128) <= dev->num_cus)
         return tile(128);
-    if (single) return F16Tile{128, 256};
+    if (single) return F16Tile{128, 256, true};
     // A grid of 128 x 256 tiles that fills the chip, where the 128 x 128 tiles take no more rounds of workgroups: the
     // wide grid's last round is then at most a third full and its last column of tiles half empty, and a round of the
     // narrower tiles is the shorter one (about 0.7).  us on 128 x 256 / 128 x 128 tiles, two rounds either way: 11008 x
@@ -837,8 +844,8 @@ static int launch_shapes(candy_hip_device *dev, const F16Job *jobs, int count, c
     constexpr bool q4k = std::is_same<F, BigQ4K>::value;
     int64_t rows[3];
     for (int s = 0; s < count; ++s) rows[s] = jobs[s].w->rows;
-    const F16Tile t = pick_tile(dev, q4k, rows, count, jobs[0].w->cols, m);
-    if (dev->opt.f16_shape == 3)
+    const F16Tile t = pick_tile(dev, jobs[0].w->fmt, rows, count, jobs[0].w->cols, m);
+    if (t.single)
         return t.bm == 128 ? launch_big<F, 128, 128, 2, 4>(dev, jobs, count, xh, m) : launch_big<F, 128, 256, 2, 4>(dev, jobs, count, xh, m);
     if constexpr (q4k) {
         if (t.bn == 112 && t.bm == 128) return launch_big<F, 112, 128, 2, 4, true>(dev, jobs, count, xh, m);
@@ -899,7 +906,7 @@ bool mmq_f16_silu_covers(const candy_hip_qtensor *gate, const candy_hip_qtensor 
     const candy_hip_qtensor *const ws[2] = {gate, up};
     const Options &opt = gate->dev->opt;
     return opt.prefill_fold_silu && opt.f16_shape == 0 && opt.f16_split == 0 && m > 128 && gate->rows == up->rows && gate->rows % 64 == 0 &&
-           mmq_f16_group_covers(ws, 2, m) && silu_fills(gate->dev, gate->rows, m);
+           mmq_f16_group_covers(ws, 2, m) && silu_fills(gate->dev, gate->rows, m) && f16_roles_fit(gate->fmt, 64, gate->cols);
 }
 
 template <class F, int BM>
@@ -942,12 +949,20 @@ int launch_mmq_f16_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, co
 
 }  // namespace candy
 
-// The rule above, for its tests (no device needed): weight rows * 1000 + activation rows of a tile.
-extern "C" int candy_test_f16_tile(int q4k, const int64_t *rows, int count, int64_t cols, int64_t m, int num_cus, int deferred) {
+// The rules above, for their tests (no device needed): weight rows * 1000 + activation rows of a tile, negative where every wavefront has
+// both roles; whether gate and up of a prompt share tiles with SiLU.
+extern "C" int candy_test_f16_tile(int fmt, const int64_t *rows, int count, int64_t cols, int64_t m, int num_cus, int deferred) {
     candy_hip_device dev;
     candy::SplitPending pend;
     dev.num_cus = num_cus;
     if (deferred) dev.defer_split = &pend;
-    const candy::F16Tile t = candy::pick_tile(&dev, q4k != 0, rows, count, cols, m);
-    return t.bn * 1000 + t.bm;
+    const candy::F16Tile t = candy::pick_tile(&dev, fmt, rows, count, cols, m);
+    return (t.single ? -1 : 1) * (t.bn * 1000 + t.bm);
+}
+extern "C" int candy_test_f16_silu(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
+    candy_hip_device dev;
+    dev.num_cus = num_cus;
+    candy_hip_qtensor w;
+    w.dev = &dev; w.fmt = fmt; w.rows = rows; w.cols = cols;
+    return candy::mmq_f16_silu_covers(&w, &w, m);
 }

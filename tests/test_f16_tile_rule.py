@@ -1,19 +1,24 @@
 """Which tile a contraction on the fp16 tiles takes, on the CPU: the rule for Q4_K rows of up to 16 super-blocks, whose narrow tiles
-spare a split of K, and where a prompt leaves them because the launch behind sums the two copies."""
+spare a split of K, and where a prompt leaves them because the launch behind sums the two copies; and rows that are too long for the
+role-split tiles' offsets."""
 import ctypes
 
 import numpy as np
 import pytest
 
-from candy_amd import hip
+from candy_amd import hip, synth
 
 LIB = ctypes.CDLL(hip.LIB_PATH)
 
 
+def code(fmt, rows, cols, m, deferred, cus):
+    n = len(rows)
+    return LIB.candy_test_f16_tile(fmt, (ctypes.c_int64 * n)(*rows), n, ctypes.c_int64(cols), ctypes.c_int64(m), cus, int(deferred))
+
+
 def tile(rows, cols, m, deferred, cus=256, q4k=True):
     """(weight rows, activation rows)."""
-    n = len(rows)
-    return divmod(LIB.candy_test_f16_tile(int(q4k), (ctypes.c_int64 * n)(*rows), n, ctypes.c_int64(cols), ctypes.c_int64(m), cus, int(deferred)), 1000)
+    return divmod(code(synth.Q4_K if q4k else synth.Q8_0, rows, cols, m, deferred, cus), 1000)
 
 
 def wide_split(rows, cols, m, cus=256):
@@ -55,3 +60,24 @@ def test_nothing_but_two_copies_moves_a_call():
             assert q4k and cols <= 4096 and m > 128 and alone[1] == 128 and wide_split(rows, cols, m, cus) == 2
         assert q4k or alone[0] == 128
     assert moved > 100
+
+
+@pytest.mark.parametrize("m", [65, 128, 129, 300])
+def test_rows_of_q8_0_past_32_bit_offsets(m):
+    # 128 rows of 17 bytes to 16 values: the last one ends at 2^32 - 1 at the most
+    last = (2 ** 32 - 1) // (128 * 272) * 256
+    for rows, longest in (((4096,), last), ((200, 128), last), ((127,), (2 ** 32 - 1) // (127 * 272) * 256), ((1,), 2 ** 31 - 256)):
+        assert code(synth.Q8_0, rows, longest, m, False, 256) > 0
+        if longest < 2 ** 31 - 256:
+            assert code(synth.Q8_0, rows, longest + 256, m, False, 256) in (-128128, -128256)
+    for fmt in (synth.Q4_K, synth.Q5_K, synth.Q6_K, synth.Q4_0, synth.Q4_0_GGML):  # through pointers
+        assert code(fmt, (4096,), 2 ** 31 - 256, m, False, 256) > 0
+
+
+def test_gate_and_up_of_q8_0_past_32_bit_offsets():
+    # 64 rows of each
+    def covers(fmt, cols):
+        return LIB.candy_test_f16_silu(fmt, ctypes.c_int64(12288), ctypes.c_int64(cols), ctypes.c_int64(300), 256)
+
+    last = (2 ** 32 - 1) // (64 * 272) * 256
+    assert covers(synth.Q8_0, 4096) and covers(synth.Q8_0, last) and not covers(synth.Q8_0, last + 256) and covers(synth.Q4_K, last + 256)
