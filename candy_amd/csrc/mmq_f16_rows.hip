@@ -129,6 +129,7 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
             request(sb + 8, k + 1 < count);
             contract(sb, k + 1 < count ? sb + 8 : sb);
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last request writes its slice, which the sums are about to take
     }
     __syncthreads();  // the slices are consumed
 #pragma unroll
