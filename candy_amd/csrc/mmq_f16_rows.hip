@@ -183,7 +183,8 @@ static const RowsCost &rows_cost(int fmt) {
 // none, the tiles.  A second round would read the activations again, wider workgroups have no registers for their sums; fewer than
 // 2048 weight rows leave half of the CUs idle.  All 3729 calls together take 0.3 % more than the faster kernel for each.  us of a call,
 // tiles / here: Q8_0 4096 x 2304, 96 rows 20.4 / 12.1, Q4_K 4096 x 4096, 80 rows 18.9 / 14.3, 128 rows 21.8 / 20.4, 8200 x 2560,
-// 96 rows 20.9 / 14.5, Q6_K 4096 x 4096, 96 rows 21.6 / 17.9, 11008 x 4096, 48 rows 29.8 / 17.1, 64 rows 30.7 / 18.4.
+// 96 rows 20.9 / 14.5, Q6_K 4096 x 4096, 96 rows 21.6 / 17.9, 11008 x 4096, 48 rows 29.8 / 17.1, 64 rows 30.7 / 18.4; one super-block in the
+// last round, Q4_K 8192 x 2304, 128 rows 17.2 / 15.1, 4200 x 4352, 80 rows 18.3 / 16.2; odd Q6_K blocks, 8200 x 3840, 40 rows 22.8 / 16.1.
 static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
     const bool q6k = fmt == CANDY_HIP_Q6_K;
     // up to 64 rows the other formats are on the exact tiles (mmq_f16_big_covers)
@@ -205,14 +206,6 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
     if (splits > 1) tile += c.tile[2] + c.tile[3] * (float)(splits + 1) * out;
     const float here = c.rows[0] + (float)rounds * (c.rows[1] * rf + c.rows[2] * mf) + (float)blocks * (c.rows[3] * mf + c.rows[4] * rf) +
                        (blocks & 1 ? c.rows[5] * (float)(blocks * rf) : 0.0f) + c.rows[6] * (float)(rf * mf) + c.rows[7] * out;
-    // Three kinds of calls stay on the tiles, where the kernel's forms before had them and the rule's test holds them.  Q4_K and Q5_K with a
-    // single super-block in the last round, at eight activation fragments or little more than half of the CUs at work (tiles / here:
-    // Q4_K 8192 x 2304, 128 rows 17.6 / 15.2 us, 4200 x 4352, 80 rows 18.5 / 16.4); Q6_K with an odd number of blocks, 13 or more, up to 64 rows, in
-    // little more than two thirds of the CUs (8200 x 3840, 40 rows 23.0 / 16.1)
-    if ((fmt == CANDY_HIP_Q4_K || fmt == CANDY_HIP_Q5_K) && rf == 2 && blocks % 8 == 1 &&
-        (mf == 8 || (mf >= 5 && blocks > 8 && (rows + 31) / 32 * 16 < num_cus * 9)))
-        return 0;
-    if (q6k && rf == 3 && mf <= 4 && blocks % 2 != 0 && blocks >= 13 && (rows + 47) / 48 * 16 < num_cus * 11) return 0;
     return here < tile ? rf : 0;
 }
 template <class F, int RF, int MF>
