@@ -166,7 +166,8 @@ int splitk_workspace(candy_hip_device *dev, size_t bytes, void **out);
 // mmq_f16.hip: y[i] = (res[i] +) part[0][i] + part[1][i] + ... in that order (count floats per part)
 int launch_splitk_sum(candy_hip_device *dev, const float *part, float *y, const float *res, size_t count, int n_split,
                       size_t stride = 0);  // copies `stride` floats apart (0: count)
-// ops.hip: the pending sum, the residual add, RMSNorm and Q8_0 quantization of the rows in one launch
+// ops.hip: the pending sum, the residual add, RMSNorm and Q8_0 quantization of the rows in one launch, rows held in registers
+constexpr int64_t SPLIT_NORM_COLS = 8192;
 int launch_split_rms_norm_quant(candy_hip_device *dev, const SplitPending &sp, const float *alpha, float eps, int64_t rows,
                                 int64_t cols, int8_t *qs, Q8Scale *scales, _Float16 *xh);
 // Formats the batch-1 kernel contracts (residual epilogue, several weights per launch): all that have a vec-dot.

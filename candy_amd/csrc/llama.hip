@@ -353,6 +353,13 @@ int candy_hip_llama::reserve_prompt(int n) {
     return rc;
 }
 
+// Whether the launch behind a layer's o or down projection is a norm that sums the projection's partial copies: its rows fit the
+// registers, and there is a launch (the last layer's down projection has none over all rows).  Elsewhere the projection is launched as any call
+// that sums its copies itself, tiles included.
+static bool norm_sums_behind(const candy_hip_llama_config &c, int layer, bool down) {
+    return c.d_model <= SPLIT_NORM_COLS && !(down && layer == c.n_layers - 1);
+}
+
 // The prompt pass: the decode step's sequence with n rows per activation. Linears go through the
 // batched contraction (MFMA tiles from 16 rows up) and attention is causal over the cache.
 int candy_hip_llama::enqueue_prompt(int n, int pos0) {
@@ -432,9 +439,9 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
         // fp16 expansion (one conversion for q/k/v, one for gate/up), and the residual add rides in the
         // projection's epilogue.
         auto xh_for = [&](const candy_hip_qtensor *w) { return mmq_f16_big_covers(w, n) ? P.xh : nullptr; };
-        auto add_linear = [&](const candy_hip_qtensor *w, const _Float16 *image = nullptr) -> int {  // P.h += (quantized activations) . w^T
+        auto add_linear = [&](const candy_hip_qtensor *w, bool down, const _Float16 *image = nullptr) -> int {  // P.h += (quantized activations) . w^T
             if (mmq_fuses_residual(w, n)) {
-                dev->defer_split = &pend;
+                if (norm_sums_behind(c, l, down)) dev->defer_split = &pend;
                 const int e = launch_contract(dev, w, P.xq, P.xs, n, P.h, image ? image : xh_for(w), P.h);
                 dev->defer_split = nullptr;
                 return e;
@@ -465,14 +472,14 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
                                       cache_stride, scale, att_xh)))
             return rc;
         if (!att_xh && (rc = launch_quantize_q8(dev, P.att, n, qd, P.xq, P.xs, nullptr, xh_for(L.wo)))) return rc;
-        if ((rc = add_linear(L.wo))) return rc;  // h += Wo . att
+        if ((rc = add_linear(L.wo, false))) return rc;  // h += Wo . att
         xh = (xh_for(L.gate) || xh_for(L.up)) ? P.xh : nullptr;
         if ((rc = norm_quant(L.ffn_norm, xh))) return rc;
         if (xh && mmq_fuses_residual(L.down, n) && mmq_f16_silu_covers(L.gate, L.up, n)) {
             // mmq_m_pad(n) rows of 2-byte values fit in gate's n > 128 rows of 4-byte ones
             _Float16 *act = (_Float16 *)P.gate;
             if ((rc = launch_mmq_f16_silu(dev, L.gate, L.up, xh, n, act))) return rc;
-            if ((rc = add_linear(L.down, act))) return rc;
+            if ((rc = add_linear(L.down, true, act))) return rc;
             continue;
         }
         const candy_hip_qtensor *gu_w[2] = {L.gate, L.up};
@@ -485,11 +492,8 @@ int candy_hip_llama::enqueue_prompt(int n, int pos0) {
         }
         if ((rc = launch_silu_mul_quant(dev, P.gate, P.up, n, c.d_ffn, nullptr, P.xq, P.xs, xh_for(L.down))))
             return rc;
-        if ((rc = add_linear(L.down))) return rc;  // h += Wdown . act
+        if ((rc = add_linear(L.down, true))) return rc;  // h += Wdown . act
     }
-    if (pend.n_split > 0 &&
-        (rc = launch_splitk_sum(dev, pend.part, pend.y, pend.res, pend.count, pend.n_split, pend.stride)))
-        return rc;
     return CANDY_HIP_OK;
 }
 
@@ -512,6 +516,14 @@ int candy_hip_llama_decode(candy_hip_llama *m, int32_t token, int32_t pos, const
 
 int candy_hip_llama_generate(candy_hip_llama *m, int32_t token, int32_t pos, int32_t n_steps, int32_t *tokens) {
     return candy_hip_decoder_generate(m, token, pos, n_steps, tokens);
+}
+
+// The rule of a prompt's deferred sums, for its test (no device needed).
+int candy_test_norm_sums_behind(int d_model, int n_layers, int layer, int down) {
+    candy_hip_llama_config c{};
+    c.d_model = d_model;
+    c.n_layers = n_layers;
+    return norm_sums_behind(c, layer, down != 0);
 }
 
 }  // extern "C"

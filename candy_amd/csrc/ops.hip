@@ -540,13 +540,14 @@ int launch_rms_norm_quant(candy_hip_device *dev, const float *x, const float *al
 }
 
 // RMSNorm + quantization of rows that a split contraction has left as partial copies (SplitPending, filled by the
-// fp16 tile launcher while dev->defer_split points at it): the sum, the residual add and the norm in one launch for
-// rows of up to 8192 values, the separate split sum first for longer ones.
+// fp16 tile launcher while dev->defer_split points at it): the sum, the residual add and the norm in one launch, for
+// rows of up to SPLIT_NORM_COLS values.
 int launch_split_rms_norm_quant(candy_hip_device *dev, const SplitPending &sp, const float *alpha, float eps, int64_t rows,
                                 int64_t cols, int8_t *qs, Q8Scale *scales, _Float16 *xh) {
     CANDY_REQUIRE(cols % 32 == 0 && cols > 0 && rows > 0 && cols <= 0x7FFFFFFF, "rms_norm_quant needs cols %% 32 == 0");
     CANDY_REQUIRE(sp.count == (size_t)rows * (size_t)cols && sp.n_split > 0, "internal: pending split sum of another shape");
-    if (cols > 8192 || !dev->opt.prefill_fold_split_sums) {
+    CANDY_REQUIRE(cols <= SPLIT_NORM_COLS, "internal: pending split sum of rows too long for the norm");
+    if (!dev->opt.prefill_fold_split_sums) {  // comparison runs
         if (int rc = launch_splitk_sum(dev, sp.part, sp.y, sp.res, sp.count, sp.n_split, sp.stride)) return rc;
         return launch_rms_norm_quant(dev, sp.y, alpha, eps, rows, cols, nullptr, qs, scales, xh);
     }

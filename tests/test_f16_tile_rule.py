@@ -81,3 +81,14 @@ def test_gate_and_up_of_q8_0_past_32_bit_offsets():
 
     last = (2 ** 32 - 1) // (64 * 272) * 256
     assert covers(synth.Q8_0, 4096) and covers(synth.Q8_0, last) and not covers(synth.Q8_0, last + 256) and covers(synth.Q4_K, last + 256)
+
+
+def test_where_the_norm_behind_sums_the_copies():
+    # rows that its registers hold, and not behind the last layer's down projection, which no norm of all rows follows: a projection that
+    # sums its own copies is no reason for the wide tiles
+    behind = LIB.candy_test_norm_sums_behind
+    for d_model in (256, 4096, 8192):
+        assert all(bool(behind(d_model, 3, layer, down)) == ((layer, down) != (2, 1)) for layer in range(3) for down in (0, 1))
+    for d_model in (8448, 11264):
+        assert not any(behind(d_model, 3, layer, down) for layer in range(3) for down in (0, 1))
+    assert tile((11264,), 1024, 200, False) == (128, 128) and tile((11264,), 1024, 200, True) != (128, 128)
