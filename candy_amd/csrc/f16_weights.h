@@ -174,8 +174,8 @@ struct BigQ5K {
 };
 
 // Q8_0: a "super-block" is eight 34-byte blocks (272 bytes); step g holds blocks 2g and 2g + 1, the task's quarter c
-// the 16 quants of half a block and that block's scale.  d * q is exact in f32 (DequantizeBlockQ8_0F32,
-// quantized.go:131-136), one rounding to fp16.
+// the 16 quants of half a block and that block's scale.  d * q (DequantizeBlockQ8_0F32, quantized.go:131-136) as one packed fp16
+// product: of two fp16 numbers, so that what is rounded, once, is the exact product.
 struct BigQ8_0 {
     static constexpr bool RUN16 = true;
     static constexpr int BLOCK = 272;
@@ -213,7 +213,7 @@ struct BigQ8_0 {
 
 // Q4_0: eight 18-byte blocks per "super-block" (144 bytes).  The task's 16 values of block 2g + c/2 are the two
 // nibbles of 8 consecutive bytes in candy's element order (quantized.go:85-93) or one nibble of all 16 bytes in
-// ggml's.  d * (q - 8) is exact in f32, one rounding to fp16.
+// ggml's.  d * (q - 8) as for Q8_0: one packed fp16 product, the exact product rounded once.
 template <bool GGML>
 struct BigQ4_0 {
     static constexpr bool RUN16 = true;

@@ -498,7 +498,7 @@ __global__ __launch_bounds__(64 * QH * KG, KVP * KG * HD * 256 > 81920 && QH * K
     // The two key groups share the end as well: group 0 takes the first 16 queries of each 32, group 1 the others; what the other
     // group needs goes through LDS, value k of thread t of group kg at (2 k + kg) * 64 QH + t.  With one group merging, dividing
     // and quantizing both halves, level by level, what is not the walk along the keys was 17 of 31 us at 512 tokens.  Kernel us, so / now:
-    // head_dim 128, 512 tokens 31.5 / 27.4, fp16 cache 24.8 / 19.9, 2000 tokens 129 / 119; head_dim 64, 1500 tokens 78 / 73.
+    // head_dim 128, 512 tokens 31.5 / 27.4, fp16 cache 24.8 / 19.9, 2000 tokens 129 / 119 (113 to 124 from run to run); head_dim 64, 1500 tokens 78 / 73.
     constexpr int NT = KG == 2 ? 1 : 2;  // 16 queries each
     const int t_own = KG == 2 ? kg : 0;
     if constexpr (KG == 2) {
