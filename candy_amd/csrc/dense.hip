@@ -38,22 +38,34 @@ __device__ __forceinline__ float epilogue(float z, const EpiArgs &e) {
 }
 
 // ------------------------------------------------------------------ one row
-// The norms in front of the contraction (launch_norm_chain's arithmetic), for a kernel that runs them in its prologue.
+// The norms in front of the contraction (launch_norm_chain's arithmetic), for a kernel that runs them in its prologue.  What its
+// first loads need are plain arguments of the kernel (they arrive in registers with the wavefront); this is the rest.  Biases, if
+// any, lie behind their weights (MvNorms::bias).
 struct NormPro {
-    const float *x, *y, *post_w, *post_b, *step, *pre_w, *pre_b;
+    const float *step;
     float *x_out;
     float mult, eps;
-    int cols, rms;
+    int cols;
 };
+struct MvNorms {  // the plain arguments
+    const float *x, *y, *post_w, *pre_w;
+    int flags;    // MV_*
+    NormPro rest;
+};
+enum { MV_Y = 1, MV_BIAS = 2, MV_RMS = 4, MV_PRE = 8 };
 
+// Sum over the workgroup's wavefronts (at most 16), in every thread.  red: 16 floats of this sum's own, zero from the last
+// wavefront on; one barrier.
 __device__ __forceinline__ float pro_sum(float v, float *red) {
     v = wave_sum(v);
-    __syncthreads();  // the last use of red is over
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    const int n = blockDim.x >> 6;
-    float t = red[0];
-    for (int w = 1; w < n; ++w) t += red[w];
+    f32x4 r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = *(const f32x4 *)(red + 4 * i);
+    float t = r[0][0];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) t += r[w >> 2][w & 3];
     return t;
 }
 
@@ -61,31 +73,40 @@ template <class AT> constexpr int mv_lds_values() { return sizeof(AT) == 2 ? 163
 template <int R> constexpr int mv_unroll() { return 8 / R; }                                  // 8 KB requested per step
 
 // One workgroup of W wavefronts per CU where the rows go round (launch_mv picks W and R so that they do), R weight rows
-// per wavefront.  The next step's weights are requested before the current ones are multiplied, the first ones before
-// the activations are staged.  NV > 0: the activations are made here, by the norm chain in front of the contraction
+// per wavefront.  Two steps of weights are in flight, the first two requested right behind the activations and in front of
+// everything that waits.  NV > 0: the activations are made here, by the norm chain in front of the contraction
 // (NV float4 per thread); every workgroup repeats it, workgroup 0 writes the new residual row.
+//   What bounds it: long weights, memory (128256 x 2048 at 6.8 TB/s); a layer's projections, the launch, the first round trip and, with
+// norms, their two to four sums over the workgroup.  Requests are served in the order they are made, so the row comes in front of the
+// weights; a step that was only requested once the row was staged (or the norms were done) cost a second round trip.  A sum is one
+// barrier with its sixteen terms read together, not two barriers and a loop.  us, one step and in that order / so: 128256 x 2048 87.6 /
+// 77.5, 102400 x 2048 70.5 / 63.2, the router of 64 experts 6.4 / 4.4; a decode step of the 1B-shaped Suvazen decoder, 1700 positions,
+// 705 / 665, of the fine Gulisun one 302 / 288.
 template <class AT, int R, int EPI, int NV>
-__global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, const bf16 *__restrict__ W, void *__restrict__ yv,
-                                                   int K, int rows, int n_store, const EpiArgs ea, const NormPro np) {
+__global__ __launch_bounds__(1024) void k_dense_mv(const void *__restrict__ xv_, const bf16 *__restrict__ W, int K, int rows,
+                                                   const float *__restrict__ ny, const float *__restrict__ post_w, const float *__restrict__ pre_w,
+                                                   int flags, void *__restrict__ yv, int n_store, const EpiArgs ea, const NormPro np) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
     constexpr int U = mv_unroll<R>(), STEP = U * 512, CH = mv_lds_values<AT>();
     __shared__ __align__(16) AT xs[CH];
-    __shared__ float red[16];
+    __shared__ __align__(16) float red[NV > 0 ? 64 : 4];  // sixteen for each sum
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int threads = blockDim.x;
     const int row0 = (blockIdx.x * (threads >> 6) + wave) * R;
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-    const bf16 *wr[R];
+    // A weight row through a descriptor of its own: a lane's place is one offset, and what lies past the row comes as zeros.
+    constexpr int NT = 2;  // nontemporal
+    __amdgpu_buffer_rsrc_t wr[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) wr[r] = W + (size_t)min(row0 + r, rows - 1) * K;
+    for (int r = 0; r < R; ++r) wr[r] = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)min(row0 + r, rows - 1) * K), 0, (int)(2u * (uint32_t)K), 0x00027000);
     auto fetch = [&](u32x4v (&w)[R][U], int k0) __attribute__((always_inline)) {
+        const uint32_t at = 2u * (uint32_t)k0 + (uint32_t)lane * 16;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = min(k0 + u * 512 + lane * 8, K - 8);  // past the row: any value of it, times x = 0
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int r = 0; r < R; ++r) w[r][u] = __builtin_nontemporal_load((const u32x4v *)(wr[r] + k));
-        }
+            for (int r = 0; r < R; ++r) w[r][u] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[r], at + u * 1024, 0, NT));
     };
     auto multiply = [&](const u32x4v (&w)[R][U], int k0) __attribute__((always_inline)) {
         const AT *xp = xs + (k0 & (CH - 1)) + lane * 8;
@@ -100,16 +121,12 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, con
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc[r] = fmaf(wf[e], xf[e], acc[r]);
             }
+            if (u & 1) __builtin_amdgcn_sched_barrier(0);  // two pieces of x at a time: all of them do not fit beside two steps of weights
         }
     };
-    auto stage = [&](int k0) __attribute__((always_inline)) {
-        if (k0) __syncthreads();  // the previous chunk is consumed
-        const int n = min(CH, (K - k0 + STEP - 1) / STEP * STEP);
-        constexpr int PER = 16 / sizeof(AT);
-        for (int i = tid * PER; i < n; i += threads * PER)
-            *(u32x4v *)&xs[i] = k0 + i < K ? *(const u32x4v *)(x + k0 + i) : u32x4v{0, 0, 0, 0};
-        __syncthreads();
-    };
+    constexpr int PER = 16 / sizeof(AT);
+    const AT *x = (const AT *)xv_;
+    auto piece = [&](int k) __attribute__((always_inline)) { return k < K ? *(const u32x4v *)(x + k) : u32x4v{0, 0, 0, 0}; };
     u32x4v wa[R][U], wb[R][U];
     if constexpr (NV > 0) {
         f32x4 xv[NV], yv4[NV];
@@ -121,23 +138,28 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, con
         f32x4 wv[NV], bv[NV], pw[NV], pb[NV];
 #pragma unroll
         for (int i = 0; i < NV; ++i) bv[i] = pb[i] = zero;
-        load(np.x, xv);
-        if (np.y) {
-            load(np.y, yv4);
-            load(np.post_w, pw);
-            if (np.post_b) load(np.post_b, pb);
+        load((const float *)xv_, xv);
+        if (flags & MV_Y) {
+            load(ny, yv4);
+            load(post_w, pw);
+            if (flags & MV_BIAS) load(post_w + K, pb);
         }
-        if (np.pre_w) load(np.pre_w, wv);
-        if (np.pre_b) load(np.pre_b, bv);
+        if (flags & MV_PRE) {
+            load(pre_w, wv);
+            if (flags & MV_BIAS) load(pre_w + K, bv);
+        }
         fetch(wa, 0);
+        if (NV == 1) fetch(wb, STEP);
+        const int n_waves = threads >> 6;
+        if (tid < 64 && (tid & 15) >= n_waves) red[tid] = 0.0f;
         const float inv_n = 1.0f / (float)np.cols;
-        auto normalize = [&](f32x4 (&d)[NV], const f32x4 (&w)[NV], const f32x4 (&b)[NV]) __attribute__((always_inline)) {
+        auto normalize = [&](f32x4 (&d)[NV], const f32x4 (&w)[NV], const f32x4 (&b)[NV], float *sums) __attribute__((always_inline)) {
             float mean = 0.0f;
-            if (!np.rms) {
+            if (!(flags & MV_RMS)) {
                 float s = 0.0f;
 #pragma unroll
                 for (int i = 0; i < NV; ++i) s += (d[i][0] + d[i][1]) + (d[i][2] + d[i][3]);
-                mean = pro_sum(s, red) * inv_n;
+                mean = pro_sum(s, sums) * inv_n;
             }
             float q = 0.0f;
 #pragma unroll
@@ -147,14 +169,14 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, con
                     d[i][j] = (tid + threads * i) * 4 + j < np.cols ? d[i][j] - mean : 0.0f;
                     q += d[i][j] * d[i][j];
                 }
-            const float rstd = 1.0f / sqrtf(pro_sum(q, red) * inv_n + np.eps);
+            const float rstd = 1.0f / sqrtf(pro_sum(q, sums + 16) * inv_n + np.eps);
 #pragma unroll
             for (int i = 0; i < NV; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) d[i][j] = d[i][j] * rstd * w[i][j] + b[i][j];  // w = b = 0 past the row
         };
-        if (np.y) {
-            normalize(yv4, pw, pb);
+        if (flags & MV_Y) {
+            normalize(yv4, pw, pb, red);
 #pragma unroll
             for (int i = 0; i < NV; ++i) xv[i] += np.mult * yv4[i];
         }
@@ -168,24 +190,43 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, con
             for (int i = 0; i < NV; ++i)
                 if ((tid + threads * i) * 4 < K) *(f32x4 *)(np.x_out + (tid + threads * i) * 4) = xv[i];
         }
-        if (np.pre_w) normalize(xv, wv, bv);
+        if (flags & MV_PRE) normalize(xv, wv, bv, red + 32);
+        if (NV > 1) fetch(wb, STEP);  // no registers for it any sooner
         typedef AT at4 __attribute__((ext_vector_type(4)));
         const int n = (K + STEP - 1) / STEP * STEP;
 #pragma unroll
         for (int i = 0; i < NV; ++i)
             if ((tid + threads * i) * 4 < n) *(at4 *)&xs[(tid + threads * i) * 4] = __builtin_convertvector(xv[i], at4);
         for (int i = (tid + threads * NV) * 4; i < n; i += threads * 4) *(at4 *)&xs[i] = __builtin_convertvector(zero, at4);
-        __syncthreads();
     } else {
+        // The first pieces of the row are requested in front of the weights: requests are served in order, and behind them the row
+        // would come last.
+        constexpr int FIRST = 2;
+        u32x4v held[FIRST];
+#pragma unroll
+        for (int i = 0; i < FIRST; ++i) held[i] = piece((tid + threads * i) * PER);
         fetch(wa, 0);
+        fetch(wb, STEP);
+        __builtin_amdgcn_sched_barrier(0);
+        const int n = min(CH, (K + STEP - 1) / STEP * STEP);
+#pragma unroll
+        for (int i = 0; i < FIRST; ++i)
+            if ((tid + threads * i) * PER < n) *(u32x4v *)&xs[(tid + threads * i) * PER] = held[i];
+        for (int i = (tid + threads * FIRST) * PER; i < n; i += threads * PER) *(u32x4v *)&xs[i] = piece(i);
     }
+    __syncthreads();
     for (int k0 = 0; k0 < K; k0 += 2 * STEP) {
-        if (NV == 0 && (k0 & (CH - 1)) == 0) stage(k0);
-        if (k0 + STEP < K) fetch(wb, k0 + STEP);
+        if (NV == 0 && k0 && (k0 & (CH - 1)) == 0) {
+            __syncthreads();  // the previous chunk is consumed
+            const int n = min(CH, (K - k0 + STEP - 1) / STEP * STEP);
+            for (int i = tid * PER; i < n; i += threads * PER) *(u32x4v *)&xs[i] = piece(k0 + i);
+            __syncthreads();
+        }
         multiply(wa, k0);
+        fetch(wa, k0 + 2 * STEP);  // (steps past the row ask for nothing)
         if (k0 + STEP >= K) break;
-        if (k0 + 2 * STEP < K) fetch(wa, k0 + 2 * STEP);
         multiply(wb, k0 + STEP);
+        fetch(wb, k0 + 3 * STEP);
     }
     float mine = 0.0f;
 #pragma unroll
@@ -198,6 +239,7 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const AT *__restrict__ x, con
         if (to_act(EPI)) ((AT *)yv)[row0 + lane] = (AT)z;
         else ((float *)yv)[row0 + lane] = z;
     }
+#endif
 }
 
 // ------------------------------------------------------------------ prompt batches, bfloat16
@@ -689,25 +731,27 @@ MvShape mv_shape(const candy_hip_device *dev, int64_t rows) {
 }
 
 template <class AT, int R, int EPI>
-static void launch_mv_nv(candy_hip_device *dev, const DenseLaunch &L, int waves, int nv, const NormPro &np) {
+static void launch_mv_nv(candy_hip_device *dev, const DenseLaunch &L, int waves, int nv, const MvNorms &np) {
     const int64_t per_wg = (int64_t)waves * R;
     const dim3 g((unsigned)((L.n_store + per_wg - 1) / per_wg)), b((unsigned)(64 * waves));
     const EpiArgs ea{L.scale, L.cap};
-    const AT *x = (const AT *)L.x;
     const bf16 *W = (const bf16 *)L.w->data;
     const int K = (int)L.w->ld, rows = (int)L.w->rows_pad, ns = (int)L.n_store;
+    auto launch = [&](auto kern, const void *x) {
+        hipLaunchKernelGGL(kern, g, b, 0, dev->stream, x, W, K, rows, np.y, np.post_w, np.pre_w, np.flags, L.y, ns, ea, np.rest);
+    };
     if constexpr (sizeof(AT) == 2 || (R == 1 && EPI == EPI_NONE)) {
         switch (nv) {
-        case 1: hipLaunchKernelGGL((k_dense_mv<AT, R, EPI, 1>), g, b, 0, dev->stream, x, W, L.y, K, rows, ns, ea, np); return;
-        case 2: hipLaunchKernelGGL((k_dense_mv<AT, R, EPI, 2>), g, b, 0, dev->stream, x, W, L.y, K, rows, ns, ea, np); return;
+        case 1: launch(k_dense_mv<AT, R, EPI, 1>, np.x); return;
+        case 2: launch(k_dense_mv<AT, R, EPI, 2>, np.x); return;
         default: break;
         }
     }
-    hipLaunchKernelGGL((k_dense_mv<AT, R, EPI, 0>), g, b, 0, dev->stream, x, W, L.y, K, rows, ns, ea, np);
+    launch(k_dense_mv<AT, R, EPI, 0>, L.x);
 }
 
 template <class AT, int R>
-static void launch_mv_epi(candy_hip_device *dev, const DenseLaunch &L, int waves, int nv, const NormPro &np) {
+static void launch_mv_epi(candy_hip_device *dev, const DenseLaunch &L, int waves, int nv, const MvNorms &np) {
     switch (L.epi) {
     case EPI_RELU2: launch_mv_nv<AT, R, EPI_RELU2>(dev, L, waves, nv, np); break;
     case EPI_CAP: launch_mv_nv<AT, R, EPI_CAP>(dev, L, waves, nv, np); break;
@@ -717,7 +761,7 @@ static void launch_mv_epi(candy_hip_device *dev, const DenseLaunch &L, int waves
 }
 
 template <class AT>
-static int launch_mv(candy_hip_device *dev, const DenseLaunch &L, const MvShape &s, int nv = 0, const NormPro &np = NormPro{}) {
+static int launch_mv(candy_hip_device *dev, const DenseLaunch &L, const MvShape &s, int nv = 0, const MvNorms &np = MvNorms{}) {
     switch (s.rows) {
     case 1: launch_mv_epi<AT, 1>(dev, L, s.waves, nv, np); break;
     case 2: launch_mv_epi<AT, 2>(dev, L, s.waves, nv, np); break;
@@ -735,8 +779,12 @@ int launch_dense_norm(candy_hip_device *dev, const DenseLaunch &L, const NormArg
         A.x == A.x_out || nv > 2 || L.w->ld > (L.f32 ? mv_lds_values<float>() : mv_lds_values<bf16>()) || L.n_store > 64 * (int64_t)dev->num_cus)
         return CANDY_HIP_ERR_UNSUPPORTED;
     CANDY_REQUIRE(pad64(A.cols) == L.w->ld, "internal: norm and contraction of different widths");
+    // biases: of both norms or of none, each behind its weights
+    const bool bias = A.pre_b || (A.y.p && A.post_b);
+    if (bias && ((A.pre_w && A.pre_b != A.pre_w + L.w->ld) || (A.y.p && A.post_b != A.post_w + L.w->ld))) return CANDY_HIP_ERR_UNSUPPORTED;
     if (L.partial) *L.partial = Partial{(const float *)L.y, 1, 0, (int)L.ldy};
-    const NormPro np{A.x, A.y.p, A.post_w, A.post_b, A.step, A.pre_w, A.pre_b, A.x_out, A.mult, A.eps, A.cols, A.rms};
+    const MvNorms np{A.x, A.y.p, A.post_w, A.pre_w, (A.y.p ? MV_Y : 0) | (bias ? MV_BIAS : 0) | (A.rms ? MV_RMS : 0) | (A.pre_w ? MV_PRE : 0),
+                     NormPro{A.step, A.x_out, A.mult, A.eps, A.cols}};
     return L.f32 ? launch_mv<float>(dev, L, s, nv, np) : launch_mv<bf16>(dev, L, s, nv, np);
 }
 

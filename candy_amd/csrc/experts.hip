@@ -18,22 +18,37 @@ namespace candy {
 __device__ __forceinline__ float ordered(float z) { return z == z ? z : -INFINITY; }
 
 // One wavefront, lane e holding score e of a token's E <= 64 (ordered()): lane k leaves with the k-th choice and its weight.
-__device__ __forceinline__ void choose64(float v, int E, int top, int &id, float &weight) {
-    const int lane = threadIdx.x & 63;
-    uint64_t left = E == 64 ? ~0ull : (1ull << E) - 1;
-    if (lane >= E) v = -INFINITY;
-    float best = wave_max(v), mine = -INFINITY;
-    const float mx = fmaxf(best, LOW), sum = wave_sum(lane < E ? expf(v - mx) : 0.0f);
-    id = 0;
-    for (int k = 0; k < top; ++k) {
-        if (k) best = wave_max(v);
-        const int e = __ffsll((unsigned long long)(__ballot(v == best) & left)) - 1;   // not empty: `left` has top - k members
-        left &= ~(1ull << e);
-        if (lane == k) { id = e; mine = best; }
-        if (lane == e) v = -INFINITY;
+struct Choice64 {
+    float v, best, mine;   // the scores left, the largest of all, lane k: the k-th choice's
+    int id;                // lane k: the k-th choice
+    __device__ __forceinline__ void pick(float score, int E, int top) {
+        const int lane = threadIdx.x & 63;
+        uint64_t left = E == 64 ? ~0ull : (1ull << E) - 1;
+        v = lane < E ? score : -INFINITY;
+        best = wave_max(v);
+        mine = -INFINITY;
+        id = 0;
+        float w = v, b = best;
+        for (int k = 0; k < top; ++k) {
+            if (k) b = wave_max(w);
+            const int e = __ffsll((unsigned long long)(__ballot(w == b) & left)) - 1;   // not empty: `left` has top - k members
+            left &= ~(1ull << e);
+            if (lane == k) { id = e; mine = b; }
+            if (lane == e) w = -INFINITY;
+        }
     }
-    const float s = lane < top ? expf(mine - mx) / sum : 0.0f;
-    weight = s / (wave_sum(s) + 1e-20f);
+    __device__ __forceinline__ float weight(int E, int top) const {
+        const int lane = threadIdx.x & 63;
+        const float mx = fmaxf(best, LOW), sum = wave_sum(lane < E ? expf(v - mx) : 0.0f);
+        const float s = lane < top ? expf(mine - mx) / sum : 0.0f;
+        return s / (wave_sum(s) + 1e-20f);
+    }
+};
+__device__ __forceinline__ void choose64(float v, int E, int top, int &id, float &weight) {
+    Choice64 c;
+    c.pick(v, E, top);
+    id = c.id;
+    weight = c.weight(E, top);
 }
 
 // The same for any number of scores z[0 .. E) in LDS; choices and weights in order of their scores.
@@ -207,31 +222,48 @@ struct RowArgs {
     int E, top, rows_e, rows_s, ld;   // rows_e / rows_s: padded inner widths of an expert and of the shared one
 };
 
-constexpr int EXP_U = 4;   // 16-byte requests per row in flight
+// 16-byte requests per row and step; two steps are in flight.  (With one of half the length, requested when the one before it was
+// consumed, the down projections were six round trips one after the other.)  us of a decode step of the fine / coarse Gulisun decoder with
+// four layers, before -> now: 288 / 396 -> 281 / 388.
+template <int R> constexpr int exp_unroll() { return 8 / R; }
 
-// Rows of the concatenated up matrices, R per wavefront.  FEW: at most 64 experts, every wavefront makes the choice for
-// itself and requests its weights before the activations are staged.  LDS: x; else also the scores and the choice.
+// Rows of the concatenated up matrices, R per wavefront.  FEW: at most 64 experts, every wavefront that has rows of chosen experts
+// makes the choice for itself; scores and activations are requested in front of everything, the weights as soon as the choice
+// stands, and its shares are worked out while they come.  LDS: x; else also the scores and the choice.
 template <class AT, int R, bool FEW>
-__global__ __launch_bounds__(1024) void k_expert_up(const RowArgs a, const float *__restrict__ x, const float *__restrict__ logits,
-                                                    AT *__restrict__ act, int *__restrict__ sel) {
+__global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x, const float *__restrict__ logits, AT *__restrict__ act,
+                                                    int *__restrict__ sel, const RowArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+    constexpr int U = exp_unroll<R>(), STEP = U * 512;
     extern __shared__ __align__(16) uint8_t lds[];
     AT *xs = (AT *)lds;
-    float *z = (float *)(xs + a.ld), *gate = z + a.E;
+    AT *nothing = xs + a.ld;   // eight zeros
+    float *z = (float *)(nothing + 8), *gate = z + a.E;
     int *ids = (int *)(gate + a.top);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x;
-    const int total = a.top * a.rows_e + a.rows_s, row0 = (blockIdx.x * (threads >> 6) + wave) * R;
-    int my_id = 0;
-    float my_weight = 0.0f;
+    const int routed = a.top * a.rows_e, total = routed + a.rows_s, row0 = (blockIdx.x * (threads >> 6) + wave) * R;
+    typedef AT at4 __attribute__((ext_vector_type(4)));
+    constexpr int FIRST = 2;
+    f32x4 held[FIRST];
+    const float score = FEW ? logits[min(lane, a.E - 1)] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) held[i] = *(const f32x4 *)(x + min((tid + threads * i) * 4, a.ld - 4));
     auto stage = [&]() __attribute__((always_inline)) {
-        typedef AT at4 __attribute__((ext_vector_type(4)));
-        for (int i = tid * 4; i < a.ld; i += threads * 4) *(at4 *)&xs[i] = __builtin_convertvector(*(const f32x4 *)(x + i), at4);
+        if (tid < 8) nothing[tid] = (AT)0.0f;
+#pragma unroll
+        for (int i = 0; i < FIRST; ++i)
+            if ((tid + threads * i) * 4 < a.ld) *(at4 *)&xs[(tid + threads * i) * 4] = __builtin_convertvector(held[i], at4);
+        for (int i = (tid + threads * FIRST) * 4; i < a.ld; i += threads * 4)
+            *(at4 *)&xs[i] = __builtin_convertvector(*(const f32x4 *)(x + i), at4);
     };
+    Choice64 choice;
     if (FEW) {
-        choose64(ordered(logits[min(lane, a.E - 1)]), a.E, a.top, my_id, my_weight);
-        if (blockIdx.x == 0 && wave == 0 && lane < a.top) sel[lane] = my_id;
+        if (row0 < routed) {
+            choice.pick(ordered(score), a.E, a.top);
+            if (blockIdx.x == 0 && wave == 0 && lane < a.top) sel[lane] = choice.id;
+        }
     } else {
         for (int e = tid; e < a.E; e += threads) z[e] = ordered(logits[e]);
-        stage();
         __syncthreads();
         if (wave == 0) {
             choose(z, a.E, a.top, ids, gate);
@@ -240,39 +272,49 @@ __global__ __launch_bounds__(1024) void k_expert_up(const RowArgs a, const float
         }
         __syncthreads();
     }
-    const bf16 *w[R];
+    // a row through a descriptor of its own: what lies past it comes as zeros
+    constexpr int NT = 2;  // nontemporal
+    __amdgpu_buffer_rsrc_t w[R];
     float scale[R];
+    int of[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int row = min(row0 + r, total - 1), k = row / a.rows_e;
+        of[r] = k;
+        const bf16 *p = a.shared + (size_t)max(row - routed, 0) * a.ld;
         if (k < a.top) {
-            const int id = FEW ? __builtin_amdgcn_readlane(my_id, k) : ids[k];
-            w[r] = a.W + ((size_t)id * a.rows_e + (row - k * a.rows_e)) * a.ld;
-            scale[r] = FEW ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_weight), k)) : gate[k];
-        } else {
-            w[r] = a.shared + (size_t)(row - a.top * a.rows_e) * a.ld;
-            scale[r] = 1.0f;
+            const int id = FEW ? __builtin_amdgcn_readlane(choice.id, k) : __builtin_amdgcn_readfirstlane(ids[k]);
+            p = a.W + ((size_t)id * a.rows_e + (row - k * a.rows_e)) * a.ld;
         }
+        w[r] = __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 2 * a.ld, 0x00027000);
     }
+    u32x4v va[R][U], vb[R][U];
+    auto fetch = [&](u32x4v (&v)[R][U], int k0) __attribute__((always_inline)) {
+        const int at = 2 * k0 + lane * 16;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[r][u] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(w[r], at + u * 1024, 0, NT));
+    };
+    fetch(va, 0);
+    fetch(vb, STEP);
+    __builtin_amdgcn_sched_barrier(0);
+    float share = 0.0f;
+    if (FEW && row0 < routed) share = choice.weight(a.E, a.top);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        scale[r] = of[r] >= a.top ? 1.0f : FEW ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(share), of[r])) : gate[of[r]];
+    stage();
+    __syncthreads();
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-    for (int k0 = 0; k0 < a.ld; k0 += EXP_U * 512) {
-        u32x4v v[R][EXP_U];
+    auto multiply = [&](const u32x4v (&v)[R][U], int k0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < EXP_U; ++u)
-#pragma unroll
-            for (int r = 0; r < R; ++r) v[r][u] = __builtin_nontemporal_load((const u32x4v *)(w[r] + min(k0 + u * 512 + lane * 8, a.ld - 8)));
-        if (FEW && k0 == 0) {
-            stage();
-            __syncthreads();
-        }
-#pragma unroll
-        for (int u = 0; u < EXP_U; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int k = k0 + u * 512 + lane * 8;
-            if (k >= a.ld) continue;
             float xf[8];
-            lds8(xs + k, xf);
+            lds8(k < a.ld ? xs + k : nothing, xf);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 float f[8];
@@ -280,58 +322,78 @@ __global__ __launch_bounds__(1024) void k_expert_up(const RowArgs a, const float
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc[r] = fmaf(f[e], xf[e], acc[r]);
             }
+            if (u & 1) __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    for (int k0 = 0; k0 < a.ld; k0 += 2 * STEP) {
+        multiply(va, k0);
+        fetch(va, k0 + 2 * STEP);  // (steps past the row ask for nothing)
+        if (k0 + STEP >= a.ld) break;
+        multiply(vb, k0 + STEP);
+        fetch(vb, k0 + 3 * STEP);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const float t = fmaxf(wave_sum(acc[r]), 0.0f);
         if (lane == r && row0 + r < total) act[row0 + r] = (AT)(t * t * scale[r]);
     }
+#endif
 }
+
+static __device__ __align__(16) const uint32_t zero_chunk[32] = {};   // 64 values
+constexpr int DOWN_STEP = 4096;   // values the table of starts is padded to, at least one chunk of zeros behind the sum
 
 // Rows of the result: an expert's inner activations meet its down matrix, all of them one long sum.  LDS: the
 // activations, and per 64 of them where their weights start.
 template <class AT, int R>
-__global__ __launch_bounds__(1024) void k_expert_down(const RowArgs a, int d_p, const AT *__restrict__ act, const int *__restrict__ sel,
-                                                      float *__restrict__ y) {
+__global__ __launch_bounds__(1024) void k_expert_down(const AT *__restrict__ act, const int *__restrict__ sel, float *__restrict__ y, int d_p,
+                                                      const RowArgs a) {
+    constexpr int U = exp_unroll<R>(), STEP = U * 512;
+    static_assert(DOWN_STEP % STEP == 0, "whole steps");
     extern __shared__ __align__(16) uint8_t lds[];
-    const int K = a.top * a.rows_e + a.rows_s, chunks = K >> 6;
-    const bf16 **base = (const bf16 **)lds;
-    int *pitch = (int *)(base + chunks);
-    AT *xs = (AT *)(pitch + ((chunks + 3) & ~3));
+    const int K = a.top * a.rows_e + a.rows_s, chunks = K >> 6, entries = (K / DOWN_STEP + 1) * (DOWN_STEP / 64);
+    int64_t *base = (int64_t *)lds;   // in bytes from a.W (a pointer out of LDS would be loaded through as a flat one)
+    AT *xs = (AT *)(base + entries), *nothing = xs + K;   // eight zeros
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x;
     const int row0 = (blockIdx.x * (threads >> 6) + wave) * R;
-    for (int i = tid; i < chunks; i += threads) {
+    // the first pieces of the activations are requested together, in front of what waits for the choice
+    constexpr int PER = 16 / sizeof(AT), FIRST = 4;
+    u32x4v held[FIRST];
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) held[i] = *(const u32x4v *)(act + min((tid + threads * i) * PER, K - PER));
+    const int routed = a.top * a.rows_e;
+    if (tid < 8) nothing[tid] = (AT)0.0f;
+    const int64_t behind = (const char *)a.shared - (const char *)a.W, none = (const char *)zero_chunk - (const char *)a.W;
+    for (int i = tid; i < entries; i += threads) {
         const int k = (i << 6) / a.rows_e;
-        if (k < a.top) {
-            base[i] = a.W + (size_t)sel[k] * d_p * a.rows_e + ((i << 6) - k * a.rows_e);
-            pitch[i] = a.rows_e;
-        } else {
-            base[i] = a.shared + ((i << 6) - a.top * a.rows_e);
-            pitch[i] = a.rows_s;
-        }
+        base[i] = i >= chunks ? none
+                              : k < a.top ? 2 * ((int64_t)sel[k] * d_p * a.rows_e + ((i << 6) - k * a.rows_e)) : behind + 2 * (int64_t)((i << 6) - routed);
     }
-    constexpr int PER = 16 / sizeof(AT);
-    for (int i = tid * PER; i < K; i += threads * PER) *(u32x4v *)&xs[i] = *(const u32x4v *)(act + i);
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i)
+        if ((tid + threads * i) * PER < K) *(u32x4v *)&xs[(tid + threads * i) * PER] = held[i];
+    for (int i = (tid + threads * FIRST) * PER; i < K; i += threads * PER) *(u32x4v *)&xs[i] = *(const u32x4v *)(act + i);
     __syncthreads();
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += EXP_U * 512) {
-        u32x4v v[R][EXP_U];
+    u32x4v va[R][U], vb[R][U];
+    auto fetch = [&](u32x4v (&v)[R][U], int k0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < EXP_U; ++u) {
-            const int k = min(k0 + u * 512 + lane * 8, K - 8), c = k >> 6;
-            const bf16 *p = base[c] + (k & 63);
+        for (int u = 0; u < U; ++u) {
+            const int k = min(k0 + u * 512, (entries << 6) - 512) + lane * 8;
+            const char *p = (const char *)a.W + base[k >> 6] + 2 * (k & 63);
+            const int pitch = 2 * (k < routed ? a.rows_e : k < K ? a.rows_s : 0);
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[r][u] = __builtin_nontemporal_load((const u32x4v *)(p + (size_t)min(row0 + r, d_p - 1) * pitch[c]));
+            for (int r = 0; r < R; ++r) v[r][u] = __builtin_nontemporal_load((const u32x4v *)(p + (size_t)min(row0 + r, d_p - 1) * pitch));
         }
+    };
+    auto multiply = [&](const u32x4v (&v)[R][U], int k0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < EXP_U; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int k = k0 + u * 512 + lane * 8;
-            if (k >= K) continue;
             float xf[8];
-            lds8(xs + k, xf);
+            lds8(k < K ? xs + k : nothing, xf);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 float f[8];
@@ -339,7 +401,17 @@ __global__ __launch_bounds__(1024) void k_expert_down(const RowArgs a, int d_p, 
 #pragma unroll
                 for (int e = 0; e < 8; ++e) acc[r] = fmaf(f[e], xf[e], acc[r]);
             }
+            if (u & 1) __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    fetch(va, 0);
+    fetch(vb, STEP);
+    for (int k0 = 0; k0 < K; k0 += 2 * STEP) {
+        multiply(va, k0);
+        fetch(va, k0 + 2 * STEP);
+        if (k0 + STEP >= K) break;
+        multiply(vb, k0 + STEP);
+        fetch(vb, k0 + 3 * STEP);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -352,10 +424,10 @@ __global__ __launch_bounds__(1024) void k_expert_down(const RowArgs a, int d_p, 
 int expert_row_values(const candy_hip_expert_spec &s) { return (int)(s.top * pad64(s.d_ff) + pad64(s.shared_ff)); }
 
 // LDS of the one-row kernels
-static size_t up_lds(const candy_hip_expert_spec &s, int64_t ld, size_t es) { return (size_t)ld * es + (size_t)(s.n_experts + 2 * s.top) * 4; }
+static size_t up_lds(const candy_hip_expert_spec &s, int64_t ld, size_t es) { return (size_t)(ld + 8) * es + (size_t)(s.n_experts + 2 * s.top) * 4; }
 static size_t down_lds(const candy_hip_expert_spec &s, size_t es) {
-    const size_t K = (size_t)expert_row_values(s), chunks = K / 64;
-    return chunks * 8 + ((chunks + 3) & ~(size_t)3) * 4 + K * es;
+    const size_t K = (size_t)expert_row_values(s);
+    return (K / DOWN_STEP + 1) * (DOWN_STEP / 64) * 8 + (K + 8) * es;
 }
 static size_t route_lds(const candy_hip_expert_spec &s) {
     return ((size_t)ROUTE_T * (s.n_experts | 1) + std::max<size_t>(ROUTE_W / 2 * 64 * 17, 2 * ROUTE_T * (size_t)s.top)) * 4;
@@ -429,8 +501,8 @@ static int experts_row(candy_hip_device *dev, const ExpertLayer &A) {
     CANDY_REQUIRE(lu <= 65536 && ldn <= 163840, "experts too wide for this activation format");
 #define CANDY_UP(R)                                                                                                          \
     do {                                                                                                                     \
-        if (s.n_experts <= 64) hipLaunchKernelGGL((k_expert_up<AT, R, true>), gu, bu, lu, dev->stream, u, A.x, A.logits, act, A.ids); \
-        else hipLaunchKernelGGL((k_expert_up<AT, R, false>), gu, bu, lu, dev->stream, u, A.x, A.logits, act, A.ids);          \
+        if (s.n_experts <= 64) hipLaunchKernelGGL((k_expert_up<AT, R, true>), gu, bu, lu, dev->stream, A.x, A.logits, act, A.ids, u); \
+        else hipLaunchKernelGGL((k_expert_up<AT, R, false>), gu, bu, lu, dev->stream, A.x, A.logits, act, A.ids, u);          \
     } while (0)
     switch (su.rows) {
     case 1: CANDY_UP(1); break;
@@ -443,9 +515,9 @@ static int experts_row(candy_hip_device *dev, const ExpertLayer &A) {
     u.shared = s.shared_ff ? (const bf16 *)A.w.shared_down->data : nullptr;
     const dim3 gd((unsigned)((d + sd.waves * sd.rows - 1) / (sd.waves * sd.rows))), bd((unsigned)(64 * sd.waves));
     switch (sd.rows) {
-    case 1: hipLaunchKernelGGL((k_expert_down<AT, 1>), gd, bd, ldn, dev->stream, u, (int)d, act, A.ids, A.y); break;
-    case 2: hipLaunchKernelGGL((k_expert_down<AT, 2>), gd, bd, ldn, dev->stream, u, (int)d, act, A.ids, A.y); break;
-    default: hipLaunchKernelGGL((k_expert_down<AT, 4>), gd, bd, ldn, dev->stream, u, (int)d, act, A.ids, A.y); break;
+    case 1: hipLaunchKernelGGL((k_expert_down<AT, 1>), gd, bd, ldn, dev->stream, act, A.ids, A.y, (int)d, u); break;
+    case 2: hipLaunchKernelGGL((k_expert_down<AT, 2>), gd, bd, ldn, dev->stream, act, A.ids, A.y, (int)d, u); break;
+    default: hipLaunchKernelGGL((k_expert_down<AT, 4>), gd, bd, ldn, dev->stream, act, A.ids, A.y, (int)d, u); break;
     }
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;

@@ -16,6 +16,7 @@ struct candy_hip_suvazen final : candy_hip_decoder {
         candy_hip_suvazen_layer c{};
         const candy_hip_dense *qk = nullptr, *o = nullptr, *up = nullptr, *down = nullptr;
         float *norm[8] = {};   // in the order of enum candy_hip_suvazen_vector
+        float *norm_room[4] = {};  // weights and bias of a norm, one behind the other
         float *sink = nullptr;
         const float *cos_t = nullptr, *sin_t = nullptr;
         int n_splits = 1;
@@ -27,7 +28,7 @@ struct candy_hip_suvazen final : candy_hip_decoder {
     std::vector<Layer> layers;
     std::vector<Run> runs;
     std::vector<float *> steps;
-    float *final_w = nullptr, *final_b = nullptr;
+    float *final_w = nullptr, *final_b = nullptr, *final_room = nullptr;
     const candy_hip_dense *head = nullptr, *embed_w = nullptr;
     bool f32 = false;
     int max_qk = 0, max_att = 0, max_ff = 0, max_q = 0;   // widest rows over the layers, padded
@@ -350,8 +351,14 @@ int candy_hip_suvazen_set_vector(candy_hip_suvazen *m, int which, int layer, con
     if (int rc = use_device(m->dev)) return rc;
     std::vector<float> padded((size_t)pad64(want), 0.0f);
     memcpy(padded.data(), host, (size_t)want * sizeof(float));
-    if (!*slot)
+    if (!*slot && (which == CANDY_HIP_SV_STEP || which == CANDY_HIP_SV_SINK)) {
         if (int rc = decoder_alloc(m, slot, padded.size())) return rc;
+    } else if (!*slot) {  // a norm's bias lies behind its weights (launch_dense_norm)
+        float **room = final_norm ? &m->final_room : &m->layers[(size_t)layer].norm_room[which >> 1];
+        if (!*room)
+            if (int rc = decoder_alloc(m, room, 2 * padded.size())) return rc;
+        *slot = *room + (which & 1 ? padded.size() : 0);
+    }
     m->graph_dirty = true;
     return candy_hip_h2d(m->dev, *slot, padded.data(), padded.size() * sizeof(float));
 }
