@@ -87,7 +87,8 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *                                         exact int8 tiles (below it the pass holds the decode step's 1e-3 end to end)
  *   "mmq.f16_api_min_m"          33       the same for one contraction through candy_hip_qmatmul / candy_hip_qmatmul_q8 (one
  *                                         matmul: 3e-4 < 1e-3): Q4_K and Q6_K from this many rows, the other formats from 65
- *                                         or this if larger
+ *                                         or this if larger; weights of few rows stay on the exact kernel up to 255 rows
+ *                                         where it is faster
  *   "prefill.kv_parts_mb"        0        prompt attention on an f32 cache: MB at most for the 16-bit parts of a layer's K and
  *                                         V that the matrix cores contract, 1 to 1.5 times one layer's cache for max_pos
  *                                         (0: no limit).  Past the limit, and where the allocation fails, the vector ALU
