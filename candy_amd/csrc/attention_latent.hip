@@ -2,6 +2,7 @@
 // equations: include/candy_hip.h).
 //   k_latent_rows          projected rows -> normed query latents, normed latent and rotated key part into the cache
 //   k_latent_prompt        bfloat16 prompts on the matrix cores over expanded keys and values, 64 queries of a head per workgroup
+//   k_latent_prompt_direct the same for keys and values of whole 64s, loaded to LDS as they lie
 //   k_latent_prompt_row    one wavefront per (query, head), vector ALU: f32 prompts, and heads too wide for the tiles
 //   k_latent_query         decode: queries contracted with Wuk, rotated part turned, the new cache row appended
 //   k_latent_decode        bfloat16 decode on the matrix cores: 16 heads against the cached rows, split over the positions
@@ -84,6 +85,130 @@ __global__ __launch_bounds__(256) void k_latent_rows(const LatentArgs a, const P
 }
 
 // ------------------------------------------------------------------ prompts, bfloat16, matrix cores
+// A query's values, rotated, as operands: lane (query, g) holds values 32 ks + 8 g .. + 7.  Everything of a step is requested before any of it is
+// used (value by value, each waiting for the one before, these loads took 20 us of a prompt's 105).
+template <int KS>
+__device__ __forceinline__ void latent_query(const LatentArgs &a, const Partial &qp, int h, int qrow, int qpos, int g, bf16x8 (&qf)[KS]) {
+    const int width = a.dim + a.rot;
+    const bool pieces = (a.half & 7) == 0 && (((uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
+    const float *src = qp.p + (size_t)qrow * qp.ld + h * width;
+    f32x4 v[KS][2];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        v[ks][0] = v[ks][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (ks * 32 < width) {
+            v[ks][0] = *(const f32x4 *)(src + ks * 32 + g * 8);
+            v[ks][1] = *(const f32x4 *)(src + ks * 32 + g * 8 + 4);
+        }
+    }
+    for (int c = 1; c < qp.copies; ++c)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            if (ks * 32 < width) {
+                const float *s = src + (size_t)c * qp.stride + ks * 32 + g * 8;
+                v[ks][0] += *(const f32x4 *)s;
+                v[ks][1] += *(const f32x4 *)(s + 4);
+            }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        if (ks * 32 >= a.dim && ks * 32 < width) {   // both multiples of 32: the whole step is rotated or none of it
+            const int j0 = ks * 32 + g * 8 - a.dim;
+            f32x4 co[2], si[2], other[2];
+            if (pieces) {  // eight values lie in one half of the rotated ones, or behind both
+                const int k = j0 < a.half ? j0 : min(j0 - a.half, a.half - 8);
+                const float *c = a.cos_t + (size_t)qpos * a.half + k, *s = a.sin_t + (size_t)qpos * a.half + k;
+                const int at = a.dim + (j0 < a.half ? j0 + a.half : k);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    co[i] = *(const f32x4 *)(c + 4 * i);
+                    si[i] = *(const f32x4 *)(s + 4 * i);
+                    other[i] = *(const f32x4 *)(src + at + 4 * i);
+                }
+                for (int c = 1; c < qp.copies; ++c)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) other[i] += *(const f32x4 *)(src + (size_t)c * qp.stride + at + 4 * i);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int j = j0 + e, k = j < a.half ? j : min(j - a.half, a.half - 1), at = a.dim + (j < a.half ? j + a.half : k);
+                    co[e >> 2][e & 3] = a.cos_t[(size_t)qpos * a.half + k];
+                    si[e >> 2][e & 3] = a.sin_t[(size_t)qpos * a.half + k];
+                    float t = src[at];
+                    for (int c = 1; c < qp.copies; ++c) t += src[(size_t)c * qp.stride + at];
+                    other[e >> 2][e & 3] = t;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int j = j0 + e;
+                const float x = v[ks][e >> 2][e & 3];
+                if (j < 2 * a.half) v[ks][e >> 2][e & 3] = 
+                        j < a.half ? x * co[e >> 2][e & 3] - other[e >> 2][e & 3] * si[e >> 2][e & 3]
+                                   : x * co[e >> 2][e & 3] + other[e >> 2][e & 3] * si[e >> 2][e & 3];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[ks][e] = (bf16)v[ks][e >> 2][e & 3];
+    }
+}
+
+// One tile of 64 keys: scores (lane: one query, keys 16 kt + 4 g + j) -> weights; the outputs and l so far in proportion.
+template <int ND>
+__device__ __forceinline__ void latent_weights(f32x4 (&s)[4], f32x4 (&o)[ND], float &m, float &l, float c_in, bool whole, int first_key, int pos) {
+    float mx = MASKED;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float z = s[kt][j] * c_in;
+            if (!whole) z = first_key + kt * 16 + j <= pos ? z : MASKED;
+            s[kt][j] = z;
+            mx = fmaxf(mx, z);
+        }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m, mx);
+    const float corr = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    float sum = 0.0f;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s[kt][j] = __builtin_amdgcn_exp2f(s[kt][j] - m_new);
+            sum += s[kt][j];
+        }
+    l = l * corr + sum;
+    if (__any(corr != 1.0f)) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) o[d] *= corr;
+    }
+}
+// The weights of keys 32 kb .. + 31 as the sum of two bfloat16
+__device__ __forceinline__ void latent_parts(const f32x4 (&s)[4], int kb, bf16x8 &hi, bf16x8 &lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float w = s[2 * kb + (e >> 2)][e & 3];
+        hi[e] = (bf16)w;
+        lo[e] = (bf16)(w - (float)hi[e]);
+    }
+}
+template <int ND>
+__device__ __forceinline__ void latent_store(const LatentArgs &a, const f32x4 (&o)[ND], float l, int h, int qi, int n, int g, bf16 *out) {
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (qi >= n) return;
+    const float inv = 1.0f / l;
+    bf16 *dst = out + (size_t)qi * a.ldo + (size_t)h * a.vdim;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        const int c = d * 16 + 4 * g;
+        if (c < a.vdim) *(bf16x4 *)(dst + c) = __builtin_convertvector(o[d] * inv, bf16x4);
+    }
+    if (h == a.H - 1)
+        for (int i = a.H * a.vdim + g; i < a.out_cols; i += 4) out[(size_t)qi * a.ldo + i] = (bf16)0.0f;
+}
+
 // grid (heads, ceil(n / 64)), 4 wavefronts of 16 queries, keys in tiles of 64 through LDS; scores transposed (keys x
 // queries), so that a lane holds scores of one query only and hands the weights to the second product from registers:
 // its K index 8 g + e stands for key 4 g + e of one 16-key tile (e < 4) or of the next (e >= 4), and V is stored
@@ -126,25 +251,7 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt(const LatentArgs a, co
     };
     request(0);
     bf16x8 qf[DK / 32];
-#pragma unroll
-    for (int ks = 0; ks < DK / 32; ++ks) {
-        const int i = ks * 32 + g * 8, base = h * (a.dim + a.rot);
-        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (i < a.dim) {
-            for (int c = 0; c < qp.copies; ++c) {
-                const float *s = qp.p + (size_t)c * qp.stride + (size_t)qrow * qp.ld + base + i;
-                const f32x4 x0 = *(const f32x4 *)s, x1 = *(const f32x4 *)(s + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { v[e] += x0[e]; v[4 + e] += x1[e]; }
-            }
-        } else if (i < a.dim + a.rot) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                v[e] = turned(a, i - a.dim + e, (size_t)qpos, [&](int j) { return partial_at(qp, (size_t)qrow, base + a.dim + j); });
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) qf[ks][e] = (bf16)v[e];
-    }
+    latent_query<DK / 32>(a, qp, h, qrow, qpos, g, qf);
     float m = a.sink ? a.sink[h] * LOG2E : LOW, l = a.sink && g == 0 ? 1.0f : 0.0f;  // l: summed over g at the end
     f32x4 o[DV / 16];
 #pragma unroll
@@ -183,44 +290,12 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt(const LatentArgs a, co
                 s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)&s_k[(kt * 16 + r16) * KP + ks * 32 + g * 8], qf[ks],
                                                                 s[kt], 0, 0, 0);
         }
-        const bool whole = p0 + KT - 1 <= wq0;  // every key visible to every query
-        float mx = MASKED;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float z = s[kt][j] * c_in;
-                if (!whole) z = p0 + kt * 16 + 4 * g + j <= pos0 + qi ? z : MASKED;
-                s[kt][j] = z;
-                mx = fmaxf(mx, z);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m, mx);
-        const float corr = __builtin_amdgcn_exp2f(m - m_new);
-        m = m_new;
-        float sum = 0.0f;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                s[kt][j] = __builtin_amdgcn_exp2f(s[kt][j] - m_new);
-                sum += s[kt][j];
-            }
-        l = l * corr + sum;
-        if (__any(corr != 1.0f)) {
-#pragma unroll
-            for (int d = 0; d < DV / 16; ++d) o[d] *= corr;
-        }
+        // whole: every key visible to every query
+        latent_weights<DV / 16>(s, o, m, l, c_in, p0 + KT - 1 <= wq0, p0 + 4 * g, pos0 + qi);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
             bf16x8 hi, lo;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float w = s[2 * kb + (e >> 2)][e & 3];
-                hi[e] = (bf16)w;
-                lo[e] = (bf16)(w - (float)hi[e]);
-            }
+            latent_parts(s, kb, hi, lo);
 #pragma unroll
             for (int d = 0; d < DV / 16; ++d) {
                 const bf16x8 vt = *(const bf16x8 *)&s_v[(d * 16 + r16) * VP + kb * 32 + g * 8];
@@ -229,18 +304,105 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt(const LatentArgs a, co
             }
         }
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    if (qi >= n) return;
-    const float inv = 1.0f / l;
-    bf16 *dst = out + (size_t)qi * a.ldo + (size_t)h * a.vdim;
+    latent_store<DV / 16>(a, o, l, h, qi, n, g, out);
+}
+
+// Heads of 64 or 128 values and 64 rotated ones, values of 64 or 128: keys and values go to LDS as they lie, by direct loads into one of two
+// tiles, so that a tile is one barrier, and a lane's keys of a column come by transposing reads.  Blocks of 64 rows x 64 values; of
+// a row's eight pieces of 16 bytes the one for place p lies at p ^ (row & 7), for the banks.  The products and their order are k_latent_prompt's:
+// the same bits.  What bounds it: a wavefront's chain of a tile, 1.9 us of which 0.5 are the scores, 0.6 the softmax, 0.5 the outputs, over the longest
+// row of keys; k_latent_prompt's 2.6 had one more for values transposed on their way to LDS between two barriers.  us, 16 heads of 128 + 64, values of
+// 128: 2048 tokens 95 -> 65 (of the 30, 13 are the queries' loads and 7 the order of the workgroups), 200 tokens 25 -> 14; 32 heads, 1000 tokens 63 -> 38.
+template <int KD, int NV>
+__global__ __launch_bounds__(256, 2) void k_latent_prompt_direct(const LatentArgs a, const Partial qp, const bf16 *__restrict__ cache,
+                                                                 const bf16 *__restrict__ kv, int ldkv, bf16 *__restrict__ out, int n, int pos0, int head) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+    constexpr int QT = 64, KT = 64, NK = KD + 1, BLOCK = 64 * 64, TILE = (NK + NV) * BLOCK, ND = NV * 4;
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    __shared__ __align__(16) bf16 s_kv[2 * TILE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    // the longest rows of keys first; where a second workgroup per CU is all that is left, the shortest of those to the longest
+    const int h = blockIdx.x, i0 = ((int)blockIdx.y < head ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y - head) * QT;
+    const int last = pos0 + min(i0 + QT, n) - 1;
+    const int qi = i0 + 16 * wave + r16, qrow = min(qi, n - 1), qpos = pos0 + qrow;
+    const int wq0 = pos0 + i0 + 16 * wave, wq1 = wq0 + 15;
+    const bf16 *kh = kv + (size_t)h * a.dim, *vh = kv + (size_t)a.H * a.dim + (size_t)h * a.vdim, *kr = cache + a.kv_p;
+
+    // a wavefront's two loads of a block: rows 16 wave + 8 i + lane / 8
+    uint32_t at_kv[2], at_kr[2];
 #pragma unroll
-    for (int d = 0; d < DV / 16; ++d) {
-        const int c = d * 16 + 4 * g;
-        if (c < a.vdim) *(bf16x4 *)(dst + c) = __builtin_convertvector(o[d] * inv, bf16x4);
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t row = wave * 16 + i * 8 + (lane >> 3), piece = ((lane & 7) ^ (lane >> 3)) * 16;
+        at_kv[i] = row * (uint32_t)ldkv * 2 + piece;
+        at_kr[i] = row * (uint32_t)a.row * 2 + piece;
     }
-    if (h == a.H - 1)
-        for (int i = a.H * a.vdim + g; i < a.out_cols; i += 4) out[(size_t)qi * a.ldo + i] = (bf16)0.0f;
+    auto request = [&](int p0, int tile) __attribute__((always_inline)) {
+        const int rows = min(KT, last + 1 - p0);   // those behind the last come as zeros
+        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(kh + (size_t)p0 * ldkv), 0, rows * ldkv * 2, 0x00027000),
+                                     rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vh + (size_t)p0 * ldkv), 0, rows * ldkv * 2, 0x00027000),
+                                     rr = __builtin_amdgcn_make_buffer_rsrc((void *)(kr + (size_t)p0 * a.row), 0, rows * a.row * 2, 0x00027000);
+        auto *to = (__attribute__((address_space(3))) bf16 *)(s_kv + tile * TILE + wave * 1024);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int b = 0; b < KD; ++b) __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, to + b * BLOCK + i * 512, 16, at_kv[i] + b * 128, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, to + KD * BLOCK + i * 512, 16, at_kr[i], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < NV; ++b) __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to + (NK + b) * BLOCK + i * 512, 16, at_kv[i] + b * 128, 0, 0, 0);
+        }
+    };
+    request(0, 0);
+    bf16x8 qf[NK * 2];
+    latent_query<NK * 2>(a, qp, h, qrow, qpos, g, qf);
+    // a lane's places in a block: of key r16, pieces g and 4 + g; of keys 4 g + r16 / 4, values 16 d + 4 (r16 & 3) .. + 3
+    int at_k[2], at_v[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) at_k[i] = r16 * 64 + ((i * 4 + g) ^ (r16 & 7)) * 8;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int row = 4 * g + (r16 >> 2);
+        at_v[d] = row * 64 + ((d * 2 + ((r16 >> 1) & 1)) ^ (row & 7)) * 8 + (r16 & 1) * 4;
+    }
+    float m = a.sink ? a.sink[h] * LOG2E : LOW, l = a.sink && g == 0 ? 1.0f : 0.0f;  // l: summed over g at the end
+    f32x4 o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float c_in = a.scale * LOG2E;
+    for (int p0 = 0, tile = 0; p0 <= last; p0 += KT, tile ^= 1) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070);  // this tile is there, and the one in front of it is read
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (p0 + KT <= last) request(p0 + KT, tile ^ 1);
+        if (p0 > wq1) continue;  // nothing of the tile is visible to these 16 queries
+        const bf16 *t = s_kv + tile * TILE;
+        f32x4 s[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < NK * 2; ++ks)
+                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(t + (ks >> 1) * BLOCK + kt * 1024 + at_k[ks & 1]), qf[ks], s[kt], 0, 0, 0);
+        }
+        latent_weights<ND>(s, o, m, l, c_in, p0 + KT - 1 <= wq0, p0 + 4 * g, pos0 + qi);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            bf16x8 hi, lo;
+            latent_parts(s, kb, hi, lo);
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                auto *v = (__attribute__((address_space(3))) s16x4 *)(t + (NK + (d >> 2)) * BLOCK + kb * 2048 + at_v[d & 3]);
+                const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(v), v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(v + 256);
+                const bf16x8 vt = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, lo, o[d], 0, 0, 0);
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, hi, o[d], 0, 0, 0);
+            }
+        }
+    }
+    latent_store<ND>(a, o, l, h, qi, n, g, out);
+#endif
 }
 
 // ------------------------------------------------------------------ one wavefront per (query, head) or (head, split)
@@ -690,6 +852,23 @@ static bool prompt_tiles(candy_hip_device *dev, const LatentAttn &A, const Laten
     return false;
 }
 
+// Two tiles of keys and values in LDS are 80 KB of heads of 128 + 64 and values of 128, two workgroups a CU; wider heads would leave one.
+static bool prompt_direct(candy_hip_device *dev, const LatentAttn &A, const LatentArgs &a, int n, int pos0) {
+    const dim3 g((unsigned)a.H, (unsigned)((n + 63) / 64)), b(256);
+    const int cus = dev->num_cus, blocks = (int)g.y, head = a.H * blocks > cus && a.H * blocks <= 2 * cus ? std::min(blocks, (cus + a.H - 1) / a.H) : blocks;
+    // a tile's rows are within the offsets of a load
+    if (a.rot != 64 || (int64_t)64 * std::max<int64_t>(A.ukv->rows_pad, a.row) * 2 > 0x7FFFFFFF) return false;
+#define CANDY_LPD(KD, NV)                                                                                                          \
+    if (a.dim == KD * 64 && a.vdim == NV * 64) {                                                                                    \
+        hipLaunchKernelGGL((k_latent_prompt_direct<KD, NV>), g, b, 0, dev->stream, a, A.q, (const bf16 *)A.cache, (const bf16 *)A.kv, \
+                           (int)A.ukv->rows_pad, (bf16 *)A.out, n, pos0, head);                                                     \
+        return true;                                                                                                                \
+    }
+    CANDY_LPD(1, 1) CANDY_LPD(1, 2) CANDY_LPD(2, 1) CANDY_LPD(2, 2)
+#undef CANDY_LPD
+    return false;
+}
+
 int launch_latent_prompt(candy_hip_device *dev, const LatentAttn &A, int n, int pos0) {
     const LatentArgs a = latent_args(A);
     CANDY_REQUIRE(A.ukv->rows == (int64_t)a.H * (a.dim + a.vdim) && A.ukv->ld == a.kv_p && (n + 63) / 64 <= 65535, "internal: attention launch");
@@ -701,8 +880,9 @@ int launch_latent_prompt(candy_hip_device *dev, const LatentAttn &A, int n, int 
     if (A.f32) return prompt_rows<float>(dev, A, n, pos0);
     CANDY_REQUIRE(A.q.ld % 4 == 0 && A.q.stride % 4 == 0 && ((uintptr_t)A.q.p & 15) == 0, "internal: unaligned queries");
     const int dk = a.dim + a.rot;
-    bool done = false;
-    if (dk <= 64) done = prompt_tiles<64>(dev, A, a, n, pos0);
+    bool done = prompt_direct(dev, A, a, n, pos0);
+    if (done) {}
+    else if (dk <= 64) done = prompt_tiles<64>(dev, A, a, n, pos0);
     else if (dk <= 96) done = prompt_tiles<96>(dev, A, a, n, pos0);
     else if (dk <= 128) done = prompt_tiles<128>(dev, A, a, n, pos0);
     else if (dk <= 192) done = prompt_tiles<192>(dev, A, a, n, pos0);
