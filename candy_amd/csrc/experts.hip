@@ -37,6 +37,32 @@ struct Choice64 {
             if (lane == e) w = -INFINITY;
         }
     }
+    // two tokens' choices at once
+    static __device__ __forceinline__ void pick2(Choice64 (&c)[2], float s0, float s1, int E, int top) {
+        const int lane = threadIdx.x & 63;
+        const uint64_t all = E == 64 ? ~0ull : (1ull << E) - 1;
+        uint64_t left[2] = {all, all};
+        float w[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            c[t].v = w[t] = lane < E ? (t ? s1 : s0) : -INFINITY;
+            c[t].mine = -INFINITY;
+            c[t].id = 0;
+        }
+        for (int k = 0; k < top; ++k) {
+            float b[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) b[t] = wave_max(w[t]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (k == 0) c[t].best = b[t];
+                const int e = __ffsll((unsigned long long)(__ballot(w[t] == b[t]) & left[t])) - 1;
+                left[t] &= ~(1ull << e);
+                if (lane == k) { c[t].id = e; c[t].mine = b[t]; }
+                if (lane == e) w[t] = -INFINITY;
+            }
+        }
+    }
     __device__ __forceinline__ float weight(int E, int top) const {
         const int lane = threadIdx.x & 63;
         const float mx = fmaxf(best, LOW), sum = wave_sum(lane < E ? expf(v - mx) : 0.0f);
@@ -90,126 +116,165 @@ __device__ __forceinline__ void choose(const float *z, int E, int top, int *ids,
 }
 
 // ------------------------------------------------------------------ prompts
-constexpr int ROUTE_T = 16, ROUTE_W = 8, ROUTE_U = 4;   // tokens and wavefronts of a workgroup, K steps requested together
-// grid ceil(n / 16), 8 wavefronts that share K; 64 experts per round
+constexpr int ROUTE_T = 16, ROUTE_W = 8, ROUTE_K = 32 * ROUTE_W;   // tokens and wavefronts of a workgroup, values of K a stage
+constexpr int ROUTE_STAGE = 64 * ROUTE_K * 2 + ROUTE_T * ROUTE_K * 4;   // bytes: router rows, token rows
+// grid ceil(n / 16), 8 wavefronts that share K, a step of 32 values of a stage each; 64 experts per round.  What bounds it: latencies and
+// the way of 384 KB into one CU, whatever the number of tokens.  Operands loaded as they are needed were 16 rows of 64 bytes, 4 KB apart, to a
+// load, and another wavefront's 64 bytes of the same lines came again; by direct loads of whole lines, three stages in LDS: us of a launch, 64 experts at
+// width 2048, 128 / 2048 tokens 18.2 / 19.2 -> 11.3 / 13.0 (of which the choices, two tokens a wavefront side by side, 1.7).
+template <int STAGES>
 __global__ __launch_bounds__(64 * ROUTE_W) void k_route(const float *__restrict__ x, int64_t ldx, const bf16 *__restrict__ W, int ld, int E,
                                                         int top, int n, int *__restrict__ ids, float *__restrict__ weights) {
-    extern __shared__ __align__(16) float z[];        // [16][E] scores, then [4][64][17] sums of pairs of wavefronts
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
+    // [STAGES] of rows of 16-byte pieces, piece p of row r in slot p ^ (r & 15); once they are read, [8][64][17] sums of wavefronts.  Then [16][E] scores
+    extern __shared__ __align__(16) uint8_t lds[];
+    float *const red = (float *)lds, *const z = (float *)(lds + STAGES * ROUTE_STAGE);
     const int Ep = E | 1;                              // odd pitch
-    float *red = z + ROUTE_T * Ep;
-    int *s_ids = (int *)red;                           // once the scores stand: [16][top], [16][top]
-    float *s_w = red + ROUTE_T * top;
+    int *const s_ids = (int *)lds;                     // once the scores stand: [16][top], [16][top]
+    float *const s_w = red + ROUTE_T * top;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
-    const int t0 = blockIdx.x * ROUTE_T, steps = ld >> 5;
-    const float *xr = x + (size_t)min(t0 + r16, n - 1) * ldx + g * 8;
+    const int t0 = blockIdx.x * ROUTE_T, steps = ld >> 5, stages = (ld + ROUTE_K - 1) / ROUTE_K, rows = min(ROUTE_T, n - t0);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(x + (size_t)t0 * ldx), 0, (int)(rows * ldx * 4), 0x00027000),
+                                 rw = __builtin_amdgcn_make_buffer_rsrc((void *)W, 0, ((E + 15) & ~15) * ld * 2, 0x00027000);
+    constexpr int LW = 64 / 2 / ROUTE_W, LX = ROUTE_T / ROUTE_W, LOADS = LW + LX;   // a wavefront's: two router rows, a token's row each
     for (int e0 = 0; e0 < E; e0 += 64) {
+        uint32_t w_off[LW], x_off[LX];
+#pragma unroll
+        for (int i = 0; i < LW; ++i) {
+            const int r = (wave * LW + i) * 2 + (lane >> 5);
+            w_off[i] = (uint32_t)(e0 + r) * (uint32_t)ld * 2 + ((lane & 31) ^ (r & 15)) * 16;
+        }
+#pragma unroll
+        for (int i = 0; i < LX; ++i) x_off[i] = (uint32_t)(wave * LX + i) * (uint32_t)ldx * 4 + (lane ^ (wave * LX + i)) * 16;
+        auto request = [&](int k, int slot) __attribute__((always_inline)) {
+            auto *to = (__attribute__((address_space(3))) uint8_t *)(lds + slot * ROUTE_STAGE);
+#pragma unroll
+            for (int i = 0; i < LW; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, to + (wave * LW + i) * 1024, 16, w_off[i], k * ROUTE_K * 2, 0, 0);
+#pragma unroll
+            for (int i = 0; i < LX; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, to + 64 * ROUTE_K * 2 + (wave * LX + i) * 1024, 16, x_off[i], k * ROUTE_K * 4, 0, 0);
+        };
         f32x4 acc[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const bf16 *w = W + (size_t)(e0 + r16) * ld + g * 8;
-        const int strips = min(4, (E - e0 + 15) >> 4);
-        for (int s0 = wave; s0 < steps; s0 += ROUTE_W * ROUTE_U) {
-            f32x4 xv[ROUTE_U][2];
-            bf16x8 wv[ROUTE_U][4];
 #pragma unroll
-            for (int u = 0; u < ROUTE_U; ++u) {
-                const int k = min(s0 + u * ROUTE_W, steps - 1) * 32;
-                xv[u][0] = *(const f32x4 *)(xr + k);
-                xv[u][1] = *(const f32x4 *)(xr + k + 4);
+        for (int k = 0; k < STAGES - 1; ++k)
+            if (k < stages) request(k, k);
+        for (int k = 0, slot = 0; k < stages; ++k, slot = slot + 1 == STAGES ? 0 : slot + 1) {
+            // this stage is there, those behind it may be on their way; the one in front of it is read
+            asm volatile("" ::: "memory");
+            if (STAGES == 3 && k + 1 < stages) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);
+            else __builtin_amdgcn_s_waitcnt(0x0070);
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (k + STAGES - 1 < stages) request(k + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);
+            if (k * ROUTE_W + wave >= steps) continue;
+            const uint8_t *at = lds + slot * ROUTE_STAGE;
+            bf16x8 w[4], part[3];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (i < strips) wv[u][i] = *(const bf16x8 *)(w + (size_t)i * 16 * ld + k);
+            for (int i = 0; i < 4; ++i) w[i] = *(const bf16x8 *)(at + (i * 16 + r16) * (ROUTE_K * 2) + ((wave * 4 + g) ^ r16) * 16);
+            f32x4 xv[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) xv[i] = *(const f32x4 *)(at + 64 * ROUTE_K * 2 + r16 * (ROUTE_K * 4) + ((wave * 8 + g * 2 + i) ^ r16) * 16);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float f = xv[j >> 2][j & 3];
+                part[0][j] = (bf16)f;
+                const float r1 = f - (float)part[0][j];
+                part[1][j] = (bf16)r1;
+                part[2][j] = (bf16)(r1 - (float)part[1][j]);
             }
 #pragma unroll
-            for (int u = 0; u < ROUTE_U; ++u) {
-                if (s0 + u * ROUTE_W >= steps) break;
-                bf16x8 part[3];
+            for (int p = 2; p >= 0; --p)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float f = xv[u][j >> 2][j & 3];
-                    part[0][j] = (bf16)f;
-                    const float r1 = f - (float)part[0][j];
-                    part[1][j] = (bf16)r1;
-                    part[2][j] = (bf16)(r1 - (float)part[1][j]);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (i < strips) {
-#pragma unroll
-                        for (int p = 2; p >= 0; --p) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u][i], part[p], acc[i], 0, 0, 0);
-                    }
-            }
+                for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], part[p], acc[i], 0, 0, 0);
         }
+        __syncthreads();
         // lane: token r16, experts e0 + 16 i + 4 g + j
-        for (int half = 1; half >= 0; --half) {   // the second four wavefronts' sums, then the first four's on top
-            if (wave >> 2 == half) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        float *s = &red[((wave & 3) * 64 + i * 16 + 4 * g + j) * 17 + r16];
-                        *s = half ? acc[i][j] : *s + acc[i][j];
-                    }
-            }
-            __syncthreads();
-        }
+            for (int j = 0; j < 4; ++j) red[(wave * 64 + i * 16 + 4 * g + j) * 17 + r16] = acc[i][j];
+        __syncthreads();
         for (int i = tid; i < 64 * ROUTE_T; i += 64 * ROUTE_W) {
             const int t = i & 15, e = i >> 4;
             if (e0 + e >= E) continue;
-            float sum = 0.0f;
+            float v[ROUTE_W], sum = 0.0f;
 #pragma unroll
-            for (int v = 0; v < ROUTE_W / 2; ++v) sum += red[(v * 64 + e) * 17 + t];
+            for (int k = 0; k < ROUTE_W; ++k) v[k] = red[(k * 64 + e) * 17 + t];
+#pragma unroll
+            for (int k = 0; k < ROUTE_W / 2; ++k) sum += v[k + ROUTE_W / 2] + v[k];
             z[t * Ep + e0 + e] = ordered(sum);
         }
         __syncthreads();
     }
-    for (int t = wave; t < ROUTE_T; t += ROUTE_W) choose(z + t * Ep, E, top, s_ids + t * top, s_w + t * top);
+    static_assert(ROUTE_T == 2 * ROUTE_W, "two tokens a wavefront");
+    if (E <= 64) {   // side by side: a choice is a chain of reductions
+        Choice64 c[2];
+        Choice64::pick2(c, lane < E ? z[wave * Ep + lane] : 0.0f, lane < E ? z[(wave + ROUTE_W) * Ep + lane] : 0.0f, E, top);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float weight = c[k].weight(E, top);
+            if (lane < top) {
+                s_ids[(wave + k * ROUTE_W) * top + lane] = c[k].id;
+                s_w[(wave + k * ROUTE_W) * top + lane] = weight;
+            }
+        }
+    } else {
+        for (int t = wave; t < ROUTE_T; t += ROUTE_W) choose(z + t * Ep, E, top, s_ids + t * top, s_w + t * top);
+    }
     __syncthreads();
     for (int i = tid; i < ROUTE_T * top; i += 64 * ROUTE_W)
         if (t0 + i / top < n) {
             ids[(size_t)t0 * top + i] = s_ids[i];
             weights[(size_t)t0 * top + i] = s_w[i];
         }
+#endif
 }
 
 constexpr int MAX_EXPERTS = 1024;
 // One workgroup of 1024: perm[0 .. count) = the slots, expert by expert; tiles of at most `rows` of one expert each.
 __global__ __launch_bounds__(1024) void k_deal(const int *__restrict__ ids, int count, int E, int rows, int *__restrict__ perm,
                                                GroupTile *__restrict__ tiles, int *__restrict__ n_tiles) {
-    __shared__ int members[MAX_EXPERTS], end[2][MAX_EXPERTS], tile_end[2][MAX_EXPERTS];
+    __shared__ int members[MAX_EXPERTS], totals[2][MAX_EXPERTS / 64];
     const int tid = threadIdx.x;
     members[tid] = 0;
     __syncthreads();
-    constexpr int AHEAD = 4;
-    for (int i0 = tid; i0 < count; i0 += 1024 * AHEAD) {
-        int e[AHEAD];
+    // a thread's slots stay in registers between the count and the deal, up to 16 of them
+    constexpr int AHEAD = 16;
+    int e[AHEAD];
+    auto request = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < AHEAD; ++k) e[k] = ids[min(i0 + 1024 * k, count - 1)];
+        for (int k = 0; k < AHEAD; ++k)
+            if (i0 + 1024 * k < count) e[k] = ids[i0 + 1024 * k];
+    };
+    for (int i0 = tid; i0 < count; i0 += 1024 * AHEAD) {
+        request(i0);
 #pragma unroll
         for (int k = 0; k < AHEAD; ++k)
             if (i0 + 1024 * k < count) atomicAdd(&members[e[k]], 1);
     }
     __syncthreads();
     const int mine = members[tid], my_tiles = (mine + rows - 1) / rows;
-    int cur = 0;
-    end[0][tid] = mine;
-    tile_end[0][tid] = my_tiles;
-    __syncthreads();
-    for (int d = 1; d < MAX_EXPERTS; d <<= 1) {   // inclusive sums
-        end[cur ^ 1][tid] = end[cur][tid] + (tid >= d ? end[cur][tid - d] : 0);
-        tile_end[cur ^ 1][tid] = tile_end[cur][tid] + (tid >= d ? tile_end[cur][tid - d] : 0);
-        cur ^= 1;
-        __syncthreads();
+    // inclusive sums of a wavefront's 64 experts, then of the wavefronts in front
+    const int lane = tid & 63, wave = tid >> 6;
+    int end = mine, tile_end = my_tiles;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int m = __shfl_up(end, d, 64), t = __shfl_up(tile_end, d, 64);
+        if (lane >= d) { end += m; tile_end += t; }
     }
-    const int begin = end[cur][tid] - mine, tile0 = tile_end[cur][tid] - my_tiles;
+    if (lane == 63) { totals[0][wave] = end; totals[1][wave] = tile_end; }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) { end += totals[0][w]; tile_end += totals[1][w]; }
+    const int begin = end - mine, tile0 = tile_end - my_tiles;
     for (int k = 0; k < my_tiles; ++k) tiles[tile0 + k] = GroupTile{tid, begin + k * rows, min(rows, mine - k * rows), (uint16_t)tile0, (uint16_t)my_tiles};
-    if (tid == MAX_EXPERTS - 1) *n_tiles = tile_end[cur][tid];
+    if (tid == E - 1) *n_tiles = tile_end;
     members[tid] = begin;
     __syncthreads();
     for (int i0 = tid; i0 < count; i0 += 1024 * AHEAD) {
-        int e[AHEAD];
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) e[k] = ids[min(i0 + 1024 * k, count - 1)];
+        if (count > 1024 * AHEAD) request(i0);
 #pragma unroll
         for (int k = 0; k < AHEAD; ++k)
             if (i0 + 1024 * k < count) perm[atomicAdd(&members[e[k]], 1)] = i0 + 1024 * k;
@@ -429,9 +494,11 @@ static size_t down_lds(const candy_hip_expert_spec &s, size_t es) {
     const size_t K = (size_t)expert_row_values(s);
     return (K / DOWN_STEP + 1) * (DOWN_STEP / 64) * 8 + (K + 8) * es;
 }
-static size_t route_lds(const candy_hip_expert_spec &s) {
-    return ((size_t)ROUTE_T * (s.n_experts | 1) + std::max<size_t>(ROUTE_W / 2 * 64 * 17, 2 * ROUTE_T * (size_t)s.top)) * 4;
+// (what k_route asks for with two stages when there are many experts; the limit on their number is older than that)
+static bool too_many_experts(const candy_hip_expert_spec &s) {
+    return ((size_t)ROUTE_T * (s.n_experts | 1) + std::max<size_t>(ROUTE_W / 2 * 64 * 17, 2 * ROUTE_T * (size_t)s.top)) * 4 > 65536;
 }
+static size_t route_lds(const candy_hip_expert_spec &s, int stages) { return (size_t)stages * ROUTE_STAGE + (size_t)ROUTE_T * (s.n_experts | 1) * 4; }
 
 int check_expert_spec(const candy_hip_expert_spec &s, int d) {
     CANDY_REQUIRE(s.n_experts > 0 && s.n_experts <= MAX_EXPERTS / 2 && s.top > 0 && s.top <= s.n_experts, "choice of %d out of %d experts unsupported",
@@ -440,7 +507,7 @@ int check_expert_spec(const candy_hip_expert_spec &s, int d) {
     // one workgroup keeps a row's activations in the 64 KB of LDS a launch gets without asking
     CANDY_REQUIRE(up_lds(s, pad64(d), 4) <= 65536 && (int64_t)s.top * pad64(s.d_ff) + pad64(s.shared_ff) <= 1 << 24 && down_lds(s, 2) <= 65536,
                   "%d experts of %d (+ %d) at width %d are too wide for one row's kernels", s.top, s.d_ff, s.shared_ff, d);
-    CANDY_REQUIRE(route_lds(s) <= 65536, "too many experts (%d)", s.n_experts);
+    CANDY_REQUIRE(!too_many_experts(s), "too many experts (%d)", s.n_experts);
     return CANDY_HIP_OK;
 }
 
@@ -455,7 +522,11 @@ size_t expert_list_ints(const candy_hip_expert_spec &s, int n) { return deal_per
 int launch_experts_prompt(candy_hip_device *dev, const ExpertLayer &A, int n) {
     const candy_hip_expert_spec &s = A.s;
     const int rows = A.f32 ? 64 : grouped_tile_rows(s.n_experts, (int64_t)n * s.top, std::max<int64_t>(A.ld_act, pad64(s.d_ff)));
-    hipLaunchKernelGGL(k_route, dim3((unsigned)((n + ROUTE_T - 1) / ROUTE_T)), dim3(64 * ROUTE_W), route_lds(s), dev->stream, A.x, A.ldx,
+    const bool three = route_lds(s, 3) <= 160 * 1024;
+    const size_t lds = route_lds(s, three ? 3 : 2);
+    auto route = three ? k_route<3> : k_route<2>;
+    CANDY_HIP_TRY(hipFuncSetAttribute((const void *)route, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(route, dim3((unsigned)((n + ROUTE_T - 1) / ROUTE_T)), dim3(64 * ROUTE_W), lds, dev->stream, A.x, A.ldx,
                        (const bf16 *)A.w.router->data, (int)A.w.router->ld, s.n_experts, s.top, n, A.ids, A.weights);
     CANDY_LAUNCH_CHECK();
     int *n_tiles = A.list, *perm = A.list + 4;
