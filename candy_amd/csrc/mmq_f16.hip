@@ -273,7 +273,8 @@ __global__ __launch_bounds__(WN * WM * 64) void k_mmq_f16(const F16Group grp, co
 // 342, 2048 rows 1124 / 1052; Llama-2-7B shape 300 rows 311 / 308, 1400 rows 847 / 824.  A CU holds one such workgroup, so
 // the epilogue's vector instructions are exposed: with q8_level's branch asked value by value and the full division in
 // silu_f half of the gain was lost (1.035 against 1.058 at 1500 rows).
-enum { EPI_PLAIN, EPI_RES, EPI_SILU };
+// EPI_TAIL: EPI_RES in a grid whose last round is split (a kernel of its own: the others' prologues stay as short as they are).
+enum { EPI_PLAIN, EPI_RES, EPI_SILU, EPI_TAIL };
 // silu_f with the quotient corrected once by its own residual: the same bits for every f32 from SILU_ONCE up.  Below, the divisor's
 // reciprocal is too small for a normal number, and the full division is asked for, once for eight values (taken at a quarter instead,
 // value by value, prompts took 0.6 to 1.5 % longer).
@@ -298,9 +299,17 @@ static bool f16_roles_fit(int fmt, int64_t tile_rows, int64_t cols) {
     return fmt != CANDY_HIP_Q8_0 || tile_rows * (cols / 256 * BigQ8_0::BLOCK) <= 0xFFFFFFFFll;
 }
 
+// Of a grid of more workgroups than CUs, the tiles of a short last round split K over the CUs that would be idle (plan_tail):
+// tiles whole .. end are dealt to several workgroups of `sb` super-blocks each, behind the whole ones, which leave BM x BN sums in
+// `part`, [split][tile], for k_tail_sum.
+struct F16Tail {
+    float *part;
+    int whole, sb;
+};
+
 template <class F, int BN, int BM, int EPI>
 __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _Float16 *__restrict__ xh, int M, int K,
-                                                    int n_tiles, int m_tiles, int sb_per, size_t split_stride) {
+                                                    int n_tiles, int m_tiles, int sb_per, size_t split_stride, const F16Tail tail) {
     constexpr int PT = 256, BNB = 128;  // BNB: weight rows an LDS buffer has room for
     constexpr int ATK = BNB * 4 / PT;   // dequantization tasks per producer thread per step
     constexpr int TNF = BN / 16;        // 16-row weight fragments of the tile
@@ -318,10 +327,14 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    const int total = n_tiles * m_tiles;
-    const int split = blockIdx.x / total;
-    int v = blockIdx.x - split * total;
-    if ((total & 7) == 0) v = (v & 7) * (total >> 3) + (v >> 3);
+    const int total = n_tiles * m_tiles, whole = EPI == EPI_TAIL ? tail.whole : total;
+    const bool in_tail = EPI == EPI_TAIL && (int)blockIdx.x >= whole;
+    const int b = blockIdx.x - (in_tail ? whole : 0), group = in_tail ? total - whole : whole;
+    const int split = b / group;
+    int v = b - split * group;
+    if (in_tail) v += whole;
+    else if ((whole & 7) == 0) v = (v & 7) * (whole >> 3) + (v >> 3);
+    if (in_tail) sb_per = tail.sb;
     const int mt = v / n_tiles, nt = v - mt * n_tiles;
     static_assert(EPI != EPI_SILU || BN == 128, "64 rows of gate and of up");
     const F16Seg seg = EPI == EPI_SILU ? grp.seg[wave >> 1 & 1] : grp.pick(nt);  // producers 0, 1 gate and 2, 3 up
@@ -334,7 +347,7 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
     const int steps = n_sb * 4;
     const uint8_t *__restrict__ W = seg.W + (size_t)sb0 * F::BLOCK;
     xh += (size_t)sb0 * 8 * 512;  // 8 fragments of 32 values further along K, in every row block
-    float *out = seg.out + (size_t)split * split_stride;
+    float *out = EPI == EPI_TAIL ? seg.out : seg.out + (size_t)split * split_stride;
     const float *res = seg.res;
 
     if (wave < 4) {
@@ -528,6 +541,17 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
         }
     }
 
+    if (in_tail) {
+        float *to = tail.part + ((size_t)split * group + (v - whole)) * (BM * BN) + 4 * (lane >> 4);
+#pragma unroll
+        for (int tn = 0; tn < TNF; ++tn)
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm) {
+                const int m = cw * (BM / 4) + tm * 16 + (lane & 15);
+                if (m0 + m < M) *(float4 *)(to + m * BN + tn * 16) = make_float4(acc[tn][tm][0], acc[tn][tm][1], acc[tn][tm][2], acc[tn][tm][3]);
+            }
+        return;
+    }
     if constexpr (EPI == EPI_SILU) {
         // the arithmetic of k_silu_mul_quant (quantize_q8_lane4 + q8_lane4_to_half) value by value
 #pragma unroll
@@ -595,7 +619,7 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
             const int n = n0 + tn * 16 + 4 * (lane >> 4);
             if (m >= M) continue;
             float *dst = out + (size_t)m * N + n;
-            const float *r = EPI == EPI_RES && res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
+            const float *r = (EPI == EPI_RES || EPI == EPI_TAIL) && res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
             if (n + 3 < N && (N & 3) == 0) {
                 float4 o = make_float4(acc[tn][tm][0], acc[tn][tm][1], acc[tn][tm][2], acc[tn][tm][3]);
                 if (r) {
@@ -644,6 +668,36 @@ int launch_splitk_sum(candy_hip_device *dev, const float *part, float *y, const 
     return CANDY_HIP_OK;
 }
 
+// The last round's tiles: y = (res +) the copies in the order of K.  grid: tile, 8 of its activation rows.
+template <int BN, int BM>
+__global__ __launch_bounds__(256) void k_tail_sum(const F16Group grp, const float *__restrict__ part, int whole, int tiles, int splits, int n_tiles, int M) {
+    constexpr int Q = BN / 4;  // threads of a row
+    const int tid = threadIdx.x, row = blockIdx.y * 8 + tid / Q, col = (tid % Q) * 4;
+    const int v = whole + blockIdx.x, mt = v / n_tiles, nt = v - mt * n_tiles;
+    const F16Seg seg = grp.pick(nt);
+    const int m = mt * BM + row, n = (nt - seg.tile0) * BN + col;
+    if (tid >= 8 * Q || m >= M || n >= seg.N) return;
+    const float *p = part + (size_t)blockIdx.x * (BM * BN) + row * BN + col;
+    float4 s = *(const float4 *)p;
+    for (int k = 1; k < splits; ++k) {
+        const float4 a = *(const float4 *)(p + (size_t)k * tiles * (BM * BN));
+        s.x += a.x; s.y += a.y; s.z += a.z; s.w += a.w;
+    }
+    float *y = seg.out + (size_t)m * seg.N + n;
+    const float *r = seg.res ? seg.res + (size_t)m * seg.N + n : nullptr;  // may alias y: read before the store
+    if (n + 3 < seg.N && (seg.N & 3) == 0) {
+        if (r) {
+            const float4 a = *(const float4 *)r;
+            s = make_float4(a.x + s.x, a.y + s.y, a.z + s.z, a.w + s.w);
+        }
+        *(float4 *)y = s;
+    } else {
+        const float o[4] = {s.x, s.y, s.z, s.w};
+        for (int l = 0; l < 4; ++l)
+            if (n + l < seg.N) y[l] = r ? r[l] + o[l] : o[l];
+    }
+}
+
 // Up to three contractions that share the activations, in one launch (a single one: count = 1).  Every tensor but the
 // last has a multiple of BN rows (a tile belongs to one tensor).
 struct F16Job {
@@ -666,6 +720,28 @@ static int plan_split(const candy_hip_device *dev, int tiles, int n_sb) {
     }
     if (dev->opt.f16_split > 0) n_split = std::min(dev->opt.f16_split, n_sb);  // comparison runs
     return n_split;
+}
+
+// A grid whose last round has tiles for half the CUs at the most (Q4_K, whose rounds are the shortest: 0.4): these tiles split K, so that the round is as much shorter (at least
+// two super-blocks a workgroup; not for short K, where the second launch costs what the round does).  us of a call, whole tiles / last
+// round split: 11008 x 4096, 700 rows (258 tiles, two rounds for one and two tiles) Q4_K 104 / 84, Q6_K 122 / 92, Q8_0 126 / 95; 1500 rows
+// (516) 159 / 149, 187 / 163, 192 / 167; 14336 x 4096, 600 rows Q8_0 (336, the last 80 in three) 122 / 110.  Q4_K, half a round in two: prompts of the 7B shape, whose
+// q / k / v are 384 tiles at 1000 tokens, 2237 / 2261 (four layers and the head): a full chip's clock falls by what the round gains.
+struct TailPlan {
+    int whole, splits = 0, sb = 0;  // tiles not split; workgroups and super-blocks of each of the others, 0: there are none
+};
+static TailPlan plan_tail(const candy_hip_device *dev, int fmt, int64_t tiles, int n_sb) {
+    TailPlan p{(int)tiles};
+    const int t = (int)(tiles % dev->num_cus);
+    if (dev->opt.f16_shape != 0 || dev->opt.f16_split != 0 || n_sb < 8 || tiles < dev->num_cus || t == 0) return p;
+    if ((fmt == CANDY_HIP_Q4_K ? 5 : 4) * t > 2 * dev->num_cus) return p;
+    const int s = std::min(std::min(dev->num_cus / t, n_sb / 2), 16), sb = (n_sb + s - 1) / s, splits = (n_sb + sb - 1) / sb;
+    // of a round's super-blocks an eighth is left, with two for the first loads and the launch that sums, and 2.5 a chip full of tiles summed
+    if (8 * (2 * (n_sb - sb - 2) * dev->num_cus - 5 * t * splits) < 2 * n_sb * dev->num_cus) return p;
+    p.whole = (int)tiles - t;
+    p.sb = sb;
+    p.splits = splits;
+    return p;
 }
 
 // LDS of the role-split kernel: weight tiles, and the producers' slices
@@ -706,15 +782,40 @@ static int launch_big(candy_hip_device *dev, const F16Job *jobs, int count, cons
             off += (size_t)m * (size_t)jobs[s].w->rows;
         }
     }
+    TailPlan tail{tiles};
+    F16Tail tail_args{};
+    if (PC && n_split == 1) {
+        tail = plan_tail(dev, jobs[0].w->fmt, tiles, n_sb);
+        void *p = nullptr;
+        if (tail.splits) {
+            const int rc = splitk_workspace(dev, (size_t)tail.splits * (tiles - tail.whole) * BM * BN * sizeof(float), &p);
+            if (rc && rc != CANDY_HIP_ERR_OOM) return rc;
+            if (rc) {  // without the memory they stay whole
+                (void)hipGetLastError();
+                tail = TailPlan{tiles};
+            } else {
+                tail_args = F16Tail{(float *)p, tail.whole, tail.sb};
+            }
+        }
+    }
     constexpr size_t smem = PC ? pc_lds<F>() : (size_t)2 * (BN + BM) * BIG_BK * sizeof(_Float16);
     const bool epi_res = any_res && n_split == 1;
-    void (*kern)(const F16Group, const _Float16 *, int, int, int, int, int, size_t);
-    if constexpr (PC) kern = epi_res ? k_mmq_f16_pc<F, BN, BM, EPI_RES> : k_mmq_f16_pc<F, BN, BM, EPI_PLAIN>;
-    else kern = epi_res ? k_mmq_f16<F, BN, BM, WN, WM, true> : k_mmq_f16<F, BN, BM, WN, WM, false>;
-    CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * n_split)), dim3(WN * WM * 64), smem, dev->stream, grp, xh, (int)m, K,
-                       n_tiles, m_tiles, sb_per, split_stride);
-    CANDY_LAUNCH_CHECK();
+    const unsigned wgs = (unsigned)(tiles * n_split + (tiles - tail.whole) * (tail.splits - (tail.splits ? 1 : 0)));
+    auto launch = [&](auto kern, auto... more) -> int {
+        CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        hipLaunchKernelGGL(kern, dim3(wgs), dim3(WN * WM * 64), smem, dev->stream, grp, xh, (int)m, K, n_tiles, m_tiles, sb_per, split_stride, more...);
+        CANDY_LAUNCH_CHECK();
+        return CANDY_HIP_OK;
+    };
+    int rc;
+    if constexpr (PC) rc = tail.splits ? launch(k_mmq_f16_pc<F, BN, BM, EPI_TAIL>, tail_args) : epi_res ? launch(k_mmq_f16_pc<F, BN, BM, EPI_RES>, tail_args) : launch(k_mmq_f16_pc<F, BN, BM, EPI_PLAIN>, tail_args);
+    else rc = epi_res ? launch(k_mmq_f16<F, BN, BM, WN, WM, true>) : launch(k_mmq_f16<F, BN, BM, WN, WM, false>);
+    if (rc) return rc;
+    if (tail.splits) {
+        hipLaunchKernelGGL((k_tail_sum<BN, BM>), dim3((unsigned)(tiles - tail.whole), BM / 8), dim3(256), 0, dev->stream, grp, tail_args.part, tail.whole,
+                           tiles - tail.whole, tail.splits, n_tiles, (int)m);
+        CANDY_LAUNCH_CHECK();
+    }
     bool one_run = true;  // outputs end to end, no residual but a single job's
     for (int s = 1; s < count; ++s)
         one_run = one_run && !jobs[0].res && !jobs[s].res && jobs[s].y == jobs[s - 1].y + (size_t)m * (size_t)jobs[s - 1].w->rows;
@@ -778,8 +879,10 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
     const int shape = dev->opt.f16_shape;  // comparison runs
     const bool single = shape == 3 || !f16_roles_fit(fmt, std::min<int64_t>(128, *std::max_element(rows, rows + count)), cols);
     const int n_sb = (int)(cols >> 8);
-    // What the busiest CU does: rounds of workgroups x weight rows per tile x super-blocks per workgroup, x 8 (a step of 192
-    // activation rows: 7, of 256: 8; measured 0.84 to 0.88, the producers' share being the same).  0: not for these rows.
+    // What the busiest CU does: rounds of workgroups x weight rows per tile x super-blocks per workgroup, x 8000 (a step of 192
+    // activation rows: 7000, of 256: 8000; measured 0.84 to 0.88, the producers' share being the same).  A last round that is split counts
+    // with its super-blocks, what plan_tail sets off, and 3 % of it all where the sides are near each other, for Q4_K 6 (prompts of the
+    // 7B shape, 1300 tokens, q / k / v on 192-row tiles, whole / 256-row tiles, last round split 3003 / 3040).  0: not for these rows.
     auto cost = [&](int bn, int bm) -> int64_t {
         const int m_tiles = (int)((m + bm - 1) / bm);
         int64_t tiles = 0;
@@ -788,8 +891,12 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
             tiles += (rows[s] + bn - 1) / bn;
         }
         const int ns = plan_split(dev, (int)(tiles * m_tiles), n_sb), sb_per = (n_sb + ns - 1) / ns;
+        const TailPlan tail = single ? TailPlan{0} : plan_tail(dev, fmt, tiles * m_tiles, n_sb);
+        if (tail.splits)
+            return (((int64_t)(tail.whole / dev->num_cus) * n_sb + tail.sb + 2) * 1000 + 2500 * (tiles * m_tiles - tail.whole) * tail.splits * bm / (256 * dev->num_cus)) *
+                   bn * (bm == 192 ? 7 : 8) * (q4k ? 106 : 103) / 100;
         const int64_t wgs = tiles * m_tiles * ((n_sb + sb_per - 1) / sb_per);
-        return ((wgs + dev->num_cus - 1) / dev->num_cus) * bn * sb_per * (bm == 192 ? 7 : 8);
+        return ((wgs + dev->num_cus - 1) / dev->num_cus) * bn * sb_per * (bm == 192 ? 7 : 8) * 1000;
     };
     // Tiles of 112 weight rows where every tensor's rows divide by 112 and the grid then takes fewer row-steps of its
     // busiest CU (14336 rows: 128 tiles instead of 112, so 256 instead of 224 workgroups at 512 activation rows, 512
@@ -802,6 +909,7 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
     auto tile = [&](int bm) { return F16Tile{narrow(bm) ? 112 : 128, bm, single}; };
     // up to 128 activation rows: 128 x 128 tiles, K split over workgroups to fill the chip
     if (shape == 2 || m <= 128) return tile(128);
+    auto wide_cost = [&](int bm) { return narrow(bm) ? cost(112, bm) : cost(128, bm); };
     // up to 256 rows where the 128 x 128 tiles fill the chip and the 128 x 256 tiles would have to split K
     // (Q4_K 14336 x 4096 at 256 rows: 70.7 us against 80.3)
     int64_t n128 = 0;
@@ -827,15 +935,24 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
     // 138 / 116; 21760 x 2048 at 300 rows (340 and 510, the fullest grids that the rule takes) 60 / 47, 70 / 60, 69 / 59,
     // 80 / 64, 77 / 65; 9300 x 1024 at 890 rows 40 / 34, 45 / 41, 45 / 40, 52 / 44, 49 / 43.  Where it costs a round
     // more the wider tiles win: 32000 x 4096 at 300 rows, two against three, Q5_K and Q4_0 0.86x on the narrow ones.
+    // Not where the wider tiles' last round is split and that leaves less to do (a step of 128 rows counts 6, for Q4_K 5): 11008 x 4096 at
+    // 513 rows Q4_K 81 / 71, Q6_K 98 / 81, Q8_0 112 / 85; at 600 rows level, 98 / 91, 113 / 93.
     auto rounds = [&](int bm) { return (n128 * ((m + bm - 1) / bm) + dev->num_cus - 1) / dev->num_cus; };
-    if (shape == 0 && !narrow(256) && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256)) return tile(128);
+    auto tail_pays = [&](int bm) {
+        int64_t tiles = 0;
+        const int bn = narrow(bm) ? 112 : 128;
+        for (int s = 0; s < count; ++s) tiles += (rows[s] + bn - 1) / bn;
+        return plan_tail(dev, fmt, tiles * ((m + bm - 1) / bm), n_sb).splits && wide_cost(bm) < 950 * rounds(128) * n_sb * 128 * (q4k ? 5 : 6);
+    };
+    if (shape == 0 && !narrow(256) && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256) && !tail_pays(192) && !tail_pays(256))
+        return tile(128);
     // Tiles of 192 activation rows where they leave the busiest CU less to do: a last column of tiles that would be mostly
     // empty (300 rows are 2 x 192 as they are 2 x 256), or a grid that fills the rounds better (1300 rows against 4096
     // weight rows: 224 workgroups instead of 192).  Over thirteen weight shapes and seventeen row counts from 140 to 2048,
     // five formats, the rule takes them at 4 points of 10, 1.09x on the geometric mean there, 0.996x to 1.225x.  us before /
     // with them: Q4_K 14336 x 4096 at 300 rows 60.6 / 51.0, 4096 x 14336 at 560 rows 101 / 87.5; Q5_K 32000 x 4096 at 560
     // rows 199 / 179; Q8_0 11008 x 4096 at 300 rows 77 / 70; Q6_K 4096 x 4096 at 1300 rows 69.9 / 63.4.
-    const bool rows192 = shape == 0 && (narrow(192) ? cost(112, 192) : cost(128, 192)) < (narrow(256) ? cost(112, 256) : cost(128, 256));
+    const bool rows192 = shape == 0 && wide_cost(192) < wide_cost(256);
     return tile(rows192 ? 192 : 256);
 }
 
@@ -919,10 +1036,10 @@ static int launch_silu(candy_hip_device *dev, const candy_hip_qtensor *gate, con
     grp.seg[0] = F16Seg{(const uint8_t *)gate->data, nullptr, nullptr, N, 0};
     grp.seg[1] = F16Seg{(const uint8_t *)up->data, nullptr, nullptr, N, 0};
     constexpr size_t smem = pc_lds<F>();
-    void (*kern)(const F16Group, const _Float16 *, int, int, int, int, int, size_t) = k_mmq_f16_pc<F, 128, BM, EPI_SILU>;
+    auto kern = k_mmq_f16_pc<F, 128, BM, EPI_SILU>;
     CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3((unsigned)(n_tiles * m_tiles)), dim3(512), smem, dev->stream, grp, xh, (int)m, K, n_tiles, m_tiles,
-                       K >> 8, (size_t)0);
+                       K >> 8, (size_t)0, F16Tail{});
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;
 }
