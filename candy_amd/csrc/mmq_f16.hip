@@ -915,6 +915,10 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
     int64_t n128 = 0;
     for (int s = 0; s < count; ++s) n128 += (rows[s] + 127) / 128;
     const int64_t fill = (3 * (int64_t)dev->num_cus) / 4;
+    // up to 192 rows: one column of 192-row tiles, K split up to four ways, instead of two columns of 128.  us, 128 x 128 / 128 x 192:
+    // 11008 x 4096, 140 rows 43.7 / 35.9, 180 rows 44.0 / 37.5; 14336 x 4096 42.6 / 36.2, 43.0 / 38.9; 8192 x 2048 23.2 / 19.5, 23.5 /
+    // 21.8; level where eight would share a tile (4096 x 4096 22.9 / 22.9)
+    if (q4k && shape == 0 && !single && m <= 192 && n_sb >= 8 && 4 * n128 >= dev->num_cus) return tile(192);
     if (q4k && m <= 256 && n128 * ((m + 127) / 128) >= fill && n128 * ((m + 255) / 256) < fill) return tile(128);
     // short K (at most 16 super-blocks) on a grid that 128 x 256 tiles would have to split: 128 x 128 tiles halve the
     // split as long as they still fit one round (Q4_K 4096 x 4096 at 512 rows 35.5 against 36.8 us, at 1024 rows 50.9
