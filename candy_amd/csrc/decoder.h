@@ -66,14 +66,15 @@ struct candy_hip_decoder {
     candy::RecurrentState state;                // empty for models without recurrent layers
     float *h = nullptr;                         // residual stream of the token being decoded
     float *logits = nullptr;
-    unsigned long long *next_key = nullptr;     // greedy token of the last step as k_argmax_key leaves it; zero before a step
+    unsigned long long *next_key = nullptr;     // greedy token as k_argmax_key leaves it, of the last step that was asked for it
     int64_t *tok_id = nullptr;
     int *d_pos = nullptr;                       // position of the token being decoded (device copy)
-    hipGraph_t graph = nullptr;                 // the captured step (layers + head + argmax)
-    hipGraphExec_t graph_exec = nullptr;
+    // the captured step, layers and head; [1]: and the argmax, for callers that ask for the greedy token (a launch of 4 us)
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     bool graph_dirty = true;
     bool use_graph = true;
-    unsigned graph_epoch = 0;                   // the device's option epoch the graph was captured under
+    unsigned graph_epoch = 0;                   // the device's option epoch the graphs were captured under
     std::vector<void *> owned;                  // freed with the model
     std::vector<void *> prompt_owned;           // prompt buffers, replaced when a longer prompt comes
     int prompt_cap = 0;
@@ -86,7 +87,7 @@ struct candy_hip_decoder {
     virtual bool has_embedding() const = 0;
     // rows of the embedding table -> f32, width_pad apart
     virtual int embed(const int64_t *dev_ids, int64_t n, float *out) = 0;
-    // h (and the position in d_pos) -> every layer -> logits -> next_key; nothing allocates or synchronises, so that the
+    // h (and the position in d_pos) -> every layer -> logits; nothing allocates or synchronises, so that the
     // sequence can be captured once and replayed for every token
     virtual int enqueue_step() = 0;
     // puts what a step counts on (tickets) back to its initial state

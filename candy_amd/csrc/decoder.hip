@@ -64,11 +64,16 @@ static int check_order(const candy_hip_decoder *m, int32_t pos) {
     return CANDY_HIP_OK;
 }
 
-// chain_to: null, or where the token chosen by the previous step is recorded while it becomes this step's input
+// choose: the greedy token is wanted, here or by the step behind.  chain_to: null, or where the token chosen by the previous step is
+// recorded while it becomes this step's input
 static int decoder_step(candy_hip_decoder *m, int32_t pos, int64_t token, const float *dev_hidden,
-                        const float **dev_logits, int32_t *next_token, int32_t *chain_to = nullptr) {
+                        const float **dev_logits, int32_t *next_token, bool choose, int32_t *chain_to = nullptr) {
     candy_hip_device *dev = m->dev;
     int rc;
+    auto enqueue = [&]() -> int {
+        if (int e = m->enqueue_step()) return e;
+        return choose ? launch_argmax_key(dev, m->logits, m->vocab, m->next_key) : CANDY_HIP_OK;
+    };
     m->state.next = -1;
     if (chain_to)
         hipLaunchKernelGGL(k_chain_step, dim3(1), dim3(1), 0, dev->stream, m->d_pos, (int)pos, m->tok_id, m->next_key, chain_to);
@@ -83,26 +88,34 @@ static int decoder_step(candy_hip_decoder *m, int32_t pos, int64_t token, const 
     if (m->use_graph) {
         if (m->graph_epoch != dev->opt_epoch) m->graph_dirty = true;  // an option changed: other kernels may be due
         if (m->graph_dirty) {
-            // a replay of the old graph may still be in flight (a caller that did not ask for the token): drain first
-            if (m->graph_exec) CANDY_HIP_TRY(hipStreamSynchronize(dev->stream));
-            if (m->graph_exec) CANDY_HIP_TRY(hipGraphExecDestroy(m->graph_exec));
-            if (m->graph) CANDY_HIP_TRY(hipGraphDestroy(m->graph));
-            m->graph_exec = nullptr;
-            m->graph = nullptr;
+            // a replay of an old graph may still be in flight (a caller that did not ask for the token): drain first
+            if (m->graph_exec[0] || m->graph_exec[1]) CANDY_HIP_TRY(hipStreamSynchronize(dev->stream));
+            for (int g = 0; g < 2; ++g) {
+                if (m->graph_exec[g]) CANDY_HIP_TRY(hipGraphExecDestroy(m->graph_exec[g]));
+                m->graph_exec[g] = nullptr;
+                if (m->graph[g]) CANDY_HIP_TRY(hipGraphDestroy(m->graph[g]));
+                m->graph[g] = nullptr;
+            }
+            m->graph_dirty = false;
+            m->graph_epoch = dev->opt_epoch;
+        }
+        hipGraph_t &graph = m->graph[choose];
+        hipGraphExec_t &exec = m->graph_exec[choose];
+        if (!exec) {
+            if (graph) CANDY_HIP_TRY(hipGraphDestroy(graph));  // of a call that failed behind its capture
+            graph = nullptr;
             // kernels may count on their tickets being zero at launch and leave them so; a step that was cut short (an
             // error, a device reset) may not have: start every new graph from the initial state
             if ((rc = m->reset_step())) return rc;
             CANDY_HIP_TRY(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
-            rc = m->enqueue_step();
-            hipError_t e = hipStreamEndCapture(dev->stream, &m->graph);
+            rc = enqueue();
+            hipError_t e = hipStreamEndCapture(dev->stream, &graph);
             if (rc) return rc;
             CANDY_HIP_TRY(e);
-            CANDY_HIP_TRY(hipGraphInstantiate(&m->graph_exec, m->graph, nullptr, nullptr, 0));
-            m->graph_dirty = false;
-            m->graph_epoch = dev->opt_epoch;
+            CANDY_HIP_TRY(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
         }
-        CANDY_HIP_TRY(hipGraphLaunch(m->graph_exec, dev->stream));
-    } else if ((rc = m->enqueue_step())) {
+        CANDY_HIP_TRY(hipGraphLaunch(exec, dev->stream));
+    } else if ((rc = enqueue())) {
         (void)m->reset_step();  // see above
         return rc;
     }
@@ -153,8 +166,10 @@ int candy_hip_decoder_free(candy_hip_decoder *m) {
     if (!m) return CANDY_HIP_OK;
     (void)hipSetDevice(m->dev->ordinal);
     (void)hipStreamSynchronize(m->dev->stream);
-    if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-    if (m->graph) (void)hipGraphDestroy(m->graph);
+    for (int g = 0; g < 2; ++g) {
+        if (m->graph_exec[g]) (void)hipGraphExecDestroy(m->graph_exec[g]);
+        if (m->graph[g]) (void)hipGraphDestroy(m->graph[g]);
+    }
     for (void *p : m->owned) (void)candy_hip_free(m->dev, p);
     for (void *p : m->prompt_owned) (void)candy_hip_free(m->dev, p);
     if (m->row_logits) (void)candy_hip_free(m->dev, m->row_logits);
@@ -198,10 +213,10 @@ int candy_hip_decoder_prefill(candy_hip_decoder *m, const int32_t *tokens, int32
                                (size_t)m->width_pad * sizeof(float)))
         return rc;
     if (int rc = m->enqueue_head()) return rc;
-    if (int rc = launch_zero(dev, m->next_key, sizeof(unsigned long long))) return rc;  // no step kernel in front here
-    if (int rc = launch_argmax_key(dev, m->logits, m->vocab, m->next_key)) return rc;
     if (dev_logits) *dev_logits = m->logits;
     if (next_token) {
+        if (int rc = launch_zero(dev, m->next_key, sizeof(unsigned long long))) return rc;  // no step kernel in front here
+        if (int rc = launch_argmax_key(dev, m->logits, m->vocab, m->next_key)) return rc;
         unsigned long long key = 0;
         if (int rc = candy_hip_d2h(dev, &key, m->next_key, sizeof(key))) return rc;
         *next_token = (int32_t)argmax_key_index(key);
@@ -237,7 +252,7 @@ int candy_hip_decoder_decode_hidden(candy_hip_decoder *m, const float *dev_hidde
     if (int rc = m->check_complete()) return rc;
     if (int rc = check_order(m, pos)) return rc;
     if (int rc = use_device(m->dev)) return rc;
-    return decoder_step(m, pos, -1, dev_hidden, dev_logits, next_token);
+    return decoder_step(m, pos, -1, dev_hidden, dev_logits, next_token, next_token != nullptr);
 }
 
 int candy_hip_decoder_decode(candy_hip_decoder *m, int32_t token, int32_t pos, const float **dev_logits,
@@ -249,7 +264,7 @@ int candy_hip_decoder_decode(candy_hip_decoder *m, int32_t token, int32_t pos, c
     if (int rc = m->check_complete()) return rc;
     if (int rc = check_order(m, pos)) return rc;
     if (int rc = use_device(m->dev)) return rc;
-    return decoder_step(m, pos, token, nullptr, dev_logits, next_token);
+    return decoder_step(m, pos, token, nullptr, dev_logits, next_token, next_token != nullptr);
 }
 
 int candy_hip_decoder_generate(candy_hip_decoder *m, int32_t token, int32_t pos, int32_t n_steps, int32_t *tokens) {
@@ -264,8 +279,8 @@ int candy_hip_decoder_generate(candy_hip_decoder *m, int32_t token, int32_t pos,
     if (int rc = use_device(m->dev)) return rc;
     int32_t *list = nullptr;  // one slot per step; slot i takes the token step i chose
     if (int rc = candy_hip_alloc(m->dev, (size_t)(n_steps + 1) * sizeof(int32_t), (void **)&list)) return rc;
-    int rc = decoder_step(m, pos, token, nullptr, nullptr, nullptr);
-    for (int i = 1; i < n_steps && !rc; ++i) rc = decoder_step(m, pos + i, -1, nullptr, nullptr, nullptr, list + i - 1);
+    int rc = decoder_step(m, pos, token, nullptr, nullptr, nullptr, true);
+    for (int i = 1; i < n_steps && !rc; ++i) rc = decoder_step(m, pos + i, -1, nullptr, nullptr, nullptr, true, list + i - 1);
     if (!rc) {
         // the last step's choice: recorded by the same kernel, into a step that is not run (position and token
         // registers are rewritten by whatever step comes next)

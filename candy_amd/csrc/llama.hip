@@ -313,8 +313,7 @@ int candy_hip_llama::enqueue_step() {
         }
         if ((rc = linear_residual(m, L.down))) return rc;  // h += Wdown . act
     }
-    if ((rc = enqueue_head())) return rc;
-    return launch_argmax_key(dev, m->logits, c.vocab, m->next_key);
+    return enqueue_head();
 }
 
 int candy_hip_llama::enqueue_head() {

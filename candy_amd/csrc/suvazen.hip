@@ -187,8 +187,7 @@ int candy_hip_suvazen::enqueue_step() {
     Buffers B = dec;
     B.x = h;
     const DenseLaunch D = head_launch(B.act, 1, logits);
-    if (int rc = layers_forward(B, 1, 0, d_pos, h, &D)) return rc;
-    return launch_argmax_key(dev, logits, vocab, next_key);
+    return layers_forward(B, 1, 0, d_pos, h, &D);
 }
 
 int candy_hip_suvazen::enqueue_prompt(int n, int pos0) {
