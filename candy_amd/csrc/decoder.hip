@@ -1,5 +1,8 @@
 // The part of a decoder that does not depend on its layers (decoder.h): one token through the captured step, a prompt
 // in one pass, greedy generation without the host in the loop.
+#include <algorithm>
+#include <vector>
+
 #include "decoder.h"
 
 namespace candy {
@@ -19,6 +22,18 @@ __global__ void k_chain_step(int *pos_dst, int pos, int64_t *tok_dst, unsigned l
     *key = 0;
     *tok_dst = (int64_t)t;
     *list = (int32_t)t;
+}
+
+// A prompt's tokens travel as kernel arguments: a copy from the caller's memory has to end before the call may go on, and what runs
+// on the stream in front of it as well, so that the chip waits for the host at the start of every prompt.
+struct PromptIds {
+    static constexpr int N = 960;  // 4 KB of arguments
+    int32_t v[N];
+};
+constexpr int32_t IDS_MOST = 16 * PromptIds::N;  // more: copied
+__global__ __launch_bounds__(256) void k_prompt_ids(const PromptIds ids, int n, int64_t *__restrict__ dst) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = ids.v[i];
 }
 
 int decoder_init(candy_hip_decoder *m) {
@@ -136,11 +151,7 @@ static int decoder_feed(candy_hip_decoder *m, const int32_t *tokens, int32_t n_t
     CANDY_REQUIRE(tokens && n_tokens > 0, "prompt is empty");
     CANDY_REQUIRE(pos0 >= 0 && (int64_t)pos0 + n_tokens <= m->max_pos,
                   "positions %d..%lld outside the cache (max_pos %d)", pos0, (long long)pos0 + n_tokens - 1, m->max_pos);
-    std::vector<int64_t> ids((size_t)n_tokens);
-    for (int32_t i = 0; i < n_tokens; ++i) {
-        CANDY_REQUIRE(tokens[i] >= 0 && tokens[i] < m->vocab, "token %d outside the vocabulary", tokens[i]);
-        ids[(size_t)i] = tokens[i];
-    }
+    for (int32_t i = 0; i < n_tokens; ++i) CANDY_REQUIRE(tokens[i] >= 0 && tokens[i] < m->vocab, "token %d outside the vocabulary", tokens[i]);
     if (int rc = m->check_complete()) return rc;
     if (int rc = check_order(m, pos0)) return rc;
     if (int rc = use_device(m->dev)) return rc;
@@ -153,7 +164,18 @@ static int decoder_feed(candy_hip_decoder *m, const int32_t *tokens, int32_t n_t
         if (int rc = m->reserve_prompt(n_tokens)) return rc;
         m->prompt_cap = n_tokens;
     }
-    if (int rc = candy_hip_h2d(m->dev, m->prompt_ids, ids.data(), ids.size() * sizeof(int64_t))) return rc;
+    if (n_tokens <= IDS_MOST) {
+        for (int32_t i0 = 0; i0 < n_tokens; i0 += PromptIds::N) {
+            PromptIds part;
+            const int32_t n = std::min<int32_t>(PromptIds::N, n_tokens - i0);
+            std::copy(tokens + i0, tokens + i0 + n, part.v);
+            hipLaunchKernelGGL(k_prompt_ids, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->dev->stream, part, (int)n, m->prompt_ids + i0);
+            CANDY_LAUNCH_CHECK();
+        }
+    } else {
+        const std::vector<int64_t> ids(tokens, tokens + n_tokens);
+        if (int rc = candy_hip_h2d(m->dev, m->prompt_ids, ids.data(), ids.size() * sizeof(int64_t))) return rc;
+    }
     m->state.next = -1;
     if (int rc = m->enqueue_prompt(n_tokens, pos0)) return rc;
     m->state.next = pos0 + n_tokens;
