@@ -30,9 +30,13 @@ namespace candy {
 template <class F>
 constexpr int pieces() { return F::BLOCK % 16 == 0 ? F::BLOCK / 16 : (F::BLOCK + 14) / 16; }
 
+// Activation fragments whose sums meet in LDS at a time: half of them where all would be more than its 160 KB
+template <int RF, int MF>
+constexpr int sums_at_once() { return RF * MF > 20 ? (MF + 1) / 2 : MF; }
+
 template <class F, int RF, int MF>
 constexpr size_t lds_bytes() {
-    const size_t sums = (size_t)8 * RF * MF * 1024, slices = (size_t)8 * 1024 * ((RF * pieces<F>() + 3) / 4);
+    const size_t sums = (size_t)8 * RF * sums_at_once<RF, MF>() * 1024, slices = (size_t)8 * 1024 * ((RF * pieces<F>() + 3) / 4);
     return sums > slices ? sums : slices;
 }
 
@@ -131,27 +135,32 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last request writes its slice, which the sums are about to take
     }
-    __syncthreads();  // the slices are consumed
+    constexpr int MP = sums_at_once<RF, MF>();
 #pragma unroll
-    for (int i = 0; i < RF; ++i)
+    for (int t0 = 0; t0 < MF; t0 += MP) {
+        __syncthreads();  // the slices, or the sums in front, are consumed
 #pragma unroll
-        for (int t = 0; t < MF; ++t) sums[((wave * RF + i) * MF + t) * 64 + lane] = acc[i][t];
-    __syncthreads();
-    for (int f = wave; f < RF * MF; f += 8) {
-        const int m = (f % MF) * 16 + r16, n = n0 + (f / MF) * 16 + 4 * c;  // activation row; weight rows n .. n + 3
-        float4v s = sums[f * 64 + lane];
+        for (int i = 0; i < RF; ++i)
 #pragma unroll
-        for (int k = 1; k < 8; ++k) s += sums[(k * RF * MF + f) * 64 + lane];
-        if (m >= M) continue;
-        float *dst = y + (size_t)m * N + n;
-        const float *r = res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
-        if (n + 3 < N && (N & 3) == 0) {
-            if (r) s = *(const float4v *)r + s;
-            *(float4v *)dst = s;
-        } else {
+            for (int t = 0; t < MP; ++t)
+                if (t0 + t < MF) sums[((wave * RF + i) * MP + t) * 64 + lane] = acc[i][t0 + t];
+        __syncthreads();
+        for (int f = wave; f < RF * MP; f += 8) {
+            const int m = (t0 + f % MP) * 16 + r16, n = n0 + (f / MP) * 16 + 4 * c;  // activation row; weight rows n .. n + 3
+            float4v s = sums[f * 64 + lane];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (n + j < N) dst[j] = r ? r[j] + s[j] : s[j];
+            for (int k = 1; k < 8; ++k) s += sums[(k * RF * MP + f) * 64 + lane];
+            if (m >= M) continue;
+            float *dst = y + (size_t)m * N + n;
+            const float *r = res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
+            if (n + 3 < N && (N & 3) == 0) {
+                if (r) s = *(const float4v *)r + s;
+                *(float4v *)dst = s;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (n + j < N) dst[j] = r ? r[j] + s[j] : s[j];
+            }
         }
     }
 #endif
@@ -193,7 +202,11 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
     int rf = 1;
     while ((rows + 16 * rf - 1) / (16 * rf) > num_cus)
         if (++rf > 3) return 0;
-    if (rf == 3 && mf > 6) return 0;
+    // 48 weight rows beside more than 96 activation rows: seven fragments of these fit the registers, but for Q6_K, and eight for Q4_0;
+    // Q4_K's nine spilled registers cost what a sixth of the CUs idle does.  us of a call, tiles / here: 11008 x 4096, 100 rows Q4_K 30.3 /
+    // 24.6, Q5_K 32.3 / 27.9, Q8_0 38.0 / 31.1, Q4_0 38.3 / 26.4, Q6_K 35.8 / 34.8 (8208 x 4096 30.2 / 33.6); 128 rows Q4_K 31.6 / 29.1 (8208 x 4096
+    // 26.4 / 28.1, 10300 x 4096 27.5 / 29.1), Q5_K 33.5 / 33.8, Q8_0 39.4 / 40.6, Q4_0 40.0 / 29.4; 11008 x 2048, 100 rows Q4_K 22.5 / 15.5, Q8_0 26.1 / 18.4
+    if (rf == 3 && m > 96 && (q6k || (m > 112 && fmt != CANDY_HIP_Q4_0 && (fmt != CANDY_HIP_Q4_K || rows < 10752)))) return 0;
     if (mf * 32 * cols > 1200000) return 0;  // not measured
     const int64_t blocks = cols / 256, rounds = (blocks + 7) / 8, tiles = (rows + 127) / 128;
     // as plan_split() deals K to the tiles' workgroups
@@ -211,7 +224,8 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
 template <class F, int RF, int MF>
 constexpr bool reached() {
     constexpr bool q4k = std::is_same<F, BigQ4K>::value, q6k = std::is_same<F, BigQ6K>::value;
-    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= 6);
+    constexpr bool most = q4k || std::is_same<F, BigQ4_0<false>>::value;
+    return (MF > 4 || q4k || q6k) && (RF < 3 || MF <= 6 || (MF == 7 && !q6k) || (MF == 8 && most));
 }
 
 template <class F, int RF, int MF>
@@ -227,12 +241,13 @@ static int launch_rf(candy_hip_device *dev, const candy_hip_qtensor *w, const _F
 
 template <class F>
 static int launch_fmt(candy_hip_device *dev, const candy_hip_qtensor *w, const _Float16 *xh, int64_t m, float *y, const float *res) {
-    const int mf = fragments(m), rf = rows_fragments(w->fmt, w->rows, w->cols, m, dev->num_cus);
+    const int rf = rows_fragments(w->fmt, w->rows, w->cols, m, dev->num_cus), mf = rf == 3 && m > 96 && m <= 112 ? 7 : fragments(m);
 #define CANDY_RF(RF, MF)                    \
     if constexpr (reached<F, RF, MF>())     \
         if (rf == RF && mf == MF) return launch_rf<F, RF, MF>(dev, w, xh, m, y, res);
 #define CANDY_MF(MF) CANDY_RF(1, MF) CANDY_RF(2, MF) CANDY_RF(3, MF)
     CANDY_MF(3) CANDY_MF(4) CANDY_MF(5) CANDY_MF(6) CANDY_MF(8)
+    CANDY_RF(3, 7)
 #undef CANDY_MF
 #undef CANDY_RF
     return fail(CANDY_HIP_ERR_INVALID, "internal: fp16 contraction of %lld rows", (long long)m);
