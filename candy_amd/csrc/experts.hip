@@ -292,6 +292,12 @@ struct RowArgs {
 // four layers, before -> now: 288 / 396 -> 281 / 388.
 template <int R> constexpr int exp_unroll() { return 8 / R; }
 
+// k_expert_up: the row that a place of the grid stands for (those behind the last row: the last row), and whether the wavefront
+// whose places start at row0 has rows of chosen experts, so that it needs the choice.  Where there is no shared expert the last row is a
+// chosen expert's, and wavefronts wholly behind it read its weights as well.
+__host__ __device__ __forceinline__ int up_row(int place, int total) { return place < total ? place : total - 1; }
+__host__ __device__ __forceinline__ bool up_chooses(int row0, int total, int routed) { return up_row(row0, total) < routed; }
+
 // Rows of the concatenated up matrices, R per wavefront.  FEW: at most 64 experts, every wavefront that has rows of chosen experts
 // makes the choice for itself; scores and activations are requested in front of everything, the weights as soon as the choice
 // stands, and its shares are worked out while they come.  LDS: x; else also the scores and the choice.
@@ -322,8 +328,9 @@ __global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x,
             *(at4 *)&xs[i] = __builtin_convertvector(*(const f32x4 *)(x + i), at4);
     };
     Choice64 choice;
+    const bool chooses = FEW && up_chooses(row0, total, routed);
     if (FEW) {
-        if (row0 < routed) {
+        if (chooses) {
             choice.pick(ordered(score), a.E, a.top);
             if (blockIdx.x == 0 && wave == 0 && lane < a.top) sel[lane] = choice.id;
         }
@@ -344,7 +351,7 @@ __global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x,
     int of[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int row = min(row0 + r, total - 1), k = row / a.rows_e;
+        const int row = up_row(row0 + r, total), k = row / a.rows_e;
         of[r] = k;
         const bf16 *p = a.shared + (size_t)max(row - routed, 0) * a.ld;
         if (k < a.top) {
@@ -365,7 +372,7 @@ __global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x,
     fetch(vb, STEP);
     __builtin_amdgcn_sched_barrier(0);
     float share = 0.0f;
-    if (FEW && row0 < routed) share = choice.weight(a.E, a.top);
+    if (chooses) share = choice.weight(a.E, a.top);
 #pragma unroll
     for (int r = 0; r < R; ++r)
         scale[r] = of[r] >= a.top ? 1.0f : FEW ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(share), of[r])) : gate[of[r]];
@@ -668,4 +675,21 @@ extern "C" int candy_hip_experts(candy_hip_device *dev, const candy_hip_expert_s
     if (ids)
         if (int rc = candy_hip_d2d(dev, ids, A.ids, slots * 4)) return rc;
     return weights ? candy_hip_d2d(dev, weights, A.weights, slots * 4) : CANDY_HIP_OK;
+}
+
+// How many wavefronts of the launch that experts_row() makes for these widths read the choice without having made it, for a test of the rule
+// (no device needed).
+extern "C" int candy_test_unmade_choices(int num_cus, int top, int rows_e, int rows_s) {
+    candy_hip_device dev;
+    dev.num_cus = num_cus;
+    const int routed = top * rows_e, total = routed + rows_s;
+    const MvShape s = mv_shape(&dev, total);
+    const int per_wg = s.waves * s.rows, places = (total + per_wg - 1) / per_wg * per_wg;
+    int unmade = 0;
+    for (int row0 = 0; row0 < places; row0 += s.rows) {
+        bool reads = false;
+        for (int r = 0; r < s.rows; ++r) reads = reads || up_row(row0 + r, total) < routed;
+        unmade += reads && !up_chooses(row0, total, routed);
+    }
+    return unmade;
 }

@@ -58,3 +58,14 @@ def test_experts_of_one_row(dev, d, experts, top, ff, shared, act):
     want = case.oracle(x)[0]
     rows = np.concatenate([dev.experts(case.spec, act, case.dense, x[t:t + 1], decode=True) for t in range(3)])
     assert own(rows, want) < (1e-5 if act == hip.ACT_F32 else 1.5e-2)
+
+
+# wavefronts wholly behind the last row, which is a chosen expert's: workgroups of 11 x 1, 9 x 4 and 11 x 4 rows on 256 CUs
+@pytest.mark.parametrize("act", ACTS)
+@pytest.mark.parametrize("d,experts,top,ff", [(200, 4, 2, 1344), (136, 7, 6, 1408), (136, 64, 8, 1408)])
+def test_experts_without_a_shared_one_and_wavefronts_without_rows(dev, d, experts, top, ff, act):
+    case = Experts(dev, d, experts, top, ff, None, d)
+    x = sm.to_bf16(np.random.default_rng(d).standard_normal((3, d)) * 1.2)
+    want = case.oracle(x)[0]
+    rows = np.concatenate([dev.experts(case.spec, act, case.dense, x[t:t + 1], decode=True) for t in range(3)])
+    assert own(rows, want) < (1e-5 if act == hip.ACT_F32 else 1.5e-2)
