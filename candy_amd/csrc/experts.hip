@@ -300,7 +300,8 @@ __host__ __device__ __forceinline__ bool up_chooses(int row0, int total, int rou
 
 // Rows of the concatenated up matrices, R per wavefront.  FEW: at most 64 experts, every wavefront that has rows of chosen experts
 // makes the choice for itself; scores and activations are requested in front of everything, the weights as soon as the choice
-// stands, and its shares are worked out while they come.  LDS: x; else also the scores and the choice.
+// stands, and its shares are worked out while they come.  LDS: x and eight zeros; else behind x the scores, where the zeros go once
+// the choice stands, and the choice.
 template <class AT, int R, bool FEW>
 __global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x, const float *__restrict__ logits, AT *__restrict__ act,
                                                     int *__restrict__ sel, const RowArgs a) {
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x,
     extern __shared__ __align__(16) uint8_t lds[];
     AT *xs = (AT *)lds;
     AT *nothing = xs + a.ld;   // eight zeros
-    float *z = (float *)(nothing + 8), *gate = z + a.E;
+    float *z = (float *)nothing, *gate = z + a.E;
     int *ids = (int *)(gate + a.top);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x;
     const int routed = a.top * a.rows_e, total = routed + a.rows_s, row0 = (blockIdx.x * (threads >> 6) + wave) * R;
@@ -496,11 +497,14 @@ __global__ __launch_bounds__(1024) void k_expert_down(const AT *__restrict__ act
 int expert_row_values(const candy_hip_expert_spec &s) { return (int)(s.top * pad64(s.d_ff) + pad64(s.shared_ff)); }
 
 // LDS of the one-row kernels
-static size_t up_lds(const candy_hip_expert_spec &s, int64_t ld, size_t es) { return (size_t)(ld + 8) * es + (size_t)(s.n_experts + 2 * s.top) * 4; }
+static size_t up_lds(const candy_hip_expert_spec &s, int64_t ld, size_t es) {
+    return (size_t)ld * es + std::max((size_t)(s.n_experts + 2 * s.top) * 4, 8 * es);
+}
 static size_t down_lds(const candy_hip_expert_spec &s, size_t es) {
     const size_t K = (size_t)expert_row_values(s);
     return (K / DOWN_STEP + 1) * (DOWN_STEP / 64) * 8 + (K + 8) * es;
 }
+constexpr int64_t MOST_INNER = 29952;   // values of a row's inner activations: in bfloat16 beside 12 bytes for 64 of them, 64 KB
 // (what k_route asks for with two stages when there are many experts; the limit on their number is older than that)
 static bool too_many_experts(const candy_hip_expert_spec &s) {
     return ((size_t)ROUTE_T * (s.n_experts | 1) + std::max<size_t>(ROUTE_W / 2 * 64 * 17, 2 * ROUTE_T * (size_t)s.top)) * 4 > 65536;
@@ -512,7 +516,7 @@ int check_expert_spec(const candy_hip_expert_spec &s, int d) {
                   s.top, s.n_experts);
     CANDY_REQUIRE(s.d_ff > 0 && s.shared_ff >= 0 && s.d_ff <= 1 << 20 && s.shared_ff <= 1 << 20, "invalid expert widths %d / %d", s.d_ff, s.shared_ff);
     // one workgroup keeps a row's activations in the 64 KB of LDS a launch gets without asking
-    CANDY_REQUIRE(up_lds(s, pad64(d), 4) <= 65536 && (int64_t)s.top * pad64(s.d_ff) + pad64(s.shared_ff) <= 1 << 24 && down_lds(s, 2) <= 65536,
+    CANDY_REQUIRE(up_lds(s, pad64(d), 4) <= 65536 && (int64_t)s.top * pad64(s.d_ff) + pad64(s.shared_ff) <= MOST_INNER,
                   "%d experts of %d (+ %d) at width %d are too wide for one row's kernels", s.top, s.d_ff, s.shared_ff, d);
     CANDY_REQUIRE(!too_many_experts(s), "too many experts (%d)", s.n_experts);
     return CANDY_HIP_OK;
@@ -675,6 +679,16 @@ extern "C" int candy_hip_experts(candy_hip_device *dev, const candy_hip_expert_s
     if (ids)
         if (int rc = candy_hip_d2d(dev, ids, A.ids, slots * 4)) return rc;
     return weights ? candy_hip_d2d(dev, weights, A.weights, slots * 4) : CANDY_HIP_OK;
+}
+
+// The limits of a spec and what its one-row launches ask for, for a test (no device needed): 0 refused, 1 taken, -1 taken without room.
+extern "C" int candy_test_expert_spec(int n_experts, int top, int d_ff, int shared_ff, int d) {
+    candy_hip_expert_spec s{};
+    s.n_experts = n_experts; s.top = top; s.d_ff = d_ff; s.shared_ff = shared_ff;
+    if (check_expert_spec(s, d)) return 0;
+    for (size_t es : {2, 4})
+        if (up_lds(s, pad64(d), es) > 65536 || down_lds(s, es) > 163840) return -1;
+    return 1;
 }
 
 // How many wavefronts of the launch that experts_row() makes for these widths read the choice without having made it, for a test of the rule

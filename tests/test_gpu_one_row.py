@@ -60,6 +60,16 @@ def test_experts_of_one_row(dev, d, experts, top, ff, shared, act):
     assert own(rows, want) < (1e-5 if act == hip.ACT_F32 else 1.5e-2)
 
 
+# rows that leave LDS no more than the scores and the choice, which the zeros share where they are in it
+@pytest.mark.parametrize("act", ACTS)
+@pytest.mark.parametrize("d,experts,top", [(16320, 40, 12), (16320, 2, 1), (16256, 100, 14)])
+def test_experts_of_the_widest_rows(dev, d, experts, top, act):
+    case = Experts(dev, d, experts, top, 5, 70, top)
+    x = sm.to_bf16(np.random.default_rng(d).standard_normal((1, d)) * 1.2)
+    rows = dev.experts(case.spec, act, case.dense, x, decode=True)
+    assert own(rows, case.oracle(x)[0]) < (1e-5 if act == hip.ACT_F32 else 1.5e-2)
+
+
 # wavefronts wholly behind the last row, which is a chosen expert's: workgroups of 11 x 1, 9 x 4 and 11 x 4 rows on 256 CUs
 @pytest.mark.parametrize("act", ACTS)
 @pytest.mark.parametrize("d,experts,top,ff", [(200, 4, 2, 1344), (136, 7, 6, 1408), (136, 64, 8, 1408)])
