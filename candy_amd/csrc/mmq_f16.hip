@@ -722,11 +722,12 @@ static int plan_split(const candy_hip_device *dev, int tiles, int n_sb) {
     return n_split;
 }
 
-// A grid whose last round has tiles for half the CUs at the most (Q4_K, whose rounds are the shortest: 0.4): these tiles split K, so that the round is as much shorter (at least
-// two super-blocks a workgroup; not for short K, where the second launch costs what the round does).  us of a call, whole tiles / last
-// round split: 11008 x 4096, 700 rows (258 tiles, two rounds for one and two tiles) Q4_K 104 / 84, Q6_K 122 / 92, Q8_0 126 / 95; 1500 rows
-// (516) 159 / 149, 187 / 163, 192 / 167; 14336 x 4096, 600 rows Q8_0 (336, the last 80 in three) 122 / 110.  Q4_K, half a round in two: prompts of the 7B shape, whose
-// q / k / v are 384 tiles at 1000 tokens, 2237 / 2261 (four layers and the head): a full chip's clock falls by what the round gains.
+// A grid whose last round has tiles for half the CUs at the most (Q4_K, whose rounds are the shortest: 0.4): these tiles split K, so
+// that the round is as much shorter (two super-blocks a workgroup or more, of the last part one; not for short K, where the second
+// launch costs what the round does).  us of a call, whole tiles / last round split: 11008 x 4096, 700 rows (258 tiles, two rounds for one
+// and two tiles) Q4_K 104 / 84, Q6_K 122 / 92, Q8_0 126 / 95; 1500 rows (516) 159 / 149, 187 / 163, 192 / 167; 14336 x 4096, 600 rows
+// Q8_0 (336, the last 80 in three) 122 / 110.  Q4_K, half a round in two: prompts of the 7B shape, whose q / k / v are 384 tiles at 1000
+// tokens, 2237 / 2261 (four layers and the head): a full chip's clock falls by what the round gains.
 struct TailPlan {
     int whole, splits = 0, sb = 0;  // tiles not split; workgroups and super-blocks of each of the others, 0: there are none
 };
@@ -1079,6 +1080,20 @@ extern "C" int candy_test_f16_tile(int fmt, const int64_t *rows, int count, int6
     if (deferred) dev.defer_split = &pend;
     const candy::F16Tile t = candy::pick_tile(&dev, fmt, rows, count, cols, m);
     return (t.single ? -1 : 1) * (t.bn * 1000 + t.bm);
+}
+// tile, and plan: tiles, those of them that are whole, workgroups and super-blocks of each of the others (0: there are none), workgroups of every
+// tile where K is split throughout.
+extern "C" int candy_test_f16_tail(int fmt, const int64_t *rows, int count, int64_t cols, int64_t m, int num_cus, int deferred, int *plan) {
+    const int code = candy_test_f16_tile(fmt, rows, count, cols, m, num_cus, deferred), bn = std::abs(code) / 1000, bm = std::abs(code) % 1000;
+    candy_hip_device dev;
+    dev.num_cus = num_cus;
+    int64_t tiles = 0;
+    for (int s = 0; s < count; ++s) tiles += (rows[s] + bn - 1) / bn;
+    tiles *= (m + bm - 1) / bm;
+    const int n_sb = (int)(cols >> 8), all = candy::plan_split(&dev, (int)tiles, n_sb);
+    const candy::TailPlan t = all == 1 && code > 0 ? candy::plan_tail(&dev, fmt, tiles, n_sb) : candy::TailPlan{(int)tiles};
+    plan[0] = (int)tiles; plan[1] = t.whole; plan[2] = t.splits; plan[3] = t.sb; plan[4] = all;
+    return code;
 }
 extern "C" int candy_test_f16_silu(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
     candy_hip_device dev;
