@@ -46,7 +46,9 @@ __global__ __launch_bounds__(512, 2) void k_mmq_f16_rows(const uint8_t *__restri
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
     constexpr bool WHOLE = F::BLOCK % 16 == 0;  // pieces
     extern __shared__ __align__(16) uint8_t smem_raw[];
-    float4v *sums = (float4v *)smem_raw;  // [wave][RF][MF][lane]
+    // [wave][RF][sums_at_once][lane]; of an odd MF in halves the last slot of the second half is not written, and its activation rows (from
+    // 16 MF on) are not there
+    float4v *sums = (float4v *)smem_raw;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, c = lane >> 4;
     const int n0 = blockIdx.x * (16 * RF), first = wave;
     const int count = ((K >> 8) - first + 7) >> 3;  // super-blocks first, first + 8, ... of this wavefront (may be none)
@@ -283,3 +285,4 @@ int launch_mmq_f16_rows(candy_hip_device *dev, const candy_hip_qtensor *w, const
 extern "C" int candy_test_rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int num_cus) {
     return candy::rows_fragments(fmt, rows, cols, m, num_cus);
 }
+extern "C" int candy_test_rows_activation_fragments(int64_t m) { return candy::fragments(m); }
