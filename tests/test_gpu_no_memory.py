@@ -90,6 +90,29 @@ def test_prompt_without_memory_for_its_operands(dev):
     assert got[0] is None and same(got[-1], exact)
 
 
+@pytest.mark.parametrize("fmt,rows,cols,m", [(synth.Q4_K, 11008, 2048, 700), (synth.Q8_0, 21951, 3328, 289)])
+def test_tiles_without_memory_for_the_parts_of_their_last_round(dev, fmt, rows, cols, m):
+    """Grids whose last round is split along K: without the workspace its tiles stay whole."""
+    L = hip.lib()
+    w = dev.qtensor(fmt, rows, cols, synth.random_weight(fmt, rows, cols, seed=m))
+    src, dst = dev.from_numpy(synth.random_activations(m, cols, seed=rows)), dev.alloc(4 * m * rows)
+
+    def call():
+        hip._check(L.candy_hip_qmatmul(dev.handle, w.handle, src.ptr, m, dst.ptr))
+        return dst.download(np.float32, m * rows)
+
+    dev.set_option("mmq.f16_split", 1)
+    whole = call()
+    dev.set_option("mmq.f16_split", 0)
+    assert dev.get_option("runtime.split_workspace_bytes") == 0
+    LIB.candy_test_fail_alloc(dev.handle, 1)
+    assert np.array_equal(call().view(np.uint32), whole.view(np.uint32))
+    assert dev.get_option("runtime.split_workspace_bytes") == 0
+    got = call()  # with memory again: sums in another order
+    assert dev.get_option("runtime.split_workspace_bytes") > 0 and np.any(got != whole)
+    assert np.max(np.abs(got - whole)) <= max(2e-6, cols ** 0.5 * 2.0 ** -24) * np.max(np.abs(whole))
+
+
 @pytest.mark.parametrize("fmt,rows,m,mib", [(synth.Q4_1, 64, 100, 5), (synth.Q4_K, 512, 8, 1), (synth.Q8_0, 4096, 40, 1)])
 def test_the_workspace_holds_what_the_call_uses(dev, fmt, rows, m, mib):
     """Quants, their fp16 image and operands only where the kernel that runs reads them (8192 values a row, in whole MiB)."""
