@@ -142,7 +142,7 @@ __device__ __forceinline__ void latent_query(const LatentArgs &a, const Partial 
             for (int e = 0; e < 8; ++e) {
                 const int j = j0 + e;
                 const float x = v[ks][e >> 2][e & 3];
-                if (j < 2 * a.half) v[ks][e >> 2][e & 3] = 
+                if (j < 2 * a.half) v[ks][e >> 2][e & 3] =
                         j < a.half ? x * co[e >> 2][e & 3] - other[e >> 2][e & 3] * si[e >> 2][e & 3]
                                    : x * co[e >> 2][e & 3] + other[e >> 2][e & 3] * si[e >> 2][e & 3];
             }
@@ -880,13 +880,14 @@ int launch_latent_prompt(candy_hip_device *dev, const LatentAttn &A, int n, int 
     if (A.f32) return prompt_rows<float>(dev, A, n, pos0);
     CANDY_REQUIRE(A.q.ld % 4 == 0 && A.q.stride % 4 == 0 && ((uintptr_t)A.q.p & 15) == 0, "internal: unaligned queries");
     const int dk = a.dim + a.rot;
-    bool done = prompt_direct(dev, A, a, n, pos0);
-    if (done) {}
-    else if (dk <= 64) done = prompt_tiles<64>(dev, A, a, n, pos0);
-    else if (dk <= 96) done = prompt_tiles<96>(dev, A, a, n, pos0);
-    else if (dk <= 128) done = prompt_tiles<128>(dev, A, a, n, pos0);
-    else if (dk <= 192) done = prompt_tiles<192>(dev, A, a, n, pos0);
-    else if (dk <= 256) done = prompt_tiles<256>(dev, A, a, n, pos0);
+    bool done = dev->opt.latent_direct && prompt_direct(dev, A, a, n, pos0);
+    if (!done) {
+        if (dk <= 64) done = prompt_tiles<64>(dev, A, a, n, pos0);
+        else if (dk <= 96) done = prompt_tiles<96>(dev, A, a, n, pos0);
+        else if (dk <= 128) done = prompt_tiles<128>(dev, A, a, n, pos0);
+        else if (dk <= 192) done = prompt_tiles<192>(dev, A, a, n, pos0);
+        else if (dk <= 256) done = prompt_tiles<256>(dev, A, a, n, pos0);
+    }
     if (!done) return prompt_rows<bf16>(dev, A, n, pos0);
     CANDY_LAUNCH_CHECK();
     return CANDY_HIP_OK;

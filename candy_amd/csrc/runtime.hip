@@ -377,6 +377,7 @@ const OptionKey OPTION_KEYS[] = {
     {"fused.wide_waves", &candy::Options::wide_waves, 8, 16},
     {"fused.down_quant", &candy::Options::down_quant, 0, 1},
     {"prefill.attention_groups", &candy::Options::prefill_attention_groups, 0, 2},
+    {"prefill.latent_direct", &candy::Options::latent_direct, 0, 1},
     {"attention.splits", &candy::Options::attn_splits, 0, 64},
 };
 const OptionKey *find_option(const char *key) {

@@ -133,6 +133,8 @@ int candy_hip_synchronize(candy_hip_device *dev);       /* device.go:81 Synchron
  *   "prefill.attention_groups"   0        comparison runs: matrix-core prompt attention with one (1) or two (2) groups of
  *                                         wavefronts per query tile that take alternate key tiles (0: two, with 64 or 128
  *                                         queries by the size of the grid)
+ *   "prefill.latent_direct"      1        comparison runs: prompt attention over latents, bfloat16, by the kernel that loads keys
+ *                                         and values straight to LDS where it can (0: the one that transposes the values)
  * A decoder whose step has been captured into a graph notices a later candy_hip_set_option on its device and captures
  * the step again at its next decode call.
  * Read-only keys (candy_hip_get_option): "runtime.workspace_bytes", "runtime.split_workspace_bytes" - what the

@@ -21,6 +21,19 @@ def dev():
     d.close()
 
 
+def transposed(dev, call):
+    """The kernel that moves values to LDS transposed: the same products in the same order."""
+    dev.set_option("prefill.latent_direct", 0)
+    try:
+        return call()
+    finally:
+        dev.set_option("prefill.latent_direct", 1)
+
+
+def same_bits(a, b):
+    return np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 # rotated halves of whole eights and not; one tile and a row, tiles cut short in front of and behind the portion's start
 @pytest.mark.parametrize("heads,dim,rot,vdim", [(2, 64, 64, 64), (3, 64, 62, 128), (2, 128, 40, 64), (1, 128, 48, 128), (5, 120, 64, 100)])
 def test_portions(dev, heads, dim, rot, vdim):
@@ -30,7 +43,9 @@ def test_portions(dev, heads, dim, rot, vdim):
     for s in (sink, None):
         want = case.oracle(s, hip.ACT_BF16)
         for portions in ([n], [2, 62, 67], [64, 2, 65], [63, 68], [129, 2]):
-            assert rel(case.device(s, hip.ACT_BF16, portions), want) < TOL, (s is None, portions)
+            got = case.device(s, hip.ACT_BF16, portions)
+            assert rel(got, want) < TOL, (s is None, portions)
+            assert same_bits(got, transposed(dev, lambda: case.device(s, hip.ACT_BF16, portions))), (s is None, portions)
 
 
 # more workgroups than CUs, the rest of them in the other order: every block of queries is somebody's
@@ -38,4 +53,6 @@ def test_portions(dev, heads, dim, rot, vdim):
 def test_order_of_the_blocks(dev, heads, n):
     case = Latent(dev, gm.latent(heads, 64, 64, 64, 64, 32, 500.0, None)["mixer"], n, n)
     want = case.oracle(None, hip.ACT_BF16)
-    assert rel(case.device(None, hip.ACT_BF16, [n]), want) < TOL
+    got = case.device(None, hip.ACT_BF16, [n])
+    assert rel(got, want) < TOL
+    assert same_bits(got, transposed(dev, lambda: case.device(None, hip.ACT_BF16, [n])))
