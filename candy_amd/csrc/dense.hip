@@ -39,8 +39,8 @@ __device__ __forceinline__ float epilogue(float z, const EpiArgs &e) {
 
 // ------------------------------------------------------------------ one row
 // The norms in front of the contraction (launch_norm_chain's arithmetic), for a kernel that runs them in its prologue.  What its
-// first loads need are plain arguments of the kernel (they arrive in registers with the wavefront); this is the rest.  Biases, if
-// any, lie behind their weights (MvNorms::bias).
+// first loads need are plain arguments of the kernel (they arrive in registers with the wavefront); this is the rest.  A norm's bias
+// lies behind its weights; of two norms both have one (every norm of a Suvazen model has) or none has (Gulisun).
 struct NormPro {
     const float *step;
     float *x_out;
@@ -779,7 +779,7 @@ int launch_dense_norm(candy_hip_device *dev, const DenseLaunch &L, const NormArg
         A.x == A.x_out || nv > 2 || L.w->ld > (L.f32 ? mv_lds_values<float>() : mv_lds_values<bf16>()) || L.n_store > 64 * (int64_t)dev->num_cus)
         return CANDY_HIP_ERR_UNSUPPORTED;
     CANDY_REQUIRE(pad64(A.cols) == L.w->ld, "internal: norm and contraction of different widths");
-    // biases: of both norms or of none, each behind its weights
+    // biases: of both norms or of none, each behind its weights (as every model has them; others take two launches)
     const bool bias = A.pre_b || (A.y.p && A.post_b);
     if (bias && ((A.pre_w && A.pre_b != A.pre_w + L.w->ld) || (A.y.p && A.post_b != A.post_w + L.w->ld))) return CANDY_HIP_ERR_UNSUPPORTED;
     if (L.partial) *L.partial = Partial{(const float *)L.y, 1, 0, (int)L.ldy};
