@@ -918,8 +918,13 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
     const int64_t fill = (3 * (int64_t)dev->num_cus) / 4;
     // up to 192 rows: one column of 192-row tiles, K split up to four ways, instead of two columns of 128.  us, 128 x 128 / 128 x 192:
     // 11008 x 4096, 140 rows 43.7 / 35.9, 180 rows 44.0 / 37.5; 14336 x 4096 42.6 / 36.2, 43.0 / 38.9; 8192 x 2048 23.2 / 19.5, 23.5 /
-    // 21.8; level where eight would share a tile (4096 x 4096 22.9 / 22.9)
-    if (q4k && shape == 0 && !single && m <= 192 && n_sb >= 8 && 4 * n128 >= dev->num_cus) return tile(192);
+    // 21.8; level where eight would share a tile (4096 x 4096 22.9 / 22.9).  Not where the two columns are one round and need no split
+    // (more tiles than half the CUs) and K is so short that the sum of the copies costs more than the empty half of a column: 129 / 192
+    // rows 9216 x 2048 24.6 / 24.1, 24.9 / 25.9, 12288 x 2048 26.3 / 27.0, 26.5 / 29.2, 14336 x 2048 24.7 / 26.2, 24.9 / 27.8, 16384 x 2048
+    // 27.2 / 27.6, 27.4 / 29.1; 14336 x 2560 28.8 / 27.8, 29.1 / 30.6, 12288 x 2560 30.4 / 28.3, 30.8 / 30.4; 14336 x 2816 31.8 / 30.3, 31.4 /
+    // 32.8, 14336 x 3072 32.9 / 30.3, 33.2 / 33.2; 18432 x 2048, two rounds, 44.4 / 29.9, 45.5 / 31.4.
+    const bool whole128 = 4 * n128 > dev->num_cus && 2 * n128 <= dev->num_cus && n_sb <= (m <= 160 ? 9 : narrow(128) ? 11 : 10);
+    if (q4k && shape == 0 && !single && m <= 192 && n_sb >= 8 && 4 * n128 >= dev->num_cus && !whole128) return tile(192);
     if (q4k && m <= 256 && n128 * ((m + 127) / 128) >= fill && n128 * ((m + 255) / 256) < fill) return tile(128);
     // short K (at most 16 super-blocks) on a grid that 128 x 256 tiles would have to split: 128 x 128 tiles halve the
     // split as long as they still fit one round (Q4_K 4096 x 4096 at 512 rows 35.5 against 36.8 us, at 1024 rows 50.9

@@ -92,3 +92,14 @@ def test_where_the_norm_behind_sums_the_copies():
     for d_model in (8448, 11264):
         assert not any(behind(d_model, 3, layer, down) for layer in range(3) for down in (0, 1))
     assert tile((11264,), 1024, 200, False) == (128, 128) and tile((11264,), 1024, 200, True) != (128, 128)
+
+
+@pytest.mark.parametrize("rows,cols,m,want", [
+    # one column of 192-row tiles with K split beside two columns of 128 rows: where those are split too, more than a round, or K is long
+    (8192, 2048, 140, (128, 192)), (18432, 2048, 192, (128, 192)), (12288, 2560, 160, (128, 192)), (14336, 3072, 192, (112, 192)), (14336, 2816, 160, (112, 192)),
+    (11008, 4096, 140, (128, 192)), (14336, 4096, 180, (112, 192)),
+    # a round of whole 128-row tiles, K short: us on 192 / 128 rows 27.0 / 26.3, 29.2 / 26.5, 26.2 / 24.7, 27.8 / 24.9, 25.9 / 24.9, 30.6 / 29.1
+    (12288, 2048, 129, (128, 128)), (12288, 2048, 192, (128, 128)), (14336, 2048, 129, (112, 128)), (14336, 2048, 192, (112, 128)),
+    (9216, 2048, 192, (128, 128)), (14336, 2560, 192, (112, 128)), (14336, 2816, 192, (112, 128)), (16384, 2304, 192, (128, 128))])
+def test_one_column_of_192_rows_or_two_of_128(rows, cols, m, want):
+    assert tile((rows,), cols, m, False) == want
