@@ -123,6 +123,14 @@ def test_where_the_fitted_costs_cross(fmt, m, rows, cols, rf):
     assert chosen(fmt, m, rows, cols) == rf
 
 
+@pytest.mark.parametrize("rows,cols,rf", [(8208, 2048, 3), (8208, 3072, 3), (10880, 3072, 3), (8208, 3328, 0), (8208, 4096, 0), (10752, 4096, 0),
+                                          (10880, 4096, 0), (10881, 4096, 3), (10881, 3328, 3), (11008, 4096, 3), (12288, 4096, 3)])
+def test_eight_fragments_of_q4_k_where_rows_are_short_or_the_tiles_many(rows, cols, rf):
+    # the tiles are ahead where they share K by three (85 columns of them on 256 CUs at most) and rows are longer than 3072: us, 128 rows, tiles /
+    # here 10880 x 4096 28.1 / 29.1, 8208 x 3328 24.8 / 25.4; 8208 x 3072 23.9 / 22.6, 10896 x 4096 31.1 / 29.1
+    assert all(chosen(synth.Q4_K, m, rows, cols) == rf for m in (113, 120, 128))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols,m", [(2049, 2304, 48), (2063, 256, 80), (4099, 2304, 64), (4111, 2048, 48), (8209, 1280, 48)])
 def test_q6_k_blocks_behind_the_start_of_a_piece(dev, rows, cols, m):
