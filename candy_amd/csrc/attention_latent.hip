@@ -85,8 +85,8 @@ __global__ __launch_bounds__(256) void k_latent_rows(const LatentArgs a, const P
 }
 
 // ------------------------------------------------------------------ prompts, bfloat16, matrix cores
-// A query's values, rotated, as operands: lane (query, g) holds values 32 ks + 8 g .. + 7.  Everything of a step is requested before any of it is
-// used (value by value, each waiting for the one before, these loads took 20 us of a prompt's 105).
+// A query's values, rotated, as operands: lane (query, g) holds values 32 ks + 8 g .. + 7.  Everything of a step is requested before
+// any of it is used (value by value, each waiting for the one before, these loads took 20 us of a prompt's 105).
 template <int KS>
 __device__ __forceinline__ void latent_query(const LatentArgs &a, const Partial &qp, int h, int qrow, int qpos, int g, bf16x8 (&qf)[KS]) {
     const int width = a.dim + a.rot;
@@ -154,7 +154,8 @@ __device__ __forceinline__ void latent_query(const LatentArgs &a, const Partial 
 
 // One tile of 64 keys: scores (lane: one query, keys 16 kt + 4 g + j) -> weights; the outputs and l so far in proportion.
 template <int ND>
-__device__ __forceinline__ void latent_weights(f32x4 (&s)[4], f32x4 (&o)[ND], float &m, float &l, float c_in, bool whole, int first_key, int pos) {
+__device__ __forceinline__ void latent_weights(f32x4 (&s)[4], f32x4 (&o)[ND], float &m, float &l, float c_in, bool whole, int first_key,
+                                               int pos) {
     float mx = MASKED;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
@@ -307,15 +308,17 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt(const LatentArgs a, co
     latent_store<DV / 16>(a, o, l, h, qi, n, g, out);
 }
 
-// Heads of 64 or 128 values and 64 rotated ones, values of 64 or 128: keys and values go to LDS as they lie, by direct loads into one of two
-// tiles, so that a tile is one barrier, and a lane's keys of a column come by transposing reads.  Blocks of 64 rows x 64 values; of
-// a row's eight pieces of 16 bytes the one for place p lies at p ^ (row & 7), for the banks.  The products and their order are k_latent_prompt's:
-// the same bits.  What bounds it: a wavefront's chain of a tile, 1.9 us of which 0.5 are the scores, 0.6 the softmax, 0.5 the outputs, over the longest
-// row of keys; k_latent_prompt's 2.6 had one more for values transposed on their way to LDS between two barriers.  us, 16 heads of 128 + 64, values of
-// 128: 2048 tokens 95 -> 65 (of the 30, 13 are the queries' loads and 7 the order of the workgroups), 200 tokens 25 -> 14; 32 heads, 1000 tokens 63 -> 38.
+// Heads of 64 or 128 values and 64 rotated ones, values of 64 or 128: keys and values go to LDS as they lie, by direct loads into one
+// of two tiles, so that a tile is one barrier, and a lane's keys of a column come by transposing reads.  Blocks of 64 rows x 64
+// values; of a row's eight pieces of 16 bytes the one for place p lies at p ^ (row & 7), for the banks.  The products and their order
+// are k_latent_prompt's: the same bits.  What bounds it: a wavefront's chain of a tile, 1.9 us of which 0.5 are the scores, 0.6 the
+// softmax, 0.5 the outputs, over the longest row of keys; k_latent_prompt's 2.6 had one more for values transposed on their way to
+// LDS between two barriers.  us, 16 heads of 128 + 64, values of 128: 2048 tokens 95 -> 65 (of the 30, 13 are the queries' loads and
+// 7 the order of the workgroups), 200 tokens 25 -> 14; 32 heads, 1000 tokens 63 -> 38.
 template <int KD, int NV>
 __global__ __launch_bounds__(256, 2) void k_latent_prompt_direct(const LatentArgs a, const Partial qp, const bf16 *__restrict__ cache,
-                                                                 const bf16 *__restrict__ kv, int ldkv, bf16 *__restrict__ out, int n, int pos0, int head) {
+                                                                 const bf16 *__restrict__ kv, int ldkv, bf16 *__restrict__ out, int n,
+                                                                 int pos0, int head) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
     constexpr int QT = 64, KT = 64, NK = KD + 1, BLOCK = 64 * 64, TILE = (NK + NV) * BLOCK, ND = NV * 4;
     typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -340,17 +343,20 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt_direct(const LatentArg
     }
     auto request = [&](int p0, int tile) __attribute__((always_inline)) {
         const int rows = min(KT, last + 1 - p0);   // those behind the last come as zeros
-        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(kh + (size_t)p0 * ldkv), 0, rows * ldkv * 2, 0x00027000),
-                                     rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vh + (size_t)p0 * ldkv), 0, rows * ldkv * 2, 0x00027000),
-                                     rr = __builtin_amdgcn_make_buffer_rsrc((void *)(kr + (size_t)p0 * a.row), 0, rows * a.row * 2, 0x00027000);
+        auto from = [&](const bf16 *p, int ld) __attribute__((always_inline)) {
+            return __builtin_amdgcn_make_buffer_rsrc((void *)(p + (size_t)p0 * ld), 0, rows * ld * 2, 0x00027000);
+        };
+        const __amdgpu_buffer_rsrc_t rk = from(kh, ldkv), rv = from(vh, ldkv), rr = from(kr, a.row);
         auto *to = (__attribute__((address_space(3))) bf16 *)(s_kv + tile * TILE + wave * 1024);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
 #pragma unroll
-            for (int b = 0; b < KD; ++b) __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, to + b * BLOCK + i * 512, 16, at_kv[i] + b * 128, 0, 0, 0);
+            for (int b = 0; b < KD; ++b)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, to + b * BLOCK + i * 512, 16, at_kv[i] + b * 128, 0, 0, 0);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, to + KD * BLOCK + i * 512, 16, at_kr[i], 0, 0, 0);
 #pragma unroll
-            for (int b = 0; b < NV; ++b) __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to + (NK + b) * BLOCK + i * 512, 16, at_kv[i] + b * 128, 0, 0, 0);
+            for (int b = 0; b < NV; ++b)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to + (NK + b) * BLOCK + i * 512, 16, at_kv[i] + b * 128, 0, 0, 0);
         }
     };
     request(0, 0);
@@ -384,7 +390,8 @@ __global__ __launch_bounds__(256, 2) void k_latent_prompt_direct(const LatentArg
             s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < NK * 2; ++ks)
-                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(t + (ks >> 1) * BLOCK + kt * 1024 + at_k[ks & 1]), qf[ks], s[kt], 0, 0, 0);
+                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(t + (ks >> 1) * BLOCK + kt * 1024 + at_k[ks & 1]), qf[ks],
+                                                                s[kt], 0, 0, 0);
         }
         latent_weights<ND>(s, o, m, l, c_in, p0 + KT - 1 <= wq0, p0 + 4 * g, pos0 + qi);
 #pragma unroll
@@ -855,7 +862,8 @@ static bool prompt_tiles(candy_hip_device *dev, const LatentAttn &A, const Laten
 // Two tiles of keys and values in LDS are 80 KB of heads of 128 + 64 and values of 128, two workgroups a CU; wider heads would leave one.
 static bool prompt_direct(candy_hip_device *dev, const LatentAttn &A, const LatentArgs &a, int n, int pos0) {
     const dim3 g((unsigned)a.H, (unsigned)((n + 63) / 64)), b(256);
-    const int cus = dev->num_cus, blocks = (int)g.y, head = a.H * blocks > cus && a.H * blocks <= 2 * cus ? std::min(blocks, (cus + a.H - 1) / a.H) : blocks;
+    const int cus = dev->num_cus, blocks = (int)g.y;
+    const int head = a.H * blocks > cus && a.H * blocks <= 2 * cus ? std::min(blocks, (cus + a.H - 1) / a.H) : blocks;
     // a tile's rows are within the offsets of a load
     if (a.rot != 64 || (int64_t)64 * std::max<int64_t>(A.ukv->rows_pad, a.row) * 2 > 0x7FFFFFFF) return false;
 #define CANDY_LPD(KD, NV)                                                                                                          \

@@ -151,7 +151,8 @@ static int decoder_feed(candy_hip_decoder *m, const int32_t *tokens, int32_t n_t
     CANDY_REQUIRE(tokens && n_tokens > 0, "prompt is empty");
     CANDY_REQUIRE(pos0 >= 0 && (int64_t)pos0 + n_tokens <= m->max_pos,
                   "positions %d..%lld outside the cache (max_pos %d)", pos0, (long long)pos0 + n_tokens - 1, m->max_pos);
-    for (int32_t i = 0; i < n_tokens; ++i) CANDY_REQUIRE(tokens[i] >= 0 && tokens[i] < m->vocab, "token %d outside the vocabulary", tokens[i]);
+    for (int32_t i = 0; i < n_tokens; ++i)
+        CANDY_REQUIRE(tokens[i] >= 0 && tokens[i] < m->vocab, "token %d outside the vocabulary", tokens[i]);
     if (int rc = m->check_complete()) return rc;
     if (int rc = check_order(m, pos0)) return rc;
     if (int rc = use_device(m->dev)) return rc;
@@ -169,7 +170,8 @@ static int decoder_feed(candy_hip_decoder *m, const int32_t *tokens, int32_t n_t
             PromptIds part;
             const int32_t n = std::min<int32_t>(PromptIds::N, n_tokens - i0);
             std::copy(tokens + i0, tokens + i0 + n, part.v);
-            hipLaunchKernelGGL(k_prompt_ids, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->dev->stream, part, (int)n, m->prompt_ids + i0);
+            hipLaunchKernelGGL(k_prompt_ids, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->dev->stream, part, (int)n,
+                               m->prompt_ids + i0);
             CANDY_LAUNCH_CHECK();
         }
     } else {

@@ -84,8 +84,8 @@ template <int R> constexpr int mv_unroll() { return 8 / R; }                    
 // 705 / 665, of the fine Gulisun one 302 / 288.
 template <class AT, int R, int EPI, int NV>
 __global__ __launch_bounds__(1024) void k_dense_mv(const void *__restrict__ xv_, const bf16 *__restrict__ W, int K, int rows,
-                                                   const float *__restrict__ ny, const float *__restrict__ post_w, const float *__restrict__ pre_w,
-                                                   int flags, void *__restrict__ yv, int n_store, const EpiArgs ea, const NormPro np) {
+                                                   const float *__restrict__ ny, const float *__restrict__ post_w,
+                                                   const float *__restrict__ pre_w, int flags, void *__restrict__ yv, int n_store, const EpiArgs ea, const NormPro np) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
     constexpr int U = mv_unroll<R>(), STEP = U * 512, CH = mv_lds_values<AT>();
     __shared__ __align__(16) AT xs[CH];
@@ -100,13 +100,15 @@ __global__ __launch_bounds__(1024) void k_dense_mv(const void *__restrict__ xv_,
     constexpr int NT = 2;  // nontemporal
     __amdgpu_buffer_rsrc_t wr[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) wr[r] = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)min(row0 + r, rows - 1) * K), 0, (int)(2u * (uint32_t)K), 0x00027000);
+    for (int r = 0; r < R; ++r)
+        wr[r] = __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)min(row0 + r, rows - 1) * K), 0, (int)(2u * (uint32_t)K), 0x00027000);
     auto fetch = [&](u32x4v (&w)[R][U], int k0) __attribute__((always_inline)) {
         const uint32_t at = 2u * (uint32_t)k0 + (uint32_t)lane * 16;
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int r = 0; r < R; ++r) w[r][u] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[r], at + u * 1024, 0, NT));
+            for (int r = 0; r < R; ++r)
+                w[r][u] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(wr[r], at + u * 1024, 0, NT));
     };
     auto multiply = [&](const u32x4v (&w)[R][U], int k0) __attribute__((always_inline)) {
         const AT *xp = xs + (k0 & (CH - 1)) + lane * 8;
@@ -783,8 +785,8 @@ int launch_dense_norm(candy_hip_device *dev, const DenseLaunch &L, const NormArg
     const bool bias = A.pre_b || (A.y.p && A.post_b);
     if (bias && ((A.pre_w && A.pre_b != A.pre_w + L.w->ld) || (A.y.p && A.post_b != A.post_w + L.w->ld))) return CANDY_HIP_ERR_UNSUPPORTED;
     if (L.partial) *L.partial = Partial{(const float *)L.y, 1, 0, (int)L.ldy};
-    const MvNorms np{A.x, A.y.p, A.post_w, A.pre_w, (A.y.p ? MV_Y : 0) | (bias ? MV_BIAS : 0) | (A.rms ? MV_RMS : 0) | (A.pre_w ? MV_PRE : 0),
-                     NormPro{A.step, A.x_out, A.mult, A.eps, A.cols}};
+    const int flags = (A.y.p ? MV_Y : 0) | (bias ? MV_BIAS : 0) | (A.rms ? MV_RMS : 0) | (A.pre_w ? MV_PRE : 0);
+    const MvNorms np{A.x, A.y.p, A.post_w, A.pre_w, flags, NormPro{A.step, A.x_out, A.mult, A.eps, A.cols}};
     return L.f32 ? launch_mv<float>(dev, L, s, nv, np) : launch_mv<bf16>(dev, L, s, nv, np);
 }
 

@@ -118,15 +118,17 @@ __device__ __forceinline__ void choose(const float *z, int E, int top, int *ids,
 // ------------------------------------------------------------------ prompts
 constexpr int ROUTE_T = 16, ROUTE_W = 8, ROUTE_K = 32 * ROUTE_W;   // tokens and wavefronts of a workgroup, values of K a stage
 constexpr int ROUTE_STAGE = 64 * ROUTE_K * 2 + ROUTE_T * ROUTE_K * 4;   // bytes: router rows, token rows
-// grid ceil(n / 16), 8 wavefronts that share K, a step of 32 values of a stage each; 64 experts per round.  What bounds it: latencies and
-// the way of 384 KB into one CU, whatever the number of tokens.  Operands loaded as they are needed were 16 rows of 64 bytes, 4 KB apart, to a
-// load, and another wavefront's 64 bytes of the same lines came again; by direct loads of whole lines, three stages in LDS: us of a launch, 64 experts at
-// width 2048, 128 / 2048 tokens 18.2 / 19.2 -> 11.3 / 13.0 (of which the choices, two tokens a wavefront side by side, 1.7).
+// grid ceil(n / 16), 8 wavefronts that share K, a step of 32 values of a stage each; 64 experts per round.  What bounds it: latencies
+// and the way of 384 KB into one CU, whatever the number of tokens.  Operands loaded as they are needed were 16 rows of 64 bytes, 4
+// KB apart, to a load, and another wavefront's 64 bytes of the same lines came again; by direct loads of whole lines, three stages in
+// LDS: us of a launch, 64 experts at width 2048, 128 / 2048 tokens 18.2 / 19.2 -> 11.3 / 13.0 (of which the choices, two tokens a
+// wavefront side by side, 1.7).
 template <int STAGES>
 __global__ __launch_bounds__(64 * ROUTE_W) void k_route(const float *__restrict__ x, int64_t ldx, const bf16 *__restrict__ W, int ld, int E,
                                                         int top, int n, int *__restrict__ ids, float *__restrict__ weights) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass knows no buffer descriptors
-    // [STAGES] of rows of 16-byte pieces, piece p of row r in slot p ^ (r & 15); once they are read, [8][64][17] sums of wavefronts.  Then [16][E] scores
+    // [STAGES] of rows of 16-byte pieces, piece p of row r in slot p ^ (r & 15); once they are read, [8][64][17] sums of wavefronts.
+    // Then [16][E] scores
     extern __shared__ __align__(16) uint8_t lds[];
     float *const red = (float *)lds, *const z = (float *)(lds + STAGES * ROUTE_STAGE);
     const int Ep = E | 1;                              // odd pitch
@@ -134,7 +136,8 @@ __global__ __launch_bounds__(64 * ROUTE_W) void k_route(const float *__restrict_
     float *const s_w = red + ROUTE_T * top;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const int t0 = blockIdx.x * ROUTE_T, steps = ld >> 5, stages = (ld + ROUTE_K - 1) / ROUTE_K, rows = min(ROUTE_T, n - t0);
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(x + (size_t)t0 * ldx), 0, (int)(rows * ldx * 4), 0x00027000),
+    const __amdgpu_buffer_rsrc_t rx =
+                                     __builtin_amdgcn_make_buffer_rsrc((void *)(x + (size_t)t0 * ldx), 0, (int)(rows * ldx * 4), 0x00027000),
                                  rw = __builtin_amdgcn_make_buffer_rsrc((void *)W, 0, ((E + 15) & ~15) * ld * 2, 0x00027000);
     constexpr int LW = 64 / 2 / ROUTE_W, LX = ROUTE_T / ROUTE_W, LOADS = LW + LX;   // a wavefront's: two router rows, a token's row each
     for (int e0 = 0; e0 < E; e0 += 64) {
@@ -153,7 +156,8 @@ __global__ __launch_bounds__(64 * ROUTE_W) void k_route(const float *__restrict_
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, to + (wave * LW + i) * 1024, 16, w_off[i], k * ROUTE_K * 2, 0, 0);
 #pragma unroll
             for (int i = 0; i < LX; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, to + 64 * ROUTE_K * 2 + (wave * LX + i) * 1024, 16, x_off[i], k * ROUTE_K * 4, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, to + 64 * ROUTE_K * 2 + (wave * LX + i) * 1024, 16, x_off[i], k * ROUTE_K * 4,
+                                                         0, 0);
         };
         f32x4 acc[4];
 #pragma unroll
@@ -176,7 +180,8 @@ __global__ __launch_bounds__(64 * ROUTE_W) void k_route(const float *__restrict_
             for (int i = 0; i < 4; ++i) w[i] = *(const bf16x8 *)(at + (i * 16 + r16) * (ROUTE_K * 2) + ((wave * 4 + g) ^ r16) * 16);
             f32x4 xv[2];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) xv[i] = *(const f32x4 *)(at + 64 * ROUTE_K * 2 + r16 * (ROUTE_K * 4) + ((wave * 8 + g * 2 + i) ^ r16) * 16);
+            for (int i = 0; i < 2; ++i)
+                xv[i] = *(const f32x4 *)(at + 64 * ROUTE_K * 2 + r16 * (ROUTE_K * 4) + ((wave * 8 + g * 2 + i) ^ r16) * 16);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float f = xv[j >> 2][j & 3];
@@ -367,7 +372,8 @@ __global__ __launch_bounds__(1024) void k_expert_up(const float *__restrict__ x,
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[r][u] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(w[r], at + u * 1024, 0, NT));
+            for (int r = 0; r < R; ++r)
+                v[r][u] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(w[r], at + u * 1024, 0, NT));
     };
     fetch(va, 0);
     fetch(vb, STEP);
@@ -419,8 +425,8 @@ constexpr int DOWN_STEP = 4096;   // values the table of starts is padded to, at
 // Rows of the result: an expert's inner activations meet its down matrix, all of them one long sum.  LDS: the
 // activations, and per 64 of them where their weights start.
 template <class AT, int R>
-__global__ __launch_bounds__(1024) void k_expert_down(const AT *__restrict__ act, const int *__restrict__ sel, float *__restrict__ y, int d_p,
-                                                      const RowArgs a) {
+__global__ __launch_bounds__(1024) void k_expert_down(const AT *__restrict__ act, const int *__restrict__ sel, float *__restrict__ y,
+                                                      int d_p, const RowArgs a) {
     constexpr int U = exp_unroll<R>(), STEP = U * 512;
     static_assert(DOWN_STEP % STEP == 0, "whole steps");
     extern __shared__ __align__(16) uint8_t lds[];
@@ -440,7 +446,8 @@ __global__ __launch_bounds__(1024) void k_expert_down(const AT *__restrict__ act
     for (int i = tid; i < entries; i += threads) {
         const int k = (i << 6) / a.rows_e;
         base[i] = i >= chunks ? none
-                              : k < a.top ? 2 * ((int64_t)sel[k] * d_p * a.rows_e + ((i << 6) - k * a.rows_e)) : behind + 2 * (int64_t)((i << 6) - routed);
+                  : k < a.top ? 2 * ((int64_t)sel[k] * d_p * a.rows_e + ((i << 6) - k * a.rows_e))
+                              : behind + 2 * (int64_t)((i << 6) - routed);
     }
 #pragma unroll
     for (int i = 0; i < FIRST; ++i)
@@ -509,7 +516,9 @@ constexpr int64_t MOST_INNER = 29952;   // values of a row's inner activations: 
 static bool too_many_experts(const candy_hip_expert_spec &s) {
     return ((size_t)ROUTE_T * (s.n_experts | 1) + std::max<size_t>(ROUTE_W / 2 * 64 * 17, 2 * ROUTE_T * (size_t)s.top)) * 4 > 65536;
 }
-static size_t route_lds(const candy_hip_expert_spec &s, int stages) { return (size_t)stages * ROUTE_STAGE + (size_t)ROUTE_T * (s.n_experts | 1) * 4; }
+static size_t route_lds(const candy_hip_expert_spec &s, int stages) {
+    return (size_t)stages * ROUTE_STAGE + (size_t)ROUTE_T * (s.n_experts | 1) * 4;
+}
 
 int check_expert_spec(const candy_hip_expert_spec &s, int d) {
     CANDY_REQUIRE(s.n_experts > 0 && s.n_experts <= MAX_EXPERTS / 2 && s.top > 0 && s.top <= s.n_experts, "choice of %d out of %d experts unsupported",
@@ -691,8 +700,8 @@ extern "C" int candy_test_expert_spec(int n_experts, int top, int d_ff, int shar
     return 1;
 }
 
-// How many wavefronts of the launch that experts_row() makes for these widths read the choice without having made it, for a test of the rule
-// (no device needed).
+// How many wavefronts of the launch that experts_row() makes for these widths read the choice without having made it, for a test of
+// the rule (no device needed).
 extern "C" int candy_test_unmade_choices(int num_cus, int top, int rows_e, int rows_s) {
     candy_hip_device dev;
     dev.num_cus = num_cus;

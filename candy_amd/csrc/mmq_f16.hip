@@ -548,7 +548,8 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
 #pragma unroll
             for (int tm = 0; tm < TM; ++tm) {
                 const int m = cw * (BM / 4) + tm * 16 + (lane & 15);
-                if (m0 + m < M) *(float4 *)(to + m * BN + tn * 16) = make_float4(acc[tn][tm][0], acc[tn][tm][1], acc[tn][tm][2], acc[tn][tm][3]);
+                if (m0 + m < M)
+                    *(float4 *)(to + m * BN + tn * 16) = make_float4(acc[tn][tm][0], acc[tn][tm][1], acc[tn][tm][2], acc[tn][tm][3]);
             }
         return;
     }
@@ -619,7 +620,8 @@ __global__ __launch_bounds__(512) void k_mmq_f16_pc(const F16Group grp, const _F
             const int n = n0 + tn * 16 + 4 * (lane >> 4);
             if (m >= M) continue;
             float *dst = out + (size_t)m * N + n;
-            const float *r = (EPI == EPI_RES || EPI == EPI_TAIL) && res ? res + (size_t)m * N + n : nullptr;  // may alias dst: read before the store
+            // may alias dst: read before the store
+            const float *r = (EPI == EPI_RES || EPI == EPI_TAIL) && res ? res + (size_t)m * N + n : nullptr;
             if (n + 3 < N && (N & 3) == 0) {
                 float4 o = make_float4(acc[tn][tm][0], acc[tn][tm][1], acc[tn][tm][2], acc[tn][tm][3]);
                 if (r) {
@@ -670,7 +672,8 @@ int launch_splitk_sum(candy_hip_device *dev, const float *part, float *y, const 
 
 // The last round's tiles: y = (res +) the copies in the order of K.  grid: tile, 8 of its activation rows.
 template <int BN, int BM>
-__global__ __launch_bounds__(256) void k_tail_sum(const F16Group grp, const float *__restrict__ part, int whole, int tiles, int splits, int n_tiles, int M) {
+__global__ __launch_bounds__(256) void k_tail_sum(const F16Group grp, const float *__restrict__ part, int whole, int tiles, int splits, int n_tiles,
+                                                  int M) {
     constexpr int Q = BN / 4;  // threads of a row
     const int tid = threadIdx.x, row = blockIdx.y * 8 + tid / Q, col = (tid % Q) * 4;
     const int v = whole + blockIdx.x, mt = v / n_tiles, nt = v - mt * n_tiles;
@@ -737,7 +740,8 @@ static TailPlan plan_tail(const candy_hip_device *dev, int fmt, int64_t tiles, i
     if (dev->opt.f16_shape != 0 || dev->opt.f16_split != 0 || n_sb < 8 || tiles < dev->num_cus || t == 0) return p;
     if ((fmt == CANDY_HIP_Q4_K ? 5 : 4) * t > 2 * dev->num_cus) return p;
     const int s = std::min(std::min(dev->num_cus / t, n_sb / 2), 16), sb = (n_sb + s - 1) / s, splits = (n_sb + sb - 1) / sb;
-    // of a round's super-blocks an eighth is left, with two for the first loads and the launch that sums, and 2.5 a chip full of tiles summed
+    // of a round's super-blocks an eighth is left, with two for the first loads and the launch that sums, and 2.5 a chip full of
+    // tiles summed
     if (8 * (2 * (n_sb - sb - 2) * dev->num_cus - 5 * t * splits) < 2 * n_sb * dev->num_cus) return p;
     p.whole = (int)tiles - t;
     p.sb = sb;
@@ -804,17 +808,22 @@ static int launch_big(candy_hip_device *dev, const F16Job *jobs, int count, cons
     const unsigned wgs = (unsigned)(tiles * n_split + (tiles - tail.whole) * (tail.splits - (tail.splits ? 1 : 0)));
     auto launch = [&](auto kern, auto... more) -> int {
         CANDY_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-        hipLaunchKernelGGL(kern, dim3(wgs), dim3(WN * WM * 64), smem, dev->stream, grp, xh, (int)m, K, n_tiles, m_tiles, sb_per, split_stride, more...);
+        hipLaunchKernelGGL(kern, dim3(wgs), dim3(WN * WM * 64), smem, dev->stream, grp, xh, (int)m, K, n_tiles, m_tiles, sb_per,
+                           split_stride, more...);
         CANDY_LAUNCH_CHECK();
         return CANDY_HIP_OK;
     };
     int rc;
-    if constexpr (PC) rc = tail.splits ? launch(k_mmq_f16_pc<F, BN, BM, EPI_TAIL>, tail_args) : epi_res ? launch(k_mmq_f16_pc<F, BN, BM, EPI_RES>, tail_args) : launch(k_mmq_f16_pc<F, BN, BM, EPI_PLAIN>, tail_args);
-    else rc = epi_res ? launch(k_mmq_f16<F, BN, BM, WN, WM, true>) : launch(k_mmq_f16<F, BN, BM, WN, WM, false>);
+    if constexpr (PC)
+        rc = tail.splits ? launch(k_mmq_f16_pc<F, BN, BM, EPI_TAIL>, tail_args)
+             : epi_res   ? launch(k_mmq_f16_pc<F, BN, BM, EPI_RES>, tail_args)
+                         : launch(k_mmq_f16_pc<F, BN, BM, EPI_PLAIN>, tail_args);
+    else
+        rc = epi_res ? launch(k_mmq_f16<F, BN, BM, WN, WM, true>) : launch(k_mmq_f16<F, BN, BM, WN, WM, false>);
     if (rc) return rc;
     if (tail.splits) {
-        hipLaunchKernelGGL((k_tail_sum<BN, BM>), dim3((unsigned)(tiles - tail.whole), BM / 8), dim3(256), 0, dev->stream, grp, tail_args.part, tail.whole,
-                           tiles - tail.whole, tail.splits, n_tiles, (int)m);
+        hipLaunchKernelGGL((k_tail_sum<BN, BM>), dim3((unsigned)(tiles - tail.whole), BM / 8), dim3(256), 0, dev->stream, grp,
+                           tail_args.part, tail.whole, tiles - tail.whole, tail.splits, n_tiles, (int)m);
         CANDY_LAUNCH_CHECK();
     }
     bool one_run = true;  // outputs end to end, no residual but a single job's
@@ -894,7 +903,8 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
         const int ns = plan_split(dev, (int)(tiles * m_tiles), n_sb), sb_per = (n_sb + ns - 1) / ns;
         const TailPlan tail = single ? TailPlan{0} : plan_tail(dev, fmt, tiles * m_tiles, n_sb);
         if (tail.splits)
-            return (((int64_t)(tail.whole / dev->num_cus) * n_sb + tail.sb + 2) * 1000 + 2500 * (tiles * m_tiles - tail.whole) * tail.splits * bm / (256 * dev->num_cus)) *
+            return (((int64_t)(tail.whole / dev->num_cus) * n_sb + tail.sb + 2) * 1000 +
+                    2500 * (tiles * m_tiles - tail.whole) * tail.splits * bm / (256 * dev->num_cus)) *
                    bn * (bm == 192 ? 7 : 8) * (q4k ? 106 : 103) / 100;
         const int64_t wgs = tiles * m_tiles * ((n_sb + sb_per - 1) / sb_per);
         return ((wgs + dev->num_cus - 1) / dev->num_cus) * bn * sb_per * (bm == 192 ? 7 : 8) * 1000;
@@ -916,13 +926,14 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
     int64_t n128 = 0;
     for (int s = 0; s < count; ++s) n128 += (rows[s] + 127) / 128;
     const int64_t fill = (3 * (int64_t)dev->num_cus) / 4;
-    // up to 192 rows: one column of 192-row tiles, K split up to four ways, instead of two columns of 128.  us, 128 x 128 / 128 x 192:
-    // 11008 x 4096, 140 rows 43.7 / 35.9, 180 rows 44.0 / 37.5; 14336 x 4096 42.6 / 36.2, 43.0 / 38.9; 8192 x 2048 23.2 / 19.5, 23.5 /
-    // 21.8; level where eight would share a tile (4096 x 4096 22.9 / 22.9).  Not where the two columns are one round and need no split
-    // (more tiles than half the CUs) and K is so short that the sum of the copies costs more than the empty half of a column: 129 / 192
-    // rows 9216 x 2048 24.6 / 24.1, 24.9 / 25.9, 12288 x 2048 26.3 / 27.0, 26.5 / 29.2, 14336 x 2048 24.7 / 26.2, 24.9 / 27.8, 16384 x 2048
-    // 27.2 / 27.6, 27.4 / 29.1; 14336 x 2560 28.8 / 27.8, 29.1 / 30.6, 12288 x 2560 30.4 / 28.3, 30.8 / 30.4; 14336 x 2816 31.8 / 30.3, 31.4 /
-    // 32.8, 14336 x 3072 32.9 / 30.3, 33.2 / 33.2; 18432 x 2048, two rounds, 44.4 / 29.9, 45.5 / 31.4.
+    // up to 192 rows: one column of 192-row tiles, K split up to four ways, instead of two columns of 128.  us, 128 x 128 / 128 x
+    // 192: 11008 x 4096, 140 rows 43.7 / 35.9, 180 rows 44.0 / 37.5; 14336 x 4096 42.6 / 36.2, 43.0 / 38.9; 8192 x 2048 23.2 / 19.5,
+    // 23.5 / 21.8; level where eight would share a tile (4096 x 4096 22.9 / 22.9).  Not where the two columns are one round and need
+    // no split (more tiles than half the CUs) and K is so short that the sum of the copies costs more than the empty half of a
+    // column: 129 / 192 rows 9216 x 2048 24.6 / 24.1, 24.9 / 25.9, 12288 x 2048 26.3 / 27.0, 26.5 / 29.2, 14336 x 2048 24.7 / 26.2,
+    // 24.9 / 27.8, 16384 x 2048 27.2 / 27.6, 27.4 / 29.1; 14336 x 2560 28.8 / 27.8, 29.1 / 30.6, 12288 x 2560 30.4 / 28.3, 30.8 /
+    // 30.4; 14336 x 2816 31.8 / 30.3, 31.4 / 32.8, 14336 x 3072 32.9 / 30.3, 33.2 / 33.2; 18432 x 2048, two rounds, 44.4 / 29.9, 45.5
+    // / 31.4.
     const bool whole128 = 4 * n128 > dev->num_cus && 2 * n128 <= dev->num_cus && n_sb <= (m <= 160 ? 9 : narrow(128) ? 11 : 10);
     if (q4k && shape == 0 && !single && m <= 192 && n_sb >= 8 && 4 * n128 >= dev->num_cus && !whole128) return tile(192);
     if (q4k && m <= 256 && n128 * ((m + 127) / 128) >= fill && n128 * ((m + 255) / 256) < fill) return tile(128);
@@ -952,7 +963,8 @@ static F16Tile pick_tile(const candy_hip_device *dev, int fmt, const int64_t *ro
         int64_t tiles = 0;
         const int bn = narrow(bm) ? 112 : 128;
         for (int s = 0; s < count; ++s) tiles += (rows[s] + bn - 1) / bn;
-        return plan_tail(dev, fmt, tiles * ((m + bm - 1) / bm), n_sb).splits && wide_cost(bm) < 950 * rounds(128) * n_sb * 128 * (q4k ? 5 : 6);
+        return plan_tail(dev, fmt, tiles * ((m + bm - 1) / bm), n_sb).splits &&
+               wide_cost(bm) < 950 * rounds(128) * n_sb * 128 * (q4k ? 5 : 6);
     };
     if (shape == 0 && !narrow(256) && n128 * ((m + 255) / 256) >= fill && rounds(128) <= rounds(256) && !tail_pays(192) && !tail_pays(256))
         return tile(128);
@@ -1086,10 +1098,11 @@ extern "C" int candy_test_f16_tile(int fmt, const int64_t *rows, int count, int6
     const candy::F16Tile t = candy::pick_tile(&dev, fmt, rows, count, cols, m);
     return (t.single ? -1 : 1) * (t.bn * 1000 + t.bm);
 }
-// tile, and plan: tiles, those of them that are whole, workgroups and super-blocks of each of the others (0: there are none), workgroups of every
-// tile where K is split throughout.
+// tile, and plan: tiles, those of them that are whole, workgroups and super-blocks of each of the others (0: there are none),
+// workgroups of every tile where K is split throughout.
 extern "C" int candy_test_f16_tail(int fmt, const int64_t *rows, int count, int64_t cols, int64_t m, int num_cus, int deferred, int *plan) {
-    const int code = candy_test_f16_tile(fmt, rows, count, cols, m, num_cus, deferred), bn = std::abs(code) / 1000, bm = std::abs(code) % 1000;
+    const int code = candy_test_f16_tile(fmt, rows, count, cols, m, num_cus, deferred);
+    const int bn = std::abs(code) / 1000, bm = std::abs(code) % 1000;
     candy_hip_device dev;
     dev.num_cus = num_cus;
     int64_t tiles = 0;

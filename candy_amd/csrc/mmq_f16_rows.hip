@@ -201,20 +201,20 @@ static int rows_fragments(int fmt, int64_t rows, int64_t cols, int64_t m, int nu
     const bool q6k = fmt == CANDY_HIP_Q6_K;
     // up to 64 rows the other formats are on the exact tiles (mmq_f16_big_covers)
     if (m > 128 || (m <= 64 && !q6k && fmt != CANDY_HIP_Q4_K) || rows < 2048 || cols % 256 != 0) return 0;
-    // (seven fragments are weighed as eight: where those were behind the tiles, the exact kernel of rows_i8.hip is ahead, 4096 x 4096, 104 rows
-    // Q4_K 15.1 there / 18.9 here)
+    // (seven fragments are weighed as eight: where those were behind the tiles, the exact kernel of rows_i8.hip is ahead, 4096 x
+    // 4096, 104 rows Q4_K 15.1 there / 18.9 here)
     const int mf = m > 96 ? 8 : fragments(m);
     int rf = 1;
     while ((rows + 16 * rf - 1) / (16 * rf) > num_cus)
         if (++rf > 3) return 0;
     const int64_t blocks = cols / 256, rounds = (blocks + 7) / 8, tiles = (rows + 127) / 128;
-    // 48 weight rows beside more than 96 activation rows: seven fragments of these fit the registers, but for Q6_K, and eight for Q4_0.
-    // us of a call, tiles / here: 11008 x 4096, 100 rows Q4_K 30.3 / 24.6, Q5_K 32.3 / 27.9, Q8_0 38.0 / 31.1, Q4_0 38.3 / 26.4, Q6_K 35.8 / 34.8
-    // (8208 x 4096 30.2 / 33.6); 128 rows Q5_K 33.5 / 33.8, Q8_0 39.4 / 40.6, Q4_0 40.0 / 29.4; 11008 x 2048, 100 rows Q4_K 22.5 / 15.5, Q8_0
-    // 26.1 / 18.4.  Q4_K beside eight spills nine registers, which it makes up for where rows are short, or where the tiles, whose number is past a
-    // third of the CUs, share their K by two and not by three: 128 rows 8208 x 3072 23.9 / 22.6, 10300 x 3072 23.9 / 23.5, 8208 x 3328 24.8 / 25.4,
-    // 10880 x 3328 25.9 / 26.2, 8208 x 4096 26.5 / 28.0, 10752 x 4096 28.6 / 29.1, 10880 x 4096 28.1 / 29.1; 10896 x 4096 31.1 / 29.1, 11008 x 4096
-    // 31.6 / 29.2, 12288 x 4096 31.8 / 29.7.
+    // 48 weight rows beside more than 96 activation rows: seven fragments of these fit the registers, but for Q6_K, and eight for
+    // Q4_0.  us of a call, tiles / here: 11008 x 4096, 100 rows Q4_K 30.3 / 24.6, Q5_K 32.3 / 27.9, Q8_0 38.0 / 31.1, Q4_0 38.3 /
+    // 26.4, Q6_K 35.8 / 34.8 (8208 x 4096 30.2 / 33.6); 128 rows Q5_K 33.5 / 33.8, Q8_0 39.4 / 40.6, Q4_0 40.0 / 29.4; 11008 x 2048,
+    // 100 rows Q4_K 22.5 / 15.5, Q8_0 26.1 / 18.4.  Q4_K beside eight spills nine registers, which it makes up for where rows are
+    // short, or where the tiles, whose number is past a third of the CUs, share their K by two and not by three: 128 rows 8208 x 3072
+    // 23.9 / 22.6, 10300 x 3072 23.9 / 23.5, 8208 x 3328 24.8 / 25.4, 10880 x 3328 25.9 / 26.2, 8208 x 4096 26.5 / 28.0, 10752 x 4096
+    // 28.6 / 29.1, 10880 x 4096 28.1 / 29.1; 10896 x 4096 31.1 / 29.1, 11008 x 4096 31.6 / 29.2, 12288 x 4096 31.8 / 29.7.
     if (rf == 3 && m > 96 && q6k) return 0;
     if (rf == 3 && m > 112 && fmt != CANDY_HIP_Q4_0 && (fmt != CANDY_HIP_Q4_K || (cols > 3072 && 3 * tiles <= num_cus))) return 0;
     if (mf * 32 * cols > 1200000) return 0;  // not measured

@@ -576,13 +576,14 @@ static bool planar_behind(const candy_hip_qtensor *w, int64_t m) {
 }
 
 // Weights of 2 million values and more that are too few rows for the fp16 kernels, which launch a workgroup for 128 weight rows
-// (mmq_f16_rows.hip: 16 to 48, from 2048 on) and sum copies of a split of K: this kernel deals K to its wavefronts, strips of 16.  us of a
-// call there / here: Q4_K 1024 x 4096, 48 / 96 / 255 rows 14.1 / 7.9, 15.7 / 9.2, 20.8 / 13.0; 2048 x 8192, 48 / 128 rows 19.4 / 11.9, 22.1 / 17.4; 4096
-// x 11008, 64 rows 26.8 / 21.5; 3000 x 2560, 160 / 255 rows 18.8 / 14.5, 22.6 / 19.0; Q6_K 1024 x 4096, 48 / 255 rows 15.8 / 8.0, 24.0 / 15.5, 2048 x 8192, 64
-// rows 21.7 / 16.2; Q8_0 2048 x 4096, 128 rows 22.7 / 13.3.  The vector ALU's work per product is what ends it, `work` below, for Q6_K at two
-// thirds (Q4_K 2.1 and 2.7 billion: 2048 x 8192, 128 / 160 rows 22.1 / 17.4, 25.5 / 26.2; 2.0 and 2.4: 1536 x 8192, 160 / 192 rows 23.2 / 17.5, 23.9 /
-// 26.0; Q6_K 1.5 and 1.8: 2048 x 5632, 128 / 160 rows 23.5 / 19.1, 23.8 / 27.7).  Below 33 rows and with a lower threshold a caller has asked for the fp16 kernels, with a
-// shape or a split for theirs.
+// (mmq_f16_rows.hip: 16 to 48, from 2048 on) and sum copies of a split of K: this kernel deals K to its wavefronts, strips of 16.  us
+// of a call there / here: Q4_K 1024 x 4096, 48 / 96 / 255 rows 14.1 / 7.9, 15.7 / 9.2, 20.8 / 13.0; 2048 x 8192, 48 / 128 rows 19.4 /
+// 11.9, 22.1 / 17.4; 4096 x 11008, 64 rows 26.8 / 21.5; 3000 x 2560, 160 / 255 rows 18.8 / 14.5, 22.6 / 19.0; Q6_K 1024 x 4096, 48 /
+// 255 rows 15.8 / 8.0, 24.0 / 15.5, 2048 x 8192, 64 rows 21.7 / 16.2; Q8_0 2048 x 4096, 128 rows 22.7 / 13.3.  The vector ALU's work
+// per product is what ends it, `work` below, for Q6_K at two thirds (Q4_K 2.1 and 2.7 billion: 2048 x 8192, 128 / 160 rows 22.1 /
+// 17.4, 25.5 / 26.2; 2.0 and 2.4: 1536 x 8192, 160 / 192 rows 23.2 / 17.5, 23.9 / 26.0; Q6_K 1.5 and 1.8: 2048 x 5632, 128 / 160 rows
+// 23.5 / 19.1, 23.8 / 27.7).  Below 33 rows and with a lower threshold a caller has asked for the fp16 kernels, with a shape or a
+// split for theirs.
 static bool ahead_of_fp16(const candy_hip_qtensor *w, int64_t m) {
     const Options &o = w->dev->opt;
     const int64_t rows = w->rows, cus = w->dev->num_cus, values = rows * w->cols, work = values * m;
@@ -606,16 +607,17 @@ static bool ahead_of_fp16(const candy_hip_qtensor *w, int64_t m) {
 //     super-blocks, two for each of its wavefronts, where a strip a CU is all there is: 2048 x 8192, 3 / 8 / 16 rows 7.7 / 8.3, 7.8 / 8.8,
 //     7.8 / 8.2 (but 28 super-blocks level, 33 10.2 / 8.0, 5120 x 8192, 16 rows 11.2 / 10.2).  Planar quants do not go there.
 //   three and four rows, the vector kernels: small weights (1024 x 4096, Q5_K 7.2 / 7.2, Q8_0 7.3 / 7.6), and Q8_0 and Q4_0 in two rounds
-//     of workgroups whose few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0, 8208 x 5120 0.89 of the vector kernels'
-//     speed, 8208 x 8192 1.01; 4096 x 4096 8.4 / 7.7), where four strips a workgroup leave slots idle (16400 x 4096 0.73 and 0.75, 24576 x
-//     8192 0.88 and 0.82, 32000 x 4096 1.01 and 1.05), and Q4_0, three rows of 2304 to 5120 values, in less than one round (5000 x 4096 0.88)
+//     of workgroups whose few super-blocks are soon done (14336 x 4096 15.5 / 18.7 and 12.7 / 15.0, 8208 x 5120 0.89 of the vector
+//     kernels' speed, 8208 x 8192 1.01; 4096 x 4096 8.4 / 7.7), where four strips a workgroup leave slots idle (16400 x 4096 0.73 and
+//     0.75, 24576 x 8192 0.88 and 0.82, 32000 x 4096 1.01 and 1.05), and Q4_0, three rows of 2304 to 5120 values, in less than one round
+//     (5000 x 4096 0.88)
 //   the fp16 kernels, whose scales are in the operands, where a call may take them (mmq.f16_api_min_m): Q4_K and Q6_K from 33 rows
-//     (11008 x 4096, 48 rows 16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 / 35.8);
-//     not small weights, where this one is ahead (ahead_of_fp16)
+//     (11008 x 4096, 48 rows 16.0 / 20.9 and 26.0 / 26.4), the others from 65 (Q8_0 11008 x 4096, 64 rows 44.5 / 24.4, 80 rows 24.7 /
+//     35.8); not small weights, where this one is ahead (ahead_of_fp16)
 // Weights under a million values are launches and nothing else whatever the kernel.
-// Not left to a faster kernel: Q8_0 and Q4_0 whose results come to four million and more (planar quants and prompts of up to 255 rows, single
-// calls of up to 64 against 44000 weight rows), which the fp16 tiles of mmq.hip took before (32000 x 4096, 200 rows 119 us there, 176 here; 100
-// rows 109 and 105).  Below the fp16 thresholds every product is exact, and this is the fastest kernel that is.
+// Not left to a faster kernel: Q8_0 and Q4_0 whose results come to four million and more (planar quants and prompts of up to 255 rows,
+// single calls of up to 64 against 44000 weight rows), which the fp16 tiles of mmq.hip took before (32000 x 4096, 200 rows 119 us
+// there, 176 here; 100 rows 109 and 105).  Below the fp16 thresholds every product is exact, and this is the fastest kernel that is.
 bool rows_i8_picks(const candy_hip_qtensor *w, int64_t m, bool exact) {
     const Options &o = w->dev->opt;
     const int64_t values = w->rows * w->cols, cus = w->dev->num_cus, strips = (w->rows + 15) / 16, nsb = w->cols >> 8;
